@@ -142,34 +142,6 @@ void launch_field_sum(hipStream_t s, int n, int pitch, const float* a, double* p
 void launch_field_fill(hipStream_t s, int n, int pitch, float value, float* a);
 void launch_set_weights(hipStream_t s, int n, int pitch, double emin, const float* x, float* w, float* xc);
 void launch_copy_pitched(hipStream_t s, int n, int pitch_in, int pitch_out, const float* in, float* out);
-
-}  // namespace homo3d
-
-namespace homo3d {
-constexpr int kMmaMaxM = 4;
-constexpr int kMmaNewtonSums = kMmaMaxM + kMmaMaxM * (kMmaMaxM + 1) / 2;
-void launch_mma_setup(hipStream_t s, int m, long n, int iter, double move, const double* x, const double* xmin,
-                      const double* xmax, const double* xold1, const double* xold2, const double* df0,
-                      const double* dfdx, double* low, double* upp, double* alfa, double* beta, double* p0, double* q0,
-                      double* P, double* Q, double* part, int nb, double* out);
-void launch_mma_resid(hipStream_t s, int m, long n, const double* lam, double epsi, const double* x,
-                      const double* xsi, const double* eta, const double* low, const double* upp, const double* alfa,
-                      const double* beta, const double* p0, const double* q0, const double* P, const double* Q,
-                      double* part, double* partmax, int nb, double* out);
-void launch_mma_newton(hipStream_t s, int m, long n, const double* lam, double epsi, const double* x,
-                       const double* xsi, const double* eta, const double* low, const double* upp, const double* alfa,
-                       const double* beta, const double* p0, const double* q0, const double* P, const double* Q,
-                       double* delx, double* diagx, double* part, int nb, double* out);
-void launch_mma_dir(hipStream_t s, int m, long n, double epsi, const double* dlam, const double* x, const double* xsi,
-                    const double* eta, const double* low, const double* upp, const double* alfa, const double* beta,
-                    const double* P, const double* Q, const double* delx, const double* diagx, double* dx,
-                    double* dxsi, double* deta, double* partmax, int nb, double* out);
-void launch_mma_step(hipStream_t s, long n, double steg, const double* xo, const double* xsio, const double* etao,
-                     const double* dx, const double* dxsi, const double* deta, double* x, double* xsi, double* eta);
-void launch_mma_init(hipStream_t s, long n, const double* alfa, const double* beta, double* x, double* xsi,
-                     double* eta);
-void launch_f32_to_f64(hipStream_t s, long n, const float* a, double* b);
-void launch_f64_to_f32(hipStream_t s, long n, const double* a, float* b);
 // Density filter with Spline4/linear radial weights (wk: normalised (2h+1)^3 box) and its adjoint (wsum: the
 // forward pass's in-grid weight sums); sgm projection and its backward.  Pitched lexicographic arrays.
 void launch_conv_filter(hipStream_t s, int n, int pitch, int h, int periodic, const float* wk, const float* in,

@@ -3760,311 +3760,6 @@ void launch_copy_pitched(hipStream_t s, int n, int pitch_in, int pitch_out, cons
 }  // namespace homo3d
 
 // =============================================================================================
-// MMA (Svanberg's method of moving asymptotes; mmasub_ker + subsolv_g, mmaOpt.cu:429-1019)
-// FP64 per-variable kernels; m <= kMmaMaxM constraints; dfdx is m x n row-major.
-// =============================================================================================
-namespace homo3d {
-namespace {
-
-struct MmaDual {          // small dual vectors of subsolv, read by every thread
-    double lam[kMmaMaxM];
-    double epsi;
-};
-
-template <int BS>
-__device__ __forceinline__ double block_max(double v, double* sh) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_down(v, off, 64));
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    if (lane == 0) sh[wid] = v;
-    __syncthreads();
-    double s = -1e300;
-    if (threadIdx.x == 0)
-        for (int i = 0; i < BS / 64; i++) s = fmax(s, sh[i]);
-    __syncthreads();
-    return s;
-}
-
-// asymptotes, move limits and the convex approximation terms (mmasub_ker, mmaOpt.cu:864-989);
-// part[i*nb + b] = block sums of P_ij/(upp-x) + Q_ij/(x-low)
-__global__ __launch_bounds__(256) void k_mma_setup(int m, long n, int iter, double move, const double* __restrict__ x,
-                                                   const double* __restrict__ xmin, const double* __restrict__ xmax,
-                                                   const double* __restrict__ xold1, const double* __restrict__ xold2,
-                                                   const double* __restrict__ df0, const double* __restrict__ dfdx,
-                                                   double* __restrict__ low, double* __restrict__ upp,
-                                                   double* __restrict__ alfa, double* __restrict__ beta,
-                                                   double* __restrict__ p0, double* __restrict__ q0,
-                                                   double* __restrict__ P, double* __restrict__ Q,
-                                                   double* __restrict__ part) {
-    __shared__ double sh[4];
-    const double raa0 = 1e-5, albefa = 0.1, asyinit = 0.5, asyincr = 1.2, asydecr = 0.7;
-    double bs[kMmaMaxM] = {0, 0, 0, 0};
-    for (long j = (long)blockIdx.x * blockDim.x + threadIdx.x; j < n; j += (long)gridDim.x * blockDim.x) {
-        const double xj = x[j], dx = xmax[j] - xmin[j];
-        double lo, up;
-        if (iter <= 2) {
-            lo = xj - asyinit * dx;
-            up = xj + asyinit * dx;
-        } else {
-            const double zzz = (xj - xold1[j]) * (xold1[j] - xold2[j]);
-            const double fac = zzz > 0 ? asyincr : (zzz < 0 ? asydecr : 1.0);
-            lo = xj - fac * (xold1[j] - low[j]);
-            up = xj + fac * (upp[j] - xold1[j]);
-            lo = fmax(lo, xj - 10 * dx);
-            lo = fmin(lo, xj - 0.01 * dx);
-            up = fmin(up, xj + 10 * dx);
-            up = fmax(up, xj + 0.01 * dx);
-        }
-        low[j] = lo;
-        upp[j] = up;
-        alfa[j] = fmax(fmax(lo + albefa * (xj - lo), xj - move * dx), xmin[j]);
-        beta[j] = fmin(fmin(up - albefa * (up - xj), xj + move * dx), xmax[j]);
-        const double xmamiinv = 1.0 / fmax(dx, 1e-5);
-        const double ux1 = up - xj, xl1 = xj - lo, ux2 = ux1 * ux1, xl2 = xl1 * xl1;
-        const double dp = fmax(df0[j], 0.0), dm = fmax(-df0[j], 0.0);
-        const double pq0 = 1e-3 * (dp + dm) + raa0 * xmamiinv;
-        p0[j] = (dp + pq0) * ux2;
-        q0[j] = (dm + pq0) * xl2;
-        for (int i = 0; i < m; i++) {
-            const double g = dfdx[(size_t)i * n + j];
-            const double pp = fmax(g, 0.0), qq = fmax(-g, 0.0), pq = 1e-3 * (pp + qq) + raa0 * xmamiinv;
-            const double Pv = (pp + pq) * ux2, Qv = (qq + pq) * xl2;
-            P[(size_t)i * n + j] = Pv;
-            Q[(size_t)i * n + j] = Qv;
-            bs[i] += Pv / ux1 + Qv / xl1;
-        }
-    }
-    for (int i = 0; i < m; i++) {
-        const double s = block_sum<256>(bs[i], sh);
-        if (threadIdx.x == 0) part[i * gridDim.x + blockIdx.x] = s;
-    }
-}
-
-// per-variable primal residual terms of subsolv at (x, xsi, eta; lam, epsi):
-// part layout per block b: [0] sum sq, [1] max abs (in part2), [2..2+m) gvec partials
-__global__ __launch_bounds__(256) void k_mma_resid(int m, long n, const MmaDual dual, const double* __restrict__ x,
-                                                   const double* __restrict__ xsi, const double* __restrict__ eta,
-                                                   const double* __restrict__ low, const double* __restrict__ upp,
-                                                   const double* __restrict__ alfa, const double* __restrict__ beta,
-                                                   const double* __restrict__ p0, const double* __restrict__ q0,
-                                                   const double* __restrict__ P, const double* __restrict__ Q,
-                                                   double* __restrict__ part, double* __restrict__ partmax) {
-    __shared__ double sh[4];
-    double ssq = 0, smax = 0;
-    double gv[kMmaMaxM] = {0, 0, 0, 0};
-    const double epsi = dual.epsi;
-    for (long j = (long)blockIdx.x * blockDim.x + threadIdx.x; j < n; j += (long)gridDim.x * blockDim.x) {
-        const double xj = x[j], ux1 = upp[j] - xj, xl1 = xj - low[j];
-        double pl = p0[j], ql = q0[j];
-        for (int i = 0; i < m; i++) {
-            const double Pv = P[(size_t)i * n + j], Qv = Q[(size_t)i * n + j];
-            pl += Pv * dual.lam[i];
-            ql += Qv * dual.lam[i];
-            gv[i] += Pv / ux1 + Qv / xl1;
-        }
-        const double dpsidx = pl / (ux1 * ux1) - ql / (xl1 * xl1);
-        const double rex = dpsidx - xsi[j] + eta[j];
-        const double rexsi = xsi[j] * (xj - alfa[j]) - epsi;
-        const double reeta = eta[j] * (beta[j] - xj) - epsi;
-        ssq += rex * rex + rexsi * rexsi + reeta * reeta;
-        smax = fmax(smax, fmax(fabs(rex), fmax(fabs(rexsi), fabs(reeta))));
-    }
-    double t = block_sum<256>(ssq, sh);
-    if (threadIdx.x == 0) part[blockIdx.x] = t;
-    for (int i = 0; i < m; i++) {
-        t = block_sum<256>(gv[i], sh);
-        if (threadIdx.x == 0) part[(1 + i) * gridDim.x + blockIdx.x] = t;
-    }
-    t = block_max<256>(smax, sh);
-    if (threadIdx.x == 0) partmax[blockIdx.x] = t;
-}
-
-// Newton system terms: delx, diagx per variable; block sums of GG_i*delx/diagx and
-// GG_i*GG_k/diagx (k >= i) for the (m+1) x (m+1) system (subsolv_g, mmaOpt.cu:560-640)
-__global__ __launch_bounds__(256) void k_mma_newton(int m, long n, const MmaDual dual, const double* __restrict__ x,
-                                                    const double* __restrict__ xsi, const double* __restrict__ eta,
-                                                    const double* __restrict__ low, const double* __restrict__ upp,
-                                                    const double* __restrict__ alfa, const double* __restrict__ beta,
-                                                    const double* __restrict__ p0, const double* __restrict__ q0,
-                                                    const double* __restrict__ P, const double* __restrict__ Q,
-                                                    double* __restrict__ delx, double* __restrict__ diagx,
-                                                    double* __restrict__ part) {
-    __shared__ double sh[4];
-    constexpr int NS = kMmaMaxM + kMmaMaxM * (kMmaMaxM + 1) / 2;
-    double acc[NS];
-#pragma unroll
-    for (int k = 0; k < NS; k++) acc[k] = 0;
-    const double epsi = dual.epsi;
-    for (long j = (long)blockIdx.x * blockDim.x + threadIdx.x; j < n; j += (long)gridDim.x * blockDim.x) {
-        const double xj = x[j], ux1 = upp[j] - xj, xl1 = xj - low[j];
-        const double ux2 = ux1 * ux1, xl2 = xl1 * xl1, ux3 = ux1 * ux2, xl3 = xl1 * xl2;
-        double pl = p0[j], ql = q0[j], gg[kMmaMaxM];
-        for (int i = 0; i < m; i++) {
-            const double Pv = P[(size_t)i * n + j], Qv = Q[(size_t)i * n + j];
-            pl += Pv * dual.lam[i];
-            ql += Qv * dual.lam[i];
-            gg[i] = Pv / ux2 - Qv / xl2;
-        }
-        const double dpsidx = pl / ux2 - ql / xl2;
-        const double dl = dpsidx - epsi / (xj - alfa[j]) + epsi / (beta[j] - xj);
-        const double dg = 2 * (pl / ux3 + ql / xl3) + xsi[j] / (xj - alfa[j]) + eta[j] / (beta[j] - xj);
-        delx[j] = dl;
-        diagx[j] = dg;
-        int k = kMmaMaxM;
-        for (int i = 0; i < m; i++) {
-            acc[i] += gg[i] * dl / dg;
-            for (int q = i; q < m; q++) acc[k + i * kMmaMaxM - i * (i - 1) / 2 + (q - i)] += gg[i] * gg[q] / dg;
-        }
-    }
-    for (int k = 0; k < NS; k++) {
-        const double t = block_sum<256>(acc[k], sh);
-        if (threadIdx.x == 0) part[k * gridDim.x + blockIdx.x] = t;
-    }
-}
-
-// Newton direction per variable and block maxima of the step-length ratios
-// (stepxx/stepalfa/stepbeta of subsolv_g, mmaOpt.cu:680-700)
-__global__ __launch_bounds__(256) void k_mma_dir(int m, long n, const MmaDual dual, const double* __restrict__ dlam,
-                                                 const double* __restrict__ x, const double* __restrict__ xsi,
-                                                 const double* __restrict__ eta, const double* __restrict__ low,
-                                                 const double* __restrict__ upp, const double* __restrict__ alfa,
-                                                 const double* __restrict__ beta, const double* __restrict__ P,
-                                                 const double* __restrict__ Q, const double* __restrict__ delx,
-                                                 const double* __restrict__ diagx, double* __restrict__ dx,
-                                                 double* __restrict__ dxsi, double* __restrict__ deta,
-                                                 double* __restrict__ partmax) {
-    __shared__ double sh[4];
-    double stm = -1e300;
-    const double epsi = dual.epsi;
-    for (long j = (long)blockIdx.x * blockDim.x + threadIdx.x; j < n; j += (long)gridDim.x * blockDim.x) {
-        const double xj = x[j], ux2 = (upp[j] - xj) * (upp[j] - xj), xl2 = (xj - low[j]) * (xj - low[j]);
-        double gt = 0;
-        for (int i = 0; i < m; i++) gt += (P[(size_t)i * n + j] / ux2 - Q[(size_t)i * n + j] / xl2) * dlam[i];
-        const double d = -delx[j] / diagx[j] - gt / diagx[j];
-        const double xa = xj - alfa[j], bx = beta[j] - xj;
-        const double ds = -xsi[j] + epsi / xa - (xsi[j] * d) / xa;
-        const double de = -eta[j] + epsi / bx + (eta[j] * d) / bx;
-        dx[j] = d;
-        dxsi[j] = ds;
-        deta[j] = de;
-        stm = fmax(stm, fmax(fmax(-1.01 * ds / xsi[j], -1.01 * de / eta[j]), fmax(-1.01 * d / xa, 1.01 * d / bx)));
-    }
-    const double t = block_max<256>(stm, sh);
-    if (threadIdx.x == 0) partmax[blockIdx.x] = t;
-}
-
-// x = xold + steg dx (and xsi, eta)
-__global__ __launch_bounds__(256) void k_mma_step(long n, double steg, const double* __restrict__ xo,
-                                                  const double* __restrict__ xsio, const double* __restrict__ etao,
-                                                  const double* __restrict__ dx, const double* __restrict__ dxsi,
-                                                  const double* __restrict__ deta, double* __restrict__ x,
-                                                  double* __restrict__ xsi, double* __restrict__ eta) {
-    const long j = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= n) return;
-    x[j] = xo[j] + steg * dx[j];
-    xsi[j] = xsio[j] + steg * dxsi[j];
-    eta[j] = etao[j] + steg * deta[j];
-}
-
-__global__ __launch_bounds__(256) void k_mma_init(long n, const double* __restrict__ alfa, const double* __restrict__ beta,
-                                                  double* __restrict__ x, double* __restrict__ xsi,
-                                                  double* __restrict__ eta) {
-    const long j = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= n) return;
-    const double xv = 0.5 * (alfa[j] + beta[j]);
-    x[j] = xv;
-    xsi[j] = fmax(1.0 / (xv - alfa[j]), 1.0);
-    eta[j] = fmax(1.0 / (beta[j] - xv), 1.0);
-}
-
-// pitched FP32 design array <-> dense FP64 vector
-__global__ __launch_bounds__(256) void k_f32_to_f64(long n, const float* __restrict__ a, double* __restrict__ b) {
-    const long j = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (j < n) b[j] = (double)a[j];
-}
-__global__ __launch_bounds__(256) void k_f64_to_f32(long n, const double* __restrict__ a, float* __restrict__ b) {
-    const long j = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (j < n) b[j] = (float)a[j];
-}
-
-__global__ void k_max_partials(int nb, const double* __restrict__ partial, double* __restrict__ out) {
-    __shared__ double sh[4];
-    double s = -1e300;
-    for (int i = threadIdx.x; i < nb; i += blockDim.x) s = fmax(s, partial[i]);
-    s = block_max<256>(s, sh);
-    if (threadIdx.x == 0) out[0] = s;
-}
-
-}  // namespace
-
-void launch_mma_setup(hipStream_t s, int m, long n, int iter, double move, const double* x, const double* xmin,
-                      const double* xmax, const double* xold1, const double* xold2, const double* df0,
-                      const double* dfdx, double* low, double* upp, double* alfa, double* beta, double* p0, double* q0,
-                      double* P, double* Q, double* part, int nb, double* out) {
-    hipLaunchKernelGGL(k_mma_setup, dim3(nb), dim3(256), 0, s, m, n, iter, move, x, xmin, xmax, xold1, xold2, df0, dfdx,
-                       low, upp, alfa, beta, p0, q0, P, Q, part);
-    hipLaunchKernelGGL(k_sum_partials, dim3(m), dim3(kSumThreads), 0, s, nb, part, out);
-}
-
-void launch_mma_resid(hipStream_t s, int m, long n, const double* lam, double epsi, const double* x,
-                      const double* xsi, const double* eta, const double* low, const double* upp, const double* alfa,
-                      const double* beta, const double* p0, const double* q0, const double* P, const double* Q,
-                      double* part, double* partmax, int nb, double* out) {
-    MmaDual d{};
-    for (int i = 0; i < m; i++) d.lam[i] = lam[i];
-    d.epsi = epsi;
-    hipLaunchKernelGGL(k_mma_resid, dim3(nb), dim3(256), 0, s, m, n, d, x, xsi, eta, low, upp, alfa, beta, p0, q0, P,
-                       Q, part, partmax);
-    hipLaunchKernelGGL(k_sum_partials, dim3(1 + m), dim3(kSumThreads), 0, s, nb, part, out);
-    hipLaunchKernelGGL(k_max_partials, dim3(1), dim3(256), 0, s, nb, partmax, out + 1 + m);
-}
-
-void launch_mma_newton(hipStream_t s, int m, long n, const double* lam, double epsi, const double* x,
-                       const double* xsi, const double* eta, const double* low, const double* upp, const double* alfa,
-                       const double* beta, const double* p0, const double* q0, const double* P, const double* Q,
-                       double* delx, double* diagx, double* part, int nb, double* out) {
-    MmaDual d{};
-    for (int i = 0; i < m; i++) d.lam[i] = lam[i];
-    d.epsi = epsi;
-    const int NS = kMmaMaxM + kMmaMaxM * (kMmaMaxM + 1) / 2;
-    hipLaunchKernelGGL(k_mma_newton, dim3(nb), dim3(256), 0, s, m, n, d, x, xsi, eta, low, upp, alfa, beta, p0, q0, P,
-                       Q, delx, diagx, part);
-    hipLaunchKernelGGL(k_sum_partials, dim3(NS), dim3(kSumThreads), 0, s, nb, part, out);
-}
-
-void launch_mma_dir(hipStream_t s, int m, long n, double epsi, const double* dlam, const double* x, const double* xsi,
-                    const double* eta, const double* low, const double* upp, const double* alfa, const double* beta,
-                    const double* P, const double* Q, const double* delx, const double* diagx, double* dx,
-                    double* dxsi, double* deta, double* partmax, int nb, double* out) {
-    MmaDual d{};
-    d.epsi = epsi;
-    hipLaunchKernelGGL(k_mma_dir, dim3(nb), dim3(256), 0, s, m, n, d, dlam, x, xsi, eta, low, upp, alfa, beta, P, Q,
-                       delx, diagx, dx, dxsi, deta, partmax);
-    hipLaunchKernelGGL(k_max_partials, dim3(1), dim3(256), 0, s, nb, partmax, out);
-}
-
-void launch_mma_step(hipStream_t s, long n, double steg, const double* xo, const double* xsio, const double* etao,
-                     const double* dx, const double* dxsi, const double* deta, double* x, double* xsi, double* eta) {
-    hipLaunchKernelGGL(k_mma_step, dim3(nblk(n)), dim3(256), 0, s, n, steg, xo, xsio, etao, dx, dxsi, deta, x, xsi,
-                       eta);
-}
-
-void launch_mma_init(hipStream_t s, long n, const double* alfa, const double* beta, double* x, double* xsi,
-                     double* eta) {
-    hipLaunchKernelGGL(k_mma_init, dim3(nblk(n)), dim3(256), 0, s, n, alfa, beta, x, xsi, eta);
-}
-
-void launch_f32_to_f64(hipStream_t s, long n, const float* a, double* b) {
-    hipLaunchKernelGGL(k_f32_to_f64, dim3(nblk(n)), dim3(256), 0, s, n, a, b);
-}
-
-void launch_f64_to_f32(hipStream_t s, long n, const double* a, float* b) {
-    hipLaunchKernelGGL(k_f64_to_f32, dim3(nblk(n)), dim3(256), 0, s, n, a, b);
-}
-
-}  // namespace homo3d
-
-// =============================================================================================
 // OC update without allocation: homo3d_oc_update_noalloc
 // =============================================================================================
 // The bisection's reduction scratch (|s| maxima of kOcBlocks workgroups, kOcBlocks FP64 partial volume
