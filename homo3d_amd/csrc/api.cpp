@@ -10,6 +10,7 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <initializer_list>
 #include <limits>
 #include <map>
 #include <string>
@@ -17,6 +18,7 @@
 #include <vector>
 
 #include "../../include/homo3d.h"
+#include "fields.h"
 #include "kernels.h"
 #include "net.h"
 
@@ -555,6 +557,22 @@ int stage_out(homo3d_handle* h, float* dst, const float* src, int pitch, int on_
                                    (size_t)n * n, kind, h->stream));
     return HOMO3D_OK;
 }
+
+// Whether the kernels can work on the caller's arrays themselves: device memory of this handle's GPU.
+// (Managed memory, another GPU's and host memory go through the staging buffer.)
+bool device_here(const homo3d_handle* h, std::initializer_list<const void*> ps) {
+    for (const void* p : ps) {
+        hipPointerAttribute_t attr;
+        if (hipPointerGetAttributes(&attr, p) != hipSuccess) {
+            (void)hipGetLastError();
+            return false;
+        }
+        if (attr.type != hipMemoryTypeDevice || attr.device != h->cfg.device) return false;
+    }
+    return true;
+}
+
+bool disjoint(const float* a, const float* b, size_t elems) { return a + elems <= b || b + elems <= a; }
 
 constexpr int kMaxOuter = 12;
 // Inner solve target per refinement round (measured at 256^3: 1e-4 and 1e-6 cost more CG steps than
@@ -1510,20 +1528,29 @@ int homo3d_oc_filter(homo3d_handle* h, float* sens, const float* rho, int pitch,
         W += wd[i];
     }
     for (size_t i = 0; i < wk.size(); i++) wk[i] = (float)(wd[i] / W);
-    HIPCHK(h, hipMemcpyAsync(h->d_ftmp, wk.data(), sizeof(float) * wk.size(), hipMemcpyHostToDevice, h->stream));
     const size_t elems = (size_t)pitch * n * n;
+    // the caller's arrays are read in place; the result takes sens's place in a copy
+    const bool here = on_device && device_here(h, {sens, rho});
     int rc = ensure_stage(h, 3 * elems);
     if (rc) return rc;
-    float* ds = h->d_stage;
-    float* dr = h->d_stage + elems;
+    const float *ds = h->d_stage, *dr = h->d_stage + elems;
     float* dout = h->d_stage + 2 * elems;
-    const hipMemcpyKind kin = on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
-    HIPCHK(h, hipMemcpyAsync(ds, sens, sizeof(float) * elems, kin, h->stream));
-    HIPCHK(h, hipMemcpyAsync(dr, rho, sizeof(float) * elems, kin, h->stream));
-    launch_oc_filter(h->stream, n, pitch, hw, periodic, h->d_ftmp, ds, dr, dout);
-    launch_copy_pitched(h->stream, n, pitch, pitch, dout, ds);
-    HIPCHK(h, hipMemcpyAsync(sens, ds, sizeof(float) * elems, on_device ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost,
-                             h->stream));
+    if (here) {
+        ds = sens;
+        dr = rho;
+    } else {
+        const hipMemcpyKind kin = on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
+        HIPCHK(h, hipMemcpyAsync(h->d_stage, sens, sizeof(float) * elems, kin, h->stream));
+        HIPCHK(h, hipMemcpyAsync(h->d_stage + elems, rho, sizeof(float) * elems, kin, h->stream));
+    }
+    if (box_filter_ok(n, hw)) {
+        launch_box_sens(h->stream, n, pitch, hw, periodic, wk.data(), reinterpret_cast<double*>(h->d_ftmp), ds, dr, dout);
+    } else {
+        HIPCHK(h, hipMemcpyAsync(h->d_ftmp, wk.data(), sizeof(float) * wk.size(), hipMemcpyHostToDevice, h->stream));
+        launch_oc_filter(h->stream, n, pitch, hw, periodic, h->d_ftmp, ds, dr, dout);
+    }
+    rc = stage_out(h, sens, dout, pitch, on_device);
+    if (rc) return rc;
     HIPCHK(h, hipStreamSynchronize(h->stream));
     return HOMO3D_OK;
 }
@@ -1659,23 +1686,40 @@ int homo3d_density_filter(homo3d_handle* h, const float* in, float* out, int pit
     }
     std::vector<float> wk(wd.size());
     for (size_t i = 0; i < wk.size(); i++) wk[i] = (float)(wd[i] / W);
-    HIPCHK(h, hipMemcpyAsync(h->d_ftmp, wk.data(), sizeof(float) * wk.size(), hipMemcpyHostToDevice, h->stream));
     const size_t elems = (size_t)pitch * n * n;
-    int rc = ensure_stage(h, 3 * elems);
-    if (rc) return rc;
-    float* din = h->d_stage;
-    float* dws = h->d_stage + elems;
-    float* dres = h->d_stage + 2 * elems;
-    HIPCHK(h, hipMemcpyAsync(din, in, sizeof(float) * elems, on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice,
-                             h->stream));
-    if (!backward) {
-        launch_conv_filter(h->stream, n, pitch, hw, periodic, h->d_ftmp, din, dres, nullptr);
-    } else {
-        launch_conv_filter(h->stream, n, pitch, hw, periodic, h->d_ftmp, din, dres, dws);  // weight sums W
-        launch_conv_filter_back(h->stream, n, pitch, hw, periodic, h->d_ftmp, din, dws, dres);
+    const bool boxed = box_filter_ok(n, hw);
+    const bool here = boxed && on_device && disjoint(in, out, elems) && device_here(h, {in, out});
+    const float* din = in;
+    float* dres = out;
+    float* dws = nullptr;
+    if (!here) {
+        int rc = ensure_stage(h, 3 * elems);
+        if (rc) return rc;
+        din = h->d_stage;
+        dws = h->d_stage + elems;
+        dres = h->d_stage + 2 * elems;
+        HIPCHK(h, hipMemcpyAsync(h->d_stage, in, sizeof(float) * elems,
+                                 on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, h->stream));
     }
-    rc = stage_out(h, out, dres, pitch, on_device);
-    if (rc) return rc;
+    if (boxed) {
+        double* table = reinterpret_cast<double*>(h->d_ftmp);
+        if (!backward)
+            launch_box_conv(h->stream, n, pitch, hw, periodic, wk.data(), table, din, dres);
+        else
+            launch_box_adjoint(h->stream, n, pitch, hw, periodic, wk.data(), table, din, dres);
+    } else {
+        HIPCHK(h, hipMemcpyAsync(h->d_ftmp, wk.data(), sizeof(float) * wk.size(), hipMemcpyHostToDevice, h->stream));
+        if (!backward) {
+            launch_conv_filter(h->stream, n, pitch, hw, periodic, h->d_ftmp, din, dres, nullptr);
+        } else {
+            launch_conv_filter(h->stream, n, pitch, hw, periodic, h->d_ftmp, din, dres, dws);  // weight sums W
+            launch_conv_filter_back(h->stream, n, pitch, hw, periodic, h->d_ftmp, din, dws, dres);
+        }
+    }
+    if (!here) {
+        int rc = stage_out(h, out, dres, pitch, on_device);
+        if (rc) return rc;
+    }
     HIPCHK(h, hipStreamSynchronize(h->stream));
     return HOMO3D_OK;
 }
@@ -1689,19 +1733,28 @@ int homo3d_projection(homo3d_handle* h, const float* in, const float* y, float* 
     const int n = h->lv[0].n;
     if (pitch < n) return set_err(h, HOMO3D_BAD_ARG, "pitch %d < n %d", pitch, n);
     const size_t elems = (size_t)pitch * n * n;
-    int rc = ensure_stage(h, 3 * elems);
-    if (rc) return rc;
-    float *din = h->d_stage, *dy = h->d_stage + elems, *dres = h->d_stage + 2 * elems;
-    const hipMemcpyKind kin = on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
-    HIPCHK(h, hipMemcpyAsync(din, in, sizeof(float) * elems, kin, h->stream));
-    if (backward) {
-        HIPCHK(h, hipMemcpyAsync(dy, y, sizeof(float) * elems, kin, h->stream));
-        launch_sgm_back(h->stream, n, pitch, k, dy, din, dres);
-    } else {
-        launch_sgm(h->stream, n, pitch, k, c, din, dres);
+    auto apart = [&](const float* a) { return a == out || disjoint(a, out, elems); };
+    const bool here = on_device && apart(in) && (!backward || apart(y)) && device_here(h, {in, out, backward ? y : in});
+    const float *din = in, *dy = y;
+    float* dres = out;
+    if (!here) {
+        int rc = ensure_stage(h, 3 * elems);
+        if (rc) return rc;
+        din = h->d_stage;
+        dy = h->d_stage + elems;
+        dres = h->d_stage + 2 * elems;
+        const hipMemcpyKind kin = on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
+        HIPCHK(h, hipMemcpyAsync(h->d_stage, in, sizeof(float) * elems, kin, h->stream));
+        if (backward) HIPCHK(h, hipMemcpyAsync(h->d_stage + elems, y, sizeof(float) * elems, kin, h->stream));
     }
-    rc = stage_out(h, out, dres, pitch, on_device);
-    if (rc) return rc;
+    if (backward)
+        launch_sgm_back(h->stream, n, pitch, k, dy, din, dres);
+    else
+        launch_sgm(h->stream, n, pitch, k, c, din, dres);
+    if (!here) {
+        int rc = stage_out(h, out, dres, pitch, on_device);
+        if (rc) return rc;
+    }
     HIPCHK(h, hipStreamSynchronize(h->stream));
     return HOMO3D_OK;
 }

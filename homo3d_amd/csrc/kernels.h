@@ -130,27 +130,14 @@ void launch_sensitivity(hipStream_t s, int n, int pitch, const float* ke, const 
                         float* sens);
 void launch_symmetrize(hipStream_t s, int n, int pitch, int ng, const int* gperm, const int* gflip, const float* in,
                        float* out);
-void launch_oc_filter(hipStream_t s, int n, int pitch, int h, int periodic, const float* wk, const float* sens,
-                      const float* rho, float* out);
 void launch_oc_trial(hipStream_t s, int n, int pitch, double g, double min_rho, double step, double damp,
                      const float* sens, const float* rho, float* out, double* partial, int nblocks, double* sum);
 void launch_absmax(hipStream_t s, int n, int pitch, const float* a, float* partial, int nblocks);
-// x = rho^p; drho = p rho^(p - 1) dx (drho may alias dx); FP64 block sums of a (nblocks partials); a = value
-void launch_density_pow(hipStream_t s, int n, int pitch, float p, const float* rho, float* x);
-void launch_density_pow_grad(hipStream_t s, int n, int pitch, float p, const float* rho, const float* dx, float* drho);
+// FP64 block sums of a (nblocks partials); a = value
 void launch_field_sum(hipStream_t s, int n, int pitch, const float* a, double* partial, int nblocks);
 void launch_field_fill(hipStream_t s, int n, int pitch, float value, float* a);
 void launch_set_weights(hipStream_t s, int n, int pitch, double emin, const float* x, float* w, float* xc);
 void launch_copy_pitched(hipStream_t s, int n, int pitch_in, int pitch_out, const float* in, float* out);
-// Density filter with Spline4/linear radial weights (wk: normalised (2h+1)^3 box) and its adjoint (wsum: the
-// forward pass's in-grid weight sums); sgm projection and its backward.  Pitched lexicographic arrays.
-void launch_conv_filter(hipStream_t s, int n, int pitch, int h, int periodic, const float* wk, const float* in,
-                        float* out, float* wsum);
-void launch_conv_filter_back(hipStream_t s, int n, int pitch, int h, int periodic, const float* wk, const float* dout,
-                             const float* wsum, float* din);
-void launch_sgm(hipStream_t s, int n, int pitch, double k, double c, const float* x, float* y);
-void launch_sgm_back(hipStream_t s, int n, int pitch, double k, const float* y, const float* gy, float* gx);
-
 // Bridges to the learned warm-start network (g | n; network tensors bf16 channels-last, see net.hip):
 // input channel 0 = mean of x^(1/3) over each coarse cell; target = scale (u - mean) / n sampled at the
 // coarse vertices, the mean weighted by the input's rho^3 (mean18: 18 doubles of device scratch); warm start = periodic trilinear upsampling of

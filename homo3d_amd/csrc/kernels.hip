@@ -2681,106 +2681,6 @@ __global__ __launch_bounds__(256) void k_symmetrize(int n, int pitch, int ng, co
     out[p[0] + ((size_t)p[1] + (size_t)p[2] * n) * pitch] = (float)(s / (double)ng);
 }
 
-// Sigmund filter (filterSens_kernel, OCOptimizer.cu:76-153): wk holds the normalised weights of the
-// (2h+1)^3 box.
-__global__ __launch_bounds__(256) void k_oc_filter(int n, int pitch, int h, int periodic, const float* __restrict__ wk,
-                                                   const float* __restrict__ sens, const float* __restrict__ rho,
-                                                   float* __restrict__ out) {
-    const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long N = (long)n * n * n;
-    if (e >= N) return;
-    const int p[3] = {(int)(e % n), (int)((e / n) % n), (int)(e / ((long)n * n))};
-    const int side = 2 * h + 1;
-    double sum = 0.0, ws = 0.0;
-    for (int i = 0; i < side * side * side; i++) {
-        int q[3] = {p[0] + i % side - h, p[1] + (i / side) % side - h, p[2] + i / (side * side) - h};
-        bool inb = true;
-        for (int k = 0; k < 3; k++) {
-            if (periodic) q[k] = ((q[k] % n) + n) % n;
-            if (q[k] < 0 || q[k] >= n) inb = false;
-        }
-        if (!inb) continue;
-        const size_t id = q[0] + ((size_t)q[1] + (size_t)q[2] * n) * pitch;
-        sum += (double)sens[id] * (double)rho[id] * (double)wk[i];
-        ws += (double)wk[i];
-    }
-    const size_t me = p[0] + ((size_t)p[1] + (size_t)p[2] * n) * pitch;
-    out[me] = (float)(sum / (ws * (double)rho[me]));
-}
-
-// Density filter conv with radial_convker_t (TensorExpression.cuh:288-368): out(i) = sum_off w(off) in(i + off)
-// / W(i), W(i) = sum of w over the neighbours inside the grid (every neighbour when periodic); wk holds the
-// normalised weights of the (2h+1)^3 box.  FP64 sums.  W is written when wsum is not null.
-__global__ __launch_bounds__(256) void k_conv_filter(int n, int pitch, int h, int periodic, const float* __restrict__ wk,
-                                                     const float* __restrict__ in, float* __restrict__ out,
-                                                     float* __restrict__ wsum) {
-    const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long N = (long)n * n * n;
-    if (e >= N) return;
-    const int p[3] = {(int)(e % n), (int)((e / n) % n), (int)(e / ((long)n * n))};
-    const int side = 2 * h + 1;
-    double sum = 0.0, ws = 0.0;
-    for (int i = 0; i < side * side * side; i++) {
-        int q[3] = {p[0] + i % side - h, p[1] + (i / side) % side - h, p[2] + i / (side * side) - h};
-        bool inb = true;
-        for (int k = 0; k < 3; k++) {
-            if (periodic) q[k] = ((q[k] % n) + n) % n;
-            if (q[k] < 0 || q[k] >= n) inb = false;
-        }
-        if (!inb) continue;
-        sum += (double)wk[i] * (double)in[q[0] + ((size_t)q[1] + (size_t)q[2] * n) * pitch];
-        ws += (double)wk[i];
-    }
-    const size_t me = p[0] + ((size_t)p[1] + (size_t)p[2] * n) * pitch;
-    out[me] = (float)(sum / ws);
-    if (wsum) wsum[me] = (float)ws;
-}
-
-// Its adjoint (conv_backward_kernel, TensorExpression.cuh:331-366): din(j) = sum_off w(off) dout(j - off) / W(j - off)
-// over the in-grid (or wrapped) j - off; wsum from k_conv_filter.
-__global__ __launch_bounds__(256) void k_conv_filter_back(int n, int pitch, int h, int periodic,
-                                                          const float* __restrict__ wk, const float* __restrict__ dout,
-                                                          const float* __restrict__ wsum, float* __restrict__ din) {
-    const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long N = (long)n * n * n;
-    if (e >= N) return;
-    const int p[3] = {(int)(e % n), (int)((e / n) % n), (int)(e / ((long)n * n))};
-    const int side = 2 * h + 1;
-    double sum = 0.0;
-    for (int i = 0; i < side * side * side; i++) {
-        int q[3] = {p[0] - (i % side - h), p[1] - ((i / side) % side - h), p[2] - (i / (side * side) - h)};
-        bool inb = true;
-        for (int k = 0; k < 3; k++) {
-            if (periodic) q[k] = ((q[k] % n) + n) % n;
-            if (q[k] < 0 || q[k] >= n) inb = false;
-        }
-        if (!inb) continue;
-        const size_t id = q[0] + ((size_t)q[1] + (size_t)q[2] * n) * pitch;
-        sum += (double)wk[i] * (double)dout[id] / (double)wsum[id];
-    }
-    din[p[0] + ((size_t)p[1] + (size_t)p[2] * n) * pitch] = (float)sum;
-}
-
-// sgm projection (sgm_exp_t, AutoDiff.h:808-823): y = 1 / (1 + exp(-k (x - c))); backward gx = gy k y (1 - y).
-__global__ __launch_bounds__(256) void k_sgm(int n, int pitch, double k, double c, const float* __restrict__ x,
-                                             float* __restrict__ y) {
-    const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long N = (long)n * n * n;
-    if (e >= N) return;
-    const size_t id = (e % n) + (size_t)(e / n) * pitch;
-    y[id] = (float)(1.0 / (1.0 + exp(-k * ((double)x[id] - c))));
-}
-
-__global__ __launch_bounds__(256) void k_sgm_back(int n, int pitch, double k, const float* __restrict__ y,
-                                                  const float* __restrict__ gy, float* __restrict__ gx) {
-    const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long N = (long)n * n * n;
-    if (e >= N) return;
-    const size_t id = (e % n) + (size_t)(e / n) * pitch;
-    const double yv = y[id];
-    gx[id] = (float)((double)gy[id] * k * yv * (1.0 - yv));
-}
-
 // OC update of one cell for multiplier g (update_kernel, OCOptimizer.cu:12-34), FP64 arithmetic rounded
 // to FP32.
 __device__ __forceinline__ float oc_cell(double r0, double sv, double g, double min_rho, double step, double damp) {
@@ -2825,30 +2725,10 @@ __global__ __launch_bounds__(256) void k_oc_apply(int n, int pitch, double g, do
     }
 }
 
-// Elementwise density maps of the optimisation loop (rho.pow(p) of the reference's expression templates
-// and its chain rule), over the n^3 live cells of pitched lexicographic arrays.  p = 3 is evaluated as
-// r * r * r and 3 r r d, the products the host loops of the drivers form.
+// index of live cell e in a pitched lexicographic array
 __device__ __forceinline__ size_t pitched(long e, int n, int pitch) {
     const int x = (int)(e % n), y = (int)((e / n) % n), z = (int)(e / ((long)n * n));
     return x + ((size_t)y + (size_t)z * n) * pitch;
-}
-__global__ __launch_bounds__(256) void k_density_pow(int n, int pitch, float p, const float* __restrict__ rho,
-                                                     float* __restrict__ x) {
-    const long N = (long)n * n * n;
-    for (long e = (long)blockIdx.x * blockDim.x + threadIdx.x; e < N; e += (long)gridDim.x * blockDim.x) {
-        const size_t id = pitched(e, n, pitch);
-        const float r = rho[id];
-        x[id] = p == 3.f ? r * r * r : powf(r, p);
-    }
-}
-__global__ __launch_bounds__(256) void k_density_pow_grad(int n, int pitch, float p, const float* __restrict__ rho,
-                                                          const float* dx, float* drho) {
-    const long N = (long)n * n * n;
-    for (long e = (long)blockIdx.x * blockDim.x + threadIdx.x; e < N; e += (long)gridDim.x * blockDim.x) {
-        const size_t id = pitched(e, n, pitch);
-        const float r = rho[id];
-        drho[id] = p == 3.f ? 3.f * r * r * dx[id] : p * powf(r, p - 1.f) * dx[id];
-    }
 }
 __global__ __launch_bounds__(256) void k_field_sum(int n, int pitch, const float* __restrict__ a,
                                                    double* __restrict__ partial) {
@@ -3579,34 +3459,6 @@ void launch_symmetrize(hipStream_t s, int n, int pitch, int ng, const int* gperm
     hipLaunchKernelGGL(k_symmetrize, dim3(nblk(N)), dim3(256), 0, s, n, pitch, ng, gperm, gflip, in, out);
 }
 
-void launch_oc_filter(hipStream_t s, int n, int pitch, int h, int periodic, const float* wk, const float* sens,
-                      const float* rho, float* out) {
-    const size_t N = (size_t)n * n * n;
-    hipLaunchKernelGGL(k_oc_filter, dim3(nblk(N)), dim3(256), 0, s, n, pitch, h, periodic, wk, sens, rho, out);
-}
-
-void launch_conv_filter(hipStream_t s, int n, int pitch, int h, int periodic, const float* wk, const float* in,
-                        float* out, float* wsum) {
-    const size_t N = (size_t)n * n * n;
-    hipLaunchKernelGGL(k_conv_filter, dim3(nblk(N)), dim3(256), 0, s, n, pitch, h, periodic, wk, in, out, wsum);
-}
-
-void launch_conv_filter_back(hipStream_t s, int n, int pitch, int h, int periodic, const float* wk, const float* dout,
-                             const float* wsum, float* din) {
-    const size_t N = (size_t)n * n * n;
-    hipLaunchKernelGGL(k_conv_filter_back, dim3(nblk(N)), dim3(256), 0, s, n, pitch, h, periodic, wk, dout, wsum, din);
-}
-
-void launch_sgm(hipStream_t s, int n, int pitch, double k, double c, const float* x, float* y) {
-    const size_t N = (size_t)n * n * n;
-    hipLaunchKernelGGL(k_sgm, dim3(nblk(N)), dim3(256), 0, s, n, pitch, k, c, x, y);
-}
-
-void launch_sgm_back(hipStream_t s, int n, int pitch, double k, const float* y, const float* gy, float* gx) {
-    const size_t N = (size_t)n * n * n;
-    hipLaunchKernelGGL(k_sgm_back, dim3(nblk(N)), dim3(256), 0, s, n, pitch, k, y, gy, gx);
-}
-
 void launch_oc_trial(hipStream_t s, int n, int pitch, double g, double min_rho, double step, double damp,
                      const float* sens, const float* rho, float* out, double* partial, int nblocks, double* sum) {
     hipLaunchKernelGGL(k_oc_trial, dim3(nblocks), dim3(256), 0, s, n, pitch, g, min_rho, step, damp, sens, rho, out,
@@ -3614,12 +3466,6 @@ void launch_oc_trial(hipStream_t s, int n, int pitch, double g, double min_rho, 
     hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(kSumThreads), 0, s, nblocks, partial, sum);
 }
 
-void launch_density_pow(hipStream_t s, int n, int pitch, float p, const float* rho, float* x) {
-    hipLaunchKernelGGL(k_density_pow, dim3(1024), dim3(256), 0, s, n, pitch, p, rho, x);
-}
-void launch_density_pow_grad(hipStream_t s, int n, int pitch, float p, const float* rho, const float* dx, float* drho) {
-    hipLaunchKernelGGL(k_density_pow_grad, dim3(1024), dim3(256), 0, s, n, pitch, p, rho, dx, drho);
-}
 void launch_field_sum(hipStream_t s, int n, int pitch, const float* a, double* partial, int nblocks) {
     hipLaunchKernelGGL(k_field_sum, dim3(nblocks), dim3(256), 0, s, n, pitch, a, partial);
 }
