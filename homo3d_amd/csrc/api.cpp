@@ -1173,7 +1173,9 @@ int homo3d_elastic_matrix(homo3d_handle* h, double C[36]) {
     int rc = require_density(h);
     if (rc) return rc;
     const Level& L0 = h->lv[0];
-    launch_elastic_matrix(h->stream, L0.n, h->d_ke, h->d_w, h->X, h->d_partial, kDotBlocks, h->d_tmp);
+    double lam, mu;
+    lame_params(h->cfg.youngs_modulus, h->cfg.poisson_ratio, lam, mu);
+    launch_elastic_matrix(h->stream, L0.n, lam, mu, h->d_w, h->X, h->d_partial, kDotBlocks, h->d_tmp);
     double acc[21];
     HIPCHK(h, hipMemcpyAsync(acc, h->d_tmp, sizeof(acc), hipMemcpyDeviceToHost, h->stream));
     HIPCHK(h, hipStreamSynchronize(h->stream));
@@ -1201,7 +1203,6 @@ static int sensitivity(homo3d_handle* h, const float dC[36], float* sens, int pi
     int k = 0;
     for (int i = 0; i < 6; i++)
         for (int j = i; j < 6; j++) wdc[k++] = dC[i * 6 + j] + (i != j ? dC[j * 6 + i] : 0.f);
-    HIPCHK(h, hipMemcpyAsync(h->d_ftmp, wdc, sizeof(wdc), hipMemcpyHostToDevice, h->stream));
     float* dst = sens;
     const size_t elems = lexi_order ? (size_t)pitch * n * n : h->lv[0].N;
     if (!on_device) {
@@ -1209,7 +1210,9 @@ static int sensitivity(homo3d_handle* h, const float dC[36], float* sens, int pi
         if (rc) return rc;
         dst = h->d_stage;
     }
-    launch_sensitivity(h->stream, n, pitch, h->d_ke, h->X, h->d_ftmp, dst);
+    double lam, mu;
+    lame_params(h->cfg.youngs_modulus, h->cfg.poisson_ratio, lam, mu);
+    launch_sensitivity(h->stream, n, pitch, lam, mu, h->X, wdc, dst);
     if (!on_device) {
         if (lexi_order)
             rc = stage_out(h, sens, dst, pitch, 0);

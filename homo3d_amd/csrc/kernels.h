@@ -124,9 +124,10 @@ hipError_t launch_set_p(hipStream_t s, size_t M, const void* z, int z_half, floa
 // per-load-case r . z -> out6 (z FP32 or packed FP16)
 void launch_dot_rz(hipStream_t s, size_t M, const float* r, const void* z, int z_half, double* partial, int nblocks,
                    double* out6);
-void launch_elastic_matrix(hipStream_t s, int n, const float* ke, const float* w, const float* chi, double* partial,
-                           int nblocks, double* out21);
-void launch_sensitivity(hipStream_t s, int n, int pitch, const float* ke, const float* chi, const float* wdc,
+// C^H sums and sensitivity of the fields chi (energy.hip); lam, mu the Lame parameters, wdc 21 host floats
+void launch_elastic_matrix(hipStream_t s, int n, double lam, double mu, const float* w, const float* chi,
+                           double* partial, int nblocks, double* out21);
+void launch_sensitivity(hipStream_t s, int n, int pitch, double lam, double mu, const float* chi, const float* wdc,
                         float* sens);
 void launch_symmetrize(hipStream_t s, int n, int pitch, int ng, const int* gperm, const int* gflip, const float* in,
                        float* out);

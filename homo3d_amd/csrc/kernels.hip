@@ -19,82 +19,12 @@
 
 #include "../../include/homo3d.h"
 #include "kernels.h"
+#include "level.h"
 #include "net.h"
 
 namespace homo3d {
 
 namespace {
-
-__device__ __forceinline__ int wrap_dec(int a, int n) { return a == 0 ? n - 1 : a - 1; }
-__device__ __forceinline__ int wrap_inc(int a, int n) { return a == n - 1 ? 0 : a + 1; }
-
-// Storage order of a level's vertices (and of the cells, which share the vertex index).  Even levels
-// are parity-blocked: the 8 coordinate-parity classes are contiguous (n/2)^3 blocks, block
-// b = (x&1) | (y&1)<<1 | (z&1)<<2, and inside a block (x>>1) + h((y>>1) + h(z>>1)).  A GS colour is
-// one block, so colour passes read their own vertices and every neighbour class contiguously.
-// The coarsest level (possibly odd) is lexicographic.  Vertex (0,0,0) has index 0 in both orders.
-struct Lay {
-    int n;        // points per axis
-    int h;        // n / 2
-    uint32_t h3;  // h^3
-    int lex;      // 1: x + n(y + n z)
-    // index contribution of (already wrapped) coordinate a on axis k
-    __device__ __forceinline__ uint32_t part(int a, int k) const {
-        if (lex) return k == 0 ? (uint32_t)a : (k == 1 ? (uint32_t)a * n : (uint32_t)a * n * n);
-        const uint32_t stride = k == 0 ? 1u : (k == 1 ? (uint32_t)h : (uint32_t)h * h);
-        return ((uint32_t)(a & 1) << k) * h3 + (uint32_t)(a >> 1) * stride;
-    }
-    __device__ __forceinline__ uint32_t idx(int x, int y, int z) const { return part(x, 0) + part(y, 1) + part(z, 2); }
-    __device__ __forceinline__ void pos(uint32_t t, int& x, int& y, int& z) const {
-        if (lex) {
-            x = (int)(t % n);
-            y = (int)((t / n) % n);
-            z = (int)(t / ((uint32_t)n * n));
-            return;
-        }
-        const uint32_t b = t / h3, l = t - b * h3;
-        x = 2 * (int)(l % h) + (int)(b & 1);
-        y = 2 * (int)((l / h) % h) + (int)((b >> 1) & 1);
-        z = 2 * (int)(l / ((uint32_t)h * h)) + (int)(b >> 2);
-    }
-    __device__ __forceinline__ int wrap(int a) const { return a < 0 ? a + n : (a >= n ? a - n : a); }
-};
-
-// Workgroup id -> work chunk.  The hardware deals workgroup g to XCD g % 8; this gives each XCD a
-// contiguous run of chunks, so the neighbour rows that adjacent chunks share stay in one L2.
-__device__ __forceinline__ uint32_t xcd_chunk(uint32_t g, uint32_t G) {
-    if (G & 7u) return g;
-    return (g & 7u) * (G >> 3) + (g >> 3);
-}
-
-// Full-level kernels run 512-thread workgroups.  On a parity-blocked level the 8 waves of a
-// workgroup take the same 64 local positions in the 8 parity blocks, so a workgroup covers a
-// 128 x 2 x 2 vertex tile and the neighbour reads of its waves overlap in L1/L2; on a
-// lexicographic level the 512 threads take consecutive vertices.  False past the end of the level.
-constexpr int kFullThreads = 512;
-__device__ __forceinline__ bool full_vertex(const Lay& L, uint32_t chunk, uint32_t& v) {
-    if (L.lex) {
-        v = chunk * (uint32_t)kFullThreads + threadIdx.x;
-        return v < (uint32_t)L.n * L.n * L.n;
-    }
-    const uint32_t t = chunk * 64u + (threadIdx.x & 63u);
-    v = (threadIdx.x >> 6) * L.h3 + t;
-    return t < L.h3;
-}
-
-// Buffer-resource loads: one SGPR descriptor per array, a 32-bit VGPR byte offset per element and an
-// SGPR byte offset per (load case, component) plane.  Offsets past the array read as zero.
-typedef __amdgpu_buffer_rsrc_t Rsrc;
-__device__ __forceinline__ Rsrc make_rsrc(const void* p, size_t bytes) {
-    const uint32_t nrec = bytes > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)bytes;
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)nrec, 0x00020000);
-}
-template <typename T>
-__device__ __forceinline__ T bload(Rsrc r, uint32_t voff, uint32_t soff);
-template <>
-__device__ __forceinline__ float bload<float>(Rsrc r, uint32_t voff, uint32_t soff) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, (int)voff, (int)soff, 0));
-}
 
 // Packed FP16 storage of a 6-load-case field: word plane (p * 3 + i) holds components i of load cases
 // 2p (.x) and 2p + 1 (.y), so a neighbour of all six load cases is 9 32-bit words.
@@ -208,21 +138,6 @@ __device__ __forceinline__ void fine_block(const W wc[8], const T* ke, T S[9]) {
     S[6] = cb[6] * fxz;
     S[5] = cb[5] * fyz;
     S[7] = cb[7] * fyz;
-}
-
-template <int BS>
-__device__ __forceinline__ double block_sum(double v, double* sh) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    if (lane == 0) sh[wid] = v;
-    __syncthreads();
-    double s = 0.0;
-    if (threadIdx.x == 0) {
-        for (int i = 0; i < BS / 64; i++) s += sh[i];
-    }
-    __syncthreads();
-    return s;
 }
 
 struct FineCtx {
@@ -2542,106 +2457,6 @@ __global__ __launch_bounds__(256) void k_pcg_update_px_h(int R, size_t M, const 
 }
 
 // ---------------------------------------------------------------------------------------------
-// C^H and sensitivity (elasticMatrix_kernel_opt homogenization.cu:208-346;
-// Sensitivity_kernel_opt_2 homogenization.cu:697-858).  One thread per cell; the six solution
-// fields of the cell's 8 nodes are read in FP32 and the cell energies accumulated in FP32.
-// ---------------------------------------------------------------------------------------------
-__device__ __forceinline__ float macro_disp(int node, int s, int c) {
-    const float px = (float)(node & 1), py = (float)((node >> 1) & 1), pz = (float)(node >> 2);
-    switch (s) {
-        case 0: return c == 0 ? px : 0.f;
-        case 1: return c == 1 ? py : 0.f;
-        case 2: return c == 2 ? pz : 0.f;
-        case 3: return c == 1 ? 0.5f * pz : (c == 2 ? 0.5f * py : 0.f);
-        case 4: return c == 0 ? 0.5f * pz : (c == 2 ? 0.5f * px : 0.f);
-        default: return c == 0 ? 0.5f * py : (c == 1 ? 0.5f * px : 0.f);
-    }
-}
-
-__device__ __forceinline__ void cell_energies(const Lay& L, size_t N, uint32_t e, const float* __restrict__ ke,
-                                              const float* __restrict__ chi, float E[21], int& x, int& y, int& z) {
-    L.pos(e, x, y, z);
-    const uint32_t xs[2] = {L.part(x, 0), L.part(wrap_inc(x, L.n), 0)};
-    const uint32_t ys[2] = {L.part(y, 1), L.part(wrap_inc(y, L.n), 1)};
-    const uint32_t zs[2] = {L.part(z, 2), L.part(wrap_inc(z, L.n), 2)};
-    float U[6][24];
-#pragma unroll
-    for (int b = 0; b < 8; b++) {
-        const uint32_t q = xs[b & 1] + ys[(b >> 1) & 1] + zs[b >> 2];
-#pragma unroll
-        for (int s = 0; s < 6; s++)
-#pragma unroll
-            for (int c = 0; c < 3; c++) U[s][3 * b + c] = macro_disp(b, s, c) - chi[(size_t)(s * 3 + c) * N + q];
-    }
-#pragma unroll
-    for (int k = 0; k < 21; k++) E[k] = 0.f;
-#pragma unroll
-    for (int i = 0; i < 24; i++) {
-        float KU[6];
-#pragma unroll
-        for (int s = 0; s < 6; s++) KU[s] = 0.f;
-#pragma unroll
-        for (int j = 0; j < 24; j++) {
-            const float kij = ke[i * 24 + j];
-#pragma unroll
-            for (int s = 0; s < 6; s++) KU[s] = fmaf(kij, U[s][j], KU[s]);
-        }
-        int k = 0;
-#pragma unroll
-        for (int a = 0; a < 6; a++)
-#pragma unroll
-            for (int b = a; b < 6; b++) {
-                E[k] = fmaf(U[a][i], KU[b], E[k]);
-                k++;
-            }
-    }
-}
-
-// partial[k * nblocks + block] = sum of w_e E_k,e over the block's cells (FP64)
-__global__ __launch_bounds__(kFullThreads) void k_elastic_matrix(Lay L, size_t N, uint32_t nchunks,
-                                                                 const float* __restrict__ ke,
-                                                                 const float* __restrict__ w,
-                                                                 const float* __restrict__ chi,
-                                                                 double* __restrict__ partial) {
-    __shared__ double sh[kFullThreads / 64];
-    double acc[21];
-#pragma unroll
-    for (int k = 0; k < 21; k++) acc[k] = 0.0;
-    for (uint32_t chunk = blockIdx.x; chunk < nchunks; chunk += gridDim.x) {
-        uint32_t e;
-        if (!full_vertex(L, chunk, e)) continue;
-        float E[21];
-        int x, y, z;
-        cell_energies(L, N, e, ke, chi, E, x, y, z);
-        const double we = w[e];
-#pragma unroll
-        for (int k = 0; k < 21; k++) acc[k] += we * (double)E[k];
-    }
-    for (int k = 0; k < 21; k++) {
-        const double s = block_sum<kFullThreads>(acc[k], sh);
-        if (threadIdx.x == 0) partial[k * gridDim.x + blockIdx.x] = s;
-    }
-}
-
-// sens[x + (y + z*n)*pitch] = (1/N) sum_{i<=j} E_ij (dC_ij + [i!=j] dC_ji)
-__global__ __launch_bounds__(kFullThreads) void k_sensitivity(Lay L, size_t N, int pitch,
-                                                              const float* __restrict__ ke,
-                                                              const float* __restrict__ chi,
-                                                              const float* __restrict__ wdc,
-                                                              float* __restrict__ sens) {
-    uint32_t e;
-    if (!full_vertex(L, xcd_chunk(blockIdx.x, gridDim.x), e)) return;
-    float E[21];
-    int x, y, z;
-    cell_energies(L, N, e, ke, chi, E, x, y, z);
-    float s = 0.f;
-#pragma unroll
-    for (int k = 0; k < 21; k++) s = fmaf(E[k], wdc[k], s);
-    // pitch 0: the level's own (parity-blocked) cell order, unpitched
-    sens[pitch ? x + ((size_t)y + (size_t)z * L.n) * pitch : (size_t)e] = s / (float)N;
-}
-
-// ---------------------------------------------------------------------------------------------
 // Density utilities
 // ---------------------------------------------------------------------------------------------
 
@@ -2786,28 +2601,13 @@ __global__ __launch_bounds__(256) void k_copy_pitched(int n, int pitch_in, int p
     out[x + ((size_t)y + (size_t)z * n) * pitch_out] = in[x + ((size_t)y + (size_t)z * n) * pitch_in];
 }
 
-inline unsigned nblk(size_t work, int bs = 256) { return (unsigned)((work + bs - 1) / bs); }
 
 }  // namespace
 
 // ---------------------------------------------------------------------------------------------
 // Launch wrappers
 // ---------------------------------------------------------------------------------------------
-static Lay make_lay(int n, int lex) {
-    Lay L;
-    L.n = n;
-    L.h = n / 2;
-    L.h3 = (uint32_t)L.h * L.h * L.h;
-    L.lex = lex;
-    return L;
-}
-
 // workgroups of a full-level kernel (see full_vertex)
-static unsigned full_grid(const Lay& L) {
-    const size_t N = (size_t)L.n * L.n * L.n;
-    return L.lex ? nblk(N, kFullThreads) : nblk(L.h3, 64);
-}
-
 int ke_mfma_table(const double* kl, const double* km, double lam, double mu, void* table, float* c0, float* c1) {
     // One exact table T = r Kl + Km (KE = mu/72 T) when r = lambda / mu is a short binary fraction
     // (nu = 0.3 gives r = 3/2) and every entry of T is an FP16 value; else Kl and Km separately.
@@ -3434,23 +3234,6 @@ void launch_dot_rz(hipStream_t s, size_t M, const float* r, const void* z, int z
     }
     hipLaunchKernelGGL(k_dot_fh, dim3(nblocks, 3), dim3(256), 0, s, M, r, static_cast<const half2_t*>(z), partial);
     hipLaunchKernelGGL(k_sum_partials, dim3(6), dim3(kSumThreads), 0, s, nblocks, partial, out6);
-}
-
-void launch_elastic_matrix(hipStream_t s, int n, const float* ke, const float* w, const float* chi, double* partial,
-                           int nblocks, double* out21) {
-    const size_t N = (size_t)n * n * n;
-    const Lay L = make_lay(n, 0);
-    const unsigned nchunks = full_grid(L);
-    const int nb = (int)std::min<unsigned>((unsigned)nblocks, nchunks);
-    hipLaunchKernelGGL(k_elastic_matrix, dim3(nb), dim3(kFullThreads), 0, s, L, N, nchunks, ke, w, chi, partial);
-    hipLaunchKernelGGL(k_sum_partials, dim3(21), dim3(kSumThreads), 0, s, nb, partial, out21);
-}
-
-void launch_sensitivity(hipStream_t s, int n, int pitch, const float* ke, const float* chi, const float* wdc,
-                        float* sens) {
-    const size_t N = (size_t)n * n * n;
-    const Lay L = make_lay(n, 0);
-    hipLaunchKernelGGL(k_sensitivity, dim3(full_grid(L)), dim3(kFullThreads), 0, s, L, N, pitch, ke, chi, wdc, sens);
 }
 
 void launch_symmetrize(hipStream_t s, int n, int pitch, int ng, const int* gperm, const int* gflip, const float* in,

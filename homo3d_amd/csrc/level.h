@@ -1,0 +1,114 @@
+// Device helpers shared by the kernels that work on a grid level: storage order, workgroup order, buffer
+// loads and workgroup sums.  Included inside each kernel file; everything has internal linkage.
+#pragma once
+#include <hip/hip_runtime.h>
+#include <stddef.h>
+#include <stdint.h>
+
+namespace homo3d {
+namespace {
+
+__device__ __forceinline__ int wrap_dec(int a, int n) { return a == 0 ? n - 1 : a - 1; }
+__device__ __forceinline__ int wrap_inc(int a, int n) { return a == n - 1 ? 0 : a + 1; }
+
+// Storage order of a level's vertices (and of the cells, which share the vertex index).  Even levels
+// are parity-blocked: the 8 coordinate-parity classes are contiguous (n/2)^3 blocks, block
+// b = (x&1) | (y&1)<<1 | (z&1)<<2, and inside a block (x>>1) + h((y>>1) + h(z>>1)).  A GS colour is
+// one block, so colour passes read their own vertices and every neighbour class contiguously.
+// The coarsest level (possibly odd) is lexicographic.  Vertex (0,0,0) has index 0 in both orders.
+struct Lay {
+    int n;        // points per axis
+    int h;        // n / 2
+    uint32_t h3;  // h^3
+    int lex;      // 1: x + n(y + n z)
+    // index contribution of (already wrapped) coordinate a on axis k
+    __device__ __forceinline__ uint32_t part(int a, int k) const {
+        if (lex) return k == 0 ? (uint32_t)a : (k == 1 ? (uint32_t)a * n : (uint32_t)a * n * n);
+        const uint32_t stride = k == 0 ? 1u : (k == 1 ? (uint32_t)h : (uint32_t)h * h);
+        return ((uint32_t)(a & 1) << k) * h3 + (uint32_t)(a >> 1) * stride;
+    }
+    __device__ __forceinline__ uint32_t idx(int x, int y, int z) const { return part(x, 0) + part(y, 1) + part(z, 2); }
+    __device__ __forceinline__ void pos(uint32_t t, int& x, int& y, int& z) const {
+        if (lex) {
+            x = (int)(t % n);
+            y = (int)((t / n) % n);
+            z = (int)(t / ((uint32_t)n * n));
+            return;
+        }
+        const uint32_t b = t / h3, l = t - b * h3;
+        x = 2 * (int)(l % h) + (int)(b & 1);
+        y = 2 * (int)((l / h) % h) + (int)((b >> 1) & 1);
+        z = 2 * (int)(l / ((uint32_t)h * h)) + (int)(b >> 2);
+    }
+    __device__ __forceinline__ int wrap(int a) const { return a < 0 ? a + n : (a >= n ? a - n : a); }
+};
+
+// Workgroup id -> work chunk.  The hardware deals workgroup g to XCD g % 8; this gives each XCD a
+// contiguous run of chunks, so the neighbour rows that adjacent chunks share stay in one L2.
+__device__ __forceinline__ uint32_t xcd_chunk(uint32_t g, uint32_t G) {
+    if (G & 7u) return g;
+    return (g & 7u) * (G >> 3) + (g >> 3);
+}
+
+// Full-level kernels run 512-thread workgroups.  On a parity-blocked level the 8 waves of a
+// workgroup take the same 64 local positions in the 8 parity blocks, so a workgroup covers a
+// 128 x 2 x 2 vertex tile and the neighbour reads of its waves overlap in L1/L2; on a
+// lexicographic level the 512 threads take consecutive vertices.  False past the end of the level.
+constexpr int kFullThreads = 512;
+__device__ __forceinline__ bool full_vertex(const Lay& L, uint32_t chunk, uint32_t& v) {
+    if (L.lex) {
+        v = chunk * (uint32_t)kFullThreads + threadIdx.x;
+        return v < (uint32_t)L.n * L.n * L.n;
+    }
+    const uint32_t t = chunk * 64u + (threadIdx.x & 63u);
+    v = (threadIdx.x >> 6) * L.h3 + t;
+    return t < L.h3;
+}
+
+// Buffer-resource loads: one SGPR descriptor per array, a 32-bit VGPR byte offset per element and an
+// SGPR byte offset per (load case, component) plane.  Offsets past the array read as zero.
+typedef __amdgpu_buffer_rsrc_t Rsrc;
+__device__ __forceinline__ Rsrc make_rsrc(const void* p, size_t bytes) {
+    const uint32_t nrec = bytes > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)bytes;
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)nrec, 0x00020000);
+}
+template <typename T>
+__device__ __forceinline__ T bload(Rsrc r, uint32_t voff, uint32_t soff);
+template <>
+__device__ __forceinline__ float bload<float>(Rsrc r, uint32_t voff, uint32_t soff) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, (int)voff, (int)soff, 0));
+}
+
+template <int BS>
+__device__ __forceinline__ double block_sum(double v, double* sh) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    if (lane == 0) sh[wid] = v;
+    __syncthreads();
+    double s = 0.0;
+    if (threadIdx.x == 0) {
+        for (int i = 0; i < BS / 64; i++) s += sh[i];
+    }
+    __syncthreads();
+    return s;
+}
+
+inline unsigned nblk(size_t work, int bs = 256) { return (unsigned)((work + bs - 1) / bs); }
+
+inline Lay make_lay(int n, int lex) {
+    Lay L;
+    L.n = n;
+    L.h = n / 2;
+    L.h3 = (uint32_t)L.h * L.h * L.h;
+    L.lex = lex;
+    return L;
+}
+
+inline unsigned full_grid(const Lay& L) {
+    const size_t N = (size_t)L.n * L.n * L.n;
+    return L.lex ? nblk(N, kFullThreads) : nblk(L.h3, 64);
+}
+
+}  // namespace
+}  // namespace homo3d
