@@ -75,14 +75,15 @@ struct homo3d_handle {
     const FineMfma* mf() const { return d_ke16 && use_mfma ? &mfma : nullptr; }
     bool stage_tiles = true;    // CG pass: z node boxes staged in LDS where fine_cg_staged_ok (homo3d_stage_tiles)
     float* d_kchi = nullptr;
-    float* d_G = nullptr;
+    double* d_G = nullptr;
+    float* d_G32 = nullptr;
     float* d_w = nullptr;
     float* d_x = nullptr;       // raw cell values x (FP32 input), for FP64 weights
     float* d_stage = nullptr;   // pitched staging buffer for host densities / sensitivities
     size_t stage_elems = 0;
     double* d_Ainv = nullptr;       // the coarsest level's dense FP64 inverse (mc x mc)
     int* d_cstat = nullptr;         // factorisation status on the device
-    double* d_cpiv = nullptr;       // its pivot rows and columns (4 mc)
+    double* d_cwork = nullptr;      // the elimination's other buffer (mc x mc)
     int mc = 0;
     // the coarsest factorisation runs on the GPU at the density update, on a stream of its own behind
     // the Galerkin kernels (ev_gal), so it overlaps the solve's finest-level work; its status is read,
@@ -769,7 +770,8 @@ int homo3d_create(const homo3d_config* cfg, homo3d_handle** out) {
         return fail(HOMO3D_HIP_ERROR);
     // element matrix, macro loads and the level-1 Galerkin table
     element_matrix(cfg->youngs_modulus, cfg->poisson_ratio, h->ke);
-    std::vector<float> kef(576), kchi(6 * 24), G(64 * 27 * 9, 0.f);
+    std::vector<float> kef(576), kchi(6 * 24);
+    std::vector<double> G(64 * 27 * 9, 0.0);
     for (int i = 0; i < 576; i++) kef[i] = (float)h->ke[i];
     for (int s = 0; s < 6; s++)
         for (int i = 0; i < 24; i++) {
@@ -794,7 +796,7 @@ int homo3d_create(const homo3d_config* cfg, homo3d_handle** out) {
                         for (int j = 0; j < 3; j++) S[i * 3 + j] += wa * wb * h->ke[(3 * a + i) * 24 + 3 * b + j];
                 }
             }
-            for (int k = 0; k < 9; k++) G[(c * 27 + D) * 9 + k] = (float)S[k];
+            for (int k = 0; k < 9; k++) G[(c * 27 + D) * 9 + k] = S[k];
         }
     }
     if (hipMalloc(&h->d_ke64, sizeof(double) * 576) || hipMalloc(&h->d_kchi64, sizeof(double) * 144))
@@ -813,7 +815,7 @@ int homo3d_create(const homo3d_config* cfg, homo3d_handle** out) {
             return fail(HOMO3D_HIP_ERROR);
     }
     if (hipMalloc(&h->d_ke, sizeof(float) * 576) || hipMalloc(&h->d_kchi, sizeof(float) * 144) ||
-        hipMalloc(&h->d_G, sizeof(float) * G.size()) || hipMalloc(&h->d_gperm, sizeof(int) * 48) ||
+        hipMalloc(&h->d_G, sizeof(double) * G.size()) || hipMalloc(&h->d_G32, sizeof(float) * G.size()) || hipMalloc(&h->d_gperm, sizeof(int) * 48) ||
         hipMalloc(&h->d_gflip, sizeof(int) * 48))
         return fail(HOMO3D_HIP_ERROR);
     double kl[576], km[576];
@@ -832,12 +834,14 @@ int homo3d_create(const homo3d_config* cfg, homo3d_handle** out) {
     }
     if (hipMemcpy(h->d_ke, kef.data(), sizeof(float) * 576, hipMemcpyHostToDevice) ||
         hipMemcpy(h->d_kchi, kchi.data(), sizeof(float) * 144, hipMemcpyHostToDevice) ||
-        hipMemcpy(h->d_G, G.data(), sizeof(float) * G.size(), hipMemcpyHostToDevice))
+        hipMemcpy(h->d_G, G.data(), sizeof(double) * G.size(), hipMemcpyHostToDevice) ||
+        hipMemcpy(h->d_G32, std::vector<float>(G.begin(), G.end()).data(), sizeof(float) * G.size(),
+                  hipMemcpyHostToDevice))
         return fail(HOMO3D_HIP_ERROR);
     const int nc = sizes[nl - 1];
     h->mc = 3 * nc * nc * nc;
     if (hipMalloc(&h->d_Ainv, sizeof(double) * h->mc * h->mc) || hipMalloc(&h->d_cstat, sizeof(int)) ||
-        hipMalloc(&h->d_cpiv, sizeof(double) * 4 * h->mc))
+        hipMalloc(&h->d_cwork, sizeof(double) * h->mc * h->mc))
         return fail(HOMO3D_HIP_ERROR);
     if (hipDeviceSynchronize() != hipSuccess) return fail(HOMO3D_HIP_ERROR);
     *out = h;
@@ -856,7 +860,7 @@ int homo3d_destroy(homo3d_handle* h) {
         (void)hipFree(h->lv[l].r);
         (void)hipFree(h->lv[l].st);
     }
-    void* ptrs[] = {h->d_x, h->U64, h->d_ke64, h->d_kchi64, h->d_ke, h->d_ke16, h->d_kchi, h->d_G, h->d_w, h->d_stage, h->d_Ainv, h->d_cstat, h->d_cpiv, h->X, h->F, h->P, h->Q, h->Z,
+    void* ptrs[] = {h->d_x, h->U64, h->d_ke64, h->d_kchi64, h->d_ke, h->d_ke16, h->d_kchi, h->d_G, h->d_G32, h->d_w, h->d_stage, h->d_Ainv, h->d_cstat, h->d_cwork, h->X, h->F, h->P, h->Q, h->Z,
                     h->Rr, h->d_partial, h->d_sc, h->d_tmp, h->d_ftmp, h->d_gperm, h->d_gflip};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
@@ -896,10 +900,12 @@ int homo3d_update_density(homo3d_handle* h, const float* x, int pitch, int on_de
     // a factorisation still running from the previous update reads the coarsest stencil rewritten below
     if (h->ev_coarse) HIPCHK(h, hipStreamWaitEvent(h->stream, h->ev_coarse, 0));
     const float clamp = (float)h->cfg.diag_clamp;
-    launch_galerkin_fine(h->stream, n, h->lv[1].lex, h->d_G, h->d_ke, h->d_w, h->lv[1].st, h->lv[1].st_half, clamp);
+    launch_galerkin_fine(h->stream, n, h->lv[1].lex, h->d_G, h->d_G32, h->d_ke64, h->d_w, h->lv[1].st,
+                         h->lv[1].st_half, clamp);
+    // (the search direction P is scratch between solves: 72 n^3 bytes, of which the product takes at most 61)
     for (int l = 2; l < h->nl; l++)
         launch_galerkin_coarse(h->stream, h->lv[l - 1].n, h->lv[l].lex, h->lv[l - 1].st, h->lv[l - 1].st_half,
-                               h->lv[l].st, h->lv[l].st_half, clamp);
+                               h->lv[l].st, h->lv[l].st_half, reinterpret_cast<double*>(h->P), clamp);
     // coarsest dense system: assembled and inverted on the GPU; its status is read at the
     // first coarse solve (coarse_factor)
     const Level& Lc = h->lv[h->nl - 1];
@@ -913,7 +919,7 @@ int homo3d_update_density(homo3d_handle* h, const float* x, int pitch, int on_de
     // solves that read the inverse)
     HIPCHK(h, hipEventRecord(h->ev_gal, h->stream));
     HIPCHK(h, hipStreamWaitEvent(h->cstream, h->ev_gal, 0));
-    launch_coarse_factor(h->cstream, Lc.n, static_cast<const float*>(Lc.st), h->d_Ainv, h->d_cpiv, h->d_cstat);
+    launch_coarse_factor(h->cstream, Lc.n, static_cast<const float*>(Lc.st), h->d_Ainv, h->d_cwork, h->d_cstat);
     HIPCHK(h, hipMemcpyAsync(h->h_cstat, h->d_cstat, sizeof(int), hipMemcpyDeviceToHost, h->cstream));
     HIPCHK(h, hipEventRecord(h->ev_coarse, h->cstream));
     h->coarse_pending = true;

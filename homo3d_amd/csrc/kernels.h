@@ -77,12 +77,11 @@ void launch_zero_pin(hipStream_t s, size_t N, void* u, int u_half);
 void launch_pack_half(hipStream_t s, size_t N, const float* u, void* z);
 void launch_unpack_half(hipStream_t s, size_t N, const void* z, float* u);
 void launch_zero_pin64(hipStream_t s, size_t N, double* u);
-// The coarsest level's dense FP64 inverse on the GPU: assembled from its FP32 stencil (lexicographic
-// n_c^3 level, m = 3 n_c^3), symmetrised and inverted in place in ainv (m x m) by Gauss-Jordan
-// elimination on the diagonal, one launch per step; piv is 4 m doubles of pivot rows and columns.
-// status (device) = 0, or 1 + the first step whose pivot is not positive (the system is not positive
-// definite; ainv is then not an inverse).
-void launch_coarse_factor(hipStream_t s, int nc, const float* st, double* ainv, double* piv, int* status);
+// The coarsest level's dense FP64 inverse on the GPU (setup.hip): assembled from its FP32 stencil
+// (lexicographic n_c^3 level, m = 3 n_c^3), symmetrised and inverted into ainv (m x m) by Gauss-Jordan
+// elimination on the diagonal; work is another m x m doubles.  status (device) = 0, or 1 + the first step
+// whose pivot is not positive (the system is not positive definite; ainv is then not an inverse).
+void launch_coarse_factor(hipStream_t s, int nc, const float* st, double* ainv, double* work, int* status);
 // Coarse stencils: FP32 [243][n^3] or, with *_half, packed FP16 [122][n^3] words (entries 2w, 2w + 1).
 // u FP32 planes, or (u_half, only where stencil_u_half_ok: six load cases per launch) packed FP16 pairs.
 int stencil_u_half_ok(int n, int lex);
@@ -103,10 +102,12 @@ void launch_stencil_residual_later(hipStream_t s, int n, const void* st, int st_
 void launch_restrict(hipStream_t s, int nf, int lexc, const float* rf, float* fc);
 // uf += P uc.  uc FP32, or packed FP16 (uc_half: parity-blocked coarse level, packed FP16 fine u).
 void launch_prolong(hipStream_t s, int nf, int lexc, const void* uc, int uc_half, void* uf, int u_half, int pin);
-void launch_galerkin_fine(hipStream_t s, int nf, int lexc, const float* G, const float* ke, const float* w, void* stc,
-                          int out_half, float clamp);
+// G: the 64 x 27 x 9 table of P-weighted element blocks, and G32 the same in FP32
+void launch_galerkin_fine(hipStream_t s, int nf, int lexc, const double* G, const float* G32, const double* ke,
+                          const float* w, void* stc, int out_half, float clamp);
+// work: 243 nf^3 / 4 doubles
 void launch_galerkin_coarse(hipStream_t s, int nf, int lexc, const void* stf, int in_half, void* stc, int out_half,
-                            float clamp);
+                            double* work, float clamp);
 void launch_coarse_solve(hipStream_t s, int nc, const double* Ainv, const float* f, float* u);
 void launch_dot6(hipStream_t s, size_t M, const float* a, const float* b, double* partial, int nblocks, double* out);
 void launch_sum_partials(hipStream_t s, int R, int nblocks, const double* partial, double* out);

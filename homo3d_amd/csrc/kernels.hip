@@ -26,14 +26,6 @@ namespace homo3d {
 
 namespace {
 
-// Packed FP16 storage of a 6-load-case field: word plane (p * 3 + i) holds components i of load cases
-// 2p (.x) and 2p + 1 (.y), so a neighbour of all six load cases is 9 32-bit words.
-typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
-template <>
-__device__ __forceinline__ half2_t bload<half2_t>(Rsrc r, uint32_t voff, uint32_t soff) {
-    return __builtin_bit_cast(half2_t, __builtin_amdgcn_raw_buffer_load_b32(r, (int)voff, (int)soff, 0));
-}
-
 // The FP64 iterate of the refinement loop stores its 18 components as nine planes of 16-byte pairs
 // (u64_index), so a neighbour of all six load cases is nine 16-byte loads rather than eighteen
 // 8-byte ones: the gather's cost is per load instruction.
@@ -1452,30 +1444,6 @@ __global__ void k_zero_pin(size_t N, int planes, T* __restrict__ u) {
 // Coarse levels (stored 27-point stencils)
 // ---------------------------------------------------------------------------------------------
 
-// A stored coarse stencil: FP32 entries [243][N] (entry e = 9d + 3i + j), or packed FP16 [122][N]
-// words, word w holding entries 2w (.x) and 2w + 1 (.y).  Both have 4-byte words per vertex.
-template <typename SA>
-struct StencilIO;
-template <>
-struct StencilIO<float> {
-    static constexpr int words = 243;
-    __device__ static float get(Rsrc rs, uint32_t vo, uint32_t plane, int e) {
-        return bload<float>(rs, vo, (uint32_t)e * plane);
-    }
-    __device__ static void put(float* st, size_t N, uint32_t v, int e, float val) { st[(size_t)e * N + v] = val; }
-};
-template <>
-struct StencilIO<half2_t> {
-    static constexpr int words = 122;
-    __device__ static float get(Rsrc rs, uint32_t vo, uint32_t plane, int e) {
-        return (float)bload<half2_t>(rs, vo, (uint32_t)(e >> 1) * plane)[e & 1];
-    }
-    // one 16-bit store per entry: the two halves of a word may come from different threads
-    __device__ static void put(half2_t* st, size_t N, uint32_t v, int e, float val) {
-        reinterpret_cast<_Float16*>(st + (size_t)(e >> 1) * N + v)[e & 1] = (_Float16)val;
-    }
-};
-
 // One neighbour of a coarse row: issue the loads of the next selected neighbour (its stencil block and
 // words), accumulate this one, recurse.  The barrier keeps the loads one neighbour ahead: with the whole
 // row unrolled freely the compiler issues every neighbour's loads at once and needs 256 VGPRs.
@@ -1713,18 +1681,6 @@ __global__ __launch_bounds__(256) void k_stencil_resid_later(Lay L, size_t N, co
     }
 }
 
-// Coarse-vertex kernels that read the fine level around 2V take coarse vertices in lexicographic
-// order whatever the coarse storage, so that consecutive lanes read consecutive fine local positions.
-__device__ __forceinline__ bool coarse_lex_vertex(const Lay& Lc, int& X, int& Y, int& Z, uint32_t& V) {
-    const uint32_t i = xcd_chunk(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
-    const uint32_t n = (uint32_t)Lc.n;
-    if (i >= n * n * n) return false;
-    X = (int)(i % n);
-    Y = (int)((i / n) % n);
-    Z = (int)(i / (n * n));
-    V = Lc.idx(X, Y, Z);
-    return true;
-}
 
 // ---------------------------------------------------------------------------------------------
 // Grid transfers (restrict_residual_kernel_1 grid.cu:917-994; prolongate_correction_kernel_1
@@ -1975,271 +1931,6 @@ __global__ __launch_bounds__(kFullThreads) void k_prolong_h(Lay Lf, Lay Lc, cons
     *f0 = make_uint4(wv[0], wv[1], wv[2], wv[3]);
     *f1 = make_uint4(wv[4], wv[5], wv[6], wv[7]);
     fw[8 * Nf + v] = wv[8];
-}
-
-// ---------------------------------------------------------------------------------------------
-// Galerkin coarse operators (restrict_stencil_otf_aos_kernel_1 grid_ex.cu:936-1061;
-// restrict_stencil_aos_kernel_1 grid_ex.cu:1065-1160; pinned-origin rows grid.cpp:1184-1325)
-// ---------------------------------------------------------------------------------------------
-
-__device__ __forceinline__ float hat(int o) { return o == 0 ? 1.f : ((o == 1 || o == -1) ? 0.5f : 0.f); }
-
-// Level-1 stencil away from the pinned origin: st[V][D] = sum_{c} w_{2V+c} G[c][D], c in {-2..1}^3.
-// G (64 x 27 x 9) is the density-independent table of P-weighted KE blocks.
-template <typename SO>
-__global__ __launch_bounds__(256) void k_galerkin_fine(Lay Lf, Lay Lc, const float* __restrict__ G,
-                                                       const float* __restrict__ w, SO* __restrict__ stc,
-                                                       float clamp) {
-    const int nf = Lf.n;
-    const size_t Nc = (size_t)Lc.n * Lc.n * Lc.n;
-    int X, Y, Z;
-    uint32_t V;
-    if (!coarse_lex_vertex(Lc, X, Y, Z, V)) return;
-    float wc[64];
-#pragma unroll
-    for (int c = 0; c < 64; c++) {
-        int cx = 2 * X + (c & 3) - 2, cy = 2 * Y + ((c >> 2) & 3) - 2, cz = 2 * Z + (c >> 4) - 2;
-        cx = cx < 0 ? cx + nf : (cx >= nf ? cx - nf : cx);
-        cy = cy < 0 ? cy + nf : (cy >= nf ? cy - nf : cy);
-        cz = cz < 0 ? cz + nf : (cz >= nf ? cz - nf : cz);
-        wc[c] = w[Lf.idx(cx, cy, cz)];
-    }
-    for (int D = 0; D < 27; D++) {
-        const int Dx = D % 3 - 1, Dy = D / 3 % 3 - 1, Dz = D / 9 - 1;
-        float S[9];
-#pragma unroll
-        for (int k = 0; k < 9; k++) S[k] = 0.f;
-#pragma unroll
-        for (int c = 0; c < 64; c++) {
-            // cell offset o from 2V per axis (-2..1): G[c][D] is zero unless the cell also touches the
-            // support of V + D, i.e. o >= 0 where D is +1 and o < 0 where D is -1 (a wave-uniform test:
-            // 8 to 64 of the 64 cells per direction, 512 of 1728 in all)
-            const int ox = (c & 3) - 2, oy = ((c >> 2) & 3) - 2, oz = (c >> 4) - 2;
-            if ((Dx > 0 && ox < 0) || (Dx < 0 && ox >= 0) || (Dy > 0 && oy < 0) || (Dy < 0 && oy >= 0) ||
-                (Dz > 0 && oz < 0) || (Dz < 0 && oz >= 0))
-                continue;
-            const float* g = G + (c * 27 + D) * 9;
-#pragma unroll
-            for (int k = 0; k < 9; k++) S[k] = fmaf(wc[c], g[k], S[k]);
-        }
-        if (D == 13) {
-            if (fabsf(S[0]) < clamp) S[0] = clamp;
-            if (fabsf(S[4]) < clamp) S[4] = clamp;
-            if (fabsf(S[8]) < clamp) S[8] = clamp;
-        }
-#pragma unroll
-        for (int k = 0; k < 9; k++) StencilIO<SO>::put(stc, Nc, V, D * 9 + k, S[k]);
-    }
-}
-
-// Level-1 stencil of the 27 coarse vertices around the pinned origin: node pairs touching the
-// origin contribute identity when they are the same node and nothing otherwise.
-template <typename SO>
-__global__ void k_galerkin_fine_pin(Lay Lf, Lay Lc, const float* __restrict__ ke, const float* __restrict__ w,
-                                    SO* __restrict__ stc, float clamp) {
-    const int nf = Lf.n, nc = Lc.n;
-    const size_t Nc = (size_t)nc * nc * nc;
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;  // (t%3-1, t/3%3-1, t/9-1) around the origin
-    if (t >= 27 * 27) return;
-    const int vi = t / 27, D = t % 27;
-    const int X = (vi % 3) - 1, Y = (vi / 3 % 3) - 1, Z = (vi / 9) - 1;
-    const int Dx = D % 3 - 1, Dy = D / 3 % 3 - 1, Dz = D / 9 - 1;
-    float S[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-    for (int c = 0; c < 64; c++) {
-        const int ox = (c & 3) - 2, oy = ((c >> 2) & 3) - 2, oz = (c >> 4) - 2;  // cell offset from 2V
-        // only the cells in the supports of both V and V + D contribute (as in k_galerkin_fine)
-        if ((Dx > 0 && ox < 0) || (Dx < 0 && ox >= 0) || (Dy > 0 && oy < 0) || (Dy < 0 && oy >= 0) ||
-            (Dz > 0 && oz < 0) || (Dz < 0 && oz >= 0))
-            continue;
-        int cx = 2 * X + ox, cy = 2 * Y + oy, cz = 2 * Z + oz;
-        const int cxw = (cx % nf + nf) % nf, cyw = (cy % nf + nf) % nf, czw = (cz % nf + nf) % nf;
-        const float we = w[Lf.idx(cxw, cyw, czw)];
-        for (int a = 0; a < 8; a++) {
-            const int ax = ox + (a & 1), ay = oy + ((a >> 1) & 1), az = oz + (a >> 2);
-            const float wa = hat(ax) * hat(ay) * hat(az);
-            if (wa == 0.f) continue;
-            const bool pa = ((cx + (a & 1)) % nf == 0) && ((cy + ((a >> 1) & 1)) % nf == 0) &&
-                            ((cz + (a >> 2)) % nf == 0);
-            for (int b = 0; b < 8; b++) {
-                const int bx = ox + (b & 1) - 2 * Dx, by = oy + ((b >> 1) & 1) - 2 * Dy, bz = oz + (b >> 2) - 2 * Dz;
-                const float wb = hat(bx) * hat(by) * hat(bz);
-                if (wb == 0.f) continue;
-                const bool pb = ((cx + (b & 1)) % nf == 0) && ((cy + ((b >> 1) & 1)) % nf == 0) &&
-                                ((cz + (b >> 2)) % nf == 0);
-                if (pa || pb) {
-                    if (a == b) {
-                        S[0] += wa * wb;
-                        S[4] += wa * wb;
-                        S[8] += wa * wb;
-                    }
-                } else {
-                    for (int i = 0; i < 3; i++)
-                        for (int j = 0; j < 3; j++) S[i * 3 + j] += wa * wb * we * ke[(3 * a + i) * 24 + 3 * b + j];
-                }
-            }
-        }
-    }
-    if (D == 13) {
-        if (fabsf(S[0]) < clamp) S[0] = clamp;
-        if (fabsf(S[4]) < clamp) S[4] = clamp;
-        if (fabsf(S[8]) < clamp) S[8] = clamp;
-    }
-    const uint32_t V = Lc.idx((X + nc) % nc, (Y + nc) % nc, (Z + nc) % nc);
-    for (int k = 0; k < 9; k++) StencilIO<SO>::put(stc, Nc, V, D * 9 + k, S[k]);
-}
-
-// Coarser stencil from a stored one: st_c[V][D] = sum_{o,d} hat(o) A_f[2V+o][d] hat3(o+d-2D).
-// One thread per coarse vertex and plane Dz (blockIdx.y): every fine block (o, d) is read once and
-// added into the nine directions (Dx, Dy) of the plane it reaches, with the weights hat3(o + d - 2D).
-template <typename SI, typename SO>
-__global__ __launch_bounds__(256) void k_galerkin_coarse(Lay Lf, Lay Lc, const SI* __restrict__ stf,
-                                                         SO* __restrict__ stc, float clamp) {
-    const int nf = Lf.n;
-    const size_t Nc = (size_t)Lc.n * Lc.n * Lc.n, Nf = (size_t)nf * nf * nf;
-    int X, Y, Z;
-    uint32_t V;
-    if (!coarse_lex_vertex(Lc, X, Y, Z, V)) return;
-    const uint32_t xs[3] = {Lf.part(wrap_dec(2 * X, nf), 0), Lf.part(2 * X, 0), Lf.part(2 * X + 1, 0)};
-    const uint32_t ys[3] = {Lf.part(wrap_dec(2 * Y, nf), 1), Lf.part(2 * Y, 1), Lf.part(2 * Y + 1, 1)};
-    const uint32_t zs[3] = {Lf.part(wrap_dec(2 * Z, nf), 2), Lf.part(2 * Z, 2), Lf.part(2 * Z + 1, 2)};
-    const Rsrc rf = make_rsrc(stf, (size_t)StencilIO<SI>::words * Nf * 4);
-    const int Dz = (int)blockIdx.y - 1;
-    float S[9][9];  // [(Dy + 1) * 3 + Dx + 1][entry]
-#pragma unroll
-    for (int j = 0; j < 9; j++)
-#pragma unroll
-        for (int k = 0; k < 9; k++) S[j][k] = 0.f;
-    for (int o = 0; o < 27; o++) {
-        const int ox = o % 3 - 1, oy = o / 3 % 3 - 1, oz = o / 9 - 1;
-        const float wo = hat(ox) * hat(oy) * hat(oz);
-        const uint32_t vf = xs[ox + 1] + ys[oy + 1] + zs[oz + 1];
-        for (int d = 0; d < 27; d++) {
-            const int kx = ox + d % 3 - 1, ky = oy + d / 3 % 3 - 1, kz = oz + d / 9 - 1;
-            const float wz = wo * hat(kz - 2 * Dz);
-            if (wz == 0.f) continue;
-            float e[9];
-#pragma unroll
-            for (int k = 0; k < 9; k++) e[k] = StencilIO<SI>::get(rf, vf * 4u, (uint32_t)(Nf * 4), d * 9 + k);
-#pragma unroll
-            for (int j = 0; j < 9; j++) {
-                // o and d are the same for the whole wave, so is wj: about two of the nine coarse
-                // directions (Dx, Dy) get a non-zero weight from a fine pair
-                const float wj = wz * hat(ky - 2 * (j / 3 - 1)) * hat(kx - 2 * (j % 3 - 1));
-                if (wj == 0.f) continue;
-#pragma unroll
-                for (int k = 0; k < 9; k++) S[j][k] = fmaf(wj, e[k], S[j][k]);
-            }
-        }
-    }
-    if (Dz == 0) {
-        if (fabsf(S[4][0]) < clamp) S[4][0] = clamp;
-        if (fabsf(S[4][4]) < clamp) S[4][4] = clamp;
-        if (fabsf(S[4][8]) < clamp) S[4][8] = clamp;
-    }
-#pragma unroll
-    for (int j = 0; j < 9; j++)
-#pragma unroll
-        for (int k = 0; k < 9; k++) StencilIO<SO>::put(stc, Nc, V, ((Dz + 1) * 9 + j) * 9 + k, S[j][k]);
-}
-
-// ---------------------------------------------------------------------------------------------
-// Coarsest level: FP64 dense solve u = A^{-1} f with the inverse formed from a Cholesky
-// factorisation of the pinned Galerkin system (replaces the host BiCGSTAB of grid.cpp:349-374).
-// One block per load case; dof order 3*v + i.
-// ---------------------------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_coarse_solve(int m, size_t Nc, const double* __restrict__ Ainv,
-                                                      const float* __restrict__ f, float* __restrict__ u) {
-    extern __shared__ double fb[];
-    const int r = blockIdx.x;
-    for (int k = threadIdx.x; k < m; k += blockDim.x) {
-        const int v = k / 3, i = k % 3;
-        fb[k] = (double)f[(size_t)(r * 3 + i) * Nc + v];
-    }
-    __syncthreads();
-    for (int row = threadIdx.x; row < m; row += blockDim.x) {
-        double s = 0.0;
-        const double* a = Ainv + (size_t)row * m;
-        for (int k = 0; k < m; k++) s = fma(a[k], fb[k], s);
-        const int v = row / 3, i = row % 3;
-        u[(size_t)(r * 3 + i) * Nc + v] = (float)s;
-    }
-}
-
-// ---------------------------------------------------------------------------------------------
-// Coarsest level: its dense FP64 operator factorised and inverted on the GPU (the reference does it
-// on the host, grid.cpp:349-424).  m = 3 n_c^3 <= 1029 (n_c = 4..7); A and T are m x m, row-major.
-// ---------------------------------------------------------------------------------------------
-
-__global__ __launch_bounds__(256) void k_fill64(size_t n, double v, double* __restrict__ a) {
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) a[i] = v;
-}
-
-// A += the coarsest stencil (lexicographic level; entry k = 9d + 3i + j of vertex v couples (v, i) with
-// (v + d, j)), one thread per row, so neighbours that coincide on the periodic grid add up.
-__global__ __launch_bounds__(256) void k_coarse_assemble(int nc, const float* __restrict__ st, double* __restrict__ A) {
-    const int Nc = nc * nc * nc, m = 3 * Nc;
-    const int row = blockIdx.x * blockDim.x + threadIdx.x;
-    if (row >= m) return;
-    const int v = row / 3, i = row % 3;
-    const int x0 = v % nc, y0 = (v / nc) % nc, z0 = v / (nc * nc);
-    double* a = A + (size_t)row * m;
-    for (int d = 0; d < 27; d++) {
-        const int xq = (x0 + d % 3 - 1 + nc) % nc, yq = (y0 + d / 3 % 3 - 1 + nc) % nc, zq = (z0 + d / 9 - 1 + nc) % nc;
-        const int q = xq + nc * (yq + nc * zq);
-        for (int j = 0; j < 3; j++) a[3 * q + j] += (double)st[(size_t)(d * 9 + i * 3 + j) * Nc + v];
-    }
-}
-
-// A = (A + A^T) / 2, one thread per pair i < j
-__global__ __launch_bounds__(256) void k_symmetrize64(int m, double* __restrict__ A) {
-    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (size_t)m * m) return;
-    const int i = (int)(t / m), j = (int)(t % m);
-    if (j <= i) return;
-    const double s = 0.5 * (A[(size_t)i * m + j] + A[(size_t)j * m + i]);
-    A[(size_t)i * m + j] = s;
-    A[(size_t)j * m + i] = s;
-}
-
-// In-place inverse of the symmetric positive definite A by Gauss-Jordan elimination on the diagonal,
-// one launch per step k over the whole matrix (one thread per element).  With p = A[k][k] (the k-th
-// Schur complement's leading entry: positive exactly when A is positive definite, the square of the
-// Cholesky pivot):
-//   A[k][j] /= p (j != k), A[k][k] = 1 / p, A[i][k] = -A[i][k] / p (i != k),
-//   A[i][j] -= A[i][k] A[k][j] / p (i, j != k).
-// Step k reads its pivot row and column from prow / pcol (their values before step k) and writes the
-// new row and column k + 1 to nrow / ncol for the next step, so no launch reads what it writes.
-// status = 0, or 1 + the first k whose pivot is not positive (every block reads the same pivot and
-// stops; later steps see the status and do nothing).
-__global__ __launch_bounds__(256) void k_gj_pivot0(int m, const double* __restrict__ A, double* __restrict__ prow,
-                                                   double* __restrict__ pcol, int* __restrict__ status) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t == 0) *status = 0;
-    if (t < m) {
-        prow[t] = A[t];
-        pcol[t] = A[(size_t)t * m];
-    }
-}
-
-__global__ __launch_bounds__(256) void k_gj_step64(int m, int k, double* __restrict__ A,
-                                                   const double* __restrict__ prow, const double* __restrict__ pcol,
-                                                   double* __restrict__ nrow, double* __restrict__ ncol,
-                                                   int* __restrict__ status) {
-    if (*status != 0) return;
-    const double piv = prow[k];
-    if (!(piv > 0.0)) {
-        if (blockIdx.x == 0 && threadIdx.x == 0) *status = 1 + k;
-        return;
-    }
-    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (size_t)m * m) return;
-    const int i = (int)(t / m), j = (int)(t - (size_t)i * m);
-    const double inv = 1.0 / piv;
-    const double rj = (j == k ? 1.0 : prow[j]) * inv;
-    const double v = i == k ? rj : (j == k ? -pcol[i] * inv : fma(-pcol[i], rj, A[t]));
-    A[t] = v;
-    if (i == k + 1) nrow[j] = v;
-    if (j == k + 1) ncol[i] = v;
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -3132,62 +2823,6 @@ void launch_prolong(hipStream_t s, int nf, int lexc, const void* uc, int uc_half
     else
         hipLaunchKernelGGL((k_prolong<1>), dim3(full_grid(Lf), 6), dim3(kFullThreads), 0, s, Lf, Lc,
                            static_cast<const float*>(uc), static_cast<float*>(uf), pin);
-}
-
-void launch_galerkin_fine(hipStream_t s, int nf, int lexc, const float* G, const float* ke, const float* w, void* stc,
-                          int out_half, float clamp) {
-    const size_t Nc = (size_t)(nf / 2) * (nf / 2) * (nf / 2);
-    const Lay Lf = make_lay(nf, 0), Lc = make_lay(nf / 2, lexc);
-    if (out_half) {
-        half2_t* o = static_cast<half2_t*>(stc);
-        hipLaunchKernelGGL(k_galerkin_fine<half2_t>, dim3(nblk(Nc)), dim3(256), 0, s, Lf, Lc, G, w, o, clamp);
-        hipLaunchKernelGGL(k_galerkin_fine_pin<half2_t>, dim3(nblk(27 * 27)), dim3(256), 0, s, Lf, Lc, ke, w, o, clamp);
-    } else {
-        float* o = static_cast<float*>(stc);
-        hipLaunchKernelGGL(k_galerkin_fine<float>, dim3(nblk(Nc)), dim3(256), 0, s, Lf, Lc, G, w, o, clamp);
-        hipLaunchKernelGGL(k_galerkin_fine_pin<float>, dim3(nblk(27 * 27)), dim3(256), 0, s, Lf, Lc, ke, w, o, clamp);
-    }
-}
-
-template <typename SI, typename SO>
-static void galerkin_coarse_case(hipStream_t s, const Lay& Lf, const Lay& Lc, const void* stf, void* stc, float clamp) {
-    const size_t Nc = (size_t)Lc.n * Lc.n * Lc.n;
-    hipLaunchKernelGGL((k_galerkin_coarse<SI, SO>), dim3(nblk(Nc), 3), dim3(256), 0, s, Lf, Lc,
-                       static_cast<const SI*>(stf), static_cast<SO*>(stc), clamp);
-}
-
-void launch_galerkin_coarse(hipStream_t s, int nf, int lexc, const void* stf, int in_half, void* stc, int out_half,
-                            float clamp) {
-    const Lay Lf = make_lay(nf, 0), Lc = make_lay(nf / 2, lexc);
-    if (in_half && out_half)
-        galerkin_coarse_case<half2_t, half2_t>(s, Lf, Lc, stf, stc, clamp);
-    else if (in_half)
-        galerkin_coarse_case<half2_t, float>(s, Lf, Lc, stf, stc, clamp);
-    else if (out_half)
-        galerkin_coarse_case<float, half2_t>(s, Lf, Lc, stf, stc, clamp);
-    else
-        galerkin_coarse_case<float, float>(s, Lf, Lc, stf, stc, clamp);
-}
-
-void launch_coarse_solve(hipStream_t s, int nc, const double* Ainv, const float* f, float* u) {
-    const size_t Nc = (size_t)nc * nc * nc;
-    const int m = (int)(3 * Nc);
-    hipLaunchKernelGGL(k_coarse_solve, dim3(6), dim3(256), sizeof(double) * m, s, m, Nc, Ainv, f, u);
-}
-
-void launch_coarse_factor(hipStream_t s, int nc, const float* st, double* ainv, double* piv, int* status) {
-    const int m = 3 * nc * nc * nc;
-    const size_t mm = (size_t)m * m;
-    hipLaunchKernelGGL(k_fill64, dim3(nblk(mm) < 1024 ? nblk(mm) : 1024), dim3(256), 0, s, mm, 0.0, ainv);
-    hipLaunchKernelGGL(k_coarse_assemble, dim3(nblk((size_t)m)), dim3(256), 0, s, nc, st, ainv);
-    hipLaunchKernelGGL(k_symmetrize64, dim3(nblk(mm)), dim3(256), 0, s, m, ainv);
-    // pivot rows and columns, double-buffered: piv = [row 0 | col 0 | row 1 | col 1], m values each
-    double* row[2] = {piv, piv + 2 * (size_t)m};
-    double* col[2] = {piv + m, piv + 3 * (size_t)m};
-    hipLaunchKernelGGL(k_gj_pivot0, dim3(nblk((size_t)m)), dim3(256), 0, s, m, ainv, row[0], col[0], status);
-    for (int k = 0; k < m; k++)
-        hipLaunchKernelGGL(k_gj_step64, dim3(nblk(mm)), dim3(256), 0, s, m, k, ainv, row[k & 1], col[k & 1],
-                           row[(k + 1) & 1], col[(k + 1) & 1], status);
 }
 
 void launch_dot6(hipStream_t s, size_t M, const float* a, const float* b, double* partial, int nblocks,

@@ -79,6 +79,54 @@ __device__ __forceinline__ float bload<float>(Rsrc r, uint32_t voff, uint32_t so
     return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, (int)voff, (int)soff, 0));
 }
 
+// Packed FP16 storage of a 6-load-case field: word plane (p * 3 + i) holds components i of load cases
+// 2p (.x) and 2p + 1 (.y), so a neighbour of all six load cases is 9 32-bit words.
+typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+template <>
+__device__ __forceinline__ half2_t bload<half2_t>(Rsrc r, uint32_t voff, uint32_t soff) {
+    return __builtin_bit_cast(half2_t, __builtin_amdgcn_raw_buffer_load_b32(r, (int)voff, (int)soff, 0));
+}
+
+// A stored coarse stencil: FP32 entries [243][N] (entry e = 9d + 3i + j), or packed FP16 [122][N]
+// words, word w holding entries 2w (.x) and 2w + 1 (.y).  Both have 4-byte words per vertex.
+template <typename SA>
+struct StencilIO;
+template <>
+struct StencilIO<float> {
+    static constexpr int words = 243;
+    __device__ static float get(Rsrc rs, uint32_t vo, uint32_t plane, int e) {
+        return bload<float>(rs, vo, (uint32_t)e * plane);
+    }
+    __device__ static void put(float* st, size_t N, uint32_t v, int e, float val) { st[(size_t)e * N + v] = val; }
+};
+template <>
+struct StencilIO<half2_t> {
+    static constexpr int words = 122;
+    __device__ static float get(Rsrc rs, uint32_t vo, uint32_t plane, int e) {
+        return (float)bload<half2_t>(rs, vo, (uint32_t)(e >> 1) * plane)[e & 1];
+    }
+    // one 16-bit store per entry: the two halves of a word may come from different threads
+    __device__ static void put(half2_t* st, size_t N, uint32_t v, int e, float val) {
+        reinterpret_cast<_Float16*>(st + (size_t)(e >> 1) * N + v)[e & 1] = (_Float16)val;
+    }
+};
+
+// Coarse-vertex kernels that read the fine level around 2V take coarse vertices in lexicographic
+// order whatever the coarse storage, so that consecutive lanes read consecutive fine local positions.
+__device__ __forceinline__ bool coarse_lex_vertex(const Lay& Lc, int& X, int& Y, int& Z, uint32_t& V) {
+    const uint32_t i = xcd_chunk(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+    const uint32_t n = (uint32_t)Lc.n;
+    if (i >= n * n * n) return false;
+    X = (int)(i % n);
+    Y = (int)((i / n) % n);
+    Z = (int)(i / (n * n));
+    V = Lc.idx(X, Y, Z);
+    return true;
+}
+
+// weight of fine offset o in the 1-D prolongation
+__device__ __forceinline__ float hat(int o) { return o == 0 ? 1.f : ((o == 1 || o == -1) ? 0.5f : 0.f); }
+
 template <int BS>
 __device__ __forceinline__ double block_sum(double v, double* sh) {
 #pragma unroll
