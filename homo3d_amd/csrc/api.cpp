@@ -39,6 +39,7 @@ struct Level {
     float* r = nullptr;
     void* st = nullptr;   // levels >= 1: FP32 [243][N], or packed FP16 [122][N] words when st_half
     int st_half = 0;
+    void* quads = nullptr;  // small levels: the stencil again, in quads (launch_stencil_quads)
 };
 
 struct ProfEvent {
@@ -358,6 +359,10 @@ bool op_smooth(homo3d_handle* h, int l, void* u, const float* f, float omega, in
         if (dot) launch_sum_partials(h->stream, kRhs, 4 * G, h->d_partial, dot_out);
         return dot;
     }
+    if (l > 0 && !u_half && L.quads) {
+        launch_plane_sweep(h->stream, L.n, omega, reverse, zs, L.quads, static_cast<float*>(u), f);
+        return false;
+    }
     if (l > 0 && stencil_gs_pairs_ok(L.n, L.lex)) {  // colours two at a time (same result as one by one)
         for (int cc = 0; cc < 8; cc += 2)
             launch_stencil_gs2(h->stream, L.n, reverse ? 7 - cc : cc, omega, reverse, zs, L.st, L.st_half, u, u_half, f,
@@ -445,7 +450,10 @@ int vcycle(homo3d_handle* h, void* u0, const float* f0, int symmetric, double* r
         if (l == 0) return u0_half;
         return u0_half && l < h->nl - 1 && stencil_u_half_ok(h->lv[l].n, h->lv[l].lex) ? 1 : 0;
     };
-    for (int l = 0; l < h->nl - 1; l++) {
+    // the last smoothed level and the coarsest in one go, where the level is small enough (and not the finest)
+    const int lt = h->nl - 2;
+    const bool tail = lt > 0 && vcycle_tail_ok(h->lv[lt].n, h->lv[lt].lex, h->lv[lt].st_half);
+    for (int l = 0; l < (tail ? lt : lt + 1); l++) {
         Level& L = h->lv[l];
         void* u = l == 0 ? u0 : L.u;
         const float* f = l == 0 ? f0 : L.f;
@@ -467,8 +475,14 @@ int vcycle(homo3d_handle* h, void* u0, const float* f0, int symmetric, double* r
     const Level& Lc = h->lv[h->nl - 1];
     int rc = coarse_factor(h);
     if (rc) return rc;
-    launch_coarse_solve(h->stream, Lc.n, h->d_Ainv, Lc.f, Lc.u);
-    for (int l = h->nl - 2; l >= 0; l--) {
+    if (tail) {
+        const Level& L = h->lv[lt];
+        launch_vcycle_tail(h->stream, L.n, omega, symmetric ? 1 : 0, L.quads, L.u, L.f, L.r, Lc.u, Lc.f,
+                           h->d_Ainv);
+    } else {
+        launch_coarse_solve(h->stream, Lc.n, h->d_Ainv, Lc.f, Lc.u);
+    }
+    for (int l = tail ? lt - 1 : lt; l >= 0; l--) {
         Level& L = h->lv[l];
         void* u = l == 0 ? u0 : L.u;
         const float* f = l == 0 ? f0 : L.f;
@@ -753,6 +767,8 @@ int homo3d_create(const homo3d_config* cfg, homo3d_handle** out) {
         if (l > 0) {
             L.st_half = cfg->coarse_half && l < nl - 1 ? 1 : 0;  // the coarsest stays FP32 for the dense solve
             if (hipMalloc(&L.st, sizeof(uint32_t) * (L.st_half ? 122 : 243) * L.N)) return fail(HOMO3D_HIP_ERROR);
+            if (small_level_ok(L.n, L.lex, L.st_half) && hipMalloc(&L.quads, stencil_quads_bytes(L.n)))
+                return fail(HOMO3D_HIP_ERROR);
         }
     }
     const size_t N0 = h->lv[0].N, vb = sizeof(float) * 3 * kRhs * N0;
@@ -859,6 +875,7 @@ int homo3d_destroy(homo3d_handle* h) {
         (void)hipFree(h->lv[l].f);
         (void)hipFree(h->lv[l].r);
         (void)hipFree(h->lv[l].st);
+        (void)hipFree(h->lv[l].quads);
     }
     void* ptrs[] = {h->d_x, h->U64, h->d_ke64, h->d_kchi64, h->d_ke, h->d_ke16, h->d_kchi, h->d_G, h->d_G32, h->d_w, h->d_stage, h->d_Ainv, h->d_cstat, h->d_cwork, h->X, h->F, h->P, h->Q, h->Z,
                     h->Rr, h->d_partial, h->d_sc, h->d_tmp, h->d_ftmp, h->d_gperm, h->d_gflip};
@@ -906,6 +923,8 @@ int homo3d_update_density(homo3d_handle* h, const float* x, int pitch, int on_de
     for (int l = 2; l < h->nl; l++)
         launch_galerkin_coarse(h->stream, h->lv[l - 1].n, h->lv[l].lex, h->lv[l - 1].st, h->lv[l - 1].st_half,
                                h->lv[l].st, h->lv[l].st_half, reinterpret_cast<double*>(h->P), clamp);
+    for (int l = 1; l < h->nl; l++)
+        if (h->lv[l].quads) launch_stencil_quads(h->stream, h->lv[l].n, h->lv[l].st, h->lv[l].quads);
     // coarsest dense system: assembled and inverted on the GPU; its status is read at the
     // first coarse solve (coarse_factor)
     const Level& Lc = h->lv[h->nl - 1];

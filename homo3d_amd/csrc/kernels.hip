@@ -39,32 +39,6 @@ __device__ __forceinline__ void bstore(float v, Rsrc r, uint32_t voff, uint32_t 
     __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), r, (int)voff, (int)soff, 0);
 }
 
-// load cases per stored word of a field type
-template <typename A>
-struct CasesPerWord {
-    static constexpr int value = 1;
-};
-template <>
-struct CasesPerWord<half2_t> {
-    static constexpr int value = 2;
-};
-
-// Packed FP16 six-load-case fields (half2_t words): word q = p * 3 + i of vertex v (component i of load
-// cases 2p (.x) and 2p + 1 (.y)) is word hw_index(q, v, N) of the field.  Words 0-3 and 4-7 form two
-// planes of 16-byte quads and word 8 a plane of single words, so the nine words of a vertex are two
-// 16-byte loads and one 4-byte load: a 27-neighbour gather costs the texture addresser per load
-// instruction, not per byte (nine 4-byte loads per neighbour take about four times as long).
-__host__ __device__ __forceinline__ size_t hw_index(int q, size_t v, size_t N) {
-    return q < 8 ? (size_t)(q >> 2) * 4 * N + 4 * v + (size_t)(q & 3) : 8 * N + v;
-}
-// word q of vertex v in a field of A words: packed FP16 as above, FP32 planes q * N + v
-template <typename A>
-__device__ __forceinline__ size_t fw_index(int q, size_t v, size_t N) {
-    if constexpr (CasesPerWord<A>::value == 2)
-        return hw_index(q, v, N);
-    else
-        return (size_t)q * N + v;
-}
 // the nine words of vertex idx of a packed FP16 field through a buffer resource over it (plane = 4 N
 // bytes; the byte offsets stay below 36 N)
 __device__ __forceinline__ void hload9(uint32_t (&wv)[9], Rsrc r, uint32_t idx, uint32_t plane) {
@@ -391,23 +365,6 @@ __device__ __forceinline__ void stage_ke(T* ke_s, const T* __restrict__ ke) {
         ke_s[kBlockConsts + t] = ke_s[(3 * (7 - e0) + i) * 24 + 3 * b0 + j];
     }
     __syncthreads();
-}
-
-// Block Gauss-Seidel / SOR update of one vertex: x, y, z in turn (z, y, x when REVERSE)
-// (gs_relaxation_otf_kernel update formula, grid.cu:530-541).
-// inv holds 1 / Ks[0], 1 / Ks[4], 1 / Ks[8] (shared by all load cases of the vertex).
-template <bool REVERSE>
-__device__ __forceinline__ void block_update(float u[3], const float f[3], const float KeU[3], const float Ks[9],
-                                             const float inv[3], float omega) {
-    if (!REVERSE) {
-        u[0] = omega * (f[0] - KeU[0] - Ks[1] * u[1] - Ks[2] * u[2]) * inv[0] + (1.f - omega) * u[0];
-        u[1] = omega * (f[1] - KeU[1] - Ks[3] * u[0] - Ks[5] * u[2]) * inv[1] + (1.f - omega) * u[1];
-        u[2] = omega * (f[2] - KeU[2] - Ks[6] * u[0] - Ks[7] * u[1]) * inv[2] + (1.f - omega) * u[2];
-    } else {
-        u[2] = omega * (f[2] - KeU[2] - Ks[6] * u[0] - Ks[7] * u[1]) * inv[2] + (1.f - omega) * u[2];
-        u[1] = omega * (f[1] - KeU[1] - Ks[3] * u[0] - Ks[5] * u[2]) * inv[1] + (1.f - omega) * u[1];
-        u[0] = omega * (f[0] - KeU[0] - Ks[1] * u[1] - Ks[2] * u[2]) * inv[0] + (1.f - omega) * u[0];
-    }
 }
 
 // GS colour c covers the vertices with coordinate parity (1-c&1, 1-c>>1&1, 1-c>>2): the reference

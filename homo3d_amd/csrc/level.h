@@ -87,6 +87,33 @@ __device__ __forceinline__ half2_t bload<half2_t>(Rsrc r, uint32_t voff, uint32_
     return __builtin_bit_cast(half2_t, __builtin_amdgcn_raw_buffer_load_b32(r, (int)voff, (int)soff, 0));
 }
 
+// load cases per stored word of a field type
+template <typename A>
+struct CasesPerWord {
+    static constexpr int value = 1;
+};
+template <>
+struct CasesPerWord<half2_t> {
+    static constexpr int value = 2;
+};
+
+// Packed FP16 six-load-case fields (half2_t words): word q = p * 3 + i of vertex v (component i of load
+// cases 2p (.x) and 2p + 1 (.y)) is word hw_index(q, v, N) of the field.  Words 0-3 and 4-7 form two
+// planes of 16-byte quads and word 8 a plane of single words, so the nine words of a vertex are two
+// 16-byte loads and one 4-byte load: a 27-neighbour gather costs the texture addresser per load
+// instruction, not per byte (nine 4-byte loads per neighbour take about four times as long).
+__host__ __device__ __forceinline__ size_t hw_index(int q, size_t v, size_t N) {
+    return q < 8 ? (size_t)(q >> 2) * 4 * N + 4 * v + (size_t)(q & 3) : 8 * N + v;
+}
+// word q of vertex v in a field of A words: packed FP16 as above, FP32 planes q * N + v
+template <typename A>
+__device__ __forceinline__ size_t fw_index(int q, size_t v, size_t N) {
+    if constexpr (CasesPerWord<A>::value == 2)
+        return hw_index(q, v, N);
+    else
+        return (size_t)q * N + v;
+}
+
 // A stored coarse stencil: FP32 entries [243][N] (entry e = 9d + 3i + j), or packed FP16 [122][N]
 // words, word w holding entries 2w (.x) and 2w + 1 (.y).  Both have 4-byte words per vertex.
 template <typename SA>
@@ -126,6 +153,23 @@ __device__ __forceinline__ bool coarse_lex_vertex(const Lay& Lc, int& X, int& Y,
 
 // weight of fine offset o in the 1-D prolongation
 __device__ __forceinline__ float hat(int o) { return o == 0 ? 1.f : ((o == 1 || o == -1) ? 0.5f : 0.f); }
+
+// Block Gauss-Seidel / SOR update of one vertex: x, y, z in turn (z, y, x when REVERSE)
+// (gs_relaxation_otf_kernel update formula, grid.cu:530-541).
+// inv holds 1 / Ks[0], 1 / Ks[4], 1 / Ks[8] (shared by all load cases of the vertex).
+template <bool REVERSE>
+__device__ __forceinline__ void block_update(float u[3], const float f[3], const float KeU[3], const float Ks[9],
+                                             const float inv[3], float omega) {
+    if (!REVERSE) {
+        u[0] = omega * (f[0] - KeU[0] - Ks[1] * u[1] - Ks[2] * u[2]) * inv[0] + (1.f - omega) * u[0];
+        u[1] = omega * (f[1] - KeU[1] - Ks[3] * u[0] - Ks[5] * u[2]) * inv[1] + (1.f - omega) * u[1];
+        u[2] = omega * (f[2] - KeU[2] - Ks[6] * u[0] - Ks[7] * u[1]) * inv[2] + (1.f - omega) * u[2];
+    } else {
+        u[2] = omega * (f[2] - KeU[2] - Ks[6] * u[0] - Ks[7] * u[1]) * inv[2] + (1.f - omega) * u[2];
+        u[1] = omega * (f[1] - KeU[1] - Ks[3] * u[0] - Ks[5] * u[2]) * inv[1] + (1.f - omega) * u[1];
+        u[0] = omega * (f[0] - KeU[0] - Ks[1] * u[1] - Ks[2] * u[2]) * inv[0] + (1.f - omega) * u[0];
+    }
+}
 
 template <int BS>
 __device__ __forceinline__ double block_sum(double v, double* sh) {
