@@ -22,10 +22,8 @@
 //       A = weights (16 output channels x 32 of (t, ci)), B = the 16 voxels' shifted inputs.  The input
 //       gradient is the same pass over dZ with the flipped, transposed weights Wb[ci][t][co] = W[co][26-t][ci].
 //   weight gradient (k_wgrad):  dW[co][t][ci] = sum_v dZ[v][co] X[v + d_t][ci]
-//       the reduction runs over voxels, so dZ and X are first transposed to channel-major rows with
-//       X in three x-shifted copies (k_to_cm); a lane's 8 voxels are then one aligned 16-byte load for
-//       every tap (y and z shifts move whole rows).  Split over voxel ranges, partial sums reduced
-//       after (k_wgrad_reduce): deterministic, no atomics.
+//       the reduction runs over voxels: tiles of dZ and X staged in LDS are read transposed.  Split over
+//       voxel ranges, partial sums reduced after (k_wgrad_reduce): deterministic, no atomics.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -52,7 +50,6 @@ constexpr int kInCh = 8;      // stored input channels (density + 7 zeros): the 
 constexpr int kPld = 24;      // row stride of the FP32 prediction
 constexpr int kDpLd = 32;     // row stride of the head's output gradient (18 used, zeros after)
 constexpr int kDpC = 24;      // channels of it read by the head's input-gradient pass (multiple of 8)
-constexpr int kWgChunks = 32; // 32-voxel chunks per wave in the weight gradient
 
 __device__ __forceinline__ bf16x8 load8(const uint16_t* p) {
     return __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(p));
@@ -161,86 +158,186 @@ __global__ __launch_bounds__(256) void k_conv(const uint16_t* __restrict__ in, i
     }
 }
 
-// Channel-major copy for the weight gradient: out[s][c][v] = in[v with x -> x + s + s0 - 1][c] for
-// slots s < ns, c < cp (zeros for c >= C).  One thread per voxel.
-__global__ __launch_bounds__(256) void k_to_cm(const uint16_t* __restrict__ in, int ldi, int C, int cp, int lg,
-                                               long nvox, int s0, int ns, uint16_t* __restrict__ out) {
-    const long v = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= nvox) return;
-    const int m = (1 << lg) - 1;
-    const int x = (int)(v & m);
-    for (int s = 0; s < ns; s++) {
-        const int dx = s + s0 - 1;
-        const long src = (v - x) + ((x + dx) & m);
-        for (int c = 0; c < cp; c++) out[((long)s * cp + c) * nvox + v] = c < C ? in[src * ldi + c] : (uint16_t)0;
-    }
+// ---------------------------------------------------------------------------------------------------
+// Weight gradient.  A block stages a tile of TX x TY x TZ voxels in LDS, 16 input channels of X with one row
+// more on each side in y and z, and 16 WC output channels of dZ with one voxel more on each side in x, both
+// as they lie in memory (a voxel's 16 channels are 32 bytes).  The tap (dx, dy, dz) pairs X at v + (dy, dz)
+// with dZ at v - dx, so a tile's 27 products need 9 X and 3 dZ operands.  The reduction over voxels wants a
+// channel's voxels in one lane: the transposing LDS reads (four voxels of 16 channels to 16 lanes with a
+// channel each) give that from any voxel on, so nothing is copied to channel-major order first.  Bound by
+// the tiles' loads, X three times over with its neighbour rows.  The 15 layers of a 64^3 x 4 gradient:
+// 0.73 ms with the sums of the partials; with channel-major copies of X (three, shifted in x) and dZ
+// through memory, one wave a block on the products and a thread or a block for each sum 7.6 ms.
+// Wave w takes output channels 16 (w % WC) and every (4 / WC)th 32-voxel chunk; a block walks a range of
+// tiles, adds its waves' sums in LDS and leaves one partial; the bias gradient is a 28th product with ones.
+// ---------------------------------------------------------------------------------------------------
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+
+constexpr int kWgTapFloats = 256;  // one 16 x 16 accumulator
+
+// Lane's 8 voxels of channel lane % 16: 4 from each of two 16-voxel reads (p0, p1: the lane's 8-byte piece).
+__device__ __forceinline__ bf16x8 read_tr(const uint16_t* p0, const uint16_t* p1) {
+    typedef __attribute__((address_space(3))) s16x4 lds4;
+    const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4*)p0), b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4*)p1);
+    return __builtin_bit_cast(bf16x8, __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
 }
 
-// Weight gradient partial sums: one wave per (voxel range, 16 output channels, 16 input channels).
-// dzc: [czp][nvox] channel-major dZ; xs: [ns][cxp][nvox] (ns = 3 x-shifted copies for 3x3x3, 1 for 1x1).
-// partial[split][czp][taps][cxp].
-template <bool TAP27>
-__global__ __launch_bounds__(64) void k_wgrad(const uint16_t* __restrict__ dzc, int czp, const uint16_t* __restrict__ xs,
-                                              int cxp, int lg, long nvox, float* __restrict__ partial) {
-    constexpr int NT = TAP27 ? 27 : 1;
-    const int lane = threadIdx.x, col = lane & 15, grp = lane >> 4;
-    const int split = blockIdx.x, cb = blockIdx.y * 16, nb = blockIdx.z * 16;
+template <int TX, int TY, int TZ, bool TAP27>
+struct WgTile {
+    static constexpr int H = TAP27 ? 1 : 0;
+    static constexpr int vox = TX * TY * TZ, xvox = TX * (TY + 2 * H) * (TZ + 2 * H), zvox = (TX + 2 * H) * TY * TZ;
+    static constexpr int taps = TAP27 ? 27 : 1;
+    static size_t lds(int wc) {  // the tile, or the waves' sums on their way to one
+        const size_t t = 32 * (size_t)(xvox + wc * zvox), r = sizeof(float) * (size_t)(taps + 1) * kWgTapFloats * 2;
+        return wc < 4 && r > t ? r : t;
+    }
+};
+
+// partial: [splits][czp][taps][cxp], bpartial: [splits][czp]
+template <int TX, int TY, int TZ, bool TAP27>
+__global__ __launch_bounds__(256, 2) void k_wgrad(const uint16_t* __restrict__ dz, int ldz, int cz,
+                                                  const uint16_t* __restrict__ x, int ldx, int cx, int lg, int tiles,
+                                                  int per, int wc, int czp, int cxp, float* __restrict__ partial,
+                                                  float* __restrict__ bpartial) {
+    using W = WgTile<TX, TY, TZ, TAP27>;
+    constexpr int H = W::H, YH = TY + 2 * H, XP = TX + 2 * H, NT = W::taps;
+    extern __shared__ __attribute__((aligned(16))) uint16_t sh[];
+    uint16_t* const xs = sh;
+    uint16_t* const zs = sh + 16 * W::xvox;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int cw = wave & (wc - 1), vw = wave / wc, nvw = 4 / wc;
+    const int cb = (int)blockIdx.y * 16 * wc, nb = (int)blockIdx.z * 16;
     const int m = (1 << lg) - 1;
-    f32x4 acc[NT];
+    f32x4 acc[NT], accb = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int t = 0; t < NT; t++) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const long vbeg = (long)split * kWgChunks * 32;
-    for (int c = 0; c < kWgChunks; c++) {
-        const long v0 = vbeg + 32L * c;
-        if (v0 >= nvox) break;
-        const long vl = v0 + 8 * grp;  // the lane's 8 voxels: one x-row segment (g >= 8)
-        const bf16x8 a = load8(dzc + (long)(cb + col) * nvox + vl);
-        const long row = vl >> lg;
-        const int xseg = (int)(vl & m);
-        const int y = (int)(row & m), z = (int)((row >> lg) & m);
-        const long sb = (row >> (2 * lg)) << (2 * lg);
+    bf16x8 ones;
 #pragma unroll
-        for (int t = 0; t < NT; t++) {
-            const int dx = TAP27 ? t % 3 - 1 : 0, dy = TAP27 ? (t / 3) % 3 - 1 : 0, dz = TAP27 ? t / 9 - 1 : 0;
-            const int s = TAP27 ? dx + 1 : 0;
-            const long r2 = sb + (((long)((z + dz) & m)) << lg) + ((y + dy) & m);
-            const bf16x8 b = load8(xs + ((long)s * cxp + nb + col) * nvox + (r2 << lg) + xseg);
-            acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[t], 0, 0, 0);
+    for (int k = 0; k < 8; k++) ones[k] = (__bf16)1.0f;
+    const int tend = min(tiles, ((int)blockIdx.x + 1) * per);
+    for (int tile = (int)blockIdx.x * per; tile < tend; tile++) {
+        // first voxel of the tile (1x1: the tiles are runs of consecutive voxels)
+        int x0 = 0, y0 = 0, z0 = 0;
+        long base = (long)tile * W::vox;
+        if (TAP27) {
+            const int nx = (1 << lg) / TX, ny = (1 << lg) / TY, nz = (1 << lg) / TZ;
+            x0 = tile % nx * TX;
+            y0 = tile / nx % ny * TY;
+            z0 = tile / (nx * ny) % nz * TZ;
+            base = (long)(tile / (nx * ny * nz)) << (3 * lg);
+        }
+        auto voxel = [&](int xx, int yy, int zz) {  // relative to the tile
+            if (!TAP27) return base + xx + (long)TX * (yy + TY * zz);
+            return base + (((long)((z0 + zz) & m) << (2 * lg)) | (long)(((y0 + yy) & m) << lg) | (long)((x0 + xx) & m));
+        };
+        if (tile != (int)blockIdx.x * per) __syncthreads();
+#pragma unroll
+        for (int k = 0; k < (2 * W::xvox + 255) / 256; k++) {
+            const int i = (int)threadIdx.x + 256 * k, r = i >> 1, row = r / TX;
+            const int c = nb + 8 * (i & 1);
+            if (2 * W::xvox % 256 == 0 || i < 2 * W::xvox) {
+                uint4 v = make_uint4(0, 0, 0, 0);
+                if (c < cx) v = *reinterpret_cast<const uint4*>(x + voxel(r % TX, row % YH - H, row / YH - H) * ldx + c);
+                *reinterpret_cast<uint4*>(xs + 8 * i) = v;
+            }
+        }
+        for (int w = 0; w < wc; w++) {
+#pragma unroll
+            for (int k = 0; k < (2 * W::zvox + 255) / 256; k++) {
+                const int i = (int)threadIdx.x + 256 * k, r = i >> 1, row = r / XP;
+                const int c = cb + 16 * w + 8 * (i & 1);
+                if (2 * W::zvox % 256 == 0 || i < 2 * W::zvox) {
+                    uint4 v = make_uint4(0, 0, 0, 0);
+                    if (c < cz) v = *reinterpret_cast<const uint4*>(dz + voxel(r % XP - H, row % TY, row / TY) * ldz + c);
+                    *reinterpret_cast<uint4*>(zs + 16 * W::zvox * w + 8 * i) = v;
+                }
+            }
+        }
+        __syncthreads();
+        for (int q = vw; q < W::vox / 32; q += nvw) {
+            // the lane's pieces: voxels 32 q + 16 r + lane / 4, channels 4 (lane % 4) ..
+            const uint16_t *px[2], *pz[2];
+#pragma unroll
+            for (int r = 0; r < 2; r++) {
+                const int v = 32 * q + 16 * r + (lane >> 2), xx = v % TX, row = v / TX, yy = row % TY, zz = row / TY;
+                px[r] = xs + 16 * ((zz + H) * YH * TX + (yy + H) * TX + xx) + 4 * (lane & 3);
+                pz[r] = zs + 16 * (cw * W::zvox + row * XP + xx + H) + 4 * (lane & 3);
+            }
+            bf16x8 a[2 * H + 1];
+#pragma unroll
+            for (int d = 0; d < 2 * H + 1; d++) a[d] = read_tr(pz[0] - 16 * (d - H), pz[1] - 16 * (d - H));
+            accb = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[H], ones, accb, 0, 0, 0);
+#pragma unroll
+            for (int d = 0; d < NT / (2 * H + 1); d++) {
+                const int o = TAP27 ? 16 * ((d / 3 - 1) * YH * TX + (d % 3 - 1) * TX) : 0;
+                const bf16x8 b = read_tr(px[0] + o, px[1] + o);
+#pragma unroll
+                for (int e = 0; e < 2 * H + 1; e++)
+                    acc[d * (2 * H + 1) + e] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[e], b, acc[d * (2 * H + 1) + e], 0, 0, 0);
+            }
         }
     }
-    // lane (col, grp) holds input channel nb + col, output channels cb + 4 grp + r
+    // the waves of the same output channels: the upper half to LDS, the lower half adds, until one is left
+    float* const fs = reinterpret_cast<float*>(sh);
+    for (int half = nvw / 2; half > 0; half /= 2) {
+        float* const mine = fs + (size_t)(cw * half + vw % half) * (NT + 1) * kWgTapFloats + 4 * lane;
+        __syncthreads();
+        if (vw >= half && vw < 2 * half) {
 #pragma unroll
-    for (int t = 0; t < NT; t++)
+            for (int t = 0; t < NT; t++) *reinterpret_cast<f32x4*>(mine + t * kWgTapFloats) = acc[t];
+            *reinterpret_cast<f32x4*>(mine + NT * kWgTapFloats) = accb;
+        }
+        __syncthreads();
+        if (vw < half) {
 #pragma unroll
-        for (int r = 0; r < 4; r++)
-            partial[(((long)split * czp + cb + 4 * grp + r) * NT + t) * cxp + nb + col] = acc[t][r];
+            for (int t = 0; t < NT; t++) acc[t] += *reinterpret_cast<const f32x4*>(mine + t * kWgTapFloats);
+            accb += *reinterpret_cast<const f32x4*>(mine + NT * kWgTapFloats);
+        }
+    }
+    // lane (col, grp) holds input channel nb + col, output channels cb + 16 cw + 4 grp + r
+    const int col = lane & 15, co = cb + 16 * cw + 4 * (lane >> 4);
+    if (vw == 0 && co < czp) {
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const long o = (long)blockIdx.x * czp + co + r;
+#pragma unroll
+            for (int t = 0; t < NT; t++) partial[(o * NT + t) * cxp + nb + col] = acc[t][r];
+            if (nb == 0 && col == 0) bpartial[o] = accb[r];
+        }
+    }
 }
 
-// dW[co][t][ci] (co < cout, ci < cin; the flat parameter layout) = sum over splits.
-__global__ __launch_bounds__(256) void k_wgrad_reduce(const float* __restrict__ partial, int splits, int czp, int taps,
-                                                      int cxp, int cout, int cin, float* __restrict__ dW) {
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long total = (long)cout * taps * cin;
-    if (i >= total) return;
-    const int ci = (int)(i % cin), t = (int)((i / cin) % taps), co = (int)(i / ((long)cin * taps));
-    float s = 0.f;
-    for (int k = 0; k < splits; k++) s += partial[(((long)k * czp + co) * taps + t) * cxp + ci];
-    dW[i] = s;
-}
-
-// db[co] = sum_v dZ[v][co], from the channel-major rows.
-__global__ __launch_bounds__(1024) void k_rowsum(const uint16_t* __restrict__ dzc, long nvox, float* __restrict__ db) {
+// dW[co][t][ci] (co < cout, ci < cin; the flat parameter layout) and db[co] = sums over the splits: a block
+// takes 64 of them, its waves every (blockDim / 64)th split: 12 us on average (one thread a parameter, a chain
+// of up to 1024 loads, was 101).
+__global__ __launch_bounds__(1024) void k_wgrad_reduce(const float* __restrict__ partial, const float* __restrict__ bpartial,
+                                                       int splits, int czp, int taps, int cxp, int cout, int cin,
+                                                       float* __restrict__ dW, float* __restrict__ db) {
     __shared__ float sh[1024];
-    const int co = blockIdx.x;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    const int i = (int)blockIdx.x * 64 + lane, total = cout * taps * cin;
+    const float* p = nullptr;
+    long stride = 0;
+    if (i < total) {
+        const int ci = i % cin, t = i / cin % taps, co = i / (cin * taps);
+        p = partial + ((long)co * taps + t) * cxp + ci;
+        stride = (long)czp * taps * cxp;
+    } else if (i < total + cout) {
+        p = bpartial + i - total;
+        stride = czp;
+    }
     float s = 0.f;
-    for (long v = threadIdx.x; v < nvox; v += blockDim.x) s += bf2f(dzc[(long)co * nvox + v]);
+    if (p) {
+#pragma unroll 8
+        for (int k = w; k < splits; k += nw) s += p[k * stride];
+    }
     sh[threadIdx.x] = s;
     __syncthreads();
-    for (int k = 512; k > 0; k >>= 1) {
-        if (threadIdx.x < k) sh[threadIdx.x] += sh[threadIdx.x + k];
+    for (int k = nw / 2; k > 0; k >>= 1) {
+        if (w < k) sh[threadIdx.x] += sh[threadIdx.x + 64 * k];
         __syncthreads();
     }
-    if (threadIdx.x == 0) db[co] = sh[0];
+    if (w == 0 && p) (i < total ? dW[i] : db[i - total]) = sh[lane];
 }
 
 // dZ = dY where Y > 0 else 0 (dY dense [v][C], overwritten; Y a strided view).
@@ -502,9 +599,7 @@ struct homo3d_net {
     int lblocks = 1024;
     float* rho = nullptr;        // host-staged densities [batch][g^3]
     float* tstage = nullptr;     // [batch][g^3][18]: host-staged targets, or a prediction on its way to the host
-    uint16_t *zc = nullptr, *xc = nullptr;  // channel-major scratch for the weight gradient
-    size_t zc_elems = 0, xc_elems = 0;
-    float* partial = nullptr;
+    float* partial = nullptr;    // the weight gradient's partial sums
     size_t partial_elems = 0;
     // dataset (device resident): inputs [count][g^3][8], targets [count][g^3][18]
     uint16_t *ds_in = nullptr, *ds_tg = nullptr;
@@ -575,28 +670,60 @@ void layer_dx(homo3d_net* n, const NetLayer& Ly, const uint16_t* dz, int ldz, in
                                       nvox);
 }
 
+// How the weight gradient of a layer is split: wc output-channel tiles a block, `splits` ranges of `per` tiles.
+struct WgPlan {
+    int czp, cxp, wc, tx, tiles, per, splits;
+    size_t partial() const { return (size_t)splits * czp; }  // rows of taps * cxp + 1 floats
+};
+
+// Tiles are whole x-rows up to 64 voxels.  Two blocks a compute unit fill the GPU (a block's tile takes 60 KB
+// of LDS in the usual layers, up to 116 KB with 64 output channels at 64 voxels), and every split more is a partial of
+// czp * taps * cxp sums written and read: 512 blocks over the channel tiles.
+WgPlan wgrad_plan(int cz, int cx, int taps, int lg, long nvox) {
+    WgPlan w;
+    w.czp = round_up(cz, 16);
+    w.cxp = round_up(cx, 16);
+    w.wc = w.czp >= 64 ? 4 : w.czp >= 32 ? 2 : 1;
+    w.czp = round_up(w.czp, 16 * w.wc);
+    w.tx = taps == 27 ? std::min(64, 1 << lg) : 64;
+    w.tiles = (int)(nvox / (w.tx * 4 * (w.tx == 64 ? 2 : 4)));
+    const int groups = w.czp / (16 * w.wc) * (w.cxp / 16);
+    w.per = (int)std::max(1L, ((long)w.tiles * groups + 511) / 512);
+    w.splits = (w.tiles + w.per - 1) / w.per;
+    return w;
+}
+
+template <int TX, int TZ, bool TAP27>
+void wgrad(hipStream_t s, const WgPlan& w, const uint16_t* dz, int ldz, int cz, const uint16_t* x, int ldx, int cx, int lg,
+           float* partial, float* bpartial) {
+    using W = WgTile<TX, 4, TZ, TAP27>;
+    const dim3 grid((unsigned)w.splits, (unsigned)(w.czp / (16 * w.wc)), (unsigned)(w.cxp / 16));
+    hipLaunchKernelGGL((k_wgrad<TX, 4, TZ, TAP27>), grid, dim3(256), W::lds(w.wc), s, dz, ldz, cz, x, ldx, cx, lg, w.tiles,
+                       w.per, w.wc, w.czp, w.cxp, partial, bpartial);
+}
+
 // weight and bias gradient of one layer into n->g: X the layer input view (ldx, cx stored channels),
-// dZ the output gradient view (ldz, cz channels with cz >= cout).
+// dZ the output gradient view (ldz, cz channels with cz >= cout; both counts multiples of 8).
 int layer_dw(homo3d_net* n, const NetLayer& Ly, const uint16_t* x, int ldx, int cx, const uint16_t* dz, int ldz, int cz,
              int lg, long nvox) {
-    const int czp = round_up(cz, 16), cxp = round_up(cx, 16);
-    const int ns = Ly.taps == 27 ? 3 : 1;
-    if ((size_t)czp * nvox > n->zc_elems || (size_t)ns * cxp * nvox > n->xc_elems)
-        return nerr(n, HOMO3D_BAD_ARG, "weight-gradient scratch too small");
-    hipLaunchKernelGGL(k_to_cm, dim3(nblk(nvox)), dim3(256), 0, n->stream, dz, ldz, cz, czp, lg, nvox, 1, 1, n->zc);
-    hipLaunchKernelGGL(k_to_cm, dim3(nblk(nvox)), dim3(256), 0, n->stream, x, ldx, cx, cxp, lg, nvox, ns == 3 ? 0 : 1, ns,
-                       n->xc);
-    const int splits = (int)((nvox + 32L * kWgChunks - 1) / (32L * kWgChunks));
-    if ((size_t)splits * czp * Ly.taps * cxp > n->partial_elems) return nerr(n, HOMO3D_BAD_ARG, "partial buffer too small");
-    const dim3 grid((unsigned)splits, (unsigned)(czp / 16), (unsigned)(cxp / 16));
-    if (Ly.taps == 27)
-        hipLaunchKernelGGL(k_wgrad<true>, grid, dim3(64), 0, n->stream, n->zc, czp, n->xc, cxp, lg, nvox, n->partial);
+    const WgPlan w = wgrad_plan(cz, cx, Ly.taps, lg, nvox);
+    if (w.partial() * (Ly.taps * w.cxp + 1) > n->partial_elems) return nerr(n, HOMO3D_BAD_ARG, "partial buffer too small");
+    float* bp = n->partial + w.partial() * Ly.taps * w.cxp;
+    if (Ly.taps != 27)
+        wgrad<64, 2, false>(n->stream, w, dz, ldz, cz, x, ldx, cx, lg, n->partial, bp);
+    else if (w.tx == 64)
+        wgrad<64, 2, true>(n->stream, w, dz, ldz, cz, x, ldx, cx, lg, n->partial, bp);
+    else if (w.tx == 32)
+        wgrad<32, 4, true>(n->stream, w, dz, ldz, cz, x, ldx, cx, lg, n->partial, bp);
+    else if (w.tx == 16)
+        wgrad<16, 4, true>(n->stream, w, dz, ldz, cz, x, ldx, cx, lg, n->partial, bp);
     else
-        hipLaunchKernelGGL(k_wgrad<false>, grid, dim3(64), 0, n->stream, n->zc, czp, n->xc, cxp, lg, nvox, n->partial);
-    const long tot = (long)Ly.cout * Ly.taps * Ly.cin;
-    hipLaunchKernelGGL(k_wgrad_reduce, dim3(nblk(tot)), dim3(256), 0, n->stream, n->partial, splits, czp, Ly.taps, cxp,
-                       Ly.cout, Ly.cin, n->g + Ly.off_w);
-    hipLaunchKernelGGL(k_rowsum, dim3(Ly.cout), dim3(1024), 0, n->stream, n->zc, nvox, n->g + Ly.off_b);
+        wgrad<8, 4, true>(n->stream, w, dz, ldz, cz, x, ldx, cx, lg, n->partial, bp);
+    const int tot = Ly.cout * Ly.taps * Ly.cin + Ly.cout;
+    int waves = 1;
+    while (waves < 16 && 2 * waves <= w.splits) waves *= 2;
+    hipLaunchKernelGGL(k_wgrad_reduce, dim3(nblk(tot, 64)), dim3(64 * waves), 0, n->stream, n->partial, bp, w.splits, w.czp,
+                       Ly.taps, w.cxp, Ly.cout, Ly.cin, n->g + Ly.off_w, n->g + Ly.off_b);
     return HOMO3D_OK;
 }
 
@@ -665,14 +792,13 @@ int loss_backward(homo3d_net* n, int batch, double* loss) {
     const double inv = 1.0 / ((double)nv0 * kOut);
     hipLaunchKernelGGL(k_head_loss, dim3(n->lblocks), dim3(256), 0, n->stream, n->P, n->mean, n->wbar, V0.in, n->T, nv0,
                        V0.lg, inv, n->dP, n->lpart);
-    NETCHK(n, hipMemsetAsync(n->g, 0, sizeof(float) * n->nparam, n->stream));
     int li = (int)n->layers.size() - 1;
     int rc;
     // head
     {
         const NetLayer& hd = n->layers[li--];
         const uint16_t* top = L > 1 ? V0.d : V0.s;
-        if ((rc = layer_dw(n, hd, top, V0.c, V0.c, n->dP, kDpLd, kOut, V0.lg, nv0))) return rc;
+        if ((rc = layer_dw(n, hd, top, V0.c, V0.c, n->dP, kDpLd, kDpC, V0.lg, nv0))) return rc;
         layer_dx(n, hd, n->dP, kDpLd, kDpC, V0.ga, V0.c, V0.lg, nv0);  // dD_0
     }
     // decoder levels, top down in the parameter list (level 0 first)
@@ -767,8 +893,7 @@ void destroy(homo3d_net* n) {
         for (void* q : ptrs)
             if (q) (void)hipFree(q);
     }
-    void* ptrs[] = {n->p, n->g, n->m1, n->m2, n->P, n->T, n->dP, n->mean, n->wbar, n->lpart, n->rho, n->tstage, n->zc, n->xc,
-                    n->partial, n->ds_in, n->ds_tg};
+    void* ptrs[] = {n->p, n->g, n->m1, n->m2, n->P, n->T, n->dP, n->mean, n->wbar, n->lpart, n->rho, n->tstage, n->partial, n->ds_in, n->ds_tg};
     for (void* q : ptrs)
         if (q) (void)hipFree(q);
     if (n->stream) (void)hipStreamDestroy(n->stream);
@@ -876,7 +1001,7 @@ int homo3d_net_create(const homo3d_net_config* cfg, homo3d_net** out) {
     if (!ok) return fail(HOMO3D_HIP_ERROR);
     // activations
     n->lv.resize(L);
-    size_t max_zc = 0, max_xc = 0, max_part = 0;
+    size_t max_part = 0;
     for (int l = 0; l < L; l++) {
         NetLevel& V = n->lv[l];
         V.g = g >> l;
@@ -896,15 +1021,17 @@ int homo3d_net_create(const homo3d_net_config* cfg, homo3d_net** out) {
             ok = ok && mal(&V.s, nv * V.c);
         if (!ok) return fail(HOMO3D_HIP_ERROR);
         if (l == 0 && hipMemset(V.in, 0, sizeof(uint16_t) * nv * kInCh)) return fail(HOMO3D_HIP_ERROR);
-        // weight-gradient scratch: the widest layer input (CAT) and output of this level
-        const int cx = round_up(std::max(cin, cu + V.c), 16);
-        max_xc = std::max(max_xc, (size_t)3 * cx * nv);
-        max_zc = std::max(max_zc, (size_t)round_up(std::max(V.c, kOut), 16) * nv);
-        const long splits = (nv + 32L * kWgChunks - 1) / (32L * kWgChunks);
-        max_part = std::max(max_part, (size_t)splits * round_up(std::max(V.c, kOut), 16) * 27 * cx);
     }
-    n->zc_elems = max_zc;
-    n->xc_elems = max_xc;
+    // weight-gradient partials, for every layer (in the parameters' order) and every batch size up to B
+    for (size_t i = 0; i < n->layers.size(); i++) {
+        const NetLayer& Ly = n->layers[i];
+        const bool head = i + 1 == n->layers.size();
+        const int l = head ? 0 : (int)i < 2 * L ? (int)i / 2 : L - 2 - ((int)i - 2 * L) / 2;
+        for (int b = 1; b <= B; b++) {
+            const WgPlan w = wgrad_plan(head ? kDpC : Ly.cout, Ly.cinp, Ly.taps, n->lv[l].lg, (long)b << (3 * n->lv[l].lg));
+            max_part = std::max(max_part, w.partial() * (Ly.taps * w.cxp + 1));
+        }
+    }
     n->partial_elems = max_part;
     const long nv0 = n->lv[0].nvox;
     if (hipMalloc(&n->p, sizeof(float) * n->nparam) || hipMalloc(&n->g, sizeof(float) * n->nparam) ||
@@ -913,7 +1040,6 @@ int homo3d_net_create(const homo3d_net_config* cfg, homo3d_net** out) {
         hipMalloc(&n->dP, sizeof(uint16_t) * nv0 * kDpLd) || hipMalloc(&n->mean, sizeof(float) * B * kOut) || hipMalloc(&n->wbar, sizeof(float) * B) ||
         hipMalloc(&n->lpart, sizeof(double) * n->lblocks) || hipMalloc(&n->rho, sizeof(float) * nv0) ||
         hipMalloc(&n->tstage, sizeof(float) * nv0 * kOut) ||
-        hipMalloc(&n->zc, sizeof(uint16_t) * max_zc) || hipMalloc(&n->xc, sizeof(uint16_t) * max_xc) ||
         hipMalloc(&n->partial, sizeof(float) * max_part))
         return fail(HOMO3D_HIP_ERROR);
     if (hipMemset(n->dP, 0, sizeof(uint16_t) * nv0 * kDpLd) || hipMemset(n->m1, 0, sizeof(float) * n->nparam) ||
