@@ -12,9 +12,13 @@
 //   head:    P = conv1(D_0) (18 channels: u of load case s, component k at channel 3 s + k)
 // conv3 is a periodic 3x3x3 correlation, tap t = (dx+1) + 3 (dy+1) + 9 (dz+1) reading X[v + (dx,dy,dz)].
 //
-// Storage: activations are bf16, channels-last [B][g^3][ld] (voxel v = x + g (y + g z) + g^3 b), so a
-// lane's 8 consecutive channels are one 16-byte load.  S_l lives inside CAT_l (channel offset
-// c_{l+1}), which makes the concatenation free.  Master weights, Adam state and gradients are FP32.
+// Storage: activations are bf16 in planes of 8 channels, [C/8][B g^3][8] (voxel v = x + g (y + g z) + g^3 b;
+// a plane is as long as the largest batch), so a matrix operand, 8 channels of 16 consecutive voxels, is
+// 256 bytes in a row.  With the voxels' channels in a row instead it was 16 bytes from each of 16 cache
+// lines, and the convolutions were bound by the lines a load touches (some 64 cycles each): 2.0 ms for a
+// 64^3 x 4 gradient's 28 of them, 1.1 ms now.  S_l lives inside
+// CAT_l (channel offset c_{l+1}), which makes the concatenation free.  Master weights, Adam state and
+// gradients are FP32.
 //
 // Matrix cores: every convolution pass is an implicit GEMM on v_mfma_f32_16x16x32_bf16 (bf16
 // operands, FP32 accumulation):
@@ -48,76 +52,95 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 constexpr int kOut = 18;      // output channels
 constexpr int kInCh = 8;      // stored input channels (density + 7 zeros): the 8-channel loads stay aligned
 constexpr int kPld = 24;      // row stride of the FP32 prediction
-constexpr int kDpLd = 32;     // row stride of the head's output gradient (18 used, zeros after)
-constexpr int kDpC = 24;      // channels of it read by the head's input-gradient pass (multiple of 8)
+constexpr int kDpC = 24;      // channels of the head's output gradient (18 used, zeros after)
+constexpr int kPlanes = kDpC / 8;
+
+// 8-channel group of channel c of voxel v; ps: length of a plane
+__device__ __forceinline__ size_t group(long v, int c, long ps) { return ((size_t)(c >> 3) * (size_t)ps + (size_t)v) * 8; }
 
 __device__ __forceinline__ bf16x8 load8(const uint16_t* p) {
     return __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(p));
 }
 
+// what a convolution reads past its last tap or chunk (selecting the address, not the loaded value, keeps the load
+// in flight, and an address in the constant segment would make it a flat one); never written
+__device__ __attribute__((aligned(16))) uint16_t kZeros[8] = {};
+
 // ---------------------------------------------------------------------------------------------------
 // Convolution (forward and input gradient): implicit GEMM.  A wave computes 16 MB output channels for
 // 16 NB voxels; a block holds 4 waves (64 NB consecutive voxels); blockIdx.y selects the channel block.
-// cin % 8 == 0; the weight rows are padded to gridDim.y * 16 MB and to kpad (multiple of 32) with zeros.
+// cin % 8 == 0; the weights lie as [kpad / 8][rows][8], rows padded to gridDim.y * 16 MB and kpad (a multiple
+// of 32) with zeros.
 // ---------------------------------------------------------------------------------------------------
 template <int MB, int NB, bool TAP27, bool RELU, bool F32OUT>
-__global__ __launch_bounds__(256) void k_conv(const uint16_t* __restrict__ in, int ldi, int cin,
-                                              const uint16_t* __restrict__ w, int kpad,
-                                              const float* __restrict__ bias, void* __restrict__ out, int ldo,
-                                              int cout, int lg, long nvox) {
+__global__ __launch_bounds__(256) void k_conv(const uint16_t* __restrict__ in, int cin, const uint16_t* __restrict__ w,
+                                              int kpad, int rows, const float* __restrict__ bias,
+                                              void* __restrict__ out, int cout, int lg, long nvox, long ps,
+                                              const uint16_t* __restrict__ relu) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int col = lane & 15, grp = lane >> 4;
     const long vb = ((long)blockIdx.x * 4 + wave) * (16 * NB);
-    if (vb >= nvox) return;
     const int cb = blockIdx.y * 16 * MB;
+    // the voxels that the taps of the wave's voxels read
+    __shared__ uint32_t nbrs[4][TAP27 ? 27 : 1][16 * NB];
+    uint32_t(*const nb)[16 * NB] = nbrs[wave];
     const int m = (1 << lg) - 1;
-    int vx[NB], vy[NB], vz[NB];
-    long vs[NB];
+    for (int v = lane; v < 16 * NB; v += 64) {
+        const uint32_t g = (uint32_t)(vb + v), x = g & m, y = (g >> lg) & m, z = (g >> (2 * lg)) & m, s0 = (g >> (3 * lg)) << (3 * lg);
+        if (TAP27) {
 #pragma unroll
-    for (int j = 0; j < NB; j++) {
-        const long v = vb + 16 * j + col;
-        vx[j] = (int)(v & m);
-        vy[j] = (int)((v >> lg) & m);
-        vz[j] = (int)((v >> (2 * lg)) & m);
-        vs[j] = (v >> (3 * lg)) << (3 * lg);
+            for (int t = 0; t < 27; t++)
+                nb[t][v] = s0 | ((z + t / 9 - 1) & m) << (2 * lg) | ((y + t / 3 % 3 - 1) & m) << lg | ((x + t % 3 - 1) & m);
+        } else {
+            nb[0][v] = g;
+        }
     }
+    if (vb >= nvox) return;
+    constexpr int D = MB + NB > 6 ? 2 : MB + NB > 3 ? 4 : 6;  // chunks of operands in flight
     f32x4 acc[MB][NB];
 #pragma unroll
     for (int i = 0; i < MB; i++)
 #pragma unroll
         for (int j = 0; j < NB; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
     const int ntaps = TAP27 ? 27 : 1;
-    int tap = 0, ci = 8 * grp;  // (tap, ci) of k0 = 32 kc + 8 grp, advanced incrementally
-    while (ci >= cin) {
-        ci -= cin;
-        tap++;
-    }
+    // (tap, ci) of k0 = 32 kc + 8 grp of the next load, advanced by 32 = dtap cin + dci
+    int tap = 8 * grp / cin, ci = 8 * grp - tap * cin;
+    const int dtap = 32 / cin, dci = 32 - dtap * cin;
     const int kch = kpad >> 5;
-    for (int kc = 0; kc < kch; kc++) {
-        const int k0 = kc * 32 + 8 * grp;
-        bf16x8 a[MB], b[NB];
+    bf16x8 a[D][MB], b[D][NB];
+    const uint16_t* wr = w + ((size_t)grp * rows + cb + col) * 8;
+    int next = 0;
+    auto load = [&](bf16x8 (&as)[MB], bf16x8 (&bs)[NB]) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < MB; i++) a[i] = load8(w + (long)(cb + 16 * i + col) * kpad + k0);
-        if (tap < ntaps) {
-            const int dx = TAP27 ? tap % 3 - 1 : 0, dy = TAP27 ? (tap / 3) % 3 - 1 : 0, dz = TAP27 ? tap / 9 - 1 : 0;
+        for (int i = 0; i < MB; i++) as[i] = load8(next < kch ? wr + 128 * i : kZeros);
+        wr += (size_t)32 * rows;
+        next++;
+        const int t = min(tap, ntaps - 1);
 #pragma unroll
-            for (int j = 0; j < NB; j++) {
-                const long nb = vs[j] + (((long)((vz[j] + dz) & m) << (2 * lg)) | ((long)((vy[j] + dy) & m) << lg) |
-                                         (long)((vx[j] + dx) & m));
-                b[j] = load8(in + nb * ldi + ci);
-            }
-        } else {
-#pragma unroll
-            for (int j = 0; j < NB; j++) b[j] = bf16x8{};
+        for (int j = 0; j < NB; j++) {
+            const uint16_t* p = in + group(nb[t][16 * j + col], ci, ps);
+            bs[j] = load8(tap < ntaps ? p : kZeros);
         }
-#pragma unroll
-        for (int i = 0; i < MB; i++)
-#pragma unroll
-            for (int j = 0; j < NB; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
-        ci += 32;
-        while (ci >= cin) {
+        tap += dtap;
+        ci += dci;
+        if (ci >= cin) {
             ci -= cin;
             tap++;
+        }
+    };
+    // D chunks ahead without a branch, whose two sides would have to wait for the same loads: a few chunks of
+    // zeros at the end instead
+#pragma unroll
+    for (int d = 0; d < D; d++) load(a[d], b[d]);
+    for (int kc = 0; kc < kch; kc += D) {
+#pragma unroll
+        for (int d = 0; d < D; d++) {
+#pragma unroll
+            for (int i = 0; i < MB; i++)
+#pragma unroll
+                for (int j = 0; j < NB; j++)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[d][i], b[d][j], acc[i][j], 0, 0, 0);
+            load(a[d], b[d]);
         }
     }
     // D layout: lane (col, grp) holds voxel vb + 16 j + col, channels cb + 16 i + 4 grp + r
@@ -134,7 +157,7 @@ __global__ __launch_bounds__(256) void k_conv(const uint16_t* __restrict__ in, i
                 if (RELU) o[r] = fmaxf(o[r], 0.f);
             }
             if (F32OUT) {
-                float* dst = reinterpret_cast<float*>(out) + v * ldo + co0;
+                float* dst = reinterpret_cast<float*>(out) + v * kPld + co0;
                 if (co0 + 3 < cout) {
                     *reinterpret_cast<float4*>(dst) = make_float4(o[0], o[1], o[2], o[3]);
                 } else {
@@ -143,16 +166,18 @@ __global__ __launch_bounds__(256) void k_conv(const uint16_t* __restrict__ in, i
                         if (co0 + r < cout) dst[r] = o[r];
                 }
             } else {
-                uint16_t* dst = reinterpret_cast<uint16_t*>(out) + v * ldo + co0;
-                if (co0 + 3 < cout) {
-                    const uint32_t lo = (uint32_t)f2bf(o[0]) | ((uint32_t)f2bf(o[1]) << 16);
-                    const uint32_t hi = (uint32_t)f2bf(o[2]) | ((uint32_t)f2bf(o[3]) << 16);
-                    *reinterpret_cast<uint2*>(dst) = make_uint2(lo, hi);
-                } else {
+                if (co0 >= cout) continue;
+                const size_t at = group(v, co0, ps) + (co0 & 7);
+                uint2 q;
+                if (!RELU && relu) {  // the layer below's ReLU: no gradient where its output is not positive
+                    q = *reinterpret_cast<const uint2*>(relu + at);
 #pragma unroll
                     for (int r = 0; r < 4; r++)
-                        if (co0 + r < cout) dst[r] = f2bf(o[r]);
+                        if (!(bf2f((uint16_t)((r < 2 ? q.x : q.y) >> (16 * (r & 1)))) > 0.f)) o[r] = 0.f;
                 }
+                q.x = (uint32_t)f2bf(o[0]) | ((uint32_t)f2bf(o[1]) << 16);
+                q.y = (uint32_t)f2bf(o[2]) | ((uint32_t)f2bf(o[3]) << 16);
+                *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(out) + at) = q;
             }
         }
     }
@@ -160,8 +185,8 @@ __global__ __launch_bounds__(256) void k_conv(const uint16_t* __restrict__ in, i
 
 // ---------------------------------------------------------------------------------------------------
 // Weight gradient.  A block stages a tile of TX x TY x TZ voxels in LDS, 16 input channels of X with one row
-// more on each side in y and z, and 16 WC output channels of dZ with one voxel more on each side in x, both
-// as they lie in memory (a voxel's 16 channels are 32 bytes).  The tap (dx, dy, dz) pairs X at v + (dy, dz)
+// more on each side in y and z, and 16 WC output channels of dZ with one voxel more on each side in x, a
+// voxel's 16 channels in 32 bytes.  The tap (dx, dy, dz) pairs X at v + (dy, dz)
 // with dZ at v - dx, so a tile's 27 products need 9 X and 3 dZ operands.  The reduction over voxels wants a
 // channel's voxels in one lane: the transposing LDS reads (four voxels of 16 channels to 16 lanes with a
 // channel each) give that from any voxel on, so nothing is copied to channel-major order first.  Bound by
@@ -195,8 +220,8 @@ struct WgTile {
 
 // partial: [splits][czp][taps][cxp], bpartial: [splits][czp]
 template <int TX, int TY, int TZ, bool TAP27>
-__global__ __launch_bounds__(256, 2) void k_wgrad(const uint16_t* __restrict__ dz, int ldz, int cz,
-                                                  const uint16_t* __restrict__ x, int ldx, int cx, int lg, int tiles,
+__global__ __launch_bounds__(256, 2) void k_wgrad(const uint16_t* __restrict__ dz, int cz,
+                                                  const uint16_t* __restrict__ x, int cx, int lg, long ps, int tiles,
                                                   int per, int wc, int czp, int cxp, float* __restrict__ partial,
                                                   float* __restrict__ bpartial) {
     using W = WgTile<TX, TY, TZ, TAP27>;
@@ -237,7 +262,7 @@ __global__ __launch_bounds__(256, 2) void k_wgrad(const uint16_t* __restrict__ d
             const int c = nb + 8 * (i & 1);
             if (2 * W::xvox % 256 == 0 || i < 2 * W::xvox) {
                 uint4 v = make_uint4(0, 0, 0, 0);
-                if (c < cx) v = *reinterpret_cast<const uint4*>(x + voxel(r % TX, row % YH - H, row / YH - H) * ldx + c);
+                if (c < cx) v = *reinterpret_cast<const uint4*>(x + group(voxel(r % TX, row % YH - H, row / YH - H), c, ps));
                 *reinterpret_cast<uint4*>(xs + 8 * i) = v;
             }
         }
@@ -248,7 +273,7 @@ __global__ __launch_bounds__(256, 2) void k_wgrad(const uint16_t* __restrict__ d
                 const int c = cb + 16 * w + 8 * (i & 1);
                 if (2 * W::zvox % 256 == 0 || i < 2 * W::zvox) {
                     uint4 v = make_uint4(0, 0, 0, 0);
-                    if (c < cz) v = *reinterpret_cast<const uint4*>(dz + voxel(r % XP - H, row % TY, row / TY) * ldz + c);
+                    if (c < cz) v = *reinterpret_cast<const uint4*>(dz + group(voxel(r % XP - H, row % TY, row / TY), c, ps));
                     *reinterpret_cast<uint4*>(zs + 16 * W::zvox * w + 8 * i) = v;
                 }
             }
@@ -340,86 +365,92 @@ __global__ __launch_bounds__(1024) void k_wgrad_reduce(const float* __restrict__
     if (w == 0 && p) (i < total ? dW[i] : db[i - total]) = sh[lane];
 }
 
-// dZ = dY where Y > 0 else 0 (dY dense [v][C], overwritten; Y a strided view).
-__global__ __launch_bounds__(256) void k_relu_mask(uint16_t* __restrict__ dy, int C, const uint16_t* __restrict__ y,
-                                                   int ldy, long nvox) {
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nvox * C) return;
-    const long v = i / C;
-    const int c = (int)(i - v * C);
-    if (!(bf2f(y[v * ldy + c]) > 0.f)) dy[i] = 0;
+// The elementwise passes between levels: a thread takes a group of 8 channels.
+__device__ __forceinline__ float group_at(const uint4& q, int k) {
+    return bf2f((uint16_t)((k < 2 ? q.x : k < 4 ? q.y : k < 6 ? q.z : q.w) >> (16 * (k & 1))));
+}
+__device__ __forceinline__ uint4 group_of(const float (&f)[8]) {
+    uint32_t w[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) w[k] = (uint32_t)f2bf(f[2 * k]) | ((uint32_t)f2bf(f[2 * k + 1]) << 16);
+    return make_uint4(w[0], w[1], w[2], w[3]);
+}
+__device__ __forceinline__ const uint4* groups(const uint16_t* p, int plane, long ps) {
+    return reinterpret_cast<const uint4*>(p) + (size_t)plane * ps;
 }
 
-// avgpool2: out[vc][c] (dense, grid g/2) = mean of the 8 children in the view (in, ldi), grid g.
-__global__ __launch_bounds__(256) void k_pool(const uint16_t* __restrict__ in, int ldi, int C, int lgc, long nvc,
+// First child (grid 2^(lgc+1)) of voxel vc of grid 2^lgc; the others are + (k & 1), + (k >> 1 & 1) rows, + (k >> 2) planes.
+__device__ __forceinline__ long child0(long vc, int lgc) {
+    const long mc = (1 << lgc) - 1, x = vc & mc, y = (vc >> lgc) & mc, z = (vc >> (2 * lgc)) & mc;
+    const int lg = lgc + 1;
+    return (vc >> (3 * lgc) << (3 * lg)) + (2 * z << (2 * lg)) + (2 * y << lg) + 2 * x;
+}
+__device__ __forceinline__ long parent(long v, int lg) {
+    const long m = (1 << lg) - 1, x = v & m, y = (v >> lg) & m, z = (v >> (2 * lg)) & m;
+    const int lgc = lg - 1;
+    return (v >> (3 * lg) << (3 * lgc)) + (z >> 1 << (2 * lgc)) + (y >> 1 << lgc) + (x >> 1);
+}
+
+// s = sum over the eight children of one group
+__device__ __forceinline__ void child_sum(const uint4* __restrict__ in, long v0, int lg, float (&s)[8]) {
+    uint4 q[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) q[k] = in[v0 + ((long)(k >> 2) << (2 * lg)) + ((long)((k >> 1) & 1) << lg) + (k & 1)];
+#pragma unroll
+    for (int c = 0; c < 8; c++) {
+        s[c] = 0.f;
+#pragma unroll
+        for (int k = 0; k < 8; k++) s[c] += group_at(q[k], c);
+    }
+}
+
+// avgpool2: out (grid g/2) = mean of the 8 children of in (grid g); blockIdx.y: plane.
+__global__ __launch_bounds__(256) void k_pool(const uint16_t* __restrict__ in, int lgc, long nvc, long ps, long psc,
                                               uint16_t* __restrict__ out) {
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nvc * C) return;
-    const long vc = i / C;
-    const int c = (int)(i - vc * C);
-    const int mc = (1 << lgc) - 1, lg = lgc + 1;
-    const int x = (int)(vc & mc), y = (int)((vc >> lgc) & mc), z = (int)((vc >> (2 * lgc)) & mc);
-    const long b = vc >> (3 * lgc);
-    float s = 0.f;
-    for (int k = 0; k < 8; k++) {
-        const long vf = (b << (3 * lg)) + ((long)(2 * z + (k >> 2)) << (2 * lg)) + ((long)(2 * y + ((k >> 1) & 1)) << lg) +
-                        (2 * x + (k & 1));
-        s += bf2f(in[vf * ldi + c]);
-    }
-    out[i] = f2bf(s * 0.125f);
+    const long vc = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (vc >= nvc) return;
+    float s[8];
+    child_sum(groups(in, blockIdx.y, ps), child0(vc, lgc), lgc + 1, s);
+#pragma unroll
+    for (int c = 0; c < 8; c++) s[c] *= 0.125f;
+    *const_cast<uint4*>(groups(out, blockIdx.y, psc) + vc) = group_of(s);
 }
 
-// up2 into the first C channels of the view (out, ldo) at grid g from the dense [vc][C] at grid g/2.
-__global__ __launch_bounds__(256) void k_up(const uint16_t* __restrict__ in, int C, int lg, long nvox,
-                                            uint16_t* __restrict__ out, int ldo) {
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nvox * C) return;
-    const long v = i / C;
-    const int c = (int)(i - v * C);
-    const int m = (1 << lg) - 1, lgc = lg - 1;
-    const int x = (int)(v & m), y = (int)((v >> lg) & m), z = (int)((v >> (2 * lg)) & m);
-    const long b = v >> (3 * lg);
-    const long vc = (b << (3 * lgc)) + ((long)(z >> 1) << (2 * lgc)) + ((long)(y >> 1) << lgc) + (x >> 1);
-    out[v * ldo + c] = in[vc * C + c];
+// up2: out (grid g) from in (grid g/2); blockIdx.y: plane.
+__global__ __launch_bounds__(256) void k_up(const uint16_t* __restrict__ in, int lg, long nvox, long ps, long psc,
+                                            uint16_t* __restrict__ out) {
+    const long v = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (v >= nvox) return;
+    *const_cast<uint4*>(groups(out, blockIdx.y, ps) + v) = groups(in, blockIdx.y, psc)[parent(v, lg)];
 }
 
-// gradient of up2: out[vc][c] (dense) = sum of the children's (in, ldi) entries c.
-__global__ __launch_bounds__(256) void k_up_back(const uint16_t* __restrict__ in, int ldi, int C, int lgc, long nvc,
-                                                 uint16_t* __restrict__ out) {
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nvc * C) return;
-    const long vc = i / C;
-    const int c = (int)(i - vc * C);
-    const int mc = (1 << lgc) - 1, lg = lgc + 1;
-    const int x = (int)(vc & mc), y = (int)((vc >> lgc) & mc), z = (int)((vc >> (2 * lgc)) & mc);
-    const long b = vc >> (3 * lgc);
-    float s = 0.f;
-    for (int k = 0; k < 8; k++) {
-        const long vf = (b << (3 * lg)) + ((long)(2 * z + (k >> 2)) << (2 * lg)) + ((long)(2 * y + ((k >> 1) & 1)) << lg) +
-                        (2 * x + (k & 1));
-        s += bf2f(in[vf * ldi + c]);
-    }
-    out[i] = f2bf(s);
+// gradient of up2: out (grid g/2) = sum of the children's entries of in (grid g) where the upsampled D (grid
+// g/2) is positive, else 0: the gradient before D's ReLU.  blockIdx.y: plane.
+__global__ __launch_bounds__(256) void k_up_back(const uint16_t* __restrict__ in, int lgc, long nvc, long ps, long psc,
+                                                 const uint16_t* __restrict__ d, uint16_t* __restrict__ out) {
+    const long vc = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (vc >= nvc) return;
+    float s[8];
+    child_sum(groups(in, blockIdx.y, ps), child0(vc, lgc), lgc + 1, s);
+    const uint4 y = groups(d, blockIdx.y, psc)[vc];
+#pragma unroll
+    for (int c = 0; c < 8; c++)
+        if (!(group_at(y, c) > 0.f)) s[c] = 0.f;
+    *const_cast<uint4*>(groups(out, blockIdx.y, psc) + vc) = group_of(s);
 }
 
-// Gradient of the skip tensor S_l (relu applied): out[v][c] = S > 0 ? dcat[v][cu + c] + dIn[parent][c] / 8 : 0,
-// where dIn is the gradient of in_{l+1} = avgpool2(S_l) (dense [vc][C], grid g/2).
-__global__ __launch_bounds__(256) void k_skip_grad(const uint16_t* __restrict__ s, const uint16_t* __restrict__ dcat,
-                                                   int ld, int cu, int C, const uint16_t* __restrict__ din, int lg,
-                                                   long nvox, uint16_t* __restrict__ out) {
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nvox * C) return;
-    const long v = i / C;
-    const int c = (int)(i - v * C);
-    if (!(bf2f(s[v * ld + cu + c]) > 0.f)) {
-        out[i] = 0;
-        return;
-    }
-    const int m = (1 << lg) - 1, lgc = lg - 1;
-    const int x = (int)(v & m), y = (int)((v >> lg) & m), z = (int)((v >> (2 * lg)) & m);
-    const long b = v >> (3 * lg);
-    const long vc = (b << (3 * lgc)) + ((long)(z >> 1) << (2 * lgc)) + ((long)(y >> 1) << lgc) + (x >> 1);
-    out[i] = f2bf(bf2f(dcat[v * ld + cu + c]) + 0.125f * bf2f(din[vc * C + c]));
+// Gradient of the skip tensor S_l (relu applied): out = S > 0 ? dS + dIn[parent] / 8 : 0, dS its part of the
+// gradient of CAT_l and dIn (grid g/2) the gradient of in_{l+1} = avgpool2(S_l).  blockIdx.y: plane.
+__global__ __launch_bounds__(256) void k_skip_grad(const uint16_t* __restrict__ s, const uint16_t* __restrict__ ds,
+                                                   const uint16_t* __restrict__ din, int lg, long nvox, long ps, long psc,
+                                                   uint16_t* __restrict__ out) {
+    const long v = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (v >= nvox) return;
+    const uint4 y = groups(s, blockIdx.y, ps)[v], a = groups(ds, blockIdx.y, ps)[v], b = groups(din, blockIdx.y, psc)[parent(v, lg)];
+    float o[8];
+#pragma unroll
+    for (int c = 0; c < 8; c++) o[c] = group_at(y, c) > 0.f ? group_at(a, c) + 0.125f * group_at(b, c) : 0.f;
+    *const_cast<uint4*>(groups(out, blockIdx.y, ps) + v) = group_of(o);
 }
 
 // Stiffness weight of voxel v: w = rho^3 of the network input (the cell stiffness of the SIMP law).
@@ -429,22 +460,41 @@ __device__ __forceinline__ float net_weight(const uint16_t* in, long v) {
 }
 
 // Per (sample, channel) stiffness-weighted mean of the prediction P [v][kPld] over the sample's g^3
-// voxels, and (channel 0 blocks) the sample's mean weight.
-__global__ __launch_bounds__(256) void k_chan_mean(const float* __restrict__ P, const uint16_t* __restrict__ in, long nsv,
-                                                   float* __restrict__ mean, float* __restrict__ wbar) {
-    __shared__ float sh[2][256];
-    const int b = blockIdx.x, c = blockIdx.y;
-    float s = 0.f, ws = 0.f;
-    for (long v = threadIdx.x; v < nsv; v += blockDim.x) {
-        const long vv = (long)b * nsv + v;
-        const float w = net_weight(in, vv);
-        s += w * P[vv * kPld + c];
+// voxels, and the sample's mean weight.  A sum is 256 chains, of the voxels t, t + 256, ..., then a tree
+// over them.  A wave takes eight chains, eight lanes each: four channels a lane, so that a row of P is read
+// once and not once a channel (36 us and 5 for the trees at 64^3 x 4, 464 with a block a channel); bound by
+// the latency of its loads, 16 of them in flight.
+constexpr int kChains = 256, kMeanRow = 20;  // kOut channels and the weight, padded to the lanes' fours
+
+__global__ __launch_bounds__(64) void k_chan_chains(const float* __restrict__ P, const uint16_t* __restrict__ in, long nsv,
+                                                    float* __restrict__ chains) {
+    const int q = threadIdx.x & 7, t = (int)blockIdx.y * 8 + (threadIdx.x >> 3);
+    const long base = (long)blockIdx.x * nsv;
+    if (q >= kMeanRow / 4) return;
+    float s[4] = {0.f, 0.f, 0.f, 0.f}, ws = 0.f;
+#pragma unroll 16
+    for (long v = t; v < nsv; v += kChains) {
+        const float w = net_weight(in, base + v);
+        const float4 p = *reinterpret_cast<const float4*>(P + (base + v) * kPld + 4 * q);
+        s[0] += w * p.x;
+        s[1] += w * p.y;
+        s[2] += w * p.z;
+        s[3] += w * p.w;
         ws += w;
     }
-    sh[0][threadIdx.x] = s;
-    sh[1][threadIdx.x] = ws;
+    if (q == kOut / 4) s[kOut % 4] = ws;
+#pragma unroll
+    for (int k = 0; k < 4; k++) chains[((long)blockIdx.x * kMeanRow + 4 * q + k) * kChains + t] = s[k];
+}
+
+__global__ __launch_bounds__(kChains) void k_chan_mean(const float* __restrict__ chains, long nsv, float* __restrict__ mean,
+                                                       float* __restrict__ wbar) {
+    __shared__ float sh[2][kChains];
+    const int b = blockIdx.x, c = blockIdx.y;
+    sh[0][threadIdx.x] = chains[((long)b * kMeanRow + c) * kChains + threadIdx.x];
+    sh[1][threadIdx.x] = chains[((long)b * kMeanRow + kOut) * kChains + threadIdx.x];
     __syncthreads();
-    for (int k = 128; k > 0; k >>= 1) {
+    for (int k = kChains / 2; k > 0; k >>= 1) {
         if (threadIdx.x < k) {
             sh[0][threadIdx.x] += sh[0][threadIdx.x + k];
             sh[1][threadIdx.x] += sh[1][threadIdx.x + k];
@@ -458,23 +508,40 @@ __global__ __launch_bounds__(256) void k_chan_mean(const float* __restrict__ P, 
 }
 
 // Loss terms with stiffness weights (w / mean w per sample): d = P - mean_w P - T;
-// dP = 2 (w / wbar) d / count (bf16, [v][kDpLd], channels >= 18 stay 0); per-block FP64 partial sums of
+// dP = 2 (w / wbar) d / count (bf16, channels >= 18 stay 0); per-block FP64 partial sums of
 // (w / wbar) d^2.  T is mean-free under the same weights, so the weighted mean needs no gradient term.
+// A thread takes a group of 8 channels (blockIdx.y: plane); bound by the prediction, target and gradient
+// rows, 190 MB at 64^3 x 4: 52 us (105 with a thread a value).
 __global__ __launch_bounds__(256) void k_head_loss(const float* __restrict__ P, const float* __restrict__ mean,
                                                    const float* __restrict__ wbar, const uint16_t* __restrict__ in,
                                                    const uint16_t* __restrict__ T, long nvox, int lgs, double inv_count,
-                                                   uint16_t* __restrict__ dP, double* __restrict__ partial) {
+                                                   long ps, uint16_t* __restrict__ dP, double* __restrict__ partial) {
     __shared__ double sh[256];
+    const int c0 = 8 * (int)blockIdx.y;
     double s = 0.0;
-    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < nvox * kOut; i += (long)gridDim.x * blockDim.x) {
-        const long v = i / kOut;
-        const int c = (int)(i - v * kOut);
+    for (long v = (long)blockIdx.x * blockDim.x + threadIdx.x; v < nvox; v += (long)gridDim.x * blockDim.x) {
         const long b = v >> (3 * lgs);
         const float wb = wbar[b];
         const float wt = wb > 0.f ? net_weight(in, v) / wb : 0.f;
-        const float d = P[v * kPld + c] - mean[b * kOut + c] - bf2f(T[i]);
-        dP[v * kDpLd + c] = f2bf((float)(2.0 * inv_count) * wt * d);
-        s += (double)wt * d * d;
+        const float4 p0 = *reinterpret_cast<const float4*>(P + v * kPld + c0), p1 = *reinterpret_cast<const float4*>(P + v * kPld + c0 + 4);
+        const float p[8] = {p0.x, p0.y, p0.z, p0.w, p1.x, p1.y, p1.z, p1.w};
+        const uint32_t* t = reinterpret_cast<const uint32_t*>(T + v * kOut + c0);  // kOut and c0 are even
+        float o[8];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const bool live = c0 + 2 * k < kOut;
+            const uint32_t tk = live ? t[k] : 0u;
+#pragma unroll
+            for (int e = 0; e < 2; e++) {
+                o[2 * k + e] = 0.f;
+                if (live) {
+                    const float d = p[2 * k + e] - mean[b * kOut + c0 + 2 * k + e] - bf2f((uint16_t)(tk >> (16 * e)));
+                    o[2 * k + e] = (float)(2.0 * inv_count) * wt * d;
+                    s += (double)wt * d * d;
+                }
+            }
+        }
+        *reinterpret_cast<uint4*>(dP + group(v, c0, ps)) = group_of(o);
     }
     sh[threadIdx.x] = s;
     __syncthreads();
@@ -482,7 +549,7 @@ __global__ __launch_bounds__(256) void k_head_loss(const float* __restrict__ P, 
         if (threadIdx.x < k) sh[threadIdx.x] += sh[threadIdx.x + k];
         __syncthreads();
     }
-    if (threadIdx.x == 0) partial[blockIdx.x] = sh[0];
+    if (threadIdx.x == 0) partial[blockIdx.y * gridDim.x + blockIdx.x] = sh[0];
 }
 
 // Adam on the FP32 master parameters (c1 = 1 / (1 - b1^t), c2 = 1 / (1 - b2^t)).
@@ -500,8 +567,8 @@ __global__ __launch_bounds__(256) void k_adam(long n, const float* __restrict__ 
 }
 
 // bf16 weight layouts of one layer from the master W[co][t][ci] (cin real input channels):
-// forward Wf[r][k], k = t cinp + ci (rows r < rows_f, zero outside co < cout, ci < cin, k < taps cinp);
-// input-gradient Wb[r][k], r = ci, k = t' coutp + co, Wb = W[co][flip t'][ci] (flip t = 26 - t for 3x3x3).
+// forward Wf[k / 8][r][k % 8], k = t cinp + ci (rows r < rows_f, zero outside co < cout, ci < cin, k < taps cinp);
+// input-gradient Wb likewise, r = ci, k = t' coutp + co, Wb = W[co][flip t'][ci] (flip t = 26 - t for 3x3x3).
 __global__ __launch_bounds__(256) void k_pack(const float* __restrict__ W, const float* __restrict__ bias, int cout,
                                               int cin, int cinp, int taps, int rows_f, int kpad_f,
                                               uint16_t* __restrict__ wf, float* __restrict__ bias_pad, int coutp,
@@ -513,7 +580,7 @@ __global__ __launch_bounds__(256) void k_pack(const float* __restrict__ W, const
         const int t = k / cinp, ci = k % cinp;
         float v = 0.f;
         if (r < cout && t < taps && ci < cin) v = W[((long)r * taps + t) * cin + ci];
-        wf[i] = f2bf(v);
+        wf[((long)(k >> 3) * rows_f + r) * 8 + (k & 7)] = f2bf(v);
         if (k == 0) bias_pad[r] = r < cout ? bias[r] : 0.f;
     } else if (i < nf + nbk) {
         const long j = i - nf;
@@ -521,7 +588,7 @@ __global__ __launch_bounds__(256) void k_pack(const float* __restrict__ W, const
         const int t = k / coutp, co = k % coutp;
         float v = 0.f;
         if (r < cin && t < taps && co < cout) v = W[((long)co * taps + (taps == 27 ? 26 - t : t)) * cin + r];
-        wb[j] = f2bf(v);
+        wb[((long)(k >> 3) * rows_b + r) * 8 + (k & 7)] = f2bf(v);
     }
 }
 
@@ -568,17 +635,17 @@ struct NetLayer {
 
 struct NetLevel {
     int g, lg, c;
-    long nvox;                   // batch_max g^3
-    uint16_t* in = nullptr;      // level 0: input [v][8]; else avgpool2(S_{l-1}) [v][c_{l-1}]
-    uint16_t* e = nullptr;       // E_l [v][c]
-    uint16_t* cat = nullptr;     // CAT_l [v][c_{l+1} + c] (S_l at offset c_{l+1}); l < L-1
-    uint16_t* s = nullptr;       // S_{L-1} [v][c] at the bottom level
-    uint16_t* d1 = nullptr;      // decoder first conv [v][c]
-    uint16_t* d = nullptr;       // D_l [v][c]
-    uint16_t* ga = nullptr;      // gradient scratch [v][c] x 2
+    long nvox;                   // batch_max g^3, the length of a plane
+    uint16_t* in = nullptr;      // level 0: input, 8 channels; else avgpool2(S_{l-1}), c_{l-1}
+    uint16_t* e = nullptr;       // E_l
+    uint16_t* cat = nullptr;     // CAT_l, c_{l+1} + c channels (S_l at offset c_{l+1}); l < L-1
+    uint16_t* s = nullptr;       // S_{L-1} at the bottom level
+    uint16_t* d1 = nullptr;      // decoder first conv
+    uint16_t* d = nullptr;       // D_l
+    uint16_t* ga = nullptr;      // gradient scratch, c channels each
     uint16_t* gb = nullptr;
     uint16_t* dcat = nullptr;    // gradient of CAT_l
-    uint16_t* din = nullptr;     // gradient of in_l (l > 0) [v][c_{l-1}]
+    uint16_t* din = nullptr;     // gradient of in_l (l > 0), c_{l-1} channels
 };
 
 struct homo3d_net {
@@ -592,11 +659,12 @@ struct homo3d_net {
     long adam_t = 0;
     float* P = nullptr;          // prediction [v][kPld]
     uint16_t* T = nullptr;       // targets [v][18]
-    uint16_t* dP = nullptr;      // [v][kDpLd]
+    uint16_t* dP = nullptr;      // kDpC channels
     float* mean = nullptr;       // [batch][18]
     float* wbar = nullptr;       // [batch] mean stiffness weight
+    float* chains = nullptr;     // [batch][kMeanRow][kChains] their sums in parts
     double* lpart = nullptr;     // loss partial sums
-    int lblocks = 1024;
+    int lblocks = 512 * kPlanes;
     float* rho = nullptr;        // host-staged densities [batch][g^3]
     float* tstage = nullptr;     // [batch][g^3][18]: host-staged targets, or a prediction on its way to the host
     float* partial = nullptr;    // the weight gradient's partial sums
@@ -629,45 +697,65 @@ int nerr(homo3d_net* n, int code, const char* fmt, ...) {
 
 int pick_mb(int cout) { return cout >= 128 ? 8 : cout >= 64 ? 4 : cout >= 32 ? 2 : 1; }
 
-template <int MB, bool TAP27, bool RELU, bool F32OUT>
-void conv_mb(hipStream_t s, const uint16_t* in, int ldi, int cin, const uint16_t* w, int kpad, const float* bias,
-             void* out, int ldo, int cout, int lg, long nvox) {
-    constexpr int NB = 8 / MB;
-    const dim3 grid((unsigned)((nvox + 64 * NB - 1) / (64 * NB)), (unsigned)((cout + 16 * MB - 1) / (16 * MB)));
-    hipLaunchKernelGGL((k_conv<MB, NB, TAP27, RELU, F32OUT>), grid, dim3(256), 0, s, in, ldi, cin, w, kpad, bias, out, ldo,
-                       cout, lg, nvox);
+struct ConvArgs {
+    const uint16_t* in;
+    int cin;
+    const uint16_t* w;
+    int kpad, rows;
+    const float* bias;
+    void* out;
+    int cout, lg;
+    long nvox, ps;
+    const uint16_t* relu;
+};
+
+template <int MB, int NB, bool TAP27, bool RELU, bool F32OUT>
+void conv_tile(hipStream_t s, const ConvArgs& a) {
+    const dim3 grid((unsigned)((a.nvox + 64 * NB - 1) / (64 * NB)), (unsigned)((a.cout + 16 * MB - 1) / (16 * MB)));
+    hipLaunchKernelGGL((k_conv<MB, NB, TAP27, RELU, F32OUT>), grid, dim3(256), 0, s, a.in, a.cin, a.w, a.kpad, a.rows,
+                       a.bias, a.out, a.cout, a.lg, a.nvox, a.ps, a.relu);
 }
 
+// A wave's tile: 8 products of 16 x 16 a chunk (mb rows of weights, the layer's padding) where that gives
+// every SIMD two waves (2048 waves), else 2, and 1 below that again: a wave walks the whole reduction, and
+// it is its latency that the small levels wait for.  64 channels at 16^3 x 4: 21 us with 2 products, and
+// 128 channels at 8^3 x 4 13 us with 1, against 58 and 86 with 8 (and operands 64 cache lines a load apart).
 template <bool TAP27, bool RELU, bool F32OUT>
-void conv_any(hipStream_t s, int mb, const uint16_t* in, int ldi, int cin, const uint16_t* w, int kpad, const float* bias,
-              void* out, int ldo, int cout, int lg, long nvox) {
-    switch (mb) {
-        case 1: conv_mb<1, TAP27, RELU, F32OUT>(s, in, ldi, cin, w, kpad, bias, out, ldo, cout, lg, nvox); break;
-        case 2: conv_mb<2, TAP27, RELU, F32OUT>(s, in, ldi, cin, w, kpad, bias, out, ldo, cout, lg, nvox); break;
-        case 4: conv_mb<4, TAP27, RELU, F32OUT>(s, in, ldi, cin, w, kpad, bias, out, ldo, cout, lg, nvox); break;
-        default: conv_mb<8, TAP27, RELU, F32OUT>(s, in, ldi, cin, w, kpad, bias, out, ldo, cout, lg, nvox); break;
-    }
-}
-
-// forward pass of one layer: out = act(conv(in) + b)
-void layer_fwd(homo3d_net* n, const NetLayer& Ly, const uint16_t* in, int ldi, void* out, int ldo, int lg, long nvox,
-               bool f32out) {
-    if (Ly.taps == 27)
-        conv_any<true, true, false>(n->stream, Ly.mb_f, in, ldi, Ly.cinp, Ly.wf, Ly.kpad_f, Ly.bias_pad, out, ldo, Ly.cout,
-                                    lg, nvox);
-    else if (f32out)
-        conv_any<false, false, true>(n->stream, Ly.mb_f, in, ldi, Ly.cinp, Ly.wf, Ly.kpad_f, Ly.bias_pad, out, ldo,
-                                     Ly.cout, lg, nvox);
-}
-
-// input gradient of one layer: dX (dense or strided [v][ldo]) = conv(dZ, Wb)
-void layer_dx(homo3d_net* n, const NetLayer& Ly, const uint16_t* dz, int ldz, int cz, uint16_t* dx, int ldo, int lg,
-              long nvox) {
-    if (Ly.taps == 27)
-        conv_any<true, false, false>(n->stream, Ly.mb_b, dz, ldz, cz, Ly.wb, Ly.kpad_b, nullptr, dx, ldo, Ly.cin, lg, nvox);
+void conv_any(hipStream_t s, int mb, const ConvArgs& a) {
+    const long products = a.nvox / 16 * ((a.cout + 15) / 16);
+    if (products < 2048 * 2)
+        conv_tile<1, 1, TAP27, RELU, F32OUT>(s, a);
+    else if (products < 2048 * 8 && mb > 1)
+        conv_tile<2, 1, TAP27, RELU, F32OUT>(s, a);
+    else if (products < 2048 * 8)
+        conv_tile<1, 2, TAP27, RELU, F32OUT>(s, a);
     else
-        conv_any<false, false, false>(n->stream, Ly.mb_b, dz, ldz, cz, Ly.wb, Ly.kpad_b, nullptr, dx, ldo, Ly.cin, lg,
-                                      nvox);
+        switch (mb) {
+            case 1: conv_tile<1, 8, TAP27, RELU, F32OUT>(s, a); break;
+            case 2: conv_tile<2, 4, TAP27, RELU, F32OUT>(s, a); break;
+            case 4: conv_tile<4, 2, TAP27, RELU, F32OUT>(s, a); break;
+            default: conv_tile<8, 1, TAP27, RELU, F32OUT>(s, a); break;
+        }
+}
+
+// forward pass of one layer at level V: out = act(conv(in) + b)
+void layer_fwd(homo3d_net* n, const NetLayer& Ly, const uint16_t* in, void* out, const NetLevel& V, long nvox, bool f32out) {
+    const ConvArgs a = {in, Ly.cinp, Ly.wf, Ly.kpad_f, Ly.rows_f, Ly.bias_pad, out, Ly.cout, V.lg, nvox, V.nvox, nullptr};
+    if (Ly.taps == 27)
+        conv_any<true, true, false>(n->stream, Ly.mb_f, a);
+    else if (f32out)
+        conv_any<false, false, true>(n->stream, Ly.mb_f, a);
+}
+
+// input gradient of one layer at level V: dX = conv(dZ, Wb), where relu (the layer's input, if that is a
+// ReLU's output) is positive; cz channels of dZ
+void layer_dx(homo3d_net* n, const NetLayer& Ly, const uint16_t* dz, int cz, uint16_t* dx, const NetLevel& V, long nvox,
+              const uint16_t* relu) {
+    const ConvArgs a = {dz, cz, Ly.wb, Ly.kpad_b, Ly.rows_b, nullptr, dx, Ly.cin, V.lg, nvox, V.nvox, relu};
+    if (Ly.taps == 27)
+        conv_any<true, false, false>(n->stream, Ly.mb_b, a);
+    else
+        conv_any<false, false, false>(n->stream, Ly.mb_b, a);
 }
 
 // How the weight gradient of a layer is split: wc output-channel tiles a block, `splits` ranges of `per` tiles.
@@ -694,41 +782,38 @@ WgPlan wgrad_plan(int cz, int cx, int taps, int lg, long nvox) {
 }
 
 template <int TX, int TZ, bool TAP27>
-void wgrad(hipStream_t s, const WgPlan& w, const uint16_t* dz, int ldz, int cz, const uint16_t* x, int ldx, int cx, int lg,
+void wgrad(hipStream_t s, const WgPlan& w, const uint16_t* dz, int cz, const uint16_t* x, int cx, int lg, long ps,
            float* partial, float* bpartial) {
     using W = WgTile<TX, 4, TZ, TAP27>;
     const dim3 grid((unsigned)w.splits, (unsigned)(w.czp / (16 * w.wc)), (unsigned)(w.cxp / 16));
-    hipLaunchKernelGGL((k_wgrad<TX, 4, TZ, TAP27>), grid, dim3(256), W::lds(w.wc), s, dz, ldz, cz, x, ldx, cx, lg, w.tiles,
+    hipLaunchKernelGGL((k_wgrad<TX, 4, TZ, TAP27>), grid, dim3(256), W::lds(w.wc), s, dz, cz, x, cx, lg, ps, w.tiles,
                        w.per, w.wc, w.czp, w.cxp, partial, bpartial);
 }
 
-// weight and bias gradient of one layer into n->g: X the layer input view (ldx, cx stored channels),
-// dZ the output gradient view (ldz, cz channels with cz >= cout; both counts multiples of 8).
-int layer_dw(homo3d_net* n, const NetLayer& Ly, const uint16_t* x, int ldx, int cx, const uint16_t* dz, int ldz, int cz,
-             int lg, long nvox) {
+// weight and bias gradient of one layer at level V into n->g: X the layer's input (cx stored channels), dZ the
+// gradient of its output (cz channels with cz >= cout; both counts multiples of 8).
+int layer_dw(homo3d_net* n, const NetLayer& Ly, const uint16_t* x, int cx, const uint16_t* dz, int cz, const NetLevel& V,
+             long nvox) {
+    const int lg = V.lg;
     const WgPlan w = wgrad_plan(cz, cx, Ly.taps, lg, nvox);
     if (w.partial() * (Ly.taps * w.cxp + 1) > n->partial_elems) return nerr(n, HOMO3D_BAD_ARG, "partial buffer too small");
     float* bp = n->partial + w.partial() * Ly.taps * w.cxp;
     if (Ly.taps != 27)
-        wgrad<64, 2, false>(n->stream, w, dz, ldz, cz, x, ldx, cx, lg, n->partial, bp);
+        wgrad<64, 2, false>(n->stream, w, dz, cz, x, cx, lg, V.nvox, n->partial, bp);
     else if (w.tx == 64)
-        wgrad<64, 2, true>(n->stream, w, dz, ldz, cz, x, ldx, cx, lg, n->partial, bp);
+        wgrad<64, 2, true>(n->stream, w, dz, cz, x, cx, lg, V.nvox, n->partial, bp);
     else if (w.tx == 32)
-        wgrad<32, 4, true>(n->stream, w, dz, ldz, cz, x, ldx, cx, lg, n->partial, bp);
+        wgrad<32, 4, true>(n->stream, w, dz, cz, x, cx, lg, V.nvox, n->partial, bp);
     else if (w.tx == 16)
-        wgrad<16, 4, true>(n->stream, w, dz, ldz, cz, x, ldx, cx, lg, n->partial, bp);
+        wgrad<16, 4, true>(n->stream, w, dz, cz, x, cx, lg, V.nvox, n->partial, bp);
     else
-        wgrad<8, 4, true>(n->stream, w, dz, ldz, cz, x, ldx, cx, lg, n->partial, bp);
+        wgrad<8, 4, true>(n->stream, w, dz, cz, x, cx, lg, V.nvox, n->partial, bp);
     const int tot = Ly.cout * Ly.taps * Ly.cin + Ly.cout;
     int waves = 1;
     while (waves < 16 && 2 * waves <= w.splits) waves *= 2;
     hipLaunchKernelGGL(k_wgrad_reduce, dim3(nblk(tot, 64)), dim3(64 * waves), 0, n->stream, n->partial, bp, w.splits, w.czp,
                        Ly.taps, w.cxp, Ly.cout, Ly.cin, n->g + Ly.off_w, n->g + Ly.off_b);
     return HOMO3D_OK;
-}
-
-void relu_mask(homo3d_net* n, uint16_t* dy, int C, const uint16_t* y, int ldy, long nvox) {
-    hipLaunchKernelGGL(k_relu_mask, dim3(nblk(nvox * C)), dim3(256), 0, n->stream, dy, C, y, ldy, nvox);
 }
 
 int pack_weights(homo3d_net* n) {
@@ -751,16 +836,15 @@ void forward(homo3d_net* n, int batch) {
         const long nv = (long)batch << (3 * V.lg);
         const NetLayer& c1 = n->layers[li++];
         const NetLayer& c2 = n->layers[li++];
-        const int ldi = l == 0 ? kInCh : n->lv[l - 1].c;
-        layer_fwd(n, c1, V.in, ldi, V.e, V.c, V.lg, nv, false);
+        layer_fwd(n, c1, V.in, V.e, V, nv, false);
         if (l < L - 1) {
-            const int cu = n->lv[l + 1].c, ld = cu + V.c;
-            layer_fwd(n, c2, V.e, V.c, V.cat + cu, ld, V.lg, nv, false);
-            const long nvc = nv / 8;
-            hipLaunchKernelGGL(k_pool, dim3(nblk(nvc * V.c)), dim3(256), 0, n->stream, V.cat + cu, ld, V.c, V.lg - 1, nvc,
-                               n->lv[l + 1].in);
+            const NetLevel& W = n->lv[l + 1];
+            uint16_t* S = V.cat + W.c * V.nvox;
+            layer_fwd(n, c2, V.e, S, V, nv, false);
+            hipLaunchKernelGGL(k_pool, dim3(nblk(nv / 8), V.c / 8), dim3(256), 0, n->stream, S, W.lg, nv / 8, V.nvox, W.nvox,
+                               W.in);
         } else {
-            layer_fwd(n, c2, V.e, V.c, V.s, V.c, V.lg, nv, false);
+            layer_fwd(n, c2, V.e, V.s, V, nv, false);
         }
     }
     // decoder
@@ -768,18 +852,16 @@ void forward(homo3d_net* n, int batch) {
         NetLevel& V = n->lv[l];
         const NetLevel& W = n->lv[l + 1];
         const long nv = (long)batch << (3 * V.lg);
-        const uint16_t* dn = l == L - 2 ? W.s : W.d;
-        const int cu = W.c, ld = cu + V.c;
-        hipLaunchKernelGGL(k_up, dim3(nblk(nv * cu)), dim3(256), 0, n->stream, dn, cu, V.lg, nv, V.cat, ld);
+        hipLaunchKernelGGL(k_up, dim3(nblk(nv), W.c / 8), dim3(256), 0, n->stream, l == L - 2 ? W.s : W.d, V.lg, nv, V.nvox,
+                           W.nvox, V.cat);
         const NetLayer& c1 = n->layers[li++];
         const NetLayer& c2 = n->layers[li++];
-        layer_fwd(n, c1, V.cat, ld, V.d1, V.c, V.lg, nv, false);
-        layer_fwd(n, c2, V.d1, V.c, V.d, V.c, V.lg, nv, false);
+        layer_fwd(n, c1, V.cat, V.d1, V, nv, false);
+        layer_fwd(n, c2, V.d1, V.d, V, nv, false);
     }
     const NetLayer& hd = n->layers[li];
     const NetLevel& V0 = n->lv[0];
-    const uint16_t* top = L > 1 ? V0.d : V0.s;
-    layer_fwd(n, hd, top, V0.c, n->P, kPld, V0.lg, (long)batch << (3 * V0.lg), true);
+    layer_fwd(n, hd, L > 1 ? V0.d : V0.s, n->P, V0, (long)batch << (3 * V0.lg), true);
 }
 
 // Loss of the prediction against n->T and the full parameter gradient into n->g.
@@ -788,62 +870,52 @@ int loss_backward(homo3d_net* n, int batch, double* loss) {
     const NetLevel& V0 = n->lv[0];
     const long nv0 = (long)batch << (3 * V0.lg);
     const long nsv = 1L << (3 * V0.lg);
-    hipLaunchKernelGGL(k_chan_mean, dim3(batch, kOut), dim3(256), 0, n->stream, n->P, V0.in, nsv, n->mean, n->wbar);
+    hipLaunchKernelGGL(k_chan_chains, dim3(batch, kChains / 8), dim3(64), 0, n->stream, n->P, V0.in, nsv, n->chains);
+    hipLaunchKernelGGL(k_chan_mean, dim3(batch, kOut), dim3(kChains), 0, n->stream, n->chains, nsv, n->mean, n->wbar);
     const double inv = 1.0 / ((double)nv0 * kOut);
-    hipLaunchKernelGGL(k_head_loss, dim3(n->lblocks), dim3(256), 0, n->stream, n->P, n->mean, n->wbar, V0.in, n->T, nv0,
-                       V0.lg, inv, n->dP, n->lpart);
+    hipLaunchKernelGGL(k_head_loss, dim3(n->lblocks / kPlanes, kPlanes), dim3(256), 0, n->stream, n->P, n->mean, n->wbar, V0.in, n->T, nv0,
+                       V0.lg, inv, V0.nvox, n->dP, n->lpart);
     int li = (int)n->layers.size() - 1;
     int rc;
     // head
     {
         const NetLayer& hd = n->layers[li--];
         const uint16_t* top = L > 1 ? V0.d : V0.s;
-        if ((rc = layer_dw(n, hd, top, V0.c, V0.c, n->dP, kDpLd, kDpC, V0.lg, nv0))) return rc;
-        layer_dx(n, hd, n->dP, kDpLd, kDpC, V0.ga, V0.c, V0.lg, nv0);  // dD_0
+        if ((rc = layer_dw(n, hd, top, V0.c, n->dP, kDpC, V0, nv0))) return rc;
+        layer_dx(n, hd, n->dP, kDpC, V0.ga, V0, nv0, top);  // dZ of dec 0.c2 (L = 1: of enc 0.c2)
     }
     // decoder levels, top down in the parameter list (level 0 first)
     for (int l = 0; l <= L - 2; l++) {
         NetLevel& V = n->lv[l];
+        NetLevel& W = n->lv[l + 1];
         const long nv = (long)batch << (3 * V.lg);
         const NetLayer& c2 = n->layers[li--];
         const NetLayer& c1 = n->layers[li--];
-        const int cu = n->lv[l + 1].c, ld = cu + V.c;
-        relu_mask(n, V.ga, V.c, V.d, V.c, nv);  // dZ of dec l.c2
-        if ((rc = layer_dw(n, c2, V.d1, V.c, V.c, V.ga, V.c, V.c, V.lg, nv))) return rc;
-        layer_dx(n, c2, V.ga, V.c, V.c, V.gb, V.c, V.lg, nv);
-        relu_mask(n, V.gb, V.c, V.d1, V.c, nv);  // dZ of dec l.c1
-        if ((rc = layer_dw(n, c1, V.cat, ld, ld, V.gb, V.c, V.c, V.lg, nv))) return rc;
-        layer_dx(n, c1, V.gb, V.c, V.c, V.dcat, ld, V.lg, nv);
-        // gradient of D_{l+1} (or S_{L-1}) = up2^T of the first cu channels
-        NetLevel& W = n->lv[l + 1];
-        const long nvc = nv / 8;
-        hipLaunchKernelGGL(k_up_back, dim3(nblk(nvc * cu)), dim3(256), 0, n->stream, V.dcat, ld, cu, W.lg, nvc, W.ga);
+        // ga: dZ of dec l.c2, gb: of dec l.c1
+        if ((rc = layer_dw(n, c2, V.d1, V.c, V.ga, V.c, V, nv))) return rc;
+        layer_dx(n, c2, V.ga, V.c, V.gb, V, nv, V.d1);
+        if ((rc = layer_dw(n, c1, V.cat, W.c + V.c, V.gb, V.c, V, nv))) return rc;
+        layer_dx(n, c1, V.gb, V.c, V.dcat, V, nv, nullptr);
+        // dZ of D_{l+1} (or S_{L-1}): up2^T of the first W.c channels
+        hipLaunchKernelGGL(k_up_back, dim3(nblk(nv / 8), W.c / 8), dim3(256), 0, n->stream, V.dcat, W.lg, nv / 8, V.nvox,
+                           W.nvox, l + 1 == L - 1 ? W.s : W.d, W.ga);
     }
-    // encoder, bottom up; lv[L-1].ga holds the gradient of S_{L-1}
+    // encoder, bottom up; lv[L-1].ga holds dZ of S_{L-1}
     for (int l = L - 1; l >= 0; l--) {
         NetLevel& V = n->lv[l];
         const long nv = (long)batch << (3 * V.lg);
         const NetLayer& c2 = n->layers[2 * l + 1];
         const NetLayer& c1 = n->layers[2 * l];
-        const uint16_t* S;
-        int lds;
-        if (l == L - 1) {
-            S = V.s;
-            lds = V.c;
-            relu_mask(n, V.ga, V.c, S, lds, nv);
-        } else {
-            const int cu = n->lv[l + 1].c;
-            S = V.cat + cu;
-            lds = cu + V.c;
-            hipLaunchKernelGGL(k_skip_grad, dim3(nblk(nv * V.c)), dim3(256), 0, n->stream, V.cat, V.dcat, lds, cu, V.c,
-                               n->lv[l + 1].din, V.lg, nv, V.ga);
+        if (l < L - 1) {
+            const NetLevel& W = n->lv[l + 1];
+            const long o = W.c * V.nvox;  // S_l's planes of CAT_l
+            hipLaunchKernelGGL(k_skip_grad, dim3(nblk(nv), V.c / 8), dim3(256), 0, n->stream, V.cat + o, V.dcat + o, W.din,
+                               V.lg, nv, V.nvox, W.nvox, V.ga);
         }
-        if ((rc = layer_dw(n, c2, V.e, V.c, V.c, V.ga, V.c, V.c, V.lg, nv))) return rc;
-        layer_dx(n, c2, V.ga, V.c, V.c, V.gb, V.c, V.lg, nv);
-        relu_mask(n, V.gb, V.c, V.e, V.c, nv);  // dZ of enc l.c1
-        const int ldi = l == 0 ? kInCh : n->lv[l - 1].c;
-        if ((rc = layer_dw(n, c1, V.in, ldi, l == 0 ? kInCh : ldi, V.gb, V.c, V.c, V.lg, nv))) return rc;
-        if (l > 0) layer_dx(n, c1, V.gb, V.c, V.c, V.din, ldi, V.lg, nv);
+        if ((rc = layer_dw(n, c2, V.e, V.c, V.ga, V.c, V, nv))) return rc;
+        layer_dx(n, c2, V.ga, V.c, V.gb, V, nv, V.e);  // dZ of enc l.c1
+        if ((rc = layer_dw(n, c1, V.in, c1.cinp, V.gb, V.c, V, nv))) return rc;
+        if (l > 0) layer_dx(n, c1, V.gb, V.c, V.din, V, nv, nullptr);
     }
     NETCHK(n, hipGetLastError());
     if (loss) {
@@ -893,7 +965,7 @@ void destroy(homo3d_net* n) {
         for (void* q : ptrs)
             if (q) (void)hipFree(q);
     }
-    void* ptrs[] = {n->p, n->g, n->m1, n->m2, n->P, n->T, n->dP, n->mean, n->wbar, n->lpart, n->rho, n->tstage, n->partial, n->ds_in, n->ds_tg};
+    void* ptrs[] = {n->p, n->g, n->m1, n->m2, n->P, n->T, n->dP, n->mean, n->wbar, n->chains, n->lpart, n->rho, n->tstage, n->partial, n->ds_in, n->ds_tg};
     for (void* q : ptrs)
         if (q) (void)hipFree(q);
     if (n->stream) (void)hipStreamDestroy(n->stream);
@@ -1037,12 +1109,13 @@ int homo3d_net_create(const homo3d_net_config* cfg, homo3d_net** out) {
     if (hipMalloc(&n->p, sizeof(float) * n->nparam) || hipMalloc(&n->g, sizeof(float) * n->nparam) ||
         hipMalloc(&n->m1, sizeof(float) * n->nparam) || hipMalloc(&n->m2, sizeof(float) * n->nparam) ||
         hipMalloc(&n->P, sizeof(float) * nv0 * kPld) || hipMalloc(&n->T, sizeof(uint16_t) * nv0 * kOut) ||
-        hipMalloc(&n->dP, sizeof(uint16_t) * nv0 * kDpLd) || hipMalloc(&n->mean, sizeof(float) * B * kOut) || hipMalloc(&n->wbar, sizeof(float) * B) ||
+        hipMalloc(&n->dP, sizeof(uint16_t) * nv0 * kDpC) || hipMalloc(&n->mean, sizeof(float) * B * kOut) || hipMalloc(&n->wbar, sizeof(float) * B) ||
+        hipMalloc(&n->chains, sizeof(float) * B * kMeanRow * kChains) ||
         hipMalloc(&n->lpart, sizeof(double) * n->lblocks) || hipMalloc(&n->rho, sizeof(float) * nv0) ||
         hipMalloc(&n->tstage, sizeof(float) * nv0 * kOut) ||
         hipMalloc(&n->partial, sizeof(float) * max_part))
         return fail(HOMO3D_HIP_ERROR);
-    if (hipMemset(n->dP, 0, sizeof(uint16_t) * nv0 * kDpLd) || hipMemset(n->m1, 0, sizeof(float) * n->nparam) ||
+    if (hipMemset(n->dP, 0, sizeof(uint16_t) * nv0 * kDpC) || hipMemset(n->m1, 0, sizeof(float) * n->nparam) ||
         hipMemset(n->m2, 0, sizeof(float) * n->nparam) || hipMemset(n->P, 0, sizeof(float) * nv0 * kPld))
         return fail(HOMO3D_HIP_ERROR);
     // He-normal initial weights (head: sqrt(1 / cin) / 4), zero biases
