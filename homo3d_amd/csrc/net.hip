@@ -650,7 +650,8 @@ struct NetLevel {
 
 struct homo3d_net {
     homo3d_net_config cfg{};
-    hipStream_t stream = nullptr;
+    hipStream_t stream = nullptr, copy = nullptr;  // copy: targets from the host during the forward pass
+    hipEvent_t copy_start = nullptr, copy_done = nullptr;
     int L = 0;
     std::vector<NetLayer> layers;
     std::vector<NetLevel> lv;
@@ -946,15 +947,21 @@ int stage_inputs(homo3d_net* n, const float* rho, int batch) {
     return HOMO3D_OK;
 }
 
+// On the copy stream, after what the network's stream held before: the 75 MB of a 64^3 x 4 batch (3 ms from
+// pageable memory, the host copying) arrive while the forward pass runs.  The caller has enqueued that pass,
+// and goes on behind copy_done.
 int stage_targets(homo3d_net* n, const float* t, int batch) {
     const long cnt = (1L << (3 * n->lv[0].lg)) * batch * kOut;
-    NETCHK(n, hipMemcpyAsync(n->tstage, t, sizeof(float) * cnt, hipMemcpyHostToDevice, n->stream));
-    hipLaunchKernelGGL(k_f32_to_bf16, dim3(nblk(cnt)), dim3(256), 0, n->stream, n->tstage, cnt, n->T);
+    NETCHK(n, hipMemcpyAsync(n->tstage, t, sizeof(float) * cnt, hipMemcpyHostToDevice, n->copy));
+    hipLaunchKernelGGL(k_f32_to_bf16, dim3(nblk(cnt)), dim3(256), 0, n->copy, n->tstage, cnt, n->T);
+    NETCHK(n, hipEventRecord(n->copy_done, n->copy));
+    NETCHK(n, hipStreamWaitEvent(n->stream, n->copy_done, 0));
     return HOMO3D_OK;
 }
 
 void destroy(homo3d_net* n) {
     if (n->stream) (void)hipStreamSynchronize(n->stream);
+    if (n->copy) (void)hipStreamSynchronize(n->copy);
     for (NetLayer& Ly : n->layers) {
         (void)hipFree(Ly.wf);
         (void)hipFree(Ly.wb);
@@ -968,6 +975,9 @@ void destroy(homo3d_net* n) {
     void* ptrs[] = {n->p, n->g, n->m1, n->m2, n->P, n->T, n->dP, n->mean, n->wbar, n->chains, n->lpart, n->rho, n->tstage, n->partial, n->ds_in, n->ds_tg};
     for (void* q : ptrs)
         if (q) (void)hipFree(q);
+    if (n->copy_start) (void)hipEventDestroy(n->copy_start);
+    if (n->copy_done) (void)hipEventDestroy(n->copy_done);
+    if (n->copy) (void)hipStreamDestroy(n->copy);
     if (n->stream) (void)hipStreamDestroy(n->stream);
     delete n;
 }
@@ -1034,7 +1044,11 @@ int homo3d_net_create(const homo3d_net_config* cfg, homo3d_net** out) {
         return code;
     };
     if (hipSetDevice(cfg->device) != hipSuccess) return fail(HOMO3D_HIP_ERROR);
-    if (hipStreamCreateWithFlags(&n->stream, hipStreamNonBlocking) != hipSuccess) return fail(HOMO3D_HIP_ERROR);
+    if (hipStreamCreateWithFlags(&n->stream, hipStreamNonBlocking) != hipSuccess ||
+        hipStreamCreateWithFlags(&n->copy, hipStreamNonBlocking) != hipSuccess ||
+        hipEventCreateWithFlags(&n->copy_start, hipEventDisableTiming) != hipSuccess ||
+        hipEventCreateWithFlags(&n->copy_done, hipEventDisableTiming) != hipSuccess)
+        return fail(HOMO3D_HIP_ERROR);
     // layers (parameter order: enc0.c1, enc0.c2, ..., enc{L-1}.c2, dec{L-2}.c1, dec{L-2}.c2, ..., dec0.c2, head)
     auto add = [&](int cin, int cinp, int cout, int taps, bool relu, bool need_dx) {
         NetLayer Ly;
@@ -1175,10 +1189,12 @@ int homo3d_net_forward(homo3d_net* n, const float* rho, int batch, float* out) {
 int homo3d_net_loss_grad(homo3d_net* n, const float* rho, const float* target, int batch, double* loss, float* grad) {
     if (!n || !rho || !target || !loss) return HOMO3D_BAD_ARG;
     if (batch < 1 || batch > n->cfg.batch) return nerr(n, HOMO3D_BAD_ARG, "batch %d outside [1, %d]", batch, n->cfg.batch);
+    NETCHK(n, hipEventRecord(n->copy_start, n->stream));
+    NETCHK(n, hipStreamWaitEvent(n->copy, n->copy_start, 0));
     int rc = stage_inputs(n, rho, batch);
-    if (!rc) rc = stage_targets(n, target, batch);
     if (rc) return rc;
     forward(n, batch);
+    if ((rc = stage_targets(n, target, batch))) return rc;
     rc = loss_backward(n, batch, loss);
     if (rc) return rc;
     if (grad) NETCHK(n, hipMemcpyAsync(grad, n->g, sizeof(float) * n->nparam, hipMemcpyDeviceToHost, n->stream));
