@@ -348,7 +348,7 @@ bool op_smooth(homo3d_handle* h, int l, void* u, const float* f, float omega, in
     const int zs = zero_start && !reverse ? 1 : 0;
     if (l == 0 && fine_gs_pairs_ok(L.n)) {  // colours two at a time (same result as one by one)
         const bool dot = dot_out && reverse && u_half;
-        const int G = (int)(L.N / 8 / 256);  // workgroups per pair launch
+        const int G = gs_pair_blocks(L.n);  // workgroups per pair launch
         for (int cc = reverse ? 0 : 2 * pair_begin; cc < (reverse ? 8 : 2 * pair_end); cc += 2) {
             ProfEvent ev;
             prof_begin(h, zs ? kProfGsZero : kProfGs, ev);
@@ -786,9 +786,10 @@ int homo3d_create(const homo3d_config* cfg, homo3d_handle** out) {
         return fail(HOMO3D_HIP_ERROR);
     // element matrix, macro loads and the level-1 Galerkin table
     element_matrix(cfg->youngs_modulus, cfg->poisson_ratio, h->ke);
-    std::vector<float> kef(576), kchi(6 * 24);
+    std::vector<float> kef(kKeFloats), kchi(6 * 24);
     std::vector<double> G(64 * 27 * 9, 0.0);
     for (int i = 0; i < 576; i++) kef[i] = (float)h->ke[i];
+    fine_block_consts(kef.data());
     for (int s = 0; s < 6; s++)
         for (int i = 0; i < 24; i++) {
             double t = 0;
@@ -830,7 +831,7 @@ int homo3d_create(const homo3d_config* cfg, homo3d_handle** out) {
             hipMemcpy(h->d_kchi64, kchi64.data(), sizeof(double) * 144, hipMemcpyHostToDevice))
             return fail(HOMO3D_HIP_ERROR);
     }
-    if (hipMalloc(&h->d_ke, sizeof(float) * 576) || hipMalloc(&h->d_kchi, sizeof(float) * 144) ||
+    if (hipMalloc(&h->d_ke, sizeof(float) * kKeFloats) || hipMalloc(&h->d_kchi, sizeof(float) * 144) ||
         hipMalloc(&h->d_G, sizeof(double) * G.size()) || hipMalloc(&h->d_G32, sizeof(float) * G.size()) || hipMalloc(&h->d_gperm, sizeof(int) * 48) ||
         hipMalloc(&h->d_gflip, sizeof(int) * 48))
         return fail(HOMO3D_HIP_ERROR);
@@ -848,7 +849,7 @@ int homo3d_create(const homo3d_config* cfg, homo3d_handle** out) {
             return fail(HOMO3D_HIP_ERROR);
         h->mfma.table = h->d_ke16;
     }
-    if (hipMemcpy(h->d_ke, kef.data(), sizeof(float) * 576, hipMemcpyHostToDevice) ||
+    if (hipMemcpy(h->d_ke, kef.data(), sizeof(float) * kKeFloats, hipMemcpyHostToDevice) ||
         hipMemcpy(h->d_kchi, kchi.data(), sizeof(float) * 144, hipMemcpyHostToDevice) ||
         hipMemcpy(h->d_G, G.data(), sizeof(double) * G.size(), hipMemcpyHostToDevice) ||
         hipMemcpy(h->d_G32, std::vector<float>(G.begin(), G.end()).data(), sizeof(float) * G.size(),
@@ -1387,10 +1388,17 @@ int homo3d_smooth16(homo3d_handle* h, double omega, int reverse) {
     return HOMO3D_OK;
 }
 
+// The grids that the presmooth entry points accept: colour pairs with every thread in use.
+static bool rows_fill_workgroups(int n) {
+    const long hn = n / 2;
+    return hn <= 256 && 256 % hn == 0 && hn * hn * hn % 256 == 0;
+}
+
 int homo3d_presmooth16(homo3d_handle* h, double omega) {
     int rc = fp16_ready(h);
     if (rc) return rc;
-    if (!residual_after_zero_sweep_ok(h)) return set_err(h, HOMO3D_NO_SUPPORT, "needs fused colour pairs at level 0");
+    if (!rows_fill_workgroups(h->lv[0].n))
+        return set_err(h, HOMO3D_NO_SUPPORT, "needs fused colour pairs at level 0");
     const Level& L = h->lv[0];
     op_smooth(h, 0, h->Z, h->F, (float)omega, 0, true, 1, nullptr, L.r);
     op_residual_after_zero_sweep(h, 0, h->Z, 1, L.r);
@@ -1405,7 +1413,7 @@ int homo3d_presmooth(homo3d_handle* h, int level, double omega) {
     if (!h || level < 1 || level >= h->nl - 1) return HOMO3D_BAD_ARG;
     int rc = require_density(h);
     if (rc) return rc;
-    if (!residual_after_zero_sweep_ok(h, level))
+    if (!residual_after_zero_sweep_ok(h, level) || !rows_fill_workgroups(h->lv[level].n))
         return set_err(h, HOMO3D_NO_SUPPORT, "level %d has no colour pairs", level);
     Level& L = h->lv[level];
     op_smooth(h, level, L.u, L.f, (float)omega, 0, true, 0, nullptr, L.r);

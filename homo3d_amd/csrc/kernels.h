@@ -20,6 +20,11 @@ struct FineMfma {
     int nt;
 };
 // n for which packed-FP16 fine operators run in element form on the matrix cores
+// The FP32 element matrix as the fine-level kernels take it: KE (576 floats), then from kKeBlocks on the
+// block constants C_d,ij = KE[7 - e0][b0](i, j) of each neighbour offset d at 12 d + 3 i + j, for the cell e0
+// with e0_m = 1 exactly where d_m = +1 and b0_m = d_m + 1 - e0_m.
+constexpr int kKeBlocks = 576, kKeFloats = kKeBlocks + 27 * 12;
+void fine_block_consts(float* ke);  // fills them from KE, on the host
 int fine_apply_mfma_ok(int n);
 // out = K u (f == nullptr) or f - K u.  With mf, packed-FP16 u and fine_apply_mfma_ok(n) the operator
 // runs in element form on the matrix cores.
@@ -41,9 +46,10 @@ void launch_fine_gs(hipStream_t s, int n, int colour, float omega, int reverse, 
                     const float* w, void* u, int u_half, const float* f);
 // Colours cfirst and cfirst + 1 (cfirst even; REVERSE: cfirst and cfirst - 1, cfirst odd) in one launch,
 // identical to two launch_fine_gs calls; only when fine_gs_pairs_ok(n).  With partial (reverse sweeps of
-// a packed-FP16 u only), each of the (n/2)^3 / 256 workgroups also writes its FP64 sums of f . u_new per
+// a packed-FP16 u only), each of the gs_pair_blocks(n) workgroups also writes its FP64 sums of f . u_new per
 // load case to partial[r * pstride + workgroup].
 int fine_gs_pairs_ok(int n);
+int gs_pair_blocks(int n);
 // rown (zero-start forward passes; ignored otherwise): both colours also store, per vertex, f minus the
 // K u terms of the colours swept so far (the vertex itself included); after the sweep,
 // launch_fine_residual_later turns these into the residual f - K u.

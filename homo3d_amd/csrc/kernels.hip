@@ -52,8 +52,7 @@ __device__ __forceinline__ void hload9(uint32_t (&wv)[9], Rsrc r, uint32_t idx, 
     wv[8] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(r, (int)(idx * 4u), (int)(8u * plane), 0);
 }
 
-// The element matrix staged in LDS: KE (576 entries) followed by 243 block constants (kBlockConsts),
-// padded so that what follows it stays 16-byte aligned.
+// The FP64 element matrix staged in LDS: KE (576 entries) followed by 243 block constants (kBlockConsts).
 constexpr int kBlockConsts = 576;
 constexpr int kKeStaged = 832;
 
@@ -86,15 +85,34 @@ __device__ __forceinline__ T cell_form(const W wc[8]) {
 // s_i s_j (i != j; s_m = +1 at the upper node of axis m, the sign of every axis along which d is
 // non-zero being the same for all the cells) and one constant (i = j), so
 // S_ij = C_d,ij * (sum of w_e, with the sign s_m(e) for each axis m in {i, j} along which d is zero).
-// C_d,ij (ke[kBlockConsts + 9 d + 3 i + j], set by stage_ke) is the entry of the cell with e_m = 1
-// exactly where d_m = +1.  Four signed sums of two to eight weights and nine products per block,
-// instead of nine FMAs per cell.
-template <int D, typename T, typename W>
-__device__ __forceinline__ void fine_block(const W wc[8], const T* ke, T S[9]) {
+// C_d,ij (BlockConsts) is the entry of the cell with e_m = 1 exactly where d_m = +1.  Four signed sums of
+// two to eight weights and nine products per block, instead of nine FMAs per cell.
+//
+// The constants are wave-uniform and come through the scalar cache (kKeBlocks floats into ke, 12 a block,
+// set when the operator is made), loaded a neighbour ahead: they cost neither vector loads, nor
+// registers, nor the staging of KE at the start of a workgroup.  At 256^3 the CG pass takes 1.67 ms and a
+// colour pair 0.37 ms (1.83 and 0.385 with the constants read from LDS).
+struct BlockConsts {
+    float v[9];
+};
+typedef const __attribute__((address_space(4))) float* KeBlocks;
+
+__device__ __forceinline__ KeBlocks ke_blocks(const float* ke) { return (KeBlocks)(uintptr_t)(ke + kKeBlocks); }
+
+template <int D>
+__device__ __forceinline__ BlockConsts block_consts(KeBlocks kb) {
+    BlockConsts c;
+#pragma unroll
+    for (int k = 0; k < 9; k++) c.v[k] = kb[12 * D + k];
+    return c;
+}
+
+template <int D>
+__device__ __forceinline__ void fine_block(const float wc[8], const BlockConsts& c, float S[9]) {
     constexpr int fm = (D % 3 == 1 ? 1 : 0) | (D / 3 % 3 == 1 ? 2 : 0) | (D / 9 == 1 ? 4 : 0);  // axes with d_m = 0
-    const T* cb = ke + kBlockConsts + 9 * D;
-    const T w0 = cell_form<D, 0, T>(wc);
-    const T fxy = cell_form<D, fm & 3, T>(wc), fxz = cell_form<D, fm & 5, T>(wc), fyz = cell_form<D, fm & 6, T>(wc);
+    const float* cb = c.v;
+    const float w0 = cell_form<D, 0, float>(wc);
+    const float fxy = cell_form<D, fm & 3, float>(wc), fxz = cell_form<D, fm & 5, float>(wc), fyz = cell_form<D, fm & 6, float>(wc);
     S[0] = cb[0] * w0;
     S[4] = cb[4] * w0;
     S[8] = cb[8] * w0;
@@ -268,91 +286,78 @@ __device__ __forceinline__ void pin_acc(T (&acc)[R][3]) {
         for (int i = 0; i < 3; i++) __asm__ volatile("" : "+v"(acc[r][i]));
 }
 
-// One neighbour of the row: issue the loads of the next neighbour, build the 3x3 block of this one
-// from the cell weights and KE (in LDS), accumulate, recurse.
-template <int R, uint32_t MASK, int D, typename T, typename A, bool XL>
-__device__ __forceinline__ void gather_step(const FineCtx& c, int n, const T* ke, Rsrc ru, uint32_t plane, int r0,
-                                            const A (&cur)[R / CasesPerWord<A>::value][3], T (&acc)[R][3],
-                                            const XNbLds<A>& xl) {
+// One neighbour of the row, the loads PF neighbours ahead (buf: a ring of the neighbours in flight, this
+// one, the K-th, in slot K % PF) and the next block's constants (k: this one's) in flight: build the 3x3
+// block from the cell weights, accumulate, recurse.
+template <int R, uint32_t MASK, int PF, int D, int DA, int K, typename A, bool XL>
+__device__ __forceinline__ void gather_step(const FineCtx& c, KeBlocks kb, Rsrc ru, uint32_t plane, int r0,
+                                            const BlockConsts& k, A (&buf)[PF][R / CasesPerWord<A>::value][3],
+                                            float (&acc)[R][3], const XNbLds<A>& xl) {
     constexpr int W = R / CasesPerWord<A>::value;
-    constexpr int DN = next_nb(MASK, D);
+    constexpr int DN = next_nb(MASK, D), DAN = DA < 27 ? next_nb(MASK, DA) : 27;
     // keep each neighbour's block build next to its use (bounds register pressure)
     __builtin_amdgcn_sched_barrier(0);
-    pin_acc<R, T>(acc);
+    pin_acc<R, float>(acc);
     A nxt[W][3];
-    if constexpr (DN < 27) load_nb_at<W, A, XL, DN>(nxt, c, ru, plane, r0, xl);
-    T S[9];
-    if constexpr (sizeof(T) == 8)
-        fine_block<D>(c.wd, ke, S);
-    else
-        fine_block<D>(c.wc, ke, S);
-    block_fma<W, T, A>(S, cur, acc);
-    if constexpr (DN < 27) gather_step<R, MASK, DN, T, A, XL>(c, n, ke, ru, plane, r0, nxt, acc, xl);
+    BlockConsts kn = {};
+    if constexpr (DN < 27) kn = block_consts<DN>(kb);
+    if constexpr (DA < 27) load_nb_at<W, A, XL, DA>(nxt, c, ru, plane, r0, xl);
+    float S[9];
+    fine_block<D>(c.wc, k, S);
+    block_fma<W, float, A>(S, buf[K % PF], acc);
+    if constexpr (DA < 27) {
+#pragma unroll
+        for (int p = 0; p < W; p++)
+#pragma unroll
+            for (int i = 0; i < 3; i++) buf[K % PF][p][i] = nxt[p][i];
+    }
+    if constexpr (DN < 27) gather_step<R, MASK, PF, DN, DAN, K + 1, A, XL>(c, kb, ru, plane, r0, kn, buf, acc, xl);
 }
 
-// The same walk with the loads issued two neighbours ahead (cur: this neighbour, nx1: the next one,
-// already in flight): more loads in flight per wave for the latency-bound gather.
-template <int R, uint32_t MASK, int D, typename T, typename A>
-__device__ __forceinline__ void gather_step2(const FineCtx& c, int n, const T* ke, Rsrc ru, uint32_t plane, int r0,
-                                             const A (&cur)[R / CasesPerWord<A>::value][3],
-                                             const A (&nx1)[R / CasesPerWord<A>::value][3], T (&acc)[R][3]) {
-    constexpr int W = R / CasesPerWord<A>::value;
-    constexpr int DN = next_nb(MASK, D);
-    constexpr int DN2 = DN < 27 ? next_nb(MASK, DN) : 27;
-    __builtin_amdgcn_sched_barrier(0);
-    pin_acc<R, T>(acc);
-    A nx2[W][3];
-    if constexpr (DN2 < 27) load_nb<W, A>(nx2, ru, c.nb(DN2) * (uint32_t)sizeof(A), plane, r0);
-    T S[9];
-    if constexpr (sizeof(T) == 8)
-        fine_block<D>(c.wd, ke, S);
-    else
-        fine_block<D>(c.wc, ke, S);
-    block_fma<W, T, A>(S, cur, acc);
-    if constexpr (DN < 27) {
-        if constexpr (DN2 < 27)
-            gather_step2<R, MASK, DN, T, A>(c, n, ke, ru, plane, r0, nx1, nx2, acc);
-        else
-            gather_step2<R, MASK, DN, T, A>(c, n, ke, ru, plane, r0, nx1, nx1, acc);
+// the first PF neighbours' loads
+template <int W, uint32_t MASK, int PF, int D, int K, typename A, bool XL>
+__device__ __forceinline__ void gather_fill(const FineCtx& c, Rsrc ru, uint32_t plane, int r0, A (&buf)[PF][W][3],
+                                            const XNbLds<A>& xl) {
+    if constexpr (K < PF && D < 27) {
+        load_nb_at<W, A, XL, D>(buf[K], c, ru, plane, r0, xl);
+        gather_fill<W, MASK, PF, next_nb(MASK, D), K + 1, A, XL>(c, ru, plane, r0, buf, xl);
     }
+}
+constexpr int nth_nb(uint32_t mask, int k) {
+    int d = next_nb(mask, -1);
+    for (int i = 0; i < k && d < 27; i++) d = next_nb(mask, d);
+    return d;
 }
 
 // acc[r][i] = sum_d S_d u_{v+d} over the neighbours d selected by MASK, load cases r0..r0+R-1.
-// ke points to the element matrix staged in LDS.  The pinned origin's entries of u are zero by
-// construction (every entry point zeroes them before the fine operator reads u).  XL: the two
-// x-neighbours come from LDS (xl).
-template <int R, uint32_t MASK, typename T, typename A, bool XL = false, int PF = 1>
-__device__ __forceinline__ void fine_gather(const FineCtx& c, int n, size_t N, const T* ke, const A* __restrict__ u,
-                                            T (&acc)[R][3], int r0 = 0, const XNbLds<A>& xl = XNbLds<A>()) {
+// The pinned origin's entries of u are zero by construction (every entry point zeroes them before the
+// fine operator reads u).  XL: the two x-neighbours come from LDS (xl).
+template <int R, uint32_t MASK, typename A, bool XL = false, int PF = 1>
+__device__ __forceinline__ void fine_gather(const FineCtx& c, size_t N, KeBlocks kb, const A* __restrict__ u,
+                                            float (&acc)[R][3], int r0 = 0, const XNbLds<A>& xl = XNbLds<A>()) {
     constexpr int W = R / CasesPerWord<A>::value;
     const Rsrc ru = make_rsrc(u, (size_t)(18 / CasesPerWord<A>::value) * N * sizeof(A));
     const uint32_t plane = (uint32_t)(N * sizeof(A));
 #pragma unroll
     for (int r = 0; r < R; r++)
 #pragma unroll
-        for (int i = 0; i < 3; i++) acc[r][i] = T(0);
+        for (int i = 0; i < 3; i++) acc[r][i] = 0.f;
     constexpr int D0 = next_nb(MASK, -1);
     if constexpr (D0 < 27) {
-        A first[W][3];
-        load_nb_at<W, A, XL, D0>(first, c, ru, plane, r0, xl);
-        if constexpr (PF == 2 && !XL && next_nb(MASK, D0) < 27) {
-            A second[W][3];
-            load_nb<W, A>(second, ru, c.nb(next_nb(MASK, D0)) * (uint32_t)sizeof(A), plane, r0);
-            gather_step2<R, MASK, D0, T, A>(c, n, ke, ru, plane, r0, first, second, acc);
-        } else {
-            gather_step<R, MASK, D0, T, A, XL>(c, n, ke, ru, plane, r0, first, acc, xl);
-        }
+        A buf[PF][W][3];
+        const BlockConsts k = block_consts<D0>(kb);
+        gather_fill<W, MASK, PF, D0, 0, A, XL>(c, ru, plane, r0, buf, xl);
+        gather_step<R, MASK, PF, D0, nth_nb(MASK, PF), 0, A, XL>(c, kb, ru, plane, r0, k, buf, acc, xl);
     }
 }
 
-// Stage the element matrix in LDS (all threads of the block take part), followed, when CONSTS (ke_s
-// then holds kKeStaged entries), by the block constants of fine_block: C_d,ij = KE[7 - e0][b0](i, j)
+// Stage the FP64 element matrix in LDS (all threads of the block take part), followed by the block
+// constants of fine_block: C_d,ij = KE[7 - e0][b0](i, j)
 // for the cell e0 with e0_m = 1 exactly where d_m = +1 and b0_m = d_m + 1 - e0_m.
-template <typename T, bool CONSTS = true>
+template <typename T>
 __device__ __forceinline__ void stage_ke(T* ke_s, const T* __restrict__ ke) {
     for (int i = threadIdx.x; i < 576; i += blockDim.x) ke_s[i] = ke[i];
     __syncthreads();
-    if constexpr (!CONSTS) return;
     for (int t = threadIdx.x; t < 243; t += blockDim.x) {
         const int d = t / 9, i = t / 3 % 3, j = t % 3;
         int e0 = 0, b0 = 0;
@@ -399,8 +404,7 @@ __global__ __launch_bounds__(kFullThreads, 4) void k_fine_apply(Lay L, size_t N,
                                                                 float* __restrict__ pp = nullptr,
                                                                 float* __restrict__ xx = nullptr,
                                                                 const double* __restrict__ alpha = nullptr) {
-    __shared__ float ke_s[kKeStaged];
-    stage_ke(ke_s, ke);
+    const KeBlocks kb = ke_blocks(ke);
     uint32_t v;
     if (!full_vertex(L, xcd_chunk(blockIdx.x, gridDim.x), v)) return;
     int x, y, z;
@@ -408,7 +412,7 @@ __global__ __launch_bounds__(kFullThreads, 4) void k_fine_apply(Lay L, size_t N,
     FineCtx c;
     fine_ctx(c, x, y, z, L, w);
     float acc[R][3];
-    fine_gather<R, kRowAll, float, A, false, PF>(c, L.n, N, ke_s, u, acc);
+    fine_gather<R, kRowAll, A, false, PF>(c, N, kb, u, acc);
     double dot[R];
 #pragma unroll
     for (int r = 0; r < R; r++) {
@@ -486,15 +490,17 @@ __device__ __forceinline__ void staged_nb(half2_t (&dst)[3][3], const uint32_t* 
 }
 
 template <int D>
-__device__ __forceinline__ void staged_step(const FineCtx& c, const float* ke, const uint32_t* zs, const int (&xb)[3],
-                                            const half2_t (&cur)[3][3], float (&acc)[6][3]) {
+__device__ __forceinline__ void staged_step(const FineCtx& c, KeBlocks kb, const BlockConsts& k, const uint32_t* zs,
+                                            const int (&xb)[3], const half2_t (&cur)[3][3], float (&acc)[6][3]) {
     __builtin_amdgcn_sched_barrier(0);
     half2_t nxt[3][3];
+    BlockConsts kn = {};
+    if constexpr (D < 26) kn = block_consts<D + 1>(kb);
     if constexpr (D < 26) staged_nb<D + 1>(nxt, zs, xb);
     float S[9];
-    fine_block<D>(c.wc, ke, S);
+    fine_block<D>(c.wc, k, S);
     block_fma<3, float, half2_t>(S, cur, acc);
-    if constexpr (D < 26) staged_step<D + 1>(c, ke, zs, xb, nxt, acc);
+    if constexpr (D < 26) staged_step<D + 1>(c, kb, kn, zs, xb, nxt, acc);
 }
 
 // Load the workgroup's node box of the packed-FP16 z (tile of chunk t0: half-x bx0.. bx0 + 63, half-y by,
@@ -551,10 +557,8 @@ __global__ __launch_bounds__(kFullThreads, 4) void k_fine_cg_staged(Lay L, size_
                                                                     float* __restrict__ pp, float* __restrict__ xx,
                                                                     const double* __restrict__ alpha) {
     static_assert(BETA == (PX == 2), "the first pass (PX 1) has no beta; later passes (PX 2) have both");
-    // one LDS array with KE first: its wave-uniform reads then take immediate offsets below 64 KB
-    __shared__ uint32_t lds[kKeStaged + 9 * kStPlane];
-    float* ke_s = reinterpret_cast<float*>(lds);
-    uint32_t* zs = lds + kKeStaged;
+    __shared__ uint32_t zs[9 * kStPlane];
+    const KeBlocks kb = ke_blocks(ke);
     const int h = L.h;
     const uint32_t t0 = xcd_chunk(blockIdx.x, gridDim.x) * 64u;
     const int bx0 = (int)(t0 % (uint32_t)h), by = (int)((t0 / (uint32_t)h) % (uint32_t)h);
@@ -595,7 +599,7 @@ __global__ __launch_bounds__(kFullThreads, 4) void k_fine_cg_staged(Lay L, size_
             }
         }
     }
-    stage_ke(ke_s, ke);  // ends with the workgroup barrier that also publishes the staged box
+    __syncthreads();  // the staged box
     const int px = b & 1, py = (b >> 1) & 1, pz = b >> 2;
     const int x = 2 * (bx0 + lane) + px, y = 2 * by + py, zc = 2 * bz + pz;
     FineCtx c;
@@ -610,7 +614,7 @@ __global__ __launch_bounds__(kFullThreads, 4) void k_fine_cg_staged(Lay L, size_
     {
         half2_t first[3][3];
         staged_nb<0>(first, zs, xb);
-        staged_step<0>(c, ke_s, zs, xb, first, acc);
+        staged_step<0>(c, kb, block_consts<0>(kb), zs, xb, first, acc);
     }
     half2_t zv[3][3];  // z of the vertex itself (d = 13)
     staged_nb<13>(zv, zs, xb);
@@ -945,6 +949,10 @@ __global__ __launch_bounds__(kEfThreads, 2) void k_fine_apply_ef(Lay L, size_t N
     }
 }
 
+// neighbours whose loads are in flight ahead of the smoother's block products
+template <typename A>
+constexpr int kGsAhead = CasesPerWord<A>::value == 2 ? 3 : 1;
+
 // GS / SOR update of the colour vertex v (load cases r0 .. r0 + R - 1), in place.  A: storage of u
 // (float, or half2_t pairs of load cases); f is FP32.  ZC >= 0: colour ZC of a forward sweep that
 // starts from u = 0 (colours above ZC are never read, so u needs no clearing beforehand; the old value
@@ -955,7 +963,7 @@ __global__ __launch_bounds__(kEfThreads, 2) void k_fine_apply_ef(Lay L, size_t N
 // stored values; once the sweep is complete, subtracting the later colours' terms gives f - K u.
 // The pinned origin keeps u = 0 (and rown = 0).
 template <int R, bool REVERSE, int ZC, typename A, bool XL, bool TO_LDS, bool DOT = false, bool ROWN = false>
-__device__ __forceinline__ void gs_vertex(const Lay& L, size_t N, uint32_t v, float omega, const float* ke_s,
+__device__ __forceinline__ void gs_vertex(const Lay& L, size_t N, uint32_t v, float omega, KeBlocks kb,
                                           const float* __restrict__ w, A* __restrict__ u,
                                           const float* __restrict__ f, int r0, const XNbLds<A>& xl, A* out_lds,
                                           float* dot = nullptr, float* __restrict__ rown = nullptr) {
@@ -966,9 +974,9 @@ __device__ __forceinline__ void gs_vertex(const Lay& L, size_t N, uint32_t v, fl
     FineCtx c;
     fine_ctx(c, x, y, z, L, w);
     float acc[R][3];
-    fine_gather<R, gs_mask(ZC), float, A, XL>(c, L.n, N, ke_s, u, acc, r0, xl);
+    fine_gather<R, gs_mask(ZC), A, XL, kGsAhead<A>>(c, N, kb, u, acc, r0, xl);
     float Ks[9];
-    fine_block<13, float>(c.wc, ke_s, Ks);
+    fine_block<13>(c.wc, block_consts<13>(kb), Ks);
     const float inv[3] = {1.f / Ks[0], 1.f / Ks[4], 1.f / Ks[8]};
     const bool pin = v == 0;
 #pragma unroll
@@ -1034,11 +1042,10 @@ template <int R, bool REVERSE, int ZC, typename A>
 __global__ __launch_bounds__(256, 4) void k_fine_gs(Lay L, size_t N, int colour, float omega,
                                                     const float* __restrict__ ke, const float* __restrict__ w,
                                                     A* __restrict__ u, const float* __restrict__ f) {
-    __shared__ float ke_s[kKeStaged];
-    stage_ke(ke_s, ke);
+    const KeBlocks kb = ke_blocks(ke);
     const uint32_t t = xcd_chunk(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
     if (t >= L.h3) return;
-    gs_vertex<R, REVERSE, ZC, A, false, false>(L, N, colour_block(colour) * L.h3 + t, omega, ke_s, w, u, f,
+    gs_vertex<R, REVERSE, ZC, A, false, false>(L, N, colour_block(colour) * L.h3 + t, omega, kb, w, u, f,
                                               R == 6 ? 0 : (int)blockIdx.y * R, XNbLds<A>(), nullptr);
 }
 
@@ -1047,9 +1054,9 @@ __global__ __launch_bounds__(256, 4) void k_fine_gs(Lay L, size_t N, int colour,
 // per load case to partial[r * pstride + blockIdx.x] (over the four pair launches of a sweep that is
 // the last to write u, this is the r . z of the CG step).  The two colours differ only in x-parity, and a vertex of the
 // second depends on the first only through its x-neighbours, which lie in the same grid row.  Each
-// workgroup owns whole rows (256 % (n/2) == 0, (n/2)^3 % 256 == 0, checked by the launcher): it
-// updates the first colour of its rows, keeps the new values in LDS, and updates the second colour
-// reading those x-neighbours from LDS.  Other workgroups never read the rows' first-colour values
+// workgroup owns as many whole rows of n/2 as 256 threads hold (pair_rows; n <= 512, the rest of the
+// threads and of the last workgroup idle): it updates the first colour of its rows, keeps the new values
+// in LDS, and updates the second colour reading those x-neighbours from LDS.  Other workgroups never read the rows' first-colour values
 // before they are final, so the result equals the two colour passes in sequence.
 // ROWN (zero-start passes): both colours also store their own-colour residuals to rown (gs_vertex).
 template <int R, bool REVERSE, int ZC, typename A, bool DOT = false, bool ROWN = false>
@@ -1059,25 +1066,29 @@ __global__ __launch_bounds__(256, 4) void k_fine_gs2(Lay L, size_t N, int cfirst
                                                      double* __restrict__ partial, int pstride,
                                                      float* __restrict__ rown) {
     constexpr int W = R / CasesPerWord<A>::value;
-    __shared__ float ke_s[kKeStaged];
     __shared__ A xs[3 * W * 256];
-    stage_ke(ke_s, ke);
-    const uint32_t t = xcd_chunk(blockIdx.x, gridDim.x) * 256u + threadIdx.x;
+    const KeBlocks kb = ke_blocks(ke);
+    const int h = L.h, span = pair_rows(h) * h;
+    const uint32_t t = xcd_chunk(blockIdx.x, gridDim.x) * (uint32_t)span + threadIdx.x;
+    const bool live = (int)threadIdx.x < span && t < L.h3;
     const int c2 = REVERSE ? cfirst - 1 : cfirst + 1;
     float dot[R];
 #pragma unroll
     for (int r = 0; r < R; r++) dot[r] = 0.f;
-    gs_vertex<R, REVERSE, ZC, A, false, true, DOT, ROWN>(L, N, colour_block(cfirst) * L.h3 + t, omega, ke_s, w, u,
-                                                        f, 0, XNbLds<A>(), xs, dot, rown);
+    if (live)
+        gs_vertex<R, REVERSE, ZC, A, false, true, DOT, ROWN>(L, N, colour_block(cfirst) * L.h3 + t, omega, kb, w, u,
+                                                            f, 0, XNbLds<A>(), xs, dot, rown);
     __syncthreads();
-    XNbLds<A> xl;
-    xl.base = xs;
-    const int h = L.h, lx = (int)(t % (uint32_t)h), row0 = (int)threadIdx.x - lx;
-    const bool odd = (colour_block(c2) & 1u) != 0;  // x-parity of the second colour
-    xl.slot[0] = row0 + (odd ? lx : (lx == 0 ? h - 1 : lx - 1));
-    xl.slot[1] = row0 + (odd ? (lx + 1 == h ? 0 : lx + 1) : lx);
-    gs_vertex<R, REVERSE, (ZC < 0 ? -1 : ZC + 1), A, true, false, DOT, ROWN>(
-        L, N, colour_block(c2) * L.h3 + t, omega, ke_s, w, u, f, 0, xl, nullptr, dot, rown);
+    if (live) {
+        XNbLds<A> xl;
+        xl.base = xs;
+        const int lx = (int)(t % (uint32_t)h), row0 = (int)threadIdx.x - lx;
+        const bool odd = (colour_block(c2) & 1u) != 0;  // x-parity of the second colour
+        xl.slot[0] = row0 + (odd ? lx : (lx == 0 ? h - 1 : lx - 1));
+        xl.slot[1] = row0 + (odd ? (lx + 1 == h ? 0 : lx + 1) : lx);
+        gs_vertex<R, REVERSE, (ZC < 0 ? -1 : ZC + 1), A, true, false, DOT, ROWN>(
+            L, N, colour_block(c2) * L.h3 + t, omega, kb, w, u, f, 0, xl, nullptr, dot, rown);
+    }
     if constexpr (DOT) {
         __shared__ double sh[4];
 #pragma unroll
@@ -1096,7 +1107,7 @@ __global__ __launch_bounds__(256, 4) void k_fine_gs2(Lay L, size_t N, int cfirst
 // gathered FP16 words inside the FMAs (v_fma_mix); with independent components it converts every word
 // up front and spills.
 template <int R, int C, typename A>
-__device__ __forceinline__ void later_vertex(const Lay& L, size_t N, uint32_t v, const float* ke_s,
+__device__ __forceinline__ void later_vertex(const Lay& L, size_t N, uint32_t v, KeBlocks kb,
                                              const float* __restrict__ w, const A* __restrict__ u,
                                              float* __restrict__ r, float zero) {
     int x, y, z;
@@ -1104,7 +1115,7 @@ __device__ __forceinline__ void later_vertex(const Lay& L, size_t N, uint32_t v,
     FineCtx c;
     fine_ctx(c, x, y, z, L, w);
     float acc[R][3];
-    fine_gather<R, later_mask(C), float, A>(c, L.n, N, ke_s, u, acc);
+    fine_gather<R, later_mask(C), A>(c, N, kb, u, acc);
 #pragma unroll
     for (int q = 0; q < R; q++) {
         float ro[3], rn[3];
@@ -1128,24 +1139,23 @@ template <int R, typename A>
 __global__ __launch_bounds__(256) void k_fine_resid_later(Lay L, size_t N, const float* __restrict__ ke,
                                                           const float* __restrict__ w, const A* __restrict__ u,
                                                           float* __restrict__ r, float zero) {
-    __shared__ float ke_s[kKeStaged];
-    stage_ke(ke_s, ke);
+    const KeBlocks kb = ke_blocks(ke);
     const uint32_t t = xcd_chunk(blockIdx.x, gridDim.x) * 64u + (threadIdx.x & 63u);
     if (t >= L.h3) return;
     const uint32_t h3 = L.h3;
     switch (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) {
-        case 0: later_vertex<R, 0, A>(L, N, 7 * h3 + t, ke_s, w, u, r, zero); break;  // colour 7: none
+        case 0: later_vertex<R, 0, A>(L, N, 7 * h3 + t, kb, w, u, r, zero); break;  // colour 7: none
         case 1:
-            later_vertex<R, 1, A>(L, N, 6 * h3 + t, ke_s, w, u, r, zero);
-            later_vertex<R, 6, A>(L, N, 1 * h3 + t, ke_s, w, u, r, zero);
+            later_vertex<R, 1, A>(L, N, 6 * h3 + t, kb, w, u, r, zero);
+            later_vertex<R, 6, A>(L, N, 1 * h3 + t, kb, w, u, r, zero);
             break;
         case 2:
-            later_vertex<R, 2, A>(L, N, 5 * h3 + t, ke_s, w, u, r, zero);
-            later_vertex<R, 5, A>(L, N, 2 * h3 + t, ke_s, w, u, r, zero);
+            later_vertex<R, 2, A>(L, N, 5 * h3 + t, kb, w, u, r, zero);
+            later_vertex<R, 5, A>(L, N, 2 * h3 + t, kb, w, u, r, zero);
             break;
         default:
-            later_vertex<R, 3, A>(L, N, 4 * h3 + t, ke_s, w, u, r, zero);
-            later_vertex<R, 4, A>(L, N, 3 * h3 + t, ke_s, w, u, r, zero);
+            later_vertex<R, 3, A>(L, N, 4 * h3 + t, kb, w, u, r, zero);
+            later_vertex<R, 4, A>(L, N, 3 * h3 + t, kb, w, u, r, zero);
             break;
     }
 }
@@ -1573,15 +1583,19 @@ __global__ __launch_bounds__(256) void k_stencil_gs2(Lay L, size_t N, int cfirst
                                                      const float* __restrict__ f, float* __restrict__ rown) {
     constexpr int W = R / CasesPerWord<A>::value;
     __shared__ A xs[3 * W * 256];
-    const uint32_t t = xcd_chunk(blockIdx.x, gridDim.x) * 256u + threadIdx.x;
+    const int h = L.h, span = pair_rows(h) * h;
+    const uint32_t t = xcd_chunk(blockIdx.x, gridDim.x) * (uint32_t)span + threadIdx.x;
+    const bool live = (int)threadIdx.x < span && t < L.h3;
     const int c2 = REVERSE ? cfirst - 1 : cfirst + 1;
     const int r0 = blockIdx.y * R;
-    stencil_gs_vertex<R, REVERSE, ZC, SA, A, false, true, ROWN>(L, N, colour_block(cfirst) * L.h3 + t, omega, st, u, f,
-                                                                r0, XNbLds<A>(), xs, rown);
+    if (live)
+        stencil_gs_vertex<R, REVERSE, ZC, SA, A, false, true, ROWN>(L, N, colour_block(cfirst) * L.h3 + t, omega, st, u,
+                                                                    f, r0, XNbLds<A>(), xs, rown);
     __syncthreads();
+    if (!live) return;
     XNbLds<A> xl;
     xl.base = xs;
-    const int h = L.h, lx = (int)(t % (uint32_t)h), row0 = (int)threadIdx.x - lx;
+    const int lx = (int)(t % (uint32_t)h), row0 = (int)threadIdx.x - lx;
     const bool odd = (colour_block(c2) & 1u) != 0;  // x-parity of the second colour
     xl.slot[0] = row0 + (odd ? lx : (lx == 0 ? h - 1 : lx - 1));
     xl.slot[1] = row0 + (odd ? (lx + 1 == h ? 0 : lx + 1) : lx);
@@ -2287,6 +2301,19 @@ int ke_mfma_table(const double* kl, const double* km, double lam, double mu, voi
     return one ? 1 : 2;
 }
 
+void fine_block_consts(float* ke) {
+    for (int t = 0; t < 243; t++) {
+        const int d = t / 9, i = t / 3 % 3, j = t % 3;
+        int e0 = 0, b0 = 0;
+        for (int m = 0; m < 3; m++) {
+            const int dm = (m == 0 ? d % 3 : (m == 1 ? d / 3 % 3 : d / 9)) - 1, em = dm > 0 ? 1 : 0;
+            e0 |= em << m;
+            b0 |= (dm + 1 - em) << m;
+        }
+        ke[kKeBlocks + 12 * d + 3 * i + j] = ke[(3 * (7 - e0) + i) * 24 + 3 * b0 + j];
+    }
+}
+
 int fine_apply_mfma_ok(int n) { return n % 32 == 0 && 72.0 * n * n * n < 4294967296.0; }
 
 static unsigned ef_grid(int n) {
@@ -2441,17 +2468,19 @@ void launch_fine_gs(hipStream_t s, int n, int colour, float omega, int reverse, 
 }
 
 // fused colour pairs need every workgroup to own whole rows of one parity block
-int fine_gs_pairs_ok(int n) {
+int fine_gs_pairs_ok(int n) { return n % 2 == 0 && n >= 4 && n / 2 <= 256; }
+
+// a multiple of 8, so that each XCD gets a contiguous run (workgroups past the last row do nothing)
+int gs_pair_blocks(int n) {
     const int h = n / 2;
-    const long h3 = (long)h * h * h;
-    return n % 2 == 0 && h <= 256 && 256 % h == 0 && h3 % 256 == 0;
+    return (int)((nblk((size_t)h * h, pair_rows(h)) + 7) / 8 * 8);
 }
 
 template <bool REV, int ZC, typename A, bool DOT = false, bool ROWN = false>
 static void fine_gs2_pair(hipStream_t s, const Lay& L, size_t N, int cfirst, float omega, const float* ke,
                           const float* w, A* u, const float* f, double* partial = nullptr, int pstride = 0,
                           float* rown = nullptr) {
-    hipLaunchKernelGGL((k_fine_gs2<6, REV, ZC, A, DOT, ROWN>), dim3(L.h3 / 256), dim3(256), 0, s, L, N, cfirst, omega,
+    hipLaunchKernelGGL((k_fine_gs2<6, REV, ZC, A, DOT, ROWN>), dim3(gs_pair_blocks(L.n)), dim3(256), 0, s, L, N, cfirst, omega,
                        ke, w, u, f, partial, pstride, rown);
 }
 
@@ -2655,7 +2684,7 @@ static void stencil_gs_st(hipStream_t s, const Lay& L, size_t N, bool split, int
 template <int R, bool REV, int ZC, typename SA, typename A, bool ROWN = false>
 static void stencil_gs2_colour(hipStream_t s, const Lay& L, size_t N, int cfirst, float omega, const SA* st, A* u,
                                const float* f, float* rown = nullptr) {
-    hipLaunchKernelGGL((k_stencil_gs2<R, REV, ZC, SA, A, ROWN>), dim3(L.h3 / 256, 6 / R), dim3(256), 0, s, L, N, cfirst,
+    hipLaunchKernelGGL((k_stencil_gs2<R, REV, ZC, SA, A, ROWN>), dim3(gs_pair_blocks(L.n), 6 / R), dim3(256), 0, s, L, N, cfirst,
                        omega, st, u, f, rown);
 }
 

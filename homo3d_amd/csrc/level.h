@@ -50,6 +50,9 @@ __device__ __forceinline__ uint32_t xcd_chunk(uint32_t g, uint32_t G) {
     return (g & 7u) * (G >> 3) + (g >> 3);
 }
 
+// Rows of n/2 = h vertices that a workgroup of a fused colour pair takes: as many as 256 threads hold.
+__host__ __device__ inline int pair_rows(int h) { return h < 256 ? 256 / h : 1; }
+
 // Full-level kernels run 512-thread workgroups.  On a parity-blocked level the 8 waves of a
 // workgroup take the same 64 local positions in the 8 parity blocks, so a workgroup covers a
 // 128 x 2 x 2 vertex tile and the neighbour reads of its waves overlap in L1/L2; on a
