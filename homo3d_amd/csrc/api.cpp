@@ -37,9 +37,8 @@ struct Level {
     float* u = nullptr;
     float* f = nullptr;
     float* r = nullptr;
-    void* st = nullptr;   // levels >= 1: FP32 [243][N], or packed FP16 [122][N] words when st_half
+    void* st = nullptr;   // levels >= 1: FP32 [243][N], or packed FP16 [31][N] quads of 8 entries when st_half
     int st_half = 0;
-    void* quads = nullptr;  // small levels: the stencil again, in quads (launch_stencil_quads)
 };
 
 struct ProfEvent {
@@ -359,8 +358,8 @@ bool op_smooth(homo3d_handle* h, int l, void* u, const float* f, float omega, in
         if (dot) launch_sum_partials(h->stream, kRhs, 4 * G, h->d_partial, dot_out);
         return dot;
     }
-    if (l > 0 && !u_half && L.quads) {
-        launch_plane_sweep(h->stream, L.n, omega, reverse, zs, L.quads, static_cast<float*>(u), f);
+    if (l > 0 && !u_half && small_level_ok(L.n, L.lex, L.st_half)) {
+        launch_plane_sweep(h->stream, L.n, omega, reverse, zs, L.st, static_cast<float*>(u), f);
         return false;
     }
     if (l > 0 && stencil_gs_pairs_ok(L.n, L.lex)) {  // colours two at a time (same result as one by one)
@@ -477,7 +476,7 @@ int vcycle(homo3d_handle* h, void* u0, const float* f0, int symmetric, double* r
     if (rc) return rc;
     if (tail) {
         const Level& L = h->lv[lt];
-        launch_vcycle_tail(h->stream, L.n, omega, symmetric ? 1 : 0, L.quads, L.u, L.f, L.r, Lc.u, Lc.f,
+        launch_vcycle_tail(h->stream, L.n, omega, symmetric ? 1 : 0, L.st, L.u, L.f, L.r, Lc.u, Lc.f,
                            h->d_Ainv);
     } else {
         launch_coarse_solve(h->stream, Lc.n, h->d_Ainv, Lc.f, Lc.u);
@@ -766,9 +765,7 @@ int homo3d_create(const homo3d_config* cfg, homo3d_handle** out) {
             return fail(HOMO3D_HIP_ERROR);
         if (l > 0) {
             L.st_half = cfg->coarse_half && l < nl - 1 ? 1 : 0;  // the coarsest stays FP32 for the dense solve
-            if (hipMalloc(&L.st, sizeof(uint32_t) * (L.st_half ? 122 : 243) * L.N)) return fail(HOMO3D_HIP_ERROR);
-            if (small_level_ok(L.n, L.lex, L.st_half) && hipMalloc(&L.quads, stencil_quads_bytes(L.n)))
-                return fail(HOMO3D_HIP_ERROR);
+            if (hipMalloc(&L.st, sizeof(uint32_t) * (L.st_half ? 124 : 243) * L.N)) return fail(HOMO3D_HIP_ERROR);
         }
     }
     const size_t N0 = h->lv[0].N, vb = sizeof(float) * 3 * kRhs * N0;
@@ -876,7 +873,6 @@ int homo3d_destroy(homo3d_handle* h) {
         (void)hipFree(h->lv[l].f);
         (void)hipFree(h->lv[l].r);
         (void)hipFree(h->lv[l].st);
-        (void)hipFree(h->lv[l].quads);
     }
     void* ptrs[] = {h->d_x, h->U64, h->d_ke64, h->d_kchi64, h->d_ke, h->d_ke16, h->d_kchi, h->d_G, h->d_G32, h->d_w, h->d_stage, h->d_Ainv, h->d_cstat, h->d_cwork, h->X, h->F, h->P, h->Q, h->Z,
                     h->Rr, h->d_partial, h->d_sc, h->d_tmp, h->d_ftmp, h->d_gperm, h->d_gflip};
@@ -924,8 +920,6 @@ int homo3d_update_density(homo3d_handle* h, const float* x, int pitch, int on_de
     for (int l = 2; l < h->nl; l++)
         launch_galerkin_coarse(h->stream, h->lv[l - 1].n, h->lv[l].lex, h->lv[l - 1].st, h->lv[l - 1].st_half,
                                h->lv[l].st, h->lv[l].st_half, reinterpret_cast<double*>(h->P), clamp);
-    for (int l = 1; l < h->nl; l++)
-        if (h->lv[l].quads) launch_stencil_quads(h->stream, h->lv[l].n, h->lv[l].st, h->lv[l].quads);
     // coarsest dense system: assembled and inverted on the GPU; its status is read at the
     // first coarse solve (coarse_factor)
     const Level& Lc = h->lv[h->nl - 1];
@@ -1491,12 +1485,12 @@ int homo3d_get_stencil(homo3d_handle* h, int level, float* host) {
     if (!h || !host || level < 1 || level >= h->nl) return HOMO3D_BAD_ARG;
     if (h->cfg.solver == HOMO3D_SOLVER_NONE) return set_err(h, HOMO3D_BAD_ARG, "density-only handle");
     const Level& L = h->lv[level];
-    const int words = L.st_half ? 122 : 243;
+    const int words = L.st_half ? 124 : 243;
     std::vector<uint32_t> soa((size_t)words * L.N);
     HIPCHK(h, hipMemcpyAsync(soa.data(), L.st, sizeof(uint32_t) * soa.size(), hipMemcpyDeviceToHost, h->stream));
     HIPCHK(h, hipStreamSynchronize(h->stream));
     auto entry = [&](int k, size_t sv) -> float {
-        const uint32_t wv = soa[(size_t)(L.st_half ? k >> 1 : k) * L.N + sv];
+        const uint32_t wv = L.st_half ? soa[((size_t)(k >> 3) * L.N + sv) * 4 + (size_t)(k >> 1 & 3)] : soa[(size_t)k * L.N + sv];
         if (!L.st_half) {
             float f;
             std::memcpy(&f, &wv, sizeof(f));

@@ -88,27 +88,24 @@ void launch_zero_pin64(hipStream_t s, size_t N, double* u);
 // elimination on the diagonal; work is another m x m doubles.  status (device) = 0, or 1 + the first step
 // whose pivot is not positive (the system is not positive definite; ainv is then not an inverse).
 void launch_coarse_factor(hipStream_t s, int nc, const float* st, double* ainv, double* work, int* status);
-// Coarse stencils: FP32 [243][n^3] or, with *_half, packed FP16 [122][n^3] words (entries 2w, 2w + 1).
+// Coarse stencils: FP32 [243][n^3] or, with *_half, packed FP16 in quads of eight entries [31][n^3].
 // u FP32 planes, or (u_half, only where stencil_u_half_ok: six load cases per launch) packed FP16 pairs.
 int stencil_u_half_ok(int n, int lex);
 void launch_stencil_apply(hipStream_t s, int n, int lex, const void* st, int st_half, const void* u, int u_half,
                           const float* f, float* out);
 void launch_stencil_gs(hipStream_t s, int n, int colour, float omega, int reverse, int zero_start, const void* st,
                        int st_half, void* u, int u_half, const float* f);
-// Small coarse levels (smallgrid.hip; parity-blocked, n <= 32, packed FP16 stencils, FP32 fields) read their
-// stencils from a copy in 16-byte quads.
+// Small coarse levels (smallgrid.hip; parity-blocked, n <= 32, packed FP16 stencils, FP32 fields).
 int small_level_ok(int n, int lex, int st_half);
-size_t stencil_quads_bytes(int n);
-void launch_stencil_quads(hipStream_t s, int n, const void* st, void* quads);
 // A whole sweep in two launches of four colours each, identical to eight launch_stencil_gs calls up to the
 // order of a vertex's 27 products.
-void launch_plane_sweep(hipStream_t s, int n, float omega, int reverse, int zero_start, const void* quads, float* u,
+void launch_plane_sweep(hipStream_t s, int n, float omega, int reverse, int zero_start, const void* st, float* u,
                         const float* f);
 // The bottom of a V(1,1) cycle from the last smoothed level (n points an axis, vcycle_tail_ok: 8 to 14) with
 // right-hand side f to its corrected and post-smoothed u (zero before): smoothing, residual (res), transfers
 // and the coarsest solve (uc, fc, ainv of the lexicographic coarsest level, n / 2 points an axis).
 int vcycle_tail_ok(int n, int lex, int st_half);
-void launch_vcycle_tail(hipStream_t s, int n, float omega, int reverse, const void* quads, float* u, const float* f,
+void launch_vcycle_tail(hipStream_t s, int n, float omega, int reverse, const void* st, float* u, const float* f,
                         float* res, float* uc, float* fc, const double* Ainv);
 // Colours cfirst and cfirst + 1 (cfirst even; reverse: cfirst and cfirst - 1, cfirst odd) of a coarse
 // parity-blocked level in one launch, identical to two launch_stencil_gs calls; only when

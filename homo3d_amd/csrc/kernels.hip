@@ -1418,11 +1418,40 @@ struct StencilRow {
     Rsrc rs, ru;
     uint32_t X[3], Y[3], Z[3], vo, plane;
 };
-template <typename SA, typename A, int W, bool XL, int D>
-__device__ __forceinline__ void stencil_nb(float (&S)[9], A (&cur)[W][3], const StencilRow& c, int r0,
-                                           const XNbLds<A>& xl) {
+// The entries of a vertex's stencil, each loaded with the neighbour that first needs it (DP: the one loaded
+// before, -1 none): packed FP16 in quads of eight, which the wave's loads fetch whole.  A word a load kept
+// the texture addresser busy: a colour pair took 20.5 us at 40^3 and 22.4 at 64^3 (55 on average at 64^3 and
+// 128^3), 17.8 and 19 (52) with quads and the vertex's own values loaded first.
+template <typename SA>
+struct StencilEntries;
+template <>
+struct StencilEntries<float> {
+    float e[243];
+    template <int DP, int D>
+    __device__ __forceinline__ void load(Rsrc rs, uint32_t vo, uint32_t plane) {
 #pragma unroll
-    for (int k = 0; k < 9; k++) S[k] = StencilIO<SA>::get(c.rs, c.vo, c.plane, D * 9 + k);
+        for (int k = 9 * D; k < 9 * D + 9; k++) e[k] = StencilIO<float>::get(rs, vo, plane, k);
+    }
+    __device__ __forceinline__ float get(int k) const { return e[k]; }
+};
+template <>
+struct StencilEntries<half2_t> {
+    typedef uint32_t Quad __attribute__((ext_vector_type(4)));
+    Quad q[31];
+    template <int DP, int D>
+    __device__ __forceinline__ void load(Rsrc rs, uint32_t vo, uint32_t plane) {
+        constexpr int before = DP < 0 ? 0 : (9 * DP + 8) / 8 + 1, first = 9 * D / 8 > before ? 9 * D / 8 : before;
+#pragma unroll
+        for (int k = first; k <= (9 * D + 8) / 8; k++)
+            q[k] = __builtin_bit_cast(Quad, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)(4u * vo), (int)((uint32_t)k * 4u * plane), 0));
+    }
+    __device__ __forceinline__ float get(int k) const {
+        return (float)__builtin_bit_cast(half2_t, (uint32_t)q[k >> 3][k >> 1 & 3])[k & 1];
+    }
+};
+
+template <typename A, int W, bool XL, int D>
+__device__ __forceinline__ void stencil_nb(A (&cur)[W][3], const StencilRow& c, int r0, const XNbLds<A>& xl) {
     if constexpr (XL && (D == 12 || D == 14)) {
         load_nb_lds<W, A>(cur, xl, D == 12 ? 0 : 1);
     } else {
@@ -1431,17 +1460,22 @@ __device__ __forceinline__ void stencil_nb(float (&S)[9], A (&cur)[W][3], const 
     }
 }
 template <int R, uint32_t MASK, int D, typename SA, typename A, bool XL>
-__device__ __forceinline__ void stencil_step(const StencilRow& c, int r0, const XNbLds<A>& xl, const float (&S)[9],
+__device__ __forceinline__ void stencil_step(const StencilRow& c, int r0, const XNbLds<A>& xl, StencilEntries<SA>& S,
                                              const A (&cur)[R / CasesPerWord<A>::value][3], float (&acc)[R][3]) {
     constexpr int W = R / CasesPerWord<A>::value;
     constexpr int DN = next_nb(MASK, D);
     __builtin_amdgcn_sched_barrier(0);
     pin_acc<R, float>(acc);
-    float Sn[9];
     A nxt[W][3];
-    if constexpr (DN < 27) stencil_nb<SA, A, W, XL, DN>(Sn, nxt, c, r0, xl);
-    block_fma<W, float, A>(S, cur, acc);
-    if constexpr (DN < 27) stencil_step<R, MASK, DN, SA, A, XL>(c, r0, xl, Sn, nxt, acc);
+    if constexpr (DN < 27) {
+        S.template load<D, DN>(c.rs, c.vo, c.plane);
+        stencil_nb<A, W, XL, DN>(nxt, c, r0, xl);
+    }
+    float e[9];
+#pragma unroll
+    for (int k = 0; k < 9; k++) e[k] = S.get(9 * D + k);
+    block_fma<W, float, A>(e, cur, acc);
+    if constexpr (DN < 27) stencil_step<R, MASK, DN, SA, A, XL>(c, r0, xl, S, nxt, acc);
 }
 
 // acc = sum over the neighbours selected by MASK of the stored 3x3 blocks times u, load cases r0 .. r0 + R - 1.
@@ -1466,9 +1500,10 @@ __device__ __forceinline__ void stencil_gather(int x, int y, int z, const Lay& L
         for (int i = 0; i < 3; i++) acc[r][i] = 0.f;
     constexpr int D0 = next_nb(MASK, -1);
     if constexpr (D0 < 27) {
-        float S[9];
+        StencilEntries<SA> S;
         A cur[W][3];
-        stencil_nb<SA, A, W, XL, D0>(S, cur, c, r0, xl);
+        S.template load<-1, D0>(c.rs, c.vo, c.plane);
+        stencil_nb<A, W, XL, D0>(cur, c, r0, xl);
         stencil_step<R, MASK, D0, SA, A, XL>(c, r0, xl, S, cur, acc);
     }
 }
@@ -1506,19 +1541,35 @@ __device__ __forceinline__ void stencil_gs_vertex(const Lay& L, size_t N, uint32
     static_assert(!ROWN || ZC >= 0, "the own-colour residual needs a zero-start forward pass");
     int x, y, z;
     L.pos(v, x, y, z);
+    constexpr int cpw = CasesPerWord<A>::value;
+    // the vertex's own values are loaded before the gather: after it, their latency would be the wave's
+    constexpr bool own = cpw == 2 && ZC < 0;
+    float fv[R][3];
+    A old[own ? R / cpw : 1][3];
+    StencilEntries<SA> diag;
+    diag.template load<-1, 13>(make_rsrc(st, (size_t)StencilIO<SA>::words * N * 4), v * 4u, (uint32_t)(N * 4));
+#pragma unroll
+    for (int r = 0; r < R; r++)
+#pragma unroll
+        for (int i = 0; i < 3; i++) fv[r][i] = f[(size_t)((r0 + r) * 3 + i) * N + v];
+    if constexpr (own) {
+#pragma unroll
+        for (int p = 0; p < R / cpw; p++)
+#pragma unroll
+            for (int i = 0; i < 3; i++) old[p][i] = u[fw_index<A>((r0 / cpw + p) * 3 + i, v, N)];
+    }
     float acc[R][3];
     stencil_gather<R, gs_mask(ZC), SA, A, XL>(x, y, z, L, N, v, st, u, acc, r0, xl);
     float Ks[9];
-    const Rsrc rs = make_rsrc(st, (size_t)StencilIO<SA>::words * N * 4);
 #pragma unroll
-    for (int k = 0; k < 9; k++) Ks[k] = StencilIO<SA>::get(rs, v * 4u, (uint32_t)(N * 4), 13 * 9 + k);
+    for (int k = 0; k < 9; k++) Ks[k] = diag.get(13 * 9 + k);
     const float inv[3] = {1.f / Ks[0], 1.f / Ks[4], 1.f / Ks[8]};
-    constexpr int cpw = CasesPerWord<A>::value;
 #pragma unroll
     for (int p = 0; p < R / cpw; p++) {
         A wd[3];
 #pragma unroll
-        for (int i = 0; i < 3; i++) wd[i] = ZC >= 0 ? A(0) : u[fw_index<A>((r0 / cpw + p) * 3 + i, v, N)];
+        for (int i = 0; i < 3; i++)
+            wd[i] = ZC >= 0 ? A(0) : own ? old[own ? p : 0][i] : u[fw_index<A>((r0 / cpw + p) * 3 + i, v, N)];
 #pragma unroll
         for (int hh = 0; hh < cpw; hh++) {
             const int r = p * cpw + hh;
@@ -1529,7 +1580,7 @@ __device__ __forceinline__ void stencil_gs_vertex(const Lay& L, size_t N, uint32
                     uu[i] = (float)wd[i][hh];
                 else
                     uu[i] = (float)wd[i];
-                ff[i] = f[(size_t)((r0 + r) * 3 + i) * N + v];
+                ff[i] = fv[r][i];
             }
             block_update<REVERSE>(uu, ff, acc[r], Ks, inv, omega);
 #pragma unroll
@@ -2714,12 +2765,10 @@ static void stencil_gs2_pick(hipStream_t s, const Lay& L, size_t N, int cfirst, 
 }
 
 template <typename SA>
-static void stencil_gs2_st(hipStream_t s, const Lay& L, size_t N, bool split, int cfirst, float omega, int reverse,
+static void stencil_gs2_st(hipStream_t s, const Lay& L, size_t N, int cfirst, float omega, int reverse,
                            int zero_start, const SA* st, void* u, int u_half, const float* f, float* rown) {
     if (u_half)
         stencil_gs2_pick<6>(s, L, N, cfirst, omega, reverse, zero_start, st, static_cast<half2_t*>(u), f, rown);
-    else if (split)
-        stencil_gs2_pick<1>(s, L, N, cfirst, omega, reverse, zero_start, st, static_cast<float*>(u), f, rown);
     else
         stencil_gs2_pick<6>(s, L, N, cfirst, omega, reverse, zero_start, st, static_cast<float*>(u), f, rown);
 }
@@ -2732,15 +2781,14 @@ void launch_stencil_gs2(hipStream_t s, int n, int cfirst, float omega, int rever
                         int st_half, void* u, int u_half, const float* f, float* rown) {
     const size_t N = (size_t)n * n * n;
     const Lay L = make_lay(n, 0);
-    const bool split = n <= kSplitLoadCasesMaxN;
     if (!stencil_gs_pairs_ok(n, 0)) return;            // the caller checks stencil_gs_pairs_ok
     if (u_half && !stencil_u_half_ok(n, 0)) return;    // ... and stencil_u_half_ok
     if (reverse || !zero_start) rown = nullptr;        // own-colour residuals only for zero-start passes
     if (st_half)
-        stencil_gs2_st(s, L, N, split, cfirst, omega, reverse, zero_start, static_cast<const half2_t*>(st), u, u_half,
+        stencil_gs2_st(s, L, N, cfirst, omega, reverse, zero_start, static_cast<const half2_t*>(st), u, u_half,
                        f, rown);
     else
-        stencil_gs2_st(s, L, N, split, cfirst, omega, reverse, zero_start, static_cast<const float*>(st), u, u_half, f,
+        stencil_gs2_st(s, L, N, cfirst, omega, reverse, zero_start, static_cast<const float*>(st), u, u_half, f,
                        rown);
 }
 

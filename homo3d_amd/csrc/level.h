@@ -117,8 +117,9 @@ __device__ __forceinline__ size_t fw_index(int q, size_t v, size_t N) {
         return (size_t)q * N + v;
 }
 
-// A stored coarse stencil: FP32 entries [243][N] (entry e = 9d + 3i + j), or packed FP16 [122][N]
-// words, word w holding entries 2w (.x) and 2w + 1 (.y).  Both have 4-byte words per vertex.
+// A stored coarse stencil: FP32 entries [243][N] (entry e = 9d + 3i + j), or packed FP16 [31][N] quads of
+// four words, quad q holding the entries 8q .. 8q + 7 (so that one load brings 16 bytes).  words: 4-byte
+// words a vertex; vo: 4 times the vertex, plane: 4 N.
 template <typename SA>
 struct StencilIO;
 template <>
@@ -127,17 +128,33 @@ struct StencilIO<float> {
     __device__ static float get(Rsrc rs, uint32_t vo, uint32_t plane, int e) {
         return bload<float>(rs, vo, (uint32_t)e * plane);
     }
+    // entries e .. e + 2 (e the same in every lane)
+    __device__ static void get3(Rsrc rs, uint32_t vo, uint32_t plane, int e, float (&out)[3]) {
+#pragma unroll
+        for (int j = 0; j < 3; j++) out[j] = get(rs, vo, plane, e + j);
+    }
     __device__ static void put(float* st, size_t N, uint32_t v, int e, float val) { st[(size_t)e * N + v] = val; }
 };
 template <>
 struct StencilIO<half2_t> {
-    static constexpr int words = 122;
+    static constexpr int words = 124;
     __device__ static float get(Rsrc rs, uint32_t vo, uint32_t plane, int e) {
-        return (float)bload<half2_t>(rs, vo, (uint32_t)(e >> 1) * plane)[e & 1];
+        return (float)bload<half2_t>(rs, 4u * vo + 4u * (uint32_t)(e >> 1 & 3), (uint32_t)(e >> 3) * 4u * plane)[e & 1];
     }
-    // one 16-bit store per entry: the two halves of a word may come from different threads
+    __device__ static void get3(Rsrc rs, uint32_t vo, uint32_t plane, int e, float (&out)[3]) {
+        const uint32_t w0 = (uint32_t)e >> 1, w1 = w0 + 1, odd = 16u * (uint32_t)(e & 1);
+        const auto word = [&](uint32_t w) {
+            return __builtin_bit_cast(uint32_t, bload<half2_t>(rs, 4u * vo, (w >> 2) * 4u * plane + 4u * (w & 3u)));
+        };
+        const uint32_t a = word(w0), b = word(w1);
+        const half2_t lo = __builtin_bit_cast(half2_t, __builtin_amdgcn_alignbit(b, a, odd));
+        out[0] = (float)lo[0];
+        out[1] = (float)lo[1];
+        out[2] = (float)__builtin_bit_cast(half2_t, b >> odd)[0];
+    }
+    // one 16-bit store per entry: the halves of a word may come from different threads
     __device__ static void put(half2_t* st, size_t N, uint32_t v, int e, float val) {
-        reinterpret_cast<_Float16*>(st + (size_t)(e >> 1) * N + v)[e & 1] = (_Float16)val;
+        reinterpret_cast<_Float16*>(st)[((size_t)(e >> 3) * N + v) * 8 + (size_t)(e & 7)] = (_Float16)val;
     }
 };
 

@@ -131,8 +131,10 @@ __global__ __launch_bounds__(64) void k_galerkin_fine_pin(Lay Lf, Lay Lc, const 
 // Coarser stencil from a stored one: st_c[V][D] = sum_{o,d} hat3(o) A_f[2V+o][d] hat3(o+d-2D), one axis
 // after another: the sum over (o, d) of one axis turns its nine blocks into three (13 products instead of
 // the 27 of a direct sum), and the axes do not mix.  The x and y axes in one pass over the fine stencil, z
-// in a second over T[((dz 3 + Dy) 3 + Dx) 9 + k][X + nc (Y + nc z)] (243 planes, z fine), one entry k of
-// the 3 x 3 blocks per thread: 81 and 9 independent loads a thread.  FP64 sums, rounded once: the coarsest
+// in a second over T[((dz 3 + Dy) 3 + Dx) 9 + k][X + nc (Y + nc z)] (243 planes, z fine), a row of the
+// 3 x 3 blocks per thread in the first pass, an entry in the second (an entry in the first as well read
+// every line of the packed stencils from nine workgroups: 430 us on average over a 256^3 solve's levels, 220
+// this way).  FP64 sums, rounded once: the coarsest
 // system is nearly singular (one node holds the translations), and its solution is as far off as the
 // stencil's rounding times that condition.  A direct sum, a thread per
 // coarse vertex and plane Dz, took 330-380 us at any small size (567 blocks in a chain) and 2 ms at
@@ -144,31 +146,40 @@ __global__ __launch_bounds__(256) void k_galerkin_xy(Lay Lf, int nc, const SI* _
     const uint32_t i = xcd_chunk(blockIdx.x, gridDim.x) * 256u + threadIdx.x, nt = (uint32_t)nc * nc * nf;
     if (i >= nt) return;
     const int X = (int)(i % nc), Y = (int)(i / nc % nc), z = (int)(i / ((uint32_t)nc * nc));
-    const int k = (int)blockIdx.y % 9, dz = (int)blockIdx.y / 9;
+    const int row = (int)blockIdx.y % 3, dz = (int)blockIdx.y / 3;
     const size_t Nf = (size_t)nf * nf * nf;
     const uint32_t xs[3] = {Lf.part(wrap_dec(2 * X, nf), 0), Lf.part(2 * X, 0), Lf.part(2 * X + 1, 0)};
     const uint32_t ys[3] = {Lf.part(wrap_dec(2 * Y, nf), 1), Lf.part(2 * Y, 1), Lf.part(2 * Y + 1, 1)};
     const uint32_t zp = Lf.part(z, 2);
     const Rsrc rf = make_rsrc(stf, (size_t)StencilIO<SI>::words * Nf * 4);
-    double S[3][3];  // [Dy + 1][Dx + 1]
+    double S[9][3];  // [(Dy + 1) 3 + Dx + 1][column]
 #pragma unroll
-    for (int j = 0; j < 9; j++) S[j / 3][j % 3] = 0.0;
+    for (int j = 0; j < 9; j++)
+#pragma unroll
+        for (int c = 0; c < 3; c++) S[j][c] = 0.0;
 #pragma unroll
     for (int oy = -1; oy <= 1; oy++)
 #pragma unroll
         for (int dy = -1; dy <= 1; dy++) {
-            double R[3] = {0.0, 0.0, 0.0};
+            double R[3][3];
+#pragma unroll
+            for (int j = 0; j < 3; j++)
+#pragma unroll
+                for (int c = 0; c < 3; c++) R[j][c] = 0.0;
 #pragma unroll
             for (int ox = -1; ox <= 1; ox++)
 #pragma unroll
                 for (int dx = -1; dx <= 1; dx++) {
                     const int d = (dx + 1) + 3 * (dy + 1) + 9 * dz;
-                    const double e = (double)StencilIO<SI>::get(rf, (xs[ox + 1] + ys[oy + 1] + zp) * 4u,
-                                                                (uint32_t)(Nf * 4), d * 9 + k);
+                    float e[3];
+                    StencilIO<SI>::get3(rf, (xs[ox + 1] + ys[oy + 1] + zp) * 4u, (uint32_t)(Nf * 4), d * 9 + 3 * row, e);
 #pragma unroll
                     for (int Dx = -1; Dx <= 1; Dx++) {
                         const int q = ox + dx - 2 * Dx;
-                        if (q >= -1 && q <= 1) R[Dx + 1] = fma((ox ? 0.5 : 1.0) * (q ? 0.5 : 1.0), e, R[Dx + 1]);
+                        if (q < -1 || q > 1) continue;
+#pragma unroll
+                        for (int c = 0; c < 3; c++)
+                            R[Dx + 1][c] = fma((ox ? 0.5 : 1.0) * (q ? 0.5 : 1.0), (double)e[c], R[Dx + 1][c]);
                     }
                 }
 #pragma unroll
@@ -177,11 +188,15 @@ __global__ __launch_bounds__(256) void k_galerkin_xy(Lay Lf, int nc, const SI* _
                 if (q < -1 || q > 1) continue;
                 const double wy = (oy ? 0.5 : 1.0) * (q ? 0.5 : 1.0);
 #pragma unroll
-                for (int j = 0; j < 3; j++) S[Dy + 1][j] = fma(wy, R[j], S[Dy + 1][j]);
+                for (int j = 0; j < 3; j++)
+#pragma unroll
+                    for (int c = 0; c < 3; c++) S[(Dy + 1) * 3 + j][c] = fma(wy, R[j][c], S[(Dy + 1) * 3 + j][c]);
             }
         }
 #pragma unroll
-    for (int j = 0; j < 9; j++) T[(size_t)((dz * 9 + j) * 9 + k) * nt + i] = S[j / 3][j % 3];
+    for (int j = 0; j < 9; j++)
+#pragma unroll
+        for (int c = 0; c < 3; c++) T[(size_t)((dz * 9 + j) * 9 + 3 * row + c) * nt + i] = S[j][c];
 }
 
 template <typename SO>
@@ -379,7 +394,7 @@ template <typename SI, typename SO>
 void galerkin_coarse_case(hipStream_t s, const Lay& Lf, const Lay& Lc, const void* stf, void* stc, double* work,
                           float clamp) {
     const size_t Nc = (size_t)Lc.n * Lc.n * Lc.n;
-    hipLaunchKernelGGL(k_galerkin_xy<SI>, dim3(nblk(2 * Nc), 27), dim3(256), 0, s, Lf, Lc.n,
+    hipLaunchKernelGGL(k_galerkin_xy<SI>, dim3(nblk(2 * Nc), 9), dim3(256), 0, s, Lf, Lc.n,
                        static_cast<const SI*>(stf), work);
     hipLaunchKernelGGL(k_galerkin_z<SO>, dim3(nblk(Nc), 81), dim3(256), 0, s, Lc, Lf.n, work, static_cast<SO*>(stc),
                        clamp);

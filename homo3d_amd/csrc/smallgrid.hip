@@ -8,7 +8,7 @@
 // depends on the others through neighbours in its own z-plane, and planes of the same parity do not meet: a
 // workgroup owns a z-plane for one load case (or one packed pair), keeps that plane and its two neighbours
 // of u in LDS, and updates the four colours in turn between barriers.  Three threads share a vertex, one per
-// neighbour plane: each has its 9 stencil blocks (11 quads of words) in flight at once, those of the next
+// neighbour plane: each has its 9 stencil blocks (11 st of words) in flight at once, those of the next
 // colour before the barriers of this one.  Bound by that load latency and the barriers: a sweep takes two
 // launches of 8 us at 8^3 to 16^3 and 12 us at 32^3, where eight of 6 us each took 65 us with their gaps.
 // Levels above 32^3 fill the GPU with one or two colours a launch and stream their stencils; FP32 stencils
@@ -25,35 +25,16 @@ namespace {
 
 constexpr int kPlaneVerts = 256;  // most vertices a workgroup updates at a time
 
-// A small level's stencils are kept a second time, a vertex's words in quads (word 4 q + k of vertex v at
-// (q N + v) 4 + k): a wave's load instruction costs the texture addresser about 11 cycles however little it
-// moves, and 41 single words for each of twelve waves were 2.2 us a colour (12 to 15 us a launch of
-// k_plane_gs, and 72 and 134 us one of k_tail at 8^3 and 10^3, against 8 to 12 and 51 and 74 with quads).
-constexpr int kStWords = StencilIO<half2_t>::words, kStQuads = (kStWords + 3) / 4;
-
-__global__ __launch_bounds__(256) void k_stencil_quads(uint32_t N, const uint32_t* __restrict__ st,
-                                                       uint4* __restrict__ quads) {
-    const uint32_t v = blockIdx.x * 256u + threadIdx.x, q = blockIdx.y;
-    if (v >= N) return;
-    uint32_t w[4];
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-        const uint32_t i = 4 * q + (uint32_t)k;
-        w[k] = i < (uint32_t)kStWords ? st[(size_t)i * N + v] : 0u;
-    }
-    quads[(size_t)q * N + v] = make_uint4(w[0], w[1], w[2], w[3]);
-}
-
 // The nine blocks of a neighbour plane g = dz + 1: entries 81 g .. 81 g + 80 of the stencil, which start g
 // entries into quad first(g).
 struct PlaneBlocks {
     typedef uint32_t Quad __attribute__((ext_vector_type(4)));
-    static constexpr int quads = 11;
-    Quad w[quads];
+    static constexpr int st = 11;
+    Quad w[st];
     __device__ __forceinline__ void load(Rsrc rs, uint32_t N, int g, uint32_t v, bool live) {
         const uint32_t q0 = (uint32_t)(81 * g / 8);
 #pragma unroll
-        for (int q = 0; q < quads; q++) {
+        for (int q = 0; q < st; q++) {
             if (live)
                 w[q] = __builtin_bit_cast(Quad, __builtin_amdgcn_raw_buffer_load_b128(
                                                     rs, (int)(v * 16u), (int)((q0 + (uint32_t)q) * N * 16u), 0));
@@ -116,7 +97,7 @@ __device__ __forceinline__ void stage_plane(A* dst, const Lay& L, size_t N, cons
 // colour are loaded while this one's are used.
 template <bool REVERSE, typename A>
 __global__ __launch_bounds__(3 * kPlaneVerts) void k_plane_gs(Lay L, size_t N, int pz, float omega, int zero,
-                                                              const uint4* __restrict__ quads, A* __restrict__ u,
+                                                              const uint4* __restrict__ st, A* __restrict__ u,
                                                               const float* __restrict__ f) {
     constexpr int cpw = CasesPerWord<A>::value, NM = 32;
     __shared__ A us[3 * 3 * NM * NM];
@@ -125,7 +106,7 @@ __global__ __launch_bounds__(3 * kPlaneVerts) void k_plane_gs(Lay L, size_t N, i
     const int vb = (int)blockDim.x / 3, g = __builtin_amdgcn_readfirstlane((int)threadIdx.x / vb);
     const int lv = (int)threadIdx.x - g * vb;
     const int kz = (int)blockIdx.x, z = 2 * kz + pz, p = (int)blockIdx.y;
-    const Rsrc rs = make_rsrc(quads, (size_t)kStQuads * N * 16);
+    const Rsrc rs = make_rsrc(st, (size_t)StencilIO<half2_t>::words * N * 4);
     const bool live = lv < h2, load = live && !(zero == 1 && g != 1);  // the neighbour planes may be zero
     const int yy = lv / h, xx = lv - yy * h;
     const uint32_t v0 = (uint32_t)pz * 4u * L.h3 + (uint32_t)lv + (uint32_t)h2 * (uint32_t)kz;
@@ -241,11 +222,11 @@ __device__ __forceinline__ int tail_verts(int h3) { return h3 <= 256 ? (h3 + 63)
 
 // One pass over the level's vertices colour by colour: a GS sweep of u, or r = f - A u.
 template <int MODE>
-__device__ __forceinline__ void tail_pass(const Lay& L, size_t N, float omega, const uint4* __restrict__ quads, float* u,
+__device__ __forceinline__ void tail_pass(const Lay& L, size_t N, float omega, const uint4* __restrict__ st, float* u,
                                           const float* f, float* r, float (*red)[kPlaneVerts][3]) {
     const int n = L.n, h = L.h, n2 = n * n, n3 = n2 * n, h3 = (int)L.h3, vb = tail_verts(h3);
     const int g = __builtin_amdgcn_readfirstlane((int)threadIdx.x / vb), lv = (int)threadIdx.x - g * vb;
-    const Rsrc rs = make_rsrc(quads, (size_t)kStQuads * N * 16);
+    const Rsrc rs = make_rsrc(st, (size_t)StencilIO<half2_t>::words * N * 4);
     const int nch = h3 <= vb ? 1 : 2, steps = 8 * nch;
     int pos[2];  // half coordinates of the thread's vertex in each chunk, 4 bits each; -1: none
 #pragma unroll
@@ -318,7 +299,7 @@ __device__ __forceinline__ void tail_pass(const Lay& L, size_t N, float omega, c
 // not run leaves or finds its fields in memory (u, f, residual of the level; uc, fc of the lexicographic
 // coarsest); the fields a run of the separate passes would leave there are written too.
 __global__ __launch_bounds__(3 * kPlaneVerts) void k_tail(Lay L, size_t N, float omega, int reverse, int down, int solve,
-                                                          int up, const uint4* __restrict__ quads, float* __restrict__ u,
+                                                          int up, const uint4* __restrict__ st, float* __restrict__ u,
                                                           const float* __restrict__ f, float* __restrict__ res,
                                                           int nc, float* __restrict__ uc, float* __restrict__ fc,
                                                           const double* __restrict__ Ainv) {
@@ -337,8 +318,8 @@ __global__ __launch_bounds__(3 * kPlaneVerts) void k_tail(Lay L, size_t N, float
     }
     __syncthreads();
     if (down) {
-        tail_pass<kTailForward>(L, N, omega, quads, su, sf, sr, red);
-        tail_pass<kTailResidual>(L, N, omega, quads, su, sf, sr, red);
+        tail_pass<kTailForward>(L, N, omega, st, su, sf, sr, red);
+        tail_pass<kTailResidual>(L, N, omega, st, su, sf, sr, red);
         for (int t = threadIdx.x; t < m; t += nt) {
             const int i = t / Nc, V = t - i * Nc, X = V % nc, Y = V / nc % nc, Z = V / (nc * nc);
             float a = 0.f;
@@ -407,9 +388,9 @@ __global__ __launch_bounds__(3 * kPlaneVerts) void k_tail(Lay L, size_t N, float
         }
         __syncthreads();
         if (reverse)
-            tail_pass<kTailReverse>(L, N, omega, quads, su, sf, sr, red);
+            tail_pass<kTailReverse>(L, N, omega, st, su, sf, sr, red);
         else
-            tail_pass<kTailForward>(L, N, omega, quads, su, sf, sr, red);
+            tail_pass<kTailForward>(L, N, omega, st, su, sf, sr, red);
     }
     for (int t = threadIdx.x; t < n3; t += nt) {
         int x, y, z;
@@ -426,17 +407,9 @@ __global__ __launch_bounds__(3 * kPlaneVerts) void k_tail(Lay L, size_t N, float
 
 int small_level_ok(int n, int lex, int st_half) { return st_half && !lex && n % 2 == 0 && n >= 4 && n <= 32; }
 
-size_t stencil_quads_bytes(int n) { return (size_t)n * n * n * 16 * kStQuads; }
-
-void launch_stencil_quads(hipStream_t s, int n, const void* st, void* quads) {
-    const uint32_t N = (uint32_t)n * n * n;
-    hipLaunchKernelGGL(k_stencil_quads, dim3(nblk(N), kStQuads), dim3(256), 0, s, N, static_cast<const uint32_t*>(st),
-                       static_cast<uint4*>(quads));
-}
-
 int vcycle_tail_ok(int n, int lex, int st_half) { return small_level_ok(n, lex, st_half) && n >= 8 && n <= kTailN; }
 
-void launch_vcycle_tail(hipStream_t s, int n, float omega, int reverse, const void* quads, float* u, const float* f,
+void launch_vcycle_tail(hipStream_t s, int n, float omega, int reverse, const void* st, float* u, const float* f,
                         float* res, float* uc, float* fc, const double* Ainv) {
     const size_t N = (size_t)n * n * n;
     const Lay L = make_lay(n, 0);
@@ -446,16 +419,16 @@ void launch_vcycle_tail(hipStream_t s, int n, float omega, int reverse, const vo
     for (int part = one ? 0 : 1; part <= (one ? 0 : 2); part++) {
         if (part == 2) launch_coarse_solve(s, n / 2, Ainv, fc, uc);
         hipLaunchKernelGGL(k_tail, dim3(6), dim3(3 * kPlaneVerts), 0, s, L, N, omega, reverse, part != 2 ? 1 : 0,
-                           part == 0 ? 1 : 0, part != 1 ? 1 : 0, static_cast<const uint4*>(quads), u, f, res, n / 2, uc,
+                           part == 0 ? 1 : 0, part != 1 ? 1 : 0, static_cast<const uint4*>(st), u, f, res, n / 2, uc,
                            fc, Ainv);
     }
 }
 
-void launch_plane_sweep(hipStream_t s, int n, float omega, int reverse, int zero_start, const void* quads, float* u,
+void launch_plane_sweep(hipStream_t s, int n, float omega, int reverse, int zero_start, const void* st, float* u,
                         const float* f) {
     const size_t N = (size_t)n * n * n;
     const Lay L = make_lay(n, 0);
-    const uint4* q = static_cast<const uint4*>(quads);
+    const uint4* q = static_cast<const uint4*>(st);
     const int vb = (L.h * L.h + 63) / 64 * 64;
     const dim3 g(L.h, 6), b(3 * vb);
     for (int k = 0; k < 2; k++) {
