@@ -111,8 +111,6 @@ struct homo3d_handle {
     double* d_sc = nullptr;
     double* d_tmp = nullptr;
     float* d_ftmp = nullptr;
-    int* d_gperm = nullptr;
-    int* d_gflip = nullptr;
     double ke[576];
     bool density_set = false;
     std::string err;
@@ -265,30 +263,18 @@ void permute_planes(const Level& L, const T* in, T* out, int planes, bool to_sto
             }
 }
 
-// Symmetry groups (TensorExpression.cuh:72-262) in the canonical order shared with the checker:
-// element = (perm, flips), out[k] = flip_k ? n-1-p[perm[k]] : p[perm[k]].
-const int kPerm[6][3] = {{0, 1, 2}, {0, 2, 1}, {1, 0, 2}, {1, 2, 0}, {2, 0, 1}, {2, 1, 0}};
+// Symmetry groups (TensorExpression.cuh:72-262) as sets of elements 8 perm + flips in the order of kSymPerm,
+// which the oracle shares (the averages are summed in it).
 const int kPermSign[6] = {1, -1, -1, 1, 1, -1};
 
-void symmetry_group(int sym, std::vector<int>& perm, std::vector<int>& flip) {
-    perm.clear();
-    flip.clear();
-    auto add = [&](int p, int f) {
-        perm.push_back(kPerm[p][0] | (kPerm[p][1] << 2) | (kPerm[p][2] << 4));
-        flip.push_back(f);
-    };
-    if (sym == HOMO3D_SYM_REFLECT3) {
-        for (int f = 0; f < 8; f++) add(0, f);
-    } else if (sym == HOMO3D_SYM_REFLECT6) {
-        for (int p = 0; p < 6; p++)
-            for (int f = 0; f < 8; f++) add(p, f);
-    } else if (sym == HOMO3D_SYM_ROTATE3) {
-        for (int p = 0; p < 6; p++)
-            for (int f = 0; f < 8; f++) {
-                const int nflip = (f & 1) + ((f >> 1) & 1) + (f >> 2);
-                if (kPermSign[p] * ((nflip & 1) ? -1 : 1) == 1) add(p, f);
-            }
-    }
+uint64_t symmetry_group(int sym) {
+    if (sym == HOMO3D_SYM_REFLECT3) return 0xFFull;
+    if (sym == HOMO3D_SYM_REFLECT6) return 0xFFFFFFFFFFFFull;
+    uint64_t g = 0;
+    for (int p = 0; p < 6; p++)
+        for (int f = 0; f < 8; f++)
+            if (kPermSign[p] * (__builtin_popcount(f) & 1 ? -1 : 1) == 1) g |= 1ull << (8 * p + f);
+    return g;
 }
 
 void prof_flush(homo3d_handle* h) {
@@ -748,8 +734,7 @@ int homo3d_create(const homo3d_config* cfg, homo3d_handle** out) {
         h->lv[0].N = (size_t)n * n * n;
         h->partial_elems = 21 * kDotBlocks;
         if (hipMalloc(&h->d_partial, sizeof(double) * h->partial_elems) || hipMalloc(&h->d_tmp, sizeof(double) * 64) ||
-            hipMalloc(&h->d_ftmp, sizeof(float) * 4096) || hipMalloc(&h->d_gperm, sizeof(int) * 48) ||
-            hipMalloc(&h->d_gflip, sizeof(int) * 48))
+            hipMalloc(&h->d_ftmp, sizeof(float) * 4096))
             return fail(HOMO3D_HIP_ERROR);
         *out = h;
         return HOMO3D_OK;
@@ -829,8 +814,7 @@ int homo3d_create(const homo3d_config* cfg, homo3d_handle** out) {
             return fail(HOMO3D_HIP_ERROR);
     }
     if (hipMalloc(&h->d_ke, sizeof(float) * kKeFloats) || hipMalloc(&h->d_kchi, sizeof(float) * 144) ||
-        hipMalloc(&h->d_G, sizeof(double) * G.size()) || hipMalloc(&h->d_G32, sizeof(float) * G.size()) || hipMalloc(&h->d_gperm, sizeof(int) * 48) ||
-        hipMalloc(&h->d_gflip, sizeof(int) * 48))
+        hipMalloc(&h->d_G, sizeof(double) * G.size()) || hipMalloc(&h->d_G32, sizeof(float) * G.size()))
         return fail(HOMO3D_HIP_ERROR);
     double kl[576], km[576];
     // the matrix-core operand table is built whenever the element form can run, so that homo3d_autotune
@@ -875,7 +859,7 @@ int homo3d_destroy(homo3d_handle* h) {
         (void)hipFree(h->lv[l].st);
     }
     void* ptrs[] = {h->d_x, h->U64, h->d_ke64, h->d_kchi64, h->d_ke, h->d_ke16, h->d_kchi, h->d_G, h->d_G32, h->d_w, h->d_stage, h->d_Ainv, h->d_cstat, h->d_cwork, h->X, h->F, h->P, h->Q, h->Z,
-                    h->Rr, h->d_partial, h->d_sc, h->d_tmp, h->d_ftmp, h->d_gperm, h->d_gflip};
+                    h->Rr, h->d_partial, h->d_sc, h->d_tmp, h->d_ftmp};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     if (h->cstream) (void)hipStreamDestroy(h->cstream);
@@ -1517,22 +1501,20 @@ int homo3d_symmetrize(homo3d_handle* h, float* field, int pitch, int sym, int on
     if (sym < 0 || sym > 3) return set_err(h, HOMO3D_BAD_ARG, "unknown symmetry %d", sym);
     const int n = h->lv[0].n;
     if (pitch < n) return set_err(h, HOMO3D_BAD_ARG, "pitch %d < n %d", pitch, n);
-    std::vector<int> perm, flip;
-    symmetry_group(sym, perm, flip);
-    HIPCHK(h, hipMemcpyAsync(h->d_gperm, perm.data(), sizeof(int) * perm.size(), hipMemcpyHostToDevice, h->stream));
-    HIPCHK(h, hipMemcpyAsync(h->d_gflip, flip.data(), sizeof(int) * flip.size(), hipMemcpyHostToDevice, h->stream));
+    const uint64_t g = symmetry_group(sym);
+    if (on_device && device_here(h, {field})) {
+        launch_symmetrize(h->stream, n, pitch, g, field);
+        HIPCHK(h, hipStreamSynchronize(h->stream));
+        return HOMO3D_OK;
+    }
     const size_t elems = (size_t)pitch * n * n;
-    int rc = ensure_stage(h, 2 * elems);
+    int rc = ensure_stage(h, elems);
     if (rc) return rc;
-    float* in = h->d_stage;
-    float* out = h->d_stage + elems;
-    if (on_device)
-        HIPCHK(h, hipMemcpyAsync(in, field, sizeof(float) * elems, hipMemcpyDeviceToDevice, h->stream));
-    else
-        HIPCHK(h, hipMemcpyAsync(in, field, sizeof(float) * elems, hipMemcpyHostToDevice, h->stream));
-    launch_symmetrize(h->stream, n, pitch, (int)perm.size(), h->d_gperm, h->d_gflip, in, out);
-    launch_copy_pitched(h->stream, n, pitch, pitch, out, in);
-    HIPCHK(h, hipMemcpyAsync(field, in, sizeof(float) * elems, on_device ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost,
+    float* d = h->d_stage;
+    HIPCHK(h, hipMemcpyAsync(d, field, sizeof(float) * elems, on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice,
+                             h->stream));
+    launch_symmetrize(h->stream, n, pitch, g, d);
+    HIPCHK(h, hipMemcpyAsync(field, d, sizeof(float) * elems, on_device ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost,
                              h->stream));
     HIPCHK(h, hipStreamSynchronize(h->stream));
     return HOMO3D_OK;

@@ -3,6 +3,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stddef.h>
+#include <stdint.h>
 
 namespace homo3d {
 
@@ -31,5 +32,10 @@ void launch_sgm(hipStream_t s, int n, int pitch, double k, double c, const float
 void launch_sgm_back(hipStream_t s, int n, int pitch, double k, const float* y, const float* gy, float* gx);
 void launch_density_pow(hipStream_t s, int n, int pitch, float p, const float* rho, float* x);
 void launch_density_pow_grad(hipStream_t s, int n, int pitch, float p, const float* rho, const float* dx, float* drho);
+
+// Symmetry projection in place over the elements 8 p + f set in `group`: axis permutation p (kSymPerm) after
+// which the axes in f are mirrored, q[a] = coordinate kSymPerm[p][a], or n - 1 minus it.
+constexpr int kSymPerm[6][3] = {{0, 1, 2}, {0, 2, 1}, {1, 0, 2}, {1, 2, 0}, {2, 0, 1}, {2, 1, 0}};
+void launch_symmetrize(hipStream_t s, int n, int pitch, uint64_t group, float* field);
 
 }  // namespace homo3d

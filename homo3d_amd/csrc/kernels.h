@@ -148,8 +148,6 @@ void launch_elastic_matrix(hipStream_t s, int n, double lam, double mu, const fl
                            double* partial, int nblocks, double* out21);
 void launch_sensitivity(hipStream_t s, int n, int pitch, double lam, double mu, const float* chi, const float* wdc,
                         float* sens);
-void launch_symmetrize(hipStream_t s, int n, int pitch, int ng, const int* gperm, const int* gflip, const float* in,
-                       float* out);
 void launch_oc_trial(hipStream_t s, int n, int pitch, double g, double min_rho, double step, double damp,
                      const float* sens, const float* rho, float* out, double* partial, int nblocks, double* sum);
 void launch_absmax(hipStream_t s, int n, int pitch, const float* a, float* partial, int nblocks);

@@ -2173,42 +2173,6 @@ __global__ __launch_bounds__(256) void k_pcg_update_px_h(int R, size_t M, const 
 // Density utilities
 // ---------------------------------------------------------------------------------------------
 
-// Symmetry projection (symetrize_tensor_kernel, TensorExpression.cuh:72-262): each cell receives
-// the FP64 average over the group applied to its orbit's smallest-index member, so every member of
-// an orbit receives the same bits.  gperm/gflip list the group elements; n cubic.
-__global__ __launch_bounds__(256) void k_symmetrize(int n, int pitch, int ng, const int* __restrict__ gperm,
-                                                    const int* __restrict__ gflip, const float* __restrict__ in,
-                                                    float* __restrict__ out) {
-    const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long N = (long)n * n * n;
-    if (e >= N) return;
-    const int p[3] = {(int)(e % n), (int)((e / n) % n), (int)(e / ((long)n * n))};
-    long best = e;
-    int bq[3] = {p[0], p[1], p[2]};
-    for (int g = 0; g < ng; g++) {
-        int q[3];
-        for (int k = 0; k < 3; k++) {
-            const int a = p[(gperm[g] >> (2 * k)) & 3];
-            q[k] = ((gflip[g] >> k) & 1) ? n - 1 - a : a;
-        }
-        const long id = q[0] + (long)n * (q[1] + (long)n * q[2]);
-        if (id < best) {
-            best = id;
-            bq[0] = q[0]; bq[1] = q[1]; bq[2] = q[2];
-        }
-    }
-    double s = 0.0;
-    for (int g = 0; g < ng; g++) {
-        int q[3];
-        for (int k = 0; k < 3; k++) {
-            const int a = bq[(gperm[g] >> (2 * k)) & 3];
-            q[k] = ((gflip[g] >> k) & 1) ? n - 1 - a : a;
-        }
-        s += (double)in[q[0] + ((size_t)q[1] + (size_t)q[2] * n) * pitch];
-    }
-    out[p[0] + ((size_t)p[1] + (size_t)p[2] * n) * pitch] = (float)(s / (double)ng);
-}
-
 // OC update of one cell for multiplier g (update_kernel, OCOptimizer.cu:12-34), FP64 arithmetic rounded
 // to FP32.
 __device__ __forceinline__ float oc_cell(double r0, double sv, double g, double min_rho, double step, double damp) {
@@ -2903,12 +2867,6 @@ void launch_dot_rz(hipStream_t s, size_t M, const float* r, const void* z, int z
     }
     hipLaunchKernelGGL(k_dot_fh, dim3(nblocks, 3), dim3(256), 0, s, M, r, static_cast<const half2_t*>(z), partial);
     hipLaunchKernelGGL(k_sum_partials, dim3(6), dim3(kSumThreads), 0, s, nblocks, partial, out6);
-}
-
-void launch_symmetrize(hipStream_t s, int n, int pitch, int ng, const int* gperm, const int* gflip, const float* in,
-                       float* out) {
-    const size_t N = (size_t)n * n * n;
-    hipLaunchKernelGGL(k_symmetrize, dim3(nblk(N)), dim3(256), 0, s, n, pitch, ng, gperm, gflip, in, out);
 }
 
 void launch_oc_trial(hipStream_t s, int n, int pitch, double g, double min_rho, double step, double damp,

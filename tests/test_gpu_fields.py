@@ -72,3 +72,13 @@ def test_maps_on_device_arrays(n, pitch, shift):
     result(3 * a * a * b, 6)
     assert L.homo3d_density_filter(hom.handle, ptr[0], ptr[2], pitch, 2.0, 0, 0, 0, 1) == 0
     result(fo.conv(a, 2.0)[0], 4)
+
+
+@pytest.mark.parametrize("n", [20, 28, 72])
+@pytest.mark.parametrize("sym", ["reflect3", "reflect6", "rotate3"])
+def test_symmetrize(orc, n, sym):
+    """Orbits across partial workgroups, bit for bit (the FP64 sums run in the group's order)."""
+    print("symmetrize: n=%d %s" % (n, sym), flush=True)
+    hom = homo3d_amd.Homogenization(homo3d_amd.HomoConfig(reso=n, solver="none"))
+    f = np.random.default_rng(n).standard_normal(n ** 3).astype(np.float32)
+    assert np.array_equal(hom.symmetrize(f, sym), orc.symmetrize(n, f, sym))
