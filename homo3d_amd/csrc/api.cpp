@@ -318,10 +318,10 @@ void prof_end(homo3d_handle* h, ProfEvent& ev) {
 // One 8-colour sweep.  zero_start: u is taken as zero on entry whatever it holds (forward sweeps
 // only); every colour pass then writes its block without reading later colours.
 // u_half: the level-0 u is packed FP16 (coarse levels are always FP32).
-// dot_out (level 0, reverse sweeps of a packed-FP16 u with fused colour pairs; returns false otherwise):
+// dot_out (level 0, reverse sweeps of a packed-FP16 u; returns false otherwise):
 // also the per-load-case f . u after the sweep, accumulated by the pair kernels as each vertex gets its
 // final value.
-// rown (zero-start forward sweeps with fused colour pairs, else ignored): the passes also store their
+// rown (zero-start forward sweeps where residual_after_zero_sweep_ok, else ignored): the passes also store their
 // own-colour residuals there, for op_residual_after_zero_sweep.  [pair_begin, pair_end): the
 // colour pairs to launch (level 0 with fused pairs, forward sweeps; a sweep split in two launches the
 // same kernels as a whole one).
@@ -331,7 +331,7 @@ bool op_smooth(homo3d_handle* h, int l, void* u, const float* f, float omega, in
     const Level& L = h->lv[l];
     if (l == 0 && !zero_start) launch_zero_pin(h->stream, L.N, u, u_half);
     const int zs = zero_start && !reverse ? 1 : 0;
-    if (l == 0 && fine_gs_pairs_ok(L.n)) {  // colours two at a time (same result as one by one)
+    if (l == 0) {  // colours two at a time (same result as one by one)
         const bool dot = dot_out && reverse && u_half;
         const int G = gs_pair_blocks(L.n);  // workgroups per pair launch
         for (int cc = reverse ? 0 : 2 * pair_begin; cc < (reverse ? 8 : 2 * pair_end); cc += 2) {
@@ -354,26 +354,18 @@ bool op_smooth(homo3d_handle* h, int l, void* u, const float* f, float omega, in
                                zs ? rown : nullptr);
         return false;
     }
-    for (int cc = 0; cc < 8; cc++) {
-        const int c = reverse ? 7 - cc : cc;
-        if (l == 0) {
-            ProfEvent ev;
-            prof_begin(h, zs ? kProfGsZero : kProfGs, ev);
-            launch_fine_gs(h->stream, L.n, c, omega, reverse, zs, h->d_ke, h->d_w, u, u_half, f);
-            prof_end(h, ev);
-        } else {
-            launch_stencil_gs(h->stream, L.n, c, omega, reverse, zs, L.st, L.st_half, u, u_half, f);
-        }
-    }
+    for (int cc = 0; cc < 8; cc++)
+        launch_stencil_gs(h->stream, L.n, reverse ? 7 - cc : cc, omega, reverse, zs, static_cast<const float*>(L.st),
+                          static_cast<float*>(u), f);
     return false;
 }
 
 // After a zero-start forward sweep that stored its own-colour residuals in r (op_smooth rown):
-// r = f - K u from the later-colour terms alone.  Level 0 needs fused colour pairs; coarse levels
+// r = f - K u from the later-colour terms alone.  Coarse levels need
 // their colour pairs (six load cases per launch).
 bool residual_after_zero_sweep_ok(const homo3d_handle* h, int l = 0) {
     const Level& L = h->lv[l];
-    return l == 0 ? fine_gs_pairs_ok(L.n) != 0 : stencil_gs_pairs_ok(L.n, L.lex) != 0;
+    return l == 0 || stencil_gs_pairs_ok(L.n, L.lex) != 0;
 }
 
 void op_residual_after_zero_sweep(homo3d_handle* h, int l, const void* u, int u_half, float* r) {
@@ -509,11 +501,9 @@ int vcycle_sweeps(homo3d_handle* h, float omega, int pre, int post) {
     return HOMO3D_OK;
 }
 
-// The first launch of a preconditioning V-cycle (u0_zero, level 0 with fused colour pairs): colour
+// The first launch of a preconditioning V-cycle (u0_zero): level 0's colour
 // pair 0 of the pre-smoothing, queued ahead so that the GPU has work while the host reads the CG
 // norms; vcycle(..., head_done = true) then continues from pair 1.
-bool vcycle_head_ok(const homo3d_handle* h) { return fine_gs_pairs_ok(h->lv[0].n) != 0; }
-
 void vcycle_head(homo3d_handle* h, void* u0, const float* f0, int u0_half) {
     Level& L = h->lv[0];
     op_smooth(h, 0, u0, f0, (float)h->cfg.sor_omega, 0, true, u0_half, nullptr,
@@ -617,7 +607,6 @@ int pcg_inner(homo3d_handle* h, const double* r0n2, const double* tol, const boo
         HIPCHK(h, hipHostMalloc((void**)&h->h_rr, sizeof(double) * kRhs, hipHostMallocDefault));
         HIPCHK(h, hipEventCreateWithFlags(&h->ev_rr, hipEventDisableTiming));
     }
-    const bool ahead = vcycle_head_ok(h);
     double rr[kRhs];
     bool x_pending = false;
     for (int it = 0; it < maxit; it++) {
@@ -633,7 +622,7 @@ int pcg_inner(homo3d_handle* h, const double* r0n2, const double* tol, const boo
         x_pending = true;  // alpha p is added by the next operator pass, or by the pass after the loop
         HIPCHK(h, hipMemcpyAsync(h->h_rr, h->d_tmp, sizeof(rr), hipMemcpyDeviceToHost, h->stream));
         HIPCHK(h, hipEventRecord(h->ev_rr, h->stream));
-        const bool head = ahead && it + 1 < maxit;
+        const bool head = it + 1 < maxit;
         if (head) vcycle_head(h, h->Z, h->Rr, zh);
         HIPCHK(h, hipEventSynchronize(h->ev_rr));
         std::copy(h->h_rr, h->h_rr + kRhs, rr);

@@ -41,14 +41,11 @@ int fine_cg_staged_ok(int n);
 void launch_fine_apply_cg(hipStream_t s, int n, const float* ke, const FineMfma* mf, const float* w, const void* z,
                           int z_half, int staged, float* p, float* x, const double* sc, int first, float* q,
                           double* partial, int dot_blocks, double* out6);
-// zero_start: colour pass of a forward sweep that starts from u = 0 (u need not be cleared)
-void launch_fine_gs(hipStream_t s, int n, int colour, float omega, int reverse, int zero_start, const float* ke,
-                    const float* w, void* u, int u_half, const float* f);
 // Colours cfirst and cfirst + 1 (cfirst even; REVERSE: cfirst and cfirst - 1, cfirst odd) in one launch,
-// identical to two launch_fine_gs calls; only when fine_gs_pairs_ok(n).  With partial (reverse sweeps of
+// the second colour reading the first one's new values.  zero_start: part of a forward sweep that starts from
+// u = 0 (u need not be cleared).  n even, at most 512.  With partial (reverse sweeps of
 // a packed-FP16 u only), each of the gs_pair_blocks(n) workgroups also writes its FP64 sums of f . u_new per
 // load case to partial[r * pstride + workgroup].
-int fine_gs_pairs_ok(int n);
 int gs_pair_blocks(int n);
 // rown (zero-start forward passes; ignored otherwise): both colours also store, per vertex, f minus the
 // K u terms of the colours swept so far (the vertex itself included); after the sweep,
@@ -93,12 +90,11 @@ void launch_coarse_factor(hipStream_t s, int nc, const float* st, double* ainv, 
 int stencil_u_half_ok(int n, int lex);
 void launch_stencil_apply(hipStream_t s, int n, int lex, const void* st, int st_half, const void* u, int u_half,
                           const float* f, float* out);
-void launch_stencil_gs(hipStream_t s, int n, int colour, float omega, int reverse, int zero_start, const void* st,
-                       int st_half, void* u, int u_half, const float* f);
+void launch_stencil_gs(hipStream_t s, int n, int colour, float omega, int reverse, int zero_start, const float* st,
+                       float* u, const float* f);  // FP32, n <= 32
 // Small coarse levels (smallgrid.hip; parity-blocked, n <= 32, packed FP16 stencils, FP32 fields).
 int small_level_ok(int n, int lex, int st_half);
-// A whole sweep in two launches of four colours each, identical to eight launch_stencil_gs calls up to the
-// order of a vertex's 27 products.
+// A whole sweep in two launches of four colours each.
 void launch_plane_sweep(hipStream_t s, int n, float omega, int reverse, int zero_start, const void* st, float* u,
                         const float* f);
 // The bottom of a V(1,1) cycle from the last smoothed level (n points an axis, vcycle_tail_ok: 8 to 14) with
@@ -108,7 +104,7 @@ int vcycle_tail_ok(int n, int lex, int st_half);
 void launch_vcycle_tail(hipStream_t s, int n, float omega, int reverse, const void* st, float* u, const float* f,
                         float* res, float* uc, float* fc, const double* Ainv);
 // Colours cfirst and cfirst + 1 (cfirst even; reverse: cfirst and cfirst - 1, cfirst odd) of a coarse
-// parity-blocked level in one launch, identical to two launch_stencil_gs calls; only when
+// parity-blocked level in one launch, the second colour reading the first one's new values; only when
 // stencil_gs_pairs_ok(n, lex) (levels above 32^3 whose grid rows fit a workgroup).
 // rown (zero-start forward passes; ignored otherwise): the own-colour residuals, as launch_fine_gs2
 // stores them; launch_stencil_residual_later completes them to f - A u after the sweep.

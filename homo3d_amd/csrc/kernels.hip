@@ -1037,19 +1037,8 @@ __device__ __forceinline__ void gs_vertex(const Lay& L, size_t N, uint32_t v, fl
     }
 }
 
-// One colour of the fine block GS / SOR sweep, in place (gs_relaxation_otf_kernel, grid.cu:323-551).
-template <int R, bool REVERSE, int ZC, typename A>
-__global__ __launch_bounds__(256, 4) void k_fine_gs(Lay L, size_t N, int colour, float omega,
-                                                    const float* __restrict__ ke, const float* __restrict__ w,
-                                                    A* __restrict__ u, const float* __restrict__ f) {
-    const KeBlocks kb = ke_blocks(ke);
-    const uint32_t t = xcd_chunk(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
-    if (t >= L.h3) return;
-    gs_vertex<R, REVERSE, ZC, A, false, false>(L, N, colour_block(colour) * L.h3 + t, omega, kb, w, u, f,
-                                              R == 6 ? 0 : (int)blockIdx.y * R, XNbLds<A>(), nullptr);
-}
-
-// Two consecutive colours of a sweep in one launch: cfirst, then cfirst + 1 (forward) or cfirst - 1
+// Two consecutive colours of a fine block GS / SOR sweep in one launch, in place
+// (gs_relaxation_otf_kernel, grid.cu:323-551): cfirst, then cfirst + 1 (forward) or cfirst - 1
 // (REVERSE), cfirst even resp. odd.  DOT: per-workgroup FP64 sums of f . u_new over the pair's vertices
 // per load case to partial[r * pstride + blockIdx.x] (over the four pair launches of a sweep that is
 // the last to write u, this is the r . z of the CG step).  The two colours differ only in x-parity, and a vertex of the
@@ -1614,15 +1603,15 @@ __device__ __forceinline__ void stencil_gs_vertex(const Lay& L, size_t N, uint32
     }
 }
 
-// One colour of the coarse block GS sweep (gs_relaxation_kernel, grid.cu:556-689); no pin on coarse levels.
-template <int R, bool REVERSE, int ZC, typename SA, typename A = float>
-__global__ __launch_bounds__(256) void k_stencil_gs(Lay L, size_t N, int colour, float omega,
-                                                    const SA* __restrict__ st, A* __restrict__ u,
-                                                    const float* __restrict__ f) {
+// One colour of the coarse block GS sweep (gs_relaxation_kernel, grid.cu:556-689) on a level of at most 32^3
+// with FP32 stencils, a load case per thread; no pin on coarse levels.
+template <bool REVERSE, int ZC>
+__global__ __launch_bounds__(256) void k_stencil_gs(Lay L, size_t N, int colour, float omega, const float* __restrict__ st,
+                                                    float* __restrict__ u, const float* __restrict__ f) {
     const uint32_t t = xcd_chunk(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
     if (t >= L.h3) return;
-    stencil_gs_vertex<R, REVERSE, ZC, SA, A, false, false>(L, N, colour_block(colour) * L.h3 + t, omega, st, u, f,
-                                                           blockIdx.y * R, XNbLds<A>(), nullptr);
+    stencil_gs_vertex<1, REVERSE, ZC, float, float, false, false>(L, N, colour_block(colour) * L.h3 + t, omega, st, u, f,
+                                                                  blockIdx.y, XNbLds<float>(), nullptr);
 }
 
 // Two consecutive colours of a coarse sweep in one launch, as k_fine_gs2 does at the finest level
@@ -2445,46 +2434,6 @@ void launch_fine_apply_cg(hipStream_t s, int n, const float* ke, const FineMfma*
     hipLaunchKernelGGL(k_sum_partials, dim3(6), dim3(kSumThreads), 0, s, (int)nb, partial, out6);
 }
 
-template <bool REV, int ZC, typename A>
-static void fine_gs_colour(hipStream_t s, const Lay& L, size_t N, int colour, float omega, const float* ke,
-                           const float* w, A* u, const float* f) {
-    hipLaunchKernelGGL((k_fine_gs<6, REV, ZC, A>), dim3(nblk(L.h3)), dim3(256), 0, s, L, N, colour, omega, ke, w, u,
-                       f);
-}
-
-template <typename A>
-static void fine_gs_pick(hipStream_t s, const Lay& L, size_t N, int colour, float omega, int reverse, int zero_start,
-                         const float* ke, const float* w, A* u, const float* f) {
-    if (reverse) {
-        fine_gs_colour<true, -1>(s, L, N, colour, omega, ke, w, u, f);
-        return;
-    }
-    switch (zero_start ? colour : -1) {
-        case 0: fine_gs_colour<false, 0>(s, L, N, colour, omega, ke, w, u, f); break;
-        case 1: fine_gs_colour<false, 1>(s, L, N, colour, omega, ke, w, u, f); break;
-        case 2: fine_gs_colour<false, 2>(s, L, N, colour, omega, ke, w, u, f); break;
-        case 3: fine_gs_colour<false, 3>(s, L, N, colour, omega, ke, w, u, f); break;
-        case 4: fine_gs_colour<false, 4>(s, L, N, colour, omega, ke, w, u, f); break;
-        case 5: fine_gs_colour<false, 5>(s, L, N, colour, omega, ke, w, u, f); break;
-        case 6: fine_gs_colour<false, 6>(s, L, N, colour, omega, ke, w, u, f); break;
-        case 7: fine_gs_colour<false, 7>(s, L, N, colour, omega, ke, w, u, f); break;
-        default: fine_gs_colour<false, -1>(s, L, N, colour, omega, ke, w, u, f); break;
-    }
-}
-
-void launch_fine_gs(hipStream_t s, int n, int colour, float omega, int reverse, int zero_start, const float* ke,
-                    const float* w, void* u, int u_half, const float* f) {
-    const size_t N = (size_t)n * n * n;
-    const Lay L = make_lay(n, 0);
-    if (u_half)
-        fine_gs_pick(s, L, N, colour, omega, reverse, zero_start, ke, w, static_cast<half2_t*>(u), f);
-    else
-        fine_gs_pick(s, L, N, colour, omega, reverse, zero_start, ke, w, static_cast<float*>(u), f);
-}
-
-// fused colour pairs need every workgroup to own whole rows of one parity block
-int fine_gs_pairs_ok(int n) { return n % 2 == 0 && n >= 4 && n / 2 <= 256; }
-
 // a multiple of 8, so that each XCD gets a contiguous run (workgroups past the last row do nothing)
 int gs_pair_blocks(int n) {
     const int h = n / 2;
@@ -2658,42 +2607,10 @@ void launch_stencil_apply(hipStream_t s, int n, int lex, const void* st, int st_
         stencil_apply_pick(s, L, N, split, static_cast<const float*>(st), u, u_half, f, out);
 }
 
-template <int R, bool REV, int ZC, typename SA, typename A>
-static void stencil_gs_colour(hipStream_t s, const Lay& L, size_t N, int colour, float omega, const SA* st, A* u,
+template <bool REV, int ZC>
+static void stencil_gs_colour(hipStream_t s, const Lay& L, size_t N, int colour, float omega, const float* st, float* u,
                               const float* f) {
-    hipLaunchKernelGGL((k_stencil_gs<R, REV, ZC, SA, A>), dim3(nblk(L.h3), 6 / R), dim3(256), 0, s, L, N, colour, omega,
-                       st, u, f);
-}
-
-template <int R, typename SA, typename A>
-static void stencil_gs_pick(hipStream_t s, const Lay& L, size_t N, int colour, float omega, int reverse,
-                            int zero_start, const SA* st, A* u, const float* f) {
-    if (reverse) {
-        stencil_gs_colour<R, true, -1>(s, L, N, colour, omega, st, u, f);
-        return;
-    }
-    switch (zero_start ? colour : -1) {
-        case 0: stencil_gs_colour<R, false, 0>(s, L, N, colour, omega, st, u, f); break;
-        case 1: stencil_gs_colour<R, false, 1>(s, L, N, colour, omega, st, u, f); break;
-        case 2: stencil_gs_colour<R, false, 2>(s, L, N, colour, omega, st, u, f); break;
-        case 3: stencil_gs_colour<R, false, 3>(s, L, N, colour, omega, st, u, f); break;
-        case 4: stencil_gs_colour<R, false, 4>(s, L, N, colour, omega, st, u, f); break;
-        case 5: stencil_gs_colour<R, false, 5>(s, L, N, colour, omega, st, u, f); break;
-        case 6: stencil_gs_colour<R, false, 6>(s, L, N, colour, omega, st, u, f); break;
-        case 7: stencil_gs_colour<R, false, 7>(s, L, N, colour, omega, st, u, f); break;
-        default: stencil_gs_colour<R, false, -1>(s, L, N, colour, omega, st, u, f); break;
-    }
-}
-
-template <typename SA>
-static void stencil_gs_st(hipStream_t s, const Lay& L, size_t N, bool split, int colour, float omega, int reverse,
-                          int zero_start, const SA* st, void* u, int u_half, const float* f) {
-    if (u_half)
-        stencil_gs_pick<6>(s, L, N, colour, omega, reverse, zero_start, st, static_cast<half2_t*>(u), f);
-    else if (split)
-        stencil_gs_pick<1>(s, L, N, colour, omega, reverse, zero_start, st, static_cast<float*>(u), f);
-    else
-        stencil_gs_pick<6>(s, L, N, colour, omega, reverse, zero_start, st, static_cast<float*>(u), f);
+    hipLaunchKernelGGL((k_stencil_gs<REV, ZC>), dim3(nblk(L.h3), 6), dim3(256), 0, s, L, N, colour, omega, st, u, f);
 }
 
 template <int R, bool REV, int ZC, typename SA, typename A, bool ROWN = false>
@@ -2739,7 +2656,7 @@ static void stencil_gs2_st(hipStream_t s, const Lay& L, size_t N, int cfirst, fl
 
 // pairs only where a launch runs six load cases per thread: on the one-case levels (<= 32^3) the
 // launch is latency-bound and two colours in one cost more than two launches (14 vs 11 us at 32^3)
-int stencil_gs_pairs_ok(int n, int lex) { return !lex && n > kSplitLoadCasesMaxN && fine_gs_pairs_ok(n); }
+int stencil_gs_pairs_ok(int n, int lex) { return !lex && n > kSplitLoadCasesMaxN; }
 
 void launch_stencil_gs2(hipStream_t s, int n, int cfirst, float omega, int reverse, int zero_start, const void* st,
                         int st_half, void* u, int u_half, const float* f, float* rown) {
@@ -2783,16 +2700,25 @@ void launch_stencil_residual_later(hipStream_t s, int n, const void* st, int st_
         stencil_resid_later_st(s, L, N, static_cast<const float*>(st), u, u_half, r);
 }
 
-void launch_stencil_gs(hipStream_t s, int n, int colour, float omega, int reverse, int zero_start, const void* st,
-                       int st_half, void* u, int u_half, const float* f) {
+void launch_stencil_gs(hipStream_t s, int n, int colour, float omega, int reverse, int zero_start, const float* st,
+                       float* u, const float* f) {
     const size_t N = (size_t)n * n * n;
     const Lay L = make_lay(n, 0);
-    const bool split = n <= kSplitLoadCasesMaxN;
-    if (u_half && !stencil_u_half_ok(n, 0)) return;  // the caller checks stencil_u_half_ok
-    if (st_half)
-        stencil_gs_st(s, L, N, split, colour, omega, reverse, zero_start, static_cast<const half2_t*>(st), u, u_half, f);
-    else
-        stencil_gs_st(s, L, N, split, colour, omega, reverse, zero_start, static_cast<const float*>(st), u, u_half, f);
+    if (reverse) {
+        stencil_gs_colour<true, -1>(s, L, N, colour, omega, st, u, f);
+        return;
+    }
+    switch (zero_start ? colour : -1) {
+        case 0: stencil_gs_colour<false, 0>(s, L, N, colour, omega, st, u, f); break;
+        case 1: stencil_gs_colour<false, 1>(s, L, N, colour, omega, st, u, f); break;
+        case 2: stencil_gs_colour<false, 2>(s, L, N, colour, omega, st, u, f); break;
+        case 3: stencil_gs_colour<false, 3>(s, L, N, colour, omega, st, u, f); break;
+        case 4: stencil_gs_colour<false, 4>(s, L, N, colour, omega, st, u, f); break;
+        case 5: stencil_gs_colour<false, 5>(s, L, N, colour, omega, st, u, f); break;
+        case 6: stencil_gs_colour<false, 6>(s, L, N, colour, omega, st, u, f); break;
+        case 7: stencil_gs_colour<false, 7>(s, L, N, colour, omega, st, u, f); break;
+        default: stencil_gs_colour<false, -1>(s, L, N, colour, omega, st, u, f); break;
+    }
 }
 
 // Transfers take one load case per thread (six grid rows): the load cases' planes are disjoint, so
