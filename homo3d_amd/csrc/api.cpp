@@ -315,6 +315,9 @@ void prof_end(homo3d_handle* h, ProfEvent& ev) {
 // ---------------------------------------------------------------------------------------------
 // Level operations
 // ---------------------------------------------------------------------------------------------
+// What follows a sum into `out`: beta, where that is the CG step's rz_new.
+int then_of(const homo3d_handle* h, const double* out) { return out == h->d_sc + 3 * kRhs ? kSumRz : kSumOnly; }
+
 // One 8-colour sweep.  zero_start: u is taken as zero on entry whatever it holds (forward sweeps
 // only); every colour pass then writes its block without reading later colours.
 // u_half: the level-0 u is packed FP16 (coarse levels are always FP32).
@@ -324,12 +327,12 @@ void prof_end(homo3d_handle* h, ProfEvent& ev) {
 // rown (zero-start forward sweeps where residual_after_zero_sweep_ok, else ignored): the passes also store their
 // own-colour residuals there, for op_residual_after_zero_sweep.  [pair_begin, pair_end): the
 // colour pairs to launch (level 0 with fused pairs, forward sweeps; a sweep split in two launches the
-// same kernels as a whole one).
+// same kernels as a whole one).  pinned: the origin of the level-0 u is zero already.
 bool op_smooth(homo3d_handle* h, int l, void* u, const float* f, float omega, int reverse, bool zero_start = false,
                int u_half = 0, double* dot_out = nullptr, float* rown = nullptr, int pair_begin = 0,
-               int pair_end = 4) {
+               int pair_end = 4, bool pinned = false) {
     const Level& L = h->lv[l];
-    if (l == 0 && !zero_start) launch_zero_pin(h->stream, L.N, u, u_half);
+    if (l == 0 && !zero_start && !pinned) launch_zero_pin(h->stream, L.N, u, u_half);
     const int zs = zero_start && !reverse ? 1 : 0;
     if (l == 0) {  // colours two at a time (same result as one by one)
         const bool dot = dot_out && reverse && u_half;
@@ -341,7 +344,7 @@ bool op_smooth(homo3d_handle* h, int l, void* u, const float* f, float omega, in
                             dot ? h->d_partial + (size_t)(cc / 2) * G : nullptr, 4 * G, zs ? rown : nullptr);
             prof_end(h, ev);
         }
-        if (dot) launch_sum_partials(h->stream, kRhs, 4 * G, h->d_partial, dot_out);
+        if (dot) launch_sum_partials(h->stream, kRhs, 4 * G, h->d_partial, dot_out, then_of(h, dot_out), h->d_sc);
         return dot;
     }
     if (l > 0 && !u_half && small_level_ok(L.n, L.lex, L.st_half)) {
@@ -467,8 +470,11 @@ int vcycle(homo3d_handle* h, void* u0, const float* f0, int symmetric, double* r
         launch_prolong(h->stream, L.n, h->lv[l + 1].lex, h->lv[l + 1].u, u_half_of(l + 1), u, uh, l == 0 ? 1 : 0);
         const int sweeps = l > 0 && L.n <= kSmallLevelN && L.n > kSmallLevelMinN ? small_sweeps : 1;
         for (int k = 1; k < sweeps; k++) op_smooth(h, l, u, f, omega, symmetric ? 1 : 0, false, uh);
-        const bool fused = op_smooth(h, l, u, f, omega, symmetric ? 1 : 0, false, uh, l == 0 ? dot_out : nullptr);
-        if (l == 0 && dot_out && !fused) launch_dot_rz(h->stream, 3 * L.N, f0, u0, uh, h->d_partial, kDotBlocks, dot_out);
+        // (the pre-smoothing zeroed the origin, and the prolongation leaves it)
+        const bool fused = op_smooth(h, l, u, f, omega, symmetric ? 1 : 0, false, uh, l == 0 ? dot_out : nullptr, nullptr, 0,
+                                     4, l == 0);
+        if (l == 0 && dot_out && !fused)
+            launch_dot_rz(h->stream, 3 * L.N, f0, u0, uh, h->d_partial, kDotBlocks, dot_out, then_of(h, dot_out), h->d_sc);
     }
     return HOMO3D_OK;
 }
@@ -614,10 +620,9 @@ int pcg_inner(homo3d_handle* h, const double* r0n2, const double* tol, const boo
             ProfEvent ev;
             prof_begin(h, it ? kProfApply : kProfApplyFirst, ev);
             launch_fine_apply_cg(h->stream, L0.n, h->d_ke, h->mf(), h->d_w, h->Z, zh, h->stage_tiles ? 1 : 0, h->P,
-                                 h->X, h->d_sc, it == 0, h->Q, h->d_partial, kDotBlocks, h->d_sc + kRhs);  // pq
+                                 h->X, h->d_sc, it == 0, h->Q, h->d_partial, kDotBlocks);  // pq and alpha
             prof_end(h, ev);
         }
-        launch_pcg_alpha(h->stream, h->d_sc);
         launch_pcg_update_r(h->stream, M, h->d_sc, h->Q, h->Rr, h->d_partial, kDotBlocks, h->d_tmp);
         x_pending = true;  // alpha p is added by the next operator pass, or by the pass after the loop
         HIPCHK(h, hipMemcpyAsync(h->h_rr, h->d_tmp, sizeof(rr), hipMemcpyDeviceToHost, h->stream));
@@ -647,9 +652,8 @@ int pcg_inner(homo3d_handle* h, const double* r0n2, const double* tol, const boo
             HIPCHK(h, hipMemcpyAsync(h->d_sc + 5 * kRhs, sc + 5 * kRhs, sizeof(double) * kRhs, hipMemcpyHostToDevice,
                                      h->stream));
         rc = vcycle(h, h->Z, h->Rr, 1, nullptr, true, zh, h->d_sc + 3 * kRhs, kPrecondSmallSweeps,
-                    head);  // with rz_new
+                    head);  // with rz_new and beta
         if (rc) return rc;
-        launch_pcg_beta(h->stream, h->d_sc);
     }
     *x_pending_out = x_pending;
     return HOMO3D_OK;

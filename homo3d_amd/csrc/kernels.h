@@ -39,8 +39,8 @@ void launch_fine_apply(hipStream_t s, int n, const float* ke, const FineMfma* mf
 // gathering the neighbours from memory; the results are the same bit for bit.
 int fine_cg_staged_ok(int n);
 void launch_fine_apply_cg(hipStream_t s, int n, const float* ke, const FineMfma* mf, const float* w, const void* z,
-                          int z_half, int staged, float* p, float* x, const double* sc, int first, float* q,
-                          double* partial, int dot_blocks, double* out6);
+                          int z_half, int staged, float* p, float* x, double* sc, int first, float* q,
+                          double* partial, int dot_blocks);
 // Colours cfirst and cfirst + 1 (cfirst even; REVERSE: cfirst and cfirst - 1, cfirst odd) in one launch,
 // the second colour reading the first one's new values.  zero_start: part of a forward sweep that starts from
 // u = 0 (u need not be cleared).  n even, at most 512.  With partial (reverse sweeps of
@@ -123,10 +123,14 @@ void launch_galerkin_fine(hipStream_t s, int nf, int lexc, const double* G, cons
 void launch_galerkin_coarse(hipStream_t s, int nf, int lexc, const void* stf, int in_half, void* stc, int out_half,
                             double* work, float clamp);
 void launch_coarse_solve(hipStream_t s, int nc, const double* Ainv, const float* f, float* u);
-void launch_dot6(hipStream_t s, size_t M, const float* a, const float* b, double* partial, int nblocks, double* out);
-void launch_sum_partials(hipStream_t s, int R, int nblocks, const double* partial, double* out);
-void launch_pcg_alpha(hipStream_t s, double* sc);
-void launch_pcg_beta(hipStream_t s, double* sc);
+// then: what else the sums' workgroups form from them for a CG step, in sc = [rz | pq | alpha | rz_new | beta |
+// active], six doubles each.  kSumPq (out = sc + 6): alpha = rz / pq; kSumRz (out = sc + 18): beta = rz_new / rz,
+// rz = rz_new.
+enum { kSumOnly = 0, kSumPq = 1, kSumRz = 2 };
+void launch_dot6(hipStream_t s, size_t M, const float* a, const float* b, double* partial, int nblocks, double* out,
+                 int then = kSumOnly, double* sc = nullptr);
+void launch_sum_partials(hipStream_t s, int R, int nblocks, const double* partial, double* out, int then = kSumOnly,
+                         double* sc = nullptr);
 // CG updates over 6 load cases of M floats each (M % 4 == 0): r -= alpha q with |r|^2 -> out6;
 // x += alpha p and, when do_p, p = z + beta p for the active load cases.
 void launch_pcg_update_r(hipStream_t s, size_t M, const double* sc, const float* q, float* r, double* partial,
@@ -138,7 +142,7 @@ void launch_pcg_update_px(hipStream_t s, size_t M, const double* sc, const void*
 hipError_t launch_set_p(hipStream_t s, size_t M, const void* z, int z_half, float* p, int nblocks);
 // per-load-case r . z -> out6 (z FP32 or packed FP16)
 void launch_dot_rz(hipStream_t s, size_t M, const float* r, const void* z, int z_half, double* partial, int nblocks,
-                   double* out6);
+                   double* out6, int then = kSumOnly, double* sc = nullptr);
 // C^H sums and sensitivity of the fields chi (energy.hip); lam, mu the Lame parameters, wdc 21 host floats
 void launch_elastic_matrix(hipStream_t s, int n, double lam, double mu, const float* w, const float* chi,
                            double* partial, int nblocks, double* out21);

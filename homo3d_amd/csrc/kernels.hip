@@ -1971,11 +1971,15 @@ __global__ __launch_bounds__(256) void k_dot(size_t M, const float* __restrict__
     if (threadIdx.x == 0) partial[r * gridDim.x + blockIdx.x] = s;
 }
 
-// out[r] = sum of partial[r * nb .. r * nb + nb), one workgroup per row r = blockIdx.x
 // out[r] = sum of partial[r * nb + i] over i < nb; one workgroup per row, four independent loads in
 // flight per thread.
-__global__ __launch_bounds__(kSumThreads) void k_sum_partials(int nb, const double* __restrict__ partial,
-                                                              double* __restrict__ out) {
+//
+// What a CG step derives from a sum is formed by the workgroup that has it (a launch of its own is 4 us and a
+// gap): sc = [rz | pq | alpha | rz_new | beta | active], six each; kSumPq: out is pq, alpha = rz / pq;
+// kSumRz: out is rz_new, beta = rz_new / rz, then rz = rz_new.  Zero for load cases no longer active.
+template <int THEN>
+__global__ __launch_bounds__(kSumThreads) void k_sum_partials(int nb, const double* __restrict__ partial, double* out,
+                                                              double* sc) {
     __shared__ double sh[kSumThreads / 64];
     const double* p = partial + (size_t)blockIdx.x * nb;
     double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
@@ -1988,24 +1992,16 @@ __global__ __launch_bounds__(kSumThreads) void k_sum_partials(int nb, const doub
     }
     for (; i < nb; i += kSumThreads) s0 += p[i];
     const double s = block_sum<kSumThreads>((s0 + s1) + (s2 + s3), sh);
-    if (threadIdx.x == 0) out[blockIdx.x] = s;
-}
-
-// PCG scalars per load case.  sc layout: [0..R) rz, [R..2R) pq, [2R..3R) alpha, [3R..4R) rz_new,
-// [4R..5R) beta, [5R..6R) active flag.
-__global__ void k_pcg_alpha(int R, double* sc) {
-    const int r = threadIdx.x;
-    if (r >= R) return;
-    const double pq = sc[R + r];
-    sc[2 * R + r] = (sc[5 * R + r] != 0.0 && pq != 0.0) ? sc[r] / pq : 0.0;
-}
-
-__global__ void k_pcg_beta(int R, double* sc) {
-    const int r = threadIdx.x;
-    if (r >= R) return;
-    const double rz = sc[r], rzn = sc[3 * R + r];
-    sc[4 * R + r] = (sc[5 * R + r] != 0.0 && rz != 0.0) ? rzn / rz : 0.0;
-    sc[r] = rzn;
+    if (threadIdx.x == 0) {
+        const int r = (int)blockIdx.x;
+        out[r] = s;
+        if constexpr (THEN == kSumPq) sc[12 + r] = sc[30 + r] != 0.0 && s != 0.0 ? sc[r] / s : 0.0;
+        if constexpr (THEN == kSumRz) {
+            const double rz = sc[r];
+            sc[24 + r] = sc[30 + r] != 0.0 && rz != 0.0 ? s / rz : 0.0;
+            sc[r] = s;
+        }
+    }
 }
 
 // CG vector updates, one grid row per load case k = blockIdx.y, grid-stride over the M values of a
@@ -2388,8 +2384,8 @@ static void fine_apply_cg_row(hipStream_t s, const Lay& L, size_t N, const float
 int fine_cg_staged_ok(int n) { return n % 128 == 0; }
 
 void launch_fine_apply_cg(hipStream_t s, int n, const float* ke, const FineMfma* mf, const float* w, const void* z,
-                          int z_half, int staged, float* p, float* x, const double* sc, int first, float* q,
-                          double* partial, int dot_blocks, double* out6) {
+                          int z_half, int staged, float* p, float* x, double* sc, int first, float* q,
+                          double* partial, int dot_blocks) {
     constexpr int R = 6;
     const size_t N = (size_t)n * n * n, M = 3 * N;
     const Lay L = make_lay(n, 0);
@@ -2408,7 +2404,7 @@ void launch_fine_apply_cg(hipStream_t s, int n, const float* ke, const FineMfma*
             launch_pcg_update_px(s, M, sc, z, 0, p, x, 1, dot_blocks);
         }
         launch_fine_apply(s, n, ke, nullptr, w, p, 0, nullptr, q);
-        launch_dot6(s, M, p, q, partial, dot_blocks, out6);
+        launch_dot6(s, M, p, q, partial, dot_blocks, sc + R, kSumPq, sc);
         return;
     } else if (z_half && staged && fine_cg_staged_ok(n)) {
         const uint32_t* zw = static_cast<const uint32_t*>(z);
@@ -2431,7 +2427,7 @@ void launch_fine_apply_cg(hipStream_t s, int n, const float* ke, const FineMfma*
         else
             fine_apply_cg_row<float, false>(s, L, N, ke, w, zf, p, x, sc, q, partial);
     }
-    hipLaunchKernelGGL(k_sum_partials, dim3(6), dim3(kSumThreads), 0, s, (int)nb, partial, out6);
+    launch_sum_partials(s, R, (int)nb, partial, sc + R, kSumPq, sc);
 }
 
 // a multiple of 8, so that each XCD gets a contiguous run (workgroups past the last row do nothing)
@@ -2519,7 +2515,7 @@ void launch_fine_residual64(hipStream_t s, int n, const double* ke, const double
         hipLaunchKernelGGL((k_fine_residual64<false>), g, b, 0, s, L, N, ke, kchi, xc, emin, u, r32, partial);
     else
         hipLaunchKernelGGL((k_fine_residual64<true>), g, b, 0, s, L, N, ke, kchi, xc, emin, u, r32, partial);
-    hipLaunchKernelGGL(k_sum_partials, dim3(6), dim3(kSumThreads), 0, s, (int)full_grid(L), partial, out6);
+    launch_sum_partials(s, 6, (int)full_grid(L), partial, out6);
 }
 
 void launch_rhs_norm64(hipStream_t s, int n, const double* kchi, const float* xc, double emin, double* partial,
@@ -2528,7 +2524,7 @@ void launch_rhs_norm64(hipStream_t s, int n, const double* kchi, const float* xc
     const Lay L = make_lay(n, 0);
     const unsigned nb = full_grid(L);
     hipLaunchKernelGGL(k_rhs_norm64, dim3(nb), dim3(kFullThreads), 0, s, L, N, kchi, xc, emin, partial);
-    hipLaunchKernelGGL(k_sum_partials, dim3(6), dim3(kSumThreads), 0, s, (int)nb, partial, out6);
+    launch_sum_partials(s, 6, (int)nb, partial, out6);
 }
 
 void launch_refine_accumulate(hipStream_t s, size_t N, const double* sc, int pending, const float* x, const float* p,
@@ -2750,22 +2746,25 @@ void launch_prolong(hipStream_t s, int nf, int lexc, const void* uc, int uc_half
 }
 
 void launch_dot6(hipStream_t s, size_t M, const float* a, const float* b, double* partial, int nblocks,
-                 double* out) {
+                 double* out, int then, double* sc) {
     hipLaunchKernelGGL(k_dot, dim3(nblocks, 6), dim3(256), 0, s, M, a, b, partial);
-    hipLaunchKernelGGL(k_sum_partials, dim3(6), dim3(kSumThreads), 0, s, nblocks, partial, out);
+    launch_sum_partials(s, 6, nblocks, partial, out, then, sc);
 }
 
-void launch_sum_partials(hipStream_t s, int R, int nblocks, const double* partial, double* out) {
-    hipLaunchKernelGGL(k_sum_partials, dim3(R), dim3(kSumThreads), 0, s, nblocks, partial, out);
+void launch_sum_partials(hipStream_t s, int R, int nblocks, const double* partial, double* out, int then, double* sc) {
+    if (then == kSumPq)
+        hipLaunchKernelGGL(k_sum_partials<kSumPq>, dim3(R), dim3(kSumThreads), 0, s, nblocks, partial, out, sc);
+    else if (then == kSumRz)
+        hipLaunchKernelGGL(k_sum_partials<kSumRz>, dim3(R), dim3(kSumThreads), 0, s, nblocks, partial, out, sc);
+    else
+        hipLaunchKernelGGL(k_sum_partials<kSumOnly>, dim3(R), dim3(kSumThreads), 0, s, nblocks, partial, out, nullptr);
 }
 
-void launch_pcg_alpha(hipStream_t s, double* sc) { hipLaunchKernelGGL(k_pcg_alpha, dim3(1), dim3(64), 0, s, 6, sc); }
-void launch_pcg_beta(hipStream_t s, double* sc) { hipLaunchKernelGGL(k_pcg_beta, dim3(1), dim3(64), 0, s, 6, sc); }
 
 void launch_pcg_update_r(hipStream_t s, size_t M, const double* sc, const float* q, float* r, double* partial,
                          int nblocks, double* out6) {
     hipLaunchKernelGGL(k_pcg_update_r, dim3(nblocks, 6), dim3(256), 0, s, 6, M, sc, q, r, partial);
-    hipLaunchKernelGGL(k_sum_partials, dim3(6), dim3(kSumThreads), 0, s, nblocks, partial, out6);
+    launch_sum_partials(s, 6, nblocks, partial, out6);
 }
 
 void launch_pcg_update_px(hipStream_t s, size_t M, const double* sc, const void* z, int z_half, float* p, float* x,
@@ -2786,20 +2785,20 @@ hipError_t launch_set_p(hipStream_t s, size_t M, const void* z, int z_half, floa
 }
 
 void launch_dot_rz(hipStream_t s, size_t M, const float* r, const void* z, int z_half, double* partial, int nblocks,
-                   double* out6) {
+                   double* out6, int then, double* sc) {
     if (!z_half) {
-        launch_dot6(s, M, r, static_cast<const float*>(z), partial, nblocks, out6);
+        launch_dot6(s, M, r, static_cast<const float*>(z), partial, nblocks, out6, then, sc);
         return;
     }
     hipLaunchKernelGGL(k_dot_fh, dim3(nblocks, 3), dim3(256), 0, s, M, r, static_cast<const half2_t*>(z), partial);
-    hipLaunchKernelGGL(k_sum_partials, dim3(6), dim3(kSumThreads), 0, s, nblocks, partial, out6);
+    launch_sum_partials(s, 6, nblocks, partial, out6, then, sc);
 }
 
 void launch_oc_trial(hipStream_t s, int n, int pitch, double g, double min_rho, double step, double damp,
                      const float* sens, const float* rho, float* out, double* partial, int nblocks, double* sum) {
     hipLaunchKernelGGL(k_oc_trial, dim3(nblocks), dim3(256), 0, s, n, pitch, g, min_rho, step, damp, sens, rho, out,
                        partial);
-    hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(kSumThreads), 0, s, nblocks, partial, sum);
+    launch_sum_partials(s, 1, nblocks, partial, sum);
 }
 
 void launch_field_sum(hipStream_t s, int n, int pitch, const float* a, double* partial, int nblocks) {
@@ -3000,7 +2999,7 @@ extern "C" int homo3d_oc_update_noalloc(const float* sens, float* rho, int n, in
         double sum = 0;
         hipLaunchKernelGGL(k_oc_trial, dim3(kOcBlocks), dim3(256), 0, s, n, pitch, g, min_rho, step, damp, sens,
                            (const float*)rho, (float*)nullptr, partial);
-        hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(kSumThreads), 0, s, kOcBlocks, (const double*)partial, total);
+        launch_sum_partials(s, 1, kOcBlocks, (const double*)partial, total);
         if (hipMemcpyAsync(&sum, total, sizeof(double), hipMemcpyDeviceToHost, s) != hipSuccess ||
             hipStreamSynchronize(s) != hipSuccess)
             return HOMO3D_HIP_ERROR;
