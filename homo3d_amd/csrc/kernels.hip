@@ -90,8 +90,8 @@ __device__ __forceinline__ T cell_form(const W wc[8]) {
 //
 // The constants are wave-uniform and come through the scalar cache (kKeBlocks floats into ke, 12 a block,
 // set when the operator is made), loaded a neighbour ahead: they cost neither vector loads, nor
-// registers, nor the staging of KE at the start of a workgroup.  At 256^3 the CG pass takes 1.67 ms and a
-// colour pair 0.37 ms (1.83 and 0.385 with the constants read from LDS).
+// registers, nor the staging of KE at the start of a workgroup.  At 256^3 the CG pass takes 1.67 to
+// 1.80 ms and a colour pair 0.37 ms (1.83 and 0.385 with the constants read from LDS).
 struct BlockConsts {
     float v[9];
 };
@@ -351,6 +351,78 @@ __device__ __forceinline__ void fine_gather(const FineCtx& c, size_t N, KeBlocks
     }
 }
 
+// The same sum for FP32 u where every 64 consecutive vertices are whole grid rows (64 % (n/2) == 0): of a
+// vertex's two x-neighbours, which alternate in the other x-parity's block, one sits at the vertex's own
+// position (x - 1 for PXP = 1, the odd vertices, x + 1 for 0) and the other is that of the next lane of the
+// row, so one load and a lane exchange (through LDS, byte address `lane`) serve both: 324 loads of single words
+// instead of 486, which the texture addresser was busy with (a colour pair at 128^3 81 us for 90, at 64^3 21
+// for 24; the residual 206 for 270 and 27 for 34).  Unit U: row U / 2, its middle or its sides.
+constexpr bool unit_in(uint32_t mask, int u) { return mask >> (3 * (u / 2) + (u & 1 ? 0 : 1)) & 1u; }
+constexpr int next_unit(uint32_t mask, int u) {
+    for (int k = u + 1; k < 18; k++)
+        if (unit_in(mask, k)) return k;
+    return 18;
+}
+
+template <int R, int PXP, bool XL, int U>
+__device__ __forceinline__ void load_unit(float (&dst)[R][3], const FineCtx& c, Rsrc ru, uint32_t plane, int r0,
+                                          const XNbLds<float>& xl) {
+    constexpr int D = 3 * (U / 2) + (U & 1 ? (PXP ? 0 : 2) : 1);
+    load_nb_at<R, float, XL, D>(dst, c, ru, plane, r0, xl);
+}
+
+template <int R, uint32_t MASK, int PXP, bool XL, int U>
+__device__ __forceinline__ void gather_unit(const FineCtx& c, KeBlocks kb, Rsrc ru, uint32_t plane, int r0, int lane,
+                                            const BlockConsts& k, const float (&cur)[R][3], float (&acc)[R][3],
+                                            const XNbLds<float>& xl) {
+    constexpr int row = U / 2, UN = next_unit(MASK, U);
+    constexpr bool sides = U & 1;
+    constexpr int D = 3 * row + (sides ? (PXP ? 0 : 2) : 1), DS = 3 * row + (PXP ? 2 : 0);
+    __builtin_amdgcn_sched_barrier(0);
+    pin_acc<R, float>(acc);
+    float nxt[R][3], far[R][3];
+    if constexpr (UN < 18) load_unit<R, PXP, XL, UN>(nxt, c, ru, plane, r0, xl);
+    BlockConsts kn = {}, ks = {};
+    if constexpr (UN < 18) kn = block_consts<3 * (UN / 2) + (UN & 1 ? (PXP ? 0 : 2) : 1)>(kb);
+    if constexpr (sides) {
+        ks = block_consts<DS>(kb);
+        if constexpr (XL && row == 4) {
+            load_nb_lds<R, float>(far, xl, PXP ? 1 : 0);
+        } else {
+#pragma unroll
+            for (int r = 0; r < R; r++)
+#pragma unroll
+                for (int i = 0; i < 3; i++)
+                    far[r][i] = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(lane, __builtin_bit_cast(int, cur[r][i])));
+        }
+    }
+    float S[9];
+    fine_block<D>(c.wc, k, S);
+    block_fma<R, float, float>(S, cur, acc);
+    if constexpr (sides) {
+        fine_block<DS>(c.wc, ks, S);
+        block_fma<R, float, float>(S, far, acc);
+    }
+    if constexpr (UN < 18) gather_unit<R, MASK, PXP, XL, UN>(c, kb, ru, plane, r0, lane, kn, nxt, acc, xl);
+}
+
+template <int R, uint32_t MASK, int PXP, bool XL>
+__device__ __forceinline__ void fine_gather_rows(const FineCtx& c, int h, size_t N, KeBlocks kb, const float* __restrict__ u,
+                                                 float (&acc)[R][3], int r0, const XNbLds<float>& xl) {
+    const Rsrc ru = make_rsrc(u, (size_t)18 * N * sizeof(float));
+    const uint32_t plane = (uint32_t)(N * sizeof(float));
+    const int l = (int)(threadIdx.x & 63u), lane = 4 * ((l & ~(h - 1)) | ((l + (PXP ? 1 : -1)) & (h - 1)));
+#pragma unroll
+    for (int r = 0; r < R; r++)
+#pragma unroll
+        for (int i = 0; i < 3; i++) acc[r][i] = 0.f;
+    constexpr int U0 = next_unit(MASK, -1);
+    float first[R][3];
+    const BlockConsts k = block_consts<3 * (U0 / 2) + (U0 & 1 ? (PXP ? 0 : 2) : 1)>(kb);
+    load_unit<R, PXP, XL, U0>(first, c, ru, plane, r0, xl);
+    gather_unit<R, MASK, PXP, XL, U0>(c, kb, ru, plane, r0, lane, k, first, acc, xl);
+}
+
 // Stage the FP64 element matrix in LDS (all threads of the block take part), followed by the block
 // constants of fine_block: C_d,ij = KE[7 - e0][b0](i, j)
 // for the cell e0 with e0_m = 1 exactly where d_m = +1 and b0_m = d_m + 1 - e0_m.
@@ -393,7 +465,7 @@ __device__ __forceinline__ uint32_t colour_block(int colour) { return (uint32_t)
 // PX (with DOT, u = z): the CG vector updates of the step, fused: p = z (PX 1, first step) or
 // x += alpha p_old, p = z + beta p_old (PX 2), per load case with alpha, beta from the device; the dot
 // is then p . out with the new p (dotv unused).  Load cases that have converged carry alpha = beta = 0.
-template <int R, int MODE, bool DOT, typename A, bool BETA = false, int PX = 0, int PF = 1>
+template <int R, int MODE, bool DOT, typename A, bool BETA = false, int PX = 0, int PF = 1, bool LANES = false>
 __global__ __launch_bounds__(kFullThreads, 4) void k_fine_apply(Lay L, size_t N, const float* __restrict__ ke,
                                                                 const float* __restrict__ w,
                                                                 const A* __restrict__ u,
@@ -412,7 +484,14 @@ __global__ __launch_bounds__(kFullThreads, 4) void k_fine_apply(Lay L, size_t N,
     FineCtx c;
     fine_ctx(c, x, y, z, L, w);
     float acc[R][3];
-    fine_gather<R, kRowAll, A, false, PF>(c, N, kb, u, acc);
+    if constexpr (LANES) {  // a wave is in one parity block
+        if (__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) & 1)
+            fine_gather_rows<R, kRowAll, 1, false>(c, L.h, N, kb, u, acc, 0, XNbLds<A>());
+        else
+            fine_gather_rows<R, kRowAll, 0, false>(c, L.h, N, kb, u, acc, 0, XNbLds<A>());
+    } else {
+        fine_gather<R, kRowAll, A, false, PF>(c, N, kb, u, acc);
+    }
     double dot[R];
 #pragma unroll
     for (int r = 0; r < R; r++) {
@@ -962,7 +1041,8 @@ constexpr int kGsAhead = CasesPerWord<A>::value == 2 ? 3 : 1;
 // rown = f - sum over the neighbours of colours up to ZC and the vertex itself of K_vj u_j, with the
 // stored values; once the sweep is complete, subtracting the later colours' terms gives f - K u.
 // The pinned origin keeps u = 0 (and rown = 0).
-template <int R, bool REVERSE, int ZC, typename A, bool XL, bool TO_LDS, bool DOT = false, bool ROWN = false>
+// PXP: the vertex's x-parity where its row is whole in the wave and u is FP32 (fine_gather_rows), else -1.
+template <int R, bool REVERSE, int ZC, typename A, bool XL, bool TO_LDS, bool DOT = false, bool ROWN = false, int PXP = -1>
 __device__ __forceinline__ void gs_vertex(const Lay& L, size_t N, uint32_t v, float omega, KeBlocks kb,
                                           const float* __restrict__ w, A* __restrict__ u,
                                           const float* __restrict__ f, int r0, const XNbLds<A>& xl, A* out_lds,
@@ -974,7 +1054,10 @@ __device__ __forceinline__ void gs_vertex(const Lay& L, size_t N, uint32_t v, fl
     FineCtx c;
     fine_ctx(c, x, y, z, L, w);
     float acc[R][3];
-    fine_gather<R, gs_mask(ZC), A, XL, kGsAhead<A>>(c, N, kb, u, acc, r0, xl);
+    if constexpr (PXP >= 0)
+        fine_gather_rows<R, gs_mask(ZC), PXP, XL>(c, L.h, N, kb, u, acc, r0, xl);
+    else
+        fine_gather<R, gs_mask(ZC), A, XL, kGsAhead<A>>(c, N, kb, u, acc, r0, xl);
     float Ks[9];
     fine_block<13>(c.wc, block_consts<13>(kb), Ks);
     const float inv[3] = {1.f / Ks[0], 1.f / Ks[4], 1.f / Ks[8]};
@@ -1048,7 +1131,8 @@ __device__ __forceinline__ void gs_vertex(const Lay& L, size_t N, uint32_t v, fl
 // in LDS, and updates the second colour reading those x-neighbours from LDS.  Other workgroups never read the rows' first-colour values
 // before they are final, so the result equals the two colour passes in sequence.
 // ROWN (zero-start passes): both colours also store their own-colour residuals to rown (gs_vertex).
-template <int R, bool REVERSE, int ZC, typename A, bool DOT = false, bool ROWN = false>
+// LANES: gs_vertex's PXP (colour c lies in block 7 - c).
+template <int R, bool REVERSE, int ZC, typename A, bool DOT = false, bool ROWN = false, bool LANES = false>
 __global__ __launch_bounds__(256, 4) void k_fine_gs2(Lay L, size_t N, int cfirst, float omega,
                                                      const float* __restrict__ ke, const float* __restrict__ w,
                                                      A* __restrict__ u, const float* __restrict__ f,
@@ -1065,7 +1149,7 @@ __global__ __launch_bounds__(256, 4) void k_fine_gs2(Lay L, size_t N, int cfirst
 #pragma unroll
     for (int r = 0; r < R; r++) dot[r] = 0.f;
     if (live)
-        gs_vertex<R, REVERSE, ZC, A, false, true, DOT, ROWN>(L, N, colour_block(cfirst) * L.h3 + t, omega, kb, w, u,
+        gs_vertex<R, REVERSE, ZC, A, false, true, DOT, ROWN, LANES ? (REVERSE ? 0 : 1) : -1>(L, N, colour_block(cfirst) * L.h3 + t, omega, kb, w, u,
                                                             f, 0, XNbLds<A>(), xs, dot, rown);
     __syncthreads();
     if (live) {
@@ -1075,7 +1159,7 @@ __global__ __launch_bounds__(256, 4) void k_fine_gs2(Lay L, size_t N, int cfirst
         const bool odd = (colour_block(c2) & 1u) != 0;  // x-parity of the second colour
         xl.slot[0] = row0 + (odd ? lx : (lx == 0 ? h - 1 : lx - 1));
         xl.slot[1] = row0 + (odd ? (lx + 1 == h ? 0 : lx + 1) : lx);
-        gs_vertex<R, REVERSE, (ZC < 0 ? -1 : ZC + 1), A, true, false, DOT, ROWN>(
+        gs_vertex<R, REVERSE, (ZC < 0 ? -1 : ZC + 1), A, true, false, DOT, ROWN, LANES ? (REVERSE ? 1 : 0) : -1>(
             L, N, colour_block(c2) * L.h3 + t, omega, kb, w, u, f, 0, xl, nullptr, dot, rown);
     }
     if constexpr (DOT) {
@@ -2360,7 +2444,10 @@ void launch_fine_apply(hipStream_t s, int n, const float* ke, const FineMfma* mf
         return;
     }
     const float* uf = static_cast<const float*>(u);
-    if (f)
+    if (f && 64 % L.h == 0)
+        hipLaunchKernelGGL((k_fine_apply<6, 1, false, float, false, 0, 1, true>), g, b, 0, s, L, N, ke, w, uf, f, out,
+                           nullptr, nullptr, nullptr, nullptr, nullptr, nullptr);
+    else if (f)
         hipLaunchKernelGGL((k_fine_apply<6, 1, false, float>), g, b, 0, s, L, N, ke, w, uf, f, out, nullptr, nullptr,
                            nullptr, nullptr, nullptr, nullptr);
     else
@@ -2440,6 +2527,13 @@ template <bool REV, int ZC, typename A, bool DOT = false, bool ROWN = false>
 static void fine_gs2_pair(hipStream_t s, const Lay& L, size_t N, int cfirst, float omega, const float* ke,
                           const float* w, A* u, const float* f, double* partial = nullptr, int pstride = 0,
                           float* rown = nullptr) {
+    if constexpr (CasesPerWord<A>::value == 1 && ZC < 0) {
+        if (64 % L.h == 0) {
+            hipLaunchKernelGGL((k_fine_gs2<6, REV, ZC, A, DOT, ROWN, true>), dim3(gs_pair_blocks(L.n)), dim3(256), 0, s, L, N,
+                               cfirst, omega, ke, w, u, f, partial, pstride, rown);
+            return;
+        }
+    }
     hipLaunchKernelGGL((k_fine_gs2<6, REV, ZC, A, DOT, ROWN>), dim3(gs_pair_blocks(L.n)), dim3(256), 0, s, L, N, cfirst, omega,
                        ke, w, u, f, partial, pstride, rown);
 }
