@@ -1603,7 +1603,7 @@ __global__ __launch_bounds__(kFullThreads) void k_stencil_apply(Lay L, size_t N,
 }
 
 // GS / SOR update of the colour vertex v of a coarse level (load cases r0 .. r0 + R - 1), in place.
-// ZC as in k_fine_gs.  A: u storage (float, or half2_t load-case pairs with FP32 arithmetic).  XL: the
+// ZC as in k_fine_gs2.  A: u storage (float, or half2_t load-case pairs with FP32 arithmetic).  XL: the
 // x-neighbours come from LDS; TO_LDS: the new words also go to slot threadIdx.x of out_lds.  ROWN
 // (ZC >= 0): also the own-colour residual f - (A u)_{colours <= ZC} to rown, as gs_vertex does.
 template <int R, bool REVERSE, int ZC, typename SA, typename A, bool XL, bool TO_LDS, bool ROWN = false>

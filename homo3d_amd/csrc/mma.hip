@@ -545,64 +545,64 @@ __global__ __launch_bounds__(kMmaCtlThreads) void k_mma_accept(MmaState* st, con
     __shared__ double total[kMmaSums];
     constexpr int per = 2 + M;
     reduce_parts(part, nb, (phase == kPhaseSearch ? kMmaCand : 1) * per, per, total);
-    if (threadIdx.x) return;
+    if (threadIdx.x >= 64) return;
+    // a lane forms each candidate's residual, the first that is taken goes on
+    const int k = (int)threadIdx.x, tries = phase == kPhaseSearch ? kMmaCand : 1, itto = st->itto;
+    const double* q = total + (k < tries ? k : 0) * per;
+    double steg = st->steg;
+    for (int i = 0; i < k && i < tries; i++) steg *= 0.5;
     MmaSmall<M> v;
-    const double* q = total;
-    double steg = st->steg, residunorm = st->residunorm;
-    int itto = st->itto;
-    const int tries = phase == kPhaseSearch ? kMmaCand : 1;
-#pragma unroll 1
-    for (int k = 0; k < tries; k++, q += per) {
-        if (phase == kPhaseSearch) {
+    if (phase == kPhaseSearch) {
 #pragma unroll
-            for (int i = 0; i < M; i++) {
-                v.y[i] = st->yo[i] + steg * st->dy[i];
-                v.lam[i] = st->lamo[i] + steg * st->dlam[i];
-                v.mu[i] = st->muo[i] + steg * st->dmu[i];
-                v.s[i] = st->so[i] + steg * st->ds[i];
-            }
-            v.z = st->zo + steg * st->dz;
-            v.zet = st->zeto + steg * st->dzet;
-        } else {
+        for (int i = 0; i < M; i++) {
+            v.y[i] = st->yo[i] + steg * st->dy[i];
+            v.lam[i] = st->lamo[i] + steg * st->dlam[i];
+            v.mu[i] = st->muo[i] + steg * st->dmu[i];
+            v.s[i] = st->so[i] + steg * st->ds[i];
+        }
+        v.z = st->zo + steg * st->dz;
+        v.zet = st->zeto + steg * st->dzet;
+    } else {
 #pragma unroll
-            for (int i = 0; i < M; i++) {
-                v.y[i] = st->y[i];
-                v.lam[i] = st->lam[i];
-                v.mu[i] = st->mu[i];
-                v.s[i] = st->s[i];
-            }
-            v.z = st->z;
-            v.zet = st->zet;
+        for (int i = 0; i < M; i++) {
+            v.y[i] = st->y[i];
+            v.lam[i] = st->lam[i];
+            v.mu[i] = st->mu[i];
+            v.s[i] = st->s[i];
         }
-        itto++;
-        double s2 = q[0], m2 = q[1 + M];
-        small_residual<M>(st, v, q + 1, s2, m2);
-        const double resinew = sqrt(s2);
-        if (phase == kPhaseSearch && resinew > residunorm && itto < 50) {
-            steg *= 0.5;
-            continue;
-        }
-        if (phase == kPhaseSearch) {
+        v.z = st->z;
+        v.zet = st->zet;
+    }
+    double s2 = q[0], m2 = q[1 + M];
+    small_residual<M>(st, v, q + 1, s2, m2);
+    const double resinew = sqrt(s2);
+    const bool taken = k < tries && !(phase == kPhaseSearch && resinew > st->residunorm && itto + k + 1 < 50);
+    const unsigned long long any = __ballot(taken);
+    if (!any) {  // every candidate refused: the next pass goes on from here
+        if (k == tries) {
+            st->itto = itto + tries;
             st->steg = steg;
-            st->pending = 1;
-#pragma unroll
-            for (int i = 0; i < M; i++) {
-                st->y[i] = v.y[i];
-                st->lam[i] = v.lam[i];
-                st->mu[i] = v.mu[i];
-                st->s[i] = v.s[i];
-            }
-            st->z = v.z;
-            st->zet = v.zet;
         }
-#pragma unroll
-        for (int i = 0; i < M; i++) st->gvec[i] = q[1 + i];
-        st->residunorm = resinew;
-        next_phase(st, m2);
         return;
     }
-    st->itto = itto;  // every candidate refused: the next pass goes on from here
-    st->steg = steg;
+    if (k != __ffsll(any) - 1) return;
+    if (phase == kPhaseSearch) {
+        st->steg = steg;
+        st->pending = 1;
+#pragma unroll
+        for (int i = 0; i < M; i++) {
+            st->y[i] = v.y[i];
+            st->lam[i] = v.lam[i];
+            st->mu[i] = v.mu[i];
+            st->s[i] = v.s[i];
+        }
+        st->z = v.z;
+        st->zet = v.zet;
+    }
+#pragma unroll
+    for (int i = 0; i < M; i++) st->gvec[i] = q[1 + i];
+    st->residunorm = resinew;
+    next_phase(st, m2);
 }
 
 // The subproblem's solution becomes the design: xold2 <- xold1 <- x <- solution (mmasub_g,
