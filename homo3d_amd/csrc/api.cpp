@@ -82,7 +82,7 @@ struct homo3d_handle {
     float* d_stage = nullptr;   // pitched staging buffer for host densities / sensitivities
     size_t stage_elems = 0;
     double* d_Ainv = nullptr;       // the coarsest level's dense FP64 inverse (mc x mc)
-    int* d_cstat = nullptr;         // factorisation status on the device
+    int* d_cstat = nullptr;         // factorisation status on the device (two words, the result in the first)
     double* d_cwork = nullptr;      // the elimination's other buffer (mc x mc)
     int mc = 0;
     // the coarsest factorisation runs on the GPU at the density update, on a stream of its own behind
@@ -831,7 +831,7 @@ int homo3d_create(const homo3d_config* cfg, homo3d_handle** out) {
         return fail(HOMO3D_HIP_ERROR);
     const int nc = sizes[nl - 1];
     h->mc = 3 * nc * nc * nc;
-    if (hipMalloc(&h->d_Ainv, sizeof(double) * h->mc * h->mc) || hipMalloc(&h->d_cstat, sizeof(int)) ||
+    if (hipMalloc(&h->d_Ainv, sizeof(double) * h->mc * h->mc) || hipMalloc(&h->d_cstat, 2 * sizeof(int)) ||
         hipMalloc(&h->d_cwork, sizeof(double) * h->mc * h->mc))
         return fail(HOMO3D_HIP_ERROR);
     if (hipDeviceSynchronize() != hipSuccess) return fail(HOMO3D_HIP_ERROR);

@@ -232,7 +232,7 @@ __global__ __launch_bounds__(256) void k_galerkin_z(Lay Lc, int nf, const double
 // ---------------------------------------------------------------------------------------------
 
 // A = (S + S^T) / 2 of the stencil's matrix S (entry k = 9d + 3i + j of vertex v couples (v, i) with
-// (v + d, j)), one thread per entry; status = 0.
+// (v + d, j)), one thread per entry; *status = 0.
 __global__ __launch_bounds__(256) void k_coarse_assemble(int nc, const float* __restrict__ st, double* __restrict__ A,
                                                          int* __restrict__ status) {
     const int Nc = nc * nc * nc, m = 3 * Nc;
@@ -267,14 +267,22 @@ __global__ __launch_bounds__(256) void k_coarse_assemble(int nc, const float* __
 // D = A[K][K]^-1:  A'[K][K] = D, A'[K][J] = D A[K][J], A'[I][K] = -A[I][K] D,
 // A'[I][J] = A[I][J] - A[I][K] D A[K][J].  Every workgroup inverts the diagonal block itself by scalar
 // Gauss-Jordan steps in registers (one barrier a step), whose pivots are the Schur complements: positive
-// exactly when A is positive definite (the squares of the Cholesky pivots).  status = 0, or 1 + the first
-// step whose pivot is not positive (every workgroup sees the same pivot and stops; later launches see the
-// status and do nothing).  A launch per scalar step took 3.2-5 us m times (0.63 ms at m = 192).
+// exactly when A is positive definite (the squares of the Cholesky pivots).  A launch finds in *before 0, or
+// 1 + the first step whose pivot was not positive (it then does nothing), and leaves the same after itself
+// in *after.  These are two words, as A and B are two buffers: a workgroup that read the word which another
+// one of the same launch may set could see it in some of its waves only, and they would part at a barrier.
+// Every workgroup forms the same pivots, so they all stop at the same one.  A launch per scalar step took
+// 3.2-5 us m times (0.63 ms at m = 192).
 constexpr int kGjB = 32;
 
 __global__ __launch_bounds__(256) void k_gj_block(int m, int k0, const double* __restrict__ A, double* __restrict__ B,
-                                                  int* __restrict__ status) {
-    if (*status != 0) return;
+                                                  const int* __restrict__ before, int* __restrict__ after) {
+    const bool writer = blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0;
+    const int failed = *before;
+    if (failed != 0) {
+        if (writer) *after = failed;
+        return;
+    }
     __shared__ double Dv[kGjB][kGjB + 1], Ct[kGjB][kGjB + 1], Rt[kGjB][kGjB + 1], prow[2][kGjB], pcol[2][kGjB];
     const int i = (int)(threadIdx.x >> 3), j0 = (int)(threadIdx.x & 7) * 4;
     const int I = (int)blockIdx.y * kGjB, J = (int)blockIdx.x * kGjB;
@@ -300,7 +308,7 @@ __global__ __launch_bounds__(256) void k_gj_block(int m, int k0, const double* _
             __syncthreads();
             const double piv = prow[buf][k];
             if (!(piv > 0.0)) {  // the same for every thread
-                if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *status = 1 + k0 + k;
+                if (writer) *after = 1 + k0 + k;
                 return;
             }
             const double inv = 1.0 / piv, ci = pcol[buf][i];
@@ -311,6 +319,7 @@ __global__ __launch_bounds__(256) void k_gj_block(int m, int k0, const double* _
             }
         }
     }
+    if (writer) *after = 0;
 #pragma unroll
     for (int q = 0; q < 4; q++) Dv[i][j0 + q] = v[q];
     __syncthreads();
@@ -432,12 +441,15 @@ void launch_coarse_solve(hipStream_t s, int nc, const double* Ainv, const float*
 
 void launch_coarse_factor(hipStream_t s, int nc, const float* st, double* ainv, double* work, int* status) {
     const int m = 3 * nc * nc * nc, nb = (m + kGjB - 1) / kGjB;
-    // the steps alternate between the two buffers and end in ainv
+    // the steps alternate between the two buffers and status words and end in ainv and status[0]
     double* buf[2] = {ainv, work};
-    hipLaunchKernelGGL(k_coarse_assemble, dim3(nblk((size_t)m * m)), dim3(256), 0, s, nc, st, buf[nb & 1], status);
-    for (int k = 0; k < nb; k++)
-        hipLaunchKernelGGL(k_gj_block, dim3(nb, nb), dim3(256), 0, s, m, k * kGjB, buf[(nb - k) & 1],
-                           buf[(nb - k - 1) & 1], status);
+    hipLaunchKernelGGL(k_coarse_assemble, dim3(nblk((size_t)m * m)), dim3(256), 0, s, nc, st, buf[nb & 1],
+                       status + (nb & 1));
+    for (int k = 0; k < nb; k++) {
+        const int from = (nb - k) & 1, to = 1 - from;
+        hipLaunchKernelGGL(k_gj_block, dim3(nb, nb), dim3(256), 0, s, m, k * kGjB, buf[from], buf[to], status + from,
+                           status + to);
+    }
 }
 
 }  // namespace homo3d
