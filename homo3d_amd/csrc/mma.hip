@@ -606,13 +606,14 @@ __global__ __launch_bounds__(kMmaCtlThreads) void k_mma_accept(MmaState* st, con
 }
 
 // The subproblem's solution becomes the design: xold2 <- xold1 <- x <- solution (mmasub_g,
-// mmaOpt.cu:1057-1059), rounded to FP32 for the caller.
+// mmaOpt.cu:1057-1059), rounded to FP32 for the caller.  out may be v.x0 itself.
 template <int M>
 __global__ __launch_bounds__(kMmaThreads) void k_mma_finish(MmaVars v, const MmaState* __restrict__ st,
                                                             double* __restrict__ xcur, double* __restrict__ xold1,
-                                                            double* __restrict__ xold2, float* __restrict__ out) {
+                                                            double* __restrict__ xold2, float* out) {
     const long j = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= v.n || st->status) return;
+    const double x0 = (double)v.x0[j];
     MmaVar<M> a;
     a.load(v, j);
     double x = a.x;
@@ -622,7 +623,7 @@ __global__ __launch_bounds__(kMmaThreads) void k_mma_finish(MmaVars v, const Mma
         x += st->steg * dx;
     }
     xold2[j] = xold1[j];
-    xold1[j] = (double)v.x0[j];
+    xold1[j] = x0;
     xcur[j] = x;
     out[j] = (float)x;
 }
