@@ -95,6 +95,10 @@ __global__ __launch_bounds__(256) void k_conv(const uint16_t* __restrict__ in, i
             nb[0][v] = g;
         }
     }
+    // the wave's lanes read each other's entries below
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     if (vb >= nvox) return;
     constexpr int D = MB + NB > 6 ? 2 : MB + NB > 3 ? 4 : 6;  // chunks of operands in flight
     f32x4 acc[MB][NB];
