@@ -364,8 +364,8 @@ bool op_smooth(homo3d_handle* h, int l, void* u, const float* f, float omega, in
 }
 
 // After a zero-start forward sweep that stored its own-colour residuals in r (op_smooth rown):
-// r = f - K u from the later-colour terms alone.  Coarse levels need
-// their colour pairs (six load cases per launch).
+// r = f - K u from the later-colour terms alone.  Coarse levels need their colour pairs (six load cases
+// per launch).
 bool residual_after_zero_sweep_ok(const homo3d_handle* h, int l = 0) {
     const Level& L = h->lv[l];
     return l == 0 || stencil_gs_pairs_ok(L.n, L.lex) != 0;
@@ -1359,17 +1359,9 @@ int homo3d_smooth16(homo3d_handle* h, double omega, int reverse) {
     return HOMO3D_OK;
 }
 
-// The grids that the presmooth entry points accept: colour pairs with every thread in use.
-static bool rows_fill_workgroups(int n) {
-    const long hn = n / 2;
-    return hn <= 256 && 256 % hn == 0 && hn * hn * hn % 256 == 0;
-}
-
 int homo3d_presmooth16(homo3d_handle* h, double omega) {
     int rc = fp16_ready(h);
     if (rc) return rc;
-    if (!rows_fill_workgroups(h->lv[0].n))
-        return set_err(h, HOMO3D_NO_SUPPORT, "needs fused colour pairs at level 0");
     const Level& L = h->lv[0];
     op_smooth(h, 0, h->Z, h->F, (float)omega, 0, true, 1, nullptr, L.r);
     op_residual_after_zero_sweep(h, 0, h->Z, 1, L.r);
@@ -1384,7 +1376,7 @@ int homo3d_presmooth(homo3d_handle* h, int level, double omega) {
     if (!h || level < 1 || level >= h->nl - 1) return HOMO3D_BAD_ARG;
     int rc = require_density(h);
     if (rc) return rc;
-    if (!residual_after_zero_sweep_ok(h, level) || !rows_fill_workgroups(h->lv[level].n))
+    if (!residual_after_zero_sweep_ok(h, level))
         return set_err(h, HOMO3D_NO_SUPPORT, "level %d has no colour pairs", level);
     Level& L = h->lv[level];
     op_smooth(h, level, L.u, L.f, (float)omega, 0, true, 0, nullptr, L.r);
