@@ -1,5 +1,5 @@
 // Density utilities on pitched lexicographic n^3 arrays: radial filters and their adjoint, projection,
-// elementwise maps, symmetry projection and the OC update.  All of them stream a few FP32 fields, so the
+// elementwise maps and symmetry projection.  All of them stream a few FP32 fields, so the
 // kernels read the caller's arrays where they lie and touch each value once; arithmetic is FP64, rounded
 // to FP32, unless noted.
 #include <hip/hip_runtime.h>
@@ -16,21 +16,6 @@ namespace {
 constexpr int kThreads = 256;
 
 inline unsigned nblk(size_t work, int bs = kThreads) { return (unsigned)((work + bs - 1) / bs); }
-
-template <int BS>
-__device__ __forceinline__ double block_sum(double v, double* sh) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    if (lane == 0) sh[wid] = v;
-    __syncthreads();
-    double s = 0.0;
-    if (threadIdx.x == 0) {
-        for (int i = 0; i < BS / 64; i++) s += sh[i];
-    }
-    __syncthreads();
-    return s;
-}
 
 // ---------------------------------------------------------------------------------------------
 // Elementwise maps.  Unpitched arrays on 16-byte boundaries run four values a thread over the whole

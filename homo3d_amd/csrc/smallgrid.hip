@@ -6,7 +6,7 @@
 // between launches, eight launches a sweep, whatever the size.  Here a launch does four colours.  The
 // colours c and c + 1, c + 2, c + 3 of one z-parity differ in x- and y-parity only, so a vertex of one
 // depends on the others through neighbours in its own z-plane, and planes of the same parity do not meet: a
-// workgroup owns a z-plane for one load case (or one packed pair), keeps that plane and its two neighbours
+// workgroup owns a z-plane for one load case, keeps that plane and its two neighbours
 // of u in LDS, and updates the four colours in turn between barriers.  Three threads share a vertex, one per
 // neighbour plane: each has its 9 stencil blocks (11 st of words) in flight at once, those of the next
 // colour before the barriers of this one.  Bound by that load latency and the barriers: a sweep takes two
@@ -46,66 +46,54 @@ struct PlaneBlocks {
     }
 };
 
-template <typename A>
-__device__ __forceinline__ float word_case(A w, int c) {
-    if constexpr (CasesPerWord<A>::value == 2)
-        return (float)w[c];
-    else
-        return (float)w;
-}
-
 // acc += the blocks of plane G times its u (pl: the plane's three components in LDS, cs words apart); the
 // vertex itself left out.
-template <int G, typename A>
-__device__ __forceinline__ void plane_sum(const PlaneBlocks& w, const A* pl, int cs, const int (&xo)[3],
-                                          const int (&yo)[3], float (&acc)[CasesPerWord<A>::value][3]) {
+template <int G>
+__device__ __forceinline__ void plane_sum(const PlaneBlocks& w, const float* pl, int cs, const int (&xo)[3],
+                                          const int (&yo)[3], float (&acc)[3]) {
 #pragma unroll
     for (int d = 0; d < 9; d++) {
         if (d == 4 && G == 1) continue;
         float S[9];
 #pragma unroll
         for (int k = 0; k < 9; k++) S[k] = w.template get<G>(9 * d + k);
-        const A* q = pl + yo[d / 3] + xo[d % 3];
-        const A u0 = q[0], u1 = q[cs], u2 = q[2 * cs];
+        const float* q = pl + yo[d / 3] + xo[d % 3];
+        const float u0 = q[0], u1 = q[cs], u2 = q[2 * cs];
 #pragma unroll
-        for (int c = 0; c < CasesPerWord<A>::value; c++) {
-            const float a0 = word_case(u0, c), a1 = word_case(u1, c), a2 = word_case(u2, c);
-#pragma unroll
-            for (int i = 0; i < 3; i++)
-                acc[c][i] = fmaf(S[3 * i], a0, fmaf(S[3 * i + 1], a1, fmaf(S[3 * i + 2], a2, acc[c][i])));
-        }
+        for (int i = 0; i < 3; i++)
+            acc[i] = fmaf(S[3 * i], u0, fmaf(S[3 * i + 1], u1, fmaf(S[3 * i + 2], u2, acc[i])));
     }
 }
 
-// Stage plane z of u (word group p) in LDS: natural (y, x) order, n2 words a component.
-template <typename A>
-__device__ __forceinline__ void stage_plane(A* dst, const Lay& L, size_t N, const A* __restrict__ u, int p, int z) {
+// Stage plane z of load case r of u in LDS: natural (y, x) order, n2 words a component.
+__device__ __forceinline__ void stage_plane(float* dst, const Lay& L, size_t N, const float* __restrict__ u, int r,
+                                            int z) {
     const int n = L.n, h = L.h, h2 = h * h, n2 = n * n;
     const uint32_t zp = L.part(z, 2);
     for (int t = threadIdx.x; t < n2; t += blockDim.x) {
         const int b = t / h2, l = t - b * h2, yy = l / h, xx = l - yy * h;
         const uint32_t v = zp + (uint32_t)(b & 1) * L.h3 + (uint32_t)(b >> 1) * 2u * L.h3 + (uint32_t)l;
-        A* q = dst + (2 * yy + (b >> 1)) * n + 2 * xx + (b & 1);
+        float* q = dst + (2 * yy + (b >> 1)) * n + 2 * xx + (b & 1);
 #pragma unroll
-        for (int i = 0; i < 3; i++) q[i * n2] = u[fw_index<A>(p * 3 + i, v, N)];
+        for (int i = 0; i < 3; i++) q[i * n2] = u[(size_t)(r * 3 + i) * N + v];
     }
 }
 
 // Colours 4 (1 - pz) .. + 3 of a sweep (in falling order when REVERSE) on the planes z of parity pz, load
-// cases of word group blockIdx.y.  zero: 0 an ordinary sweep; u = 0 before the sweep whatever it holds, and
+// case blockIdx.y.  zero: 0 an ordinary sweep; u = 0 before the sweep whatever it holds, and
 // this is its first (1: the neighbouring planes are zero too) or second launch (2).  The blocks of the next
 // colour are loaded while this one's are used.
-template <bool REVERSE, typename A>
+template <bool REVERSE>
 __global__ __launch_bounds__(3 * kPlaneVerts) void k_plane_gs(Lay L, size_t N, int pz, float omega, int zero,
-                                                              const uint4* __restrict__ st, A* __restrict__ u,
+                                                              const uint4* __restrict__ st, float* __restrict__ u,
                                                               const float* __restrict__ f) {
-    constexpr int cpw = CasesPerWord<A>::value, NM = 32;
-    __shared__ A us[3 * 3 * NM * NM];
-    __shared__ float red[2][kPlaneVerts][3 * cpw];
+    constexpr int NM = 32;
+    __shared__ float us[3 * 3 * NM * NM];
+    __shared__ float red[2][kPlaneVerts][3];
     const int n = L.n, h = L.h, n2 = n * n, h2 = h * h;
     const int vb = (int)blockDim.x / 3, g = __builtin_amdgcn_readfirstlane((int)threadIdx.x / vb);
     const int lv = (int)threadIdx.x - g * vb;
-    const int kz = (int)blockIdx.x, z = 2 * kz + pz, p = (int)blockIdx.y;
+    const int kz = (int)blockIdx.x, z = 2 * kz + pz, r = (int)blockIdx.y;
     const Rsrc rs = make_rsrc(st, (size_t)StencilIO<half2_t>::words * N * 4);
     const bool live = lv < h2, load = live && !(zero == 1 && g != 1);  // the neighbour planes may be zero
     const int yy = lv / h, xx = lv - yy * h;
@@ -115,93 +103,72 @@ __global__ __launch_bounds__(3 * kPlaneVerts) void k_plane_gs(Lay L, size_t N, i
         const int c = colour(s);
         return v0 + (uint32_t)((1 - (c & 1)) + 2 * (1 - (c >> 1))) * L.h3;
     };
-    auto load_f = [&](int s, float (&ff)[cpw][3]) __attribute__((always_inline)) {
+    auto load_f = [&](int s, float (&ff)[3]) __attribute__((always_inline)) {
         if (g == 1 && live && s < 4) {
 #pragma unroll
-            for (int c = 0; c < cpw; c++)
-#pragma unroll
-                for (int i = 0; i < 3; i++) ff[c][i] = f[(size_t)((p * cpw + c) * 3 + i) * N + vertex(s)];
+            for (int i = 0; i < 3; i++) ff[i] = f[(size_t)(r * 3 + i) * N + vertex(s)];
         }
     };
     PlaneBlocks cur;
-    float ff[cpw][3];
+    float ff[3];
     cur.load(rs, (uint32_t)N, g, vertex(0), load);
     load_f(0, ff);
     if (zero) {
-        for (int t = threadIdx.x; t < 3 * n2; t += blockDim.x) us[3 * n2 + t] = A(0);
+        for (int t = threadIdx.x; t < 3 * n2; t += blockDim.x) us[3 * n2 + t] = 0.f;
     } else {
-        stage_plane(us + 3 * n2, L, N, u, p, z);
+        stage_plane(us + 3 * n2, L, N, u, r, z);
     }
     if (zero != 1) {
-        stage_plane(us, L, N, u, p, z == 0 ? n - 1 : z - 1);
-        stage_plane(us + 6 * n2, L, N, u, p, z == n - 1 ? 0 : z + 1);
+        stage_plane(us, L, N, u, r, z == 0 ? n - 1 : z - 1);
+        stage_plane(us + 6 * n2, L, N, u, r, z == n - 1 ? 0 : z + 1);
     }
     __syncthreads();
 #pragma unroll 1
     for (int s = 0; s < 4; s++) {
         PlaneBlocks nxt;
-        float fn[cpw][3];
+        float fn[3];
         nxt.load(rs, (uint32_t)N, g, vertex(s + 1), load && s < 3);
         load_f(s + 1, fn);
-        float acc[cpw][3], Ks[9];
-#pragma unroll
-        for (int c = 0; c < cpw; c++)
-#pragma unroll
-            for (int i = 0; i < 3; i++) acc[c][i] = 0.f;
+        float acc[3] = {0.f, 0.f, 0.f}, Ks[9];
         const int c4 = colour(s), x = 2 * xx + 1 - (c4 & 1), y = 2 * yy + 1 - (c4 >> 1), me = y * n + x;
         if (load) {
             const int xo[3] = {x == 0 ? n - 1 : x - 1, x, x == n - 1 ? 0 : x + 1};
             const int yo[3] = {(y == 0 ? n - 1 : y - 1) * n, y * n, (y == n - 1 ? 0 : y + 1) * n};
-            const A* pl = us + 3 * n2 * g;
+            const float* pl = us + 3 * n2 * g;
             if (g == 1) {
-                plane_sum<1, A>(cur, pl, n2, xo, yo, acc);
+                plane_sum<1>(cur, pl, n2, xo, yo, acc);
 #pragma unroll
                 for (int k = 0; k < 9; k++) Ks[k] = cur.template get<1>(36 + k);
             } else {
                 if (g == 0)
-                    plane_sum<0, A>(cur, pl, n2, xo, yo, acc);
+                    plane_sum<0>(cur, pl, n2, xo, yo, acc);
                 else
-                    plane_sum<2, A>(cur, pl, n2, xo, yo, acc);
+                    plane_sum<2>(cur, pl, n2, xo, yo, acc);
 #pragma unroll
-                for (int c = 0; c < cpw; c++)
-#pragma unroll
-                    for (int i = 0; i < 3; i++) red[g >> 1][lv][c * 3 + i] = acc[c][i];
+                for (int i = 0; i < 3; i++) red[g >> 1][lv][i] = acc[i];
             }
         }
         __syncthreads();
         if (g == 1 && live) {
             const float inv[3] = {1.f / Ks[0], 1.f / Ks[4], 1.f / Ks[8]};
-            A* own = us + 3 * n2 + me;
-            A wd[3] = {own[0], own[n2], own[2 * n2]};
-#pragma unroll
-            for (int c = 0; c < cpw; c++) {
-                float uu[3];
-#pragma unroll
-                for (int i = 0; i < 3; i++) {
-                    uu[i] = word_case(wd[i], c);
-                    if (zero != 1) acc[c][i] += red[0][lv][c * 3 + i] + red[1][lv][c * 3 + i];
-                }
-                block_update<REVERSE>(uu, ff[c], acc[c], Ks, inv, omega);
-#pragma unroll
-                for (int i = 0; i < 3; i++) {
-                    if constexpr (cpw == 2)
-                        wd[i][c] = (_Float16)uu[i];
-                    else
-                        wd[i] = uu[i];
-                }
-            }
+            float* own = us + 3 * n2 + me;
+            float uu[3];
 #pragma unroll
             for (int i = 0; i < 3; i++) {
-                own[i * n2] = wd[i];
-                u[fw_index<A>(p * 3 + i, vertex(s), N)] = wd[i];
+                uu[i] = own[i * n2];
+                if (zero != 1) acc[i] += red[0][lv][i] + red[1][lv][i];
+            }
+            block_update<REVERSE>(uu, ff, acc, Ks, inv, omega);
+#pragma unroll
+            for (int i = 0; i < 3; i++) {
+                own[i * n2] = uu[i];
+                u[(size_t)(r * 3 + i) * N + vertex(s)] = uu[i];
             }
         }
         __syncthreads();
         cur = nxt;
 #pragma unroll
-        for (int c = 0; c < cpw; c++)
-#pragma unroll
-            for (int i = 0; i < 3; i++) ff[c][i] = fn[c][i];
+        for (int i = 0; i < 3; i++) ff[i] = fn[i];
     }
 }
 
@@ -247,7 +214,7 @@ __device__ __forceinline__ void tail_pass(const Lay& L, size_t N, float omega, c
         const int nk = s + 1 < steps ? (chunk(s + 1) ? pos[1] : pos[0]) : -1;
         PlaneBlocks nxt;
         nxt.load(rs, (uint32_t)N, g, vertex(s + 1), nk >= 0);
-        float acc[1][3] = {{0.f, 0.f, 0.f}}, Ks[9];
+        float acc[3] = {0.f, 0.f, 0.f}, Ks[9];
         const int me3 = chunk(s) ? pos[1] : pos[0];
         int me = 0;
         if (me3 >= 0) {
@@ -257,16 +224,16 @@ __device__ __forceinline__ void tail_pass(const Lay& L, size_t N, float omega, c
             const int xo[3] = {x == 0 ? n - 1 : x - 1, x, x == n - 1 ? 0 : x + 1};
             const int yo[3] = {(y == 0 ? n - 1 : y - 1) * n, y * n, (y == n - 1 ? 0 : y + 1) * n};
             if (g == 1) {
-                plane_sum<1, float>(cur, u + n2 * z, n3, xo, yo, acc);
+                plane_sum<1>(cur, u + n2 * z, n3, xo, yo, acc);
 #pragma unroll
                 for (int k = 0; k < 9; k++) Ks[k] = cur.template get<1>(36 + k);
             } else {
                 if (g == 0)
-                    plane_sum<0, float>(cur, u + n2 * (z == 0 ? n - 1 : z - 1), n3, xo, yo, acc);
+                    plane_sum<0>(cur, u + n2 * (z == 0 ? n - 1 : z - 1), n3, xo, yo, acc);
                 else
-                    plane_sum<2, float>(cur, u + n2 * (z == n - 1 ? 0 : z + 1), n3, xo, yo, acc);
+                    plane_sum<2>(cur, u + n2 * (z == n - 1 ? 0 : z + 1), n3, xo, yo, acc);
 #pragma unroll
-                for (int i = 0; i < 3; i++) red[g >> 1][lv][i] = acc[0][i];
+                for (int i = 0; i < 3; i++) red[g >> 1][lv][i] = acc[i];
             }
         }
         __syncthreads();
@@ -276,16 +243,16 @@ __device__ __forceinline__ void tail_pass(const Lay& L, size_t N, float omega, c
             for (int i = 0; i < 3; i++) {
                 uu[i] = u[me + i * n3];
                 ff[i] = f[me + i * n3];
-                acc[0][i] += red[0][lv][i] + red[1][lv][i];
+                acc[i] += red[0][lv][i] + red[1][lv][i];
             }
             if constexpr (MODE == kTailResidual) {
 #pragma unroll
                 for (int i = 0; i < 3; i++)
-                    r[me + i * n3] = ff[i] - acc[0][i] -
+                    r[me + i * n3] = ff[i] - acc[i] -
                                      fmaf(Ks[3 * i], uu[0], fmaf(Ks[3 * i + 1], uu[1], Ks[3 * i + 2] * uu[2]));
             } else {
                 const float inv[3] = {1.f / Ks[0], 1.f / Ks[4], 1.f / Ks[8]};
-                block_update<MODE == kTailReverse>(uu, ff, acc[0], Ks, inv, omega);
+                block_update<MODE == kTailReverse>(uu, ff, acc, Ks, inv, omega);
 #pragma unroll
                 for (int i = 0; i < 3; i++) u[me + i * n3] = uu[i];
             }
@@ -434,9 +401,9 @@ void launch_plane_sweep(hipStream_t s, int n, float omega, int reverse, int zero
     for (int k = 0; k < 2; k++) {
         const int pz = reverse ? k : 1 - k;  // colours 0..3 are the odd planes
         if (reverse)
-            hipLaunchKernelGGL((k_plane_gs<true, float>), g, b, 0, s, L, N, pz, omega, 0, q, u, f);
+            hipLaunchKernelGGL((k_plane_gs<true>), g, b, 0, s, L, N, pz, omega, 0, q, u, f);
         else
-            hipLaunchKernelGGL((k_plane_gs<false, float>), g, b, 0, s, L, N, pz, omega, zero_start ? k + 1 : 0, q, u, f);
+            hipLaunchKernelGGL((k_plane_gs<false>), g, b, 0, s, L, N, pz, omega, zero_start ? k + 1 : 0, q, u, f);
     }
 }
 
