@@ -19,12 +19,12 @@ struct FineMfma {
     float c0, c1;
     int nt;
 };
-// n for which packed-FP16 fine operators run in element form on the matrix cores
 // The FP32 element matrix as the fine-level kernels take it: KE (576 floats), then from kKeBlocks on the
 // block constants C_d,ij = KE[7 - e0][b0](i, j) of each neighbour offset d at 12 d + 3 i + j, for the cell e0
 // with e0_m = 1 exactly where d_m = +1 and b0_m = d_m + 1 - e0_m.
 constexpr int kKeBlocks = 576, kKeFloats = kKeBlocks + 27 * 12;
 void fine_block_consts(float* ke);  // fills them from KE, on the host
+// n for which packed-FP16 fine operators run in element form on the matrix cores
 int fine_apply_mfma_ok(int n);
 // out = K u (f == nullptr) or f - K u.  With mf, packed-FP16 u and fine_apply_mfma_ok(n) the operator
 // runs in element form on the matrix cores.

@@ -90,8 +90,9 @@ __device__ __forceinline__ T cell_form(const W wc[8]) {
 //
 // The constants are wave-uniform and come through the scalar cache (kKeBlocks floats into ke, 12 a block,
 // set when the operator is made), loaded a neighbour ahead: they cost neither vector loads, nor
-// registers, nor the staging of KE at the start of a workgroup.  At 256^3 the CG pass takes 1.67 to
-// 1.80 ms and a colour pair 0.37 ms (1.83 and 0.385 with the constants read from LDS).
+// registers, nor the staging of KE at the start of a workgroup.  At 256^3 the CG pass takes 1.80 ms (1.87
+// with the constants read from LDS) and a reverse colour pair 0.376 ms (0.389 with that and with its
+// neighbours loaded one ahead instead of three).
 struct BlockConsts {
     float v[9];
 };
@@ -2353,7 +2354,6 @@ __global__ __launch_bounds__(256) void k_copy_pitched(int n, int pitch_in, int p
 // ---------------------------------------------------------------------------------------------
 // Launch wrappers
 // ---------------------------------------------------------------------------------------------
-// workgroups of a full-level kernel (see full_vertex)
 int ke_mfma_table(const double* kl, const double* km, double lam, double mu, void* table, float* c0, float* c1) {
     // One exact table T = r Kl + Km (KE = mu/72 T) when r = lambda / mu is a short binary fraction
     // (nu = 0.3 gives r = 3/2) and every entry of T is an FP16 value; else Kl and Km separately.

@@ -12,11 +12,12 @@
 // each pass from those (72 bytes a variable for m = 2 instead of 104, and no coefficient is ever
 // written), and so is the Newton direction (from the last point and multipliers) instead of being
 // stored.  The line search tries kMmaCand halvings per pass over the variables: it needs 5.2 on average
-// at 128^3, m = 2 (4 a pass: 39.1 ms a step, 8 a pass: 36.1).  There a step of 269 Newton steps takes
-// 34.9 ms (188 with the direction and every trial point stored, a trial per pass and three host waits
-// a Newton step); the passes 31.6 us (Newton sums, with the iterate's update), 24.5 us (step length,
-// 6.2 TB/s of the 151 MB it reads, which stay in the last-level cache) and 49 us (eight trials, bound by
-// FP64 arithmetic), the control kernels 5-8 us each.
+// at 128^3, m = 2 (a step took 39.1 ms with four a pass where it took 36.1 with eight, both with as many
+// search workgroups as the other passes have).  There a step of 269 Newton steps takes 35 ms (188 with the
+// direction and every trial point stored, a trial per pass and three host waits a Newton step); the passes
+// 31.3 us (Newton sums, with the iterate's update), 24.2 us (step length, 6.2 TB/s of the 151 MB it reads,
+// which stay in the last-level cache) and 48.7 us (eight trials, bound by FP64 arithmetic), the control
+// kernels 5-8 us each.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

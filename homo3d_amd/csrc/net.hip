@@ -195,7 +195,7 @@ __global__ __launch_bounds__(256) void k_conv(const uint16_t* __restrict__ in, i
 // channel's voxels in one lane: the transposing LDS reads (four voxels of 16 channels to 16 lanes with a
 // channel each) give that from any voxel on, so nothing is copied to channel-major order first.  Bound by
 // the tiles' loads, X three times over with its neighbour rows.  The 15 layers of a 64^3 x 4 gradient:
-// 0.73 ms with the sums of the partials; with channel-major copies of X (three, shifted in x) and dZ
+// 0.68 ms with the sums of the partials; with channel-major copies of X (three, shifted in x) and dZ
 // through memory, one wave a block on the products and a thread or a block for each sum 7.6 ms.
 // Wave w takes output channels 16 (w % WC) and every (4 / WC)th 32-voxel chunk; a block walks a range of
 // tiles, adds its waves' sums in LDS and leaves one partial; the bias gradient is a 28th product with ones.
@@ -466,7 +466,7 @@ __device__ __forceinline__ float net_weight(const uint16_t* in, long v) {
 // Per (sample, channel) stiffness-weighted mean of the prediction P [v][kPld] over the sample's g^3
 // voxels, and the sample's mean weight.  A sum is 256 chains, of the voxels t, t + 256, ..., then a tree
 // over them.  A wave takes eight chains, eight lanes each: four channels a lane, so that a row of P is read
-// once and not once a channel (36 us and 5 for the trees at 64^3 x 4, 464 with a block a channel); bound by
+// once and not once a channel (109 us and 5 for the trees at 64^3 x 4, 464 with a block a channel); bound by
 // the latency of its loads, 16 of them in flight.
 constexpr int kChains = 256, kMeanRow = 20;  // kOut channels and the weight, padded to the lanes' fours
 
@@ -515,7 +515,7 @@ __global__ __launch_bounds__(kChains) void k_chan_mean(const float* __restrict__
 // dP = 2 (w / wbar) d / count (bf16, channels >= 18 stay 0); per-block FP64 partial sums of
 // (w / wbar) d^2.  T is mean-free under the same weights, so the weighted mean needs no gradient term.
 // A thread takes a group of 8 channels (blockIdx.y: plane); bound by the prediction, target and gradient
-// rows, 190 MB at 64^3 x 4: 52 us (105 with a thread a value).
+// rows, 190 MB at 64^3 x 4: 50 us (105 with a thread a value).
 __global__ __launch_bounds__(256) void k_head_loss(const float* __restrict__ P, const float* __restrict__ mean,
                                                    const float* __restrict__ wbar, const uint16_t* __restrict__ in,
                                                    const uint16_t* __restrict__ T, long nvox, int lgs, double inv_count,
@@ -770,7 +770,7 @@ struct WgPlan {
 };
 
 // Tiles are whole x-rows up to 64 voxels.  Two blocks a compute unit fill the GPU (a block's tile takes 60 KB
-// of LDS in the usual layers, up to 116 KB with 64 output channels at 64 voxels), and every split more is a partial of
+// of LDS in the usual layers, up to 117 KB with 64 output channels at 64 voxels), and every split more is a partial of
 // czp * taps * cxp sums written and read: 512 blocks over the channel tiles.
 WgPlan wgrad_plan(int cz, int cx, int taps, int lg, long nvox) {
     WgPlan w;

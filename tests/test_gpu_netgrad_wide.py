@@ -1,4 +1,4 @@
-"""GPU test of the weight gradient with four tiles of output channels on rows of 32 and 64 voxels (104 and 114 KB
+"""GPU test of the weight gradient with four tiles of output channels on rows of 32 and 64 voxels (106 and 117 KB
 of LDS a workgroup), against the FP64 oracle with the tolerances of the other gradient tests."""
 import pytest
 
