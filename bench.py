@@ -44,13 +44,6 @@ def log(*a):
     print(*a, file=sys.stderr, flush=True)
 
 
-def gs_colours_per_launch(n):
-    """Colours per finest-level GS launch: two when whole grid rows of a parity block fit a 256-thread
-    workgroup (the library fuses colour pairs then), else one."""
-    h = n // 2
-    return 2 if (n % 2 == 0 and h <= 256 and 256 % h == 0 and h ** 3 % 256 == 0) else 1
-
-
 def kernel_bytes(name, n, R=6, s_z=2, s_f=4, s_w=4):
     """Algorithmic HBM bytes per launch of a finest-level kernel.  p, q, r, f, x are FP32 (s_f); the
     preconditioner iterate z (u of the V-cycle's finest level) is packed FP16 (s_z = 2) when n % 8 == 0."""
@@ -61,18 +54,17 @@ def kernel_bytes(name, n, R=6, s_z=2, s_f=4, s_w=4):
         return N * (3 * R * (s_z + 2 * s_f) + s_w)
     if name == "fine_residual":   # r = f - K z: read z, f, write r, read w
         return N * (3 * R * (s_z + s_f + s_f) + s_w)
-    if name == "fine_gs":         # c colours = c/8 of an in-place sweep: z read+write, f read, w read
-        return N * (3 * R * (2 * s_z + s_f) + s_w) * gs_colours_per_launch(n) / 8.0
+    if name == "fine_gs":         # a colour pair, a quarter of an in-place sweep: z read+write, f read, w read
+        return N * (3 * R * (2 * s_z + s_f) + s_w) / 4.0
     return None
 
 
 def gs_pair_must_read(n, R=6, s_z=2, s_f=4, s_w=4):
     """HBM bytes a colour-pair GS launch must move at least: every vertex neighbours the pair's colours, so
     the whole z field and every cell weight is read; f of the pair's vertices is read and their z words
-    written (c/8 of the vertices)."""
+    written (a quarter of the vertices)."""
     N = n ** 3
-    c = gs_colours_per_launch(n) / 8.0
-    return N * (3 * R * s_z + s_w) + N * c * (3 * R * s_f + 3 * R * s_z)
+    return N * (3 * R * s_z + s_w) + N / 4.0 * (3 * R * s_f + 3 * R * s_z)
 
 
 def measured_traffic(name, n):
@@ -229,10 +221,10 @@ def main():
                 "frac": round(achieved / HBM_PEAK_GBS, 5), "traffic": measured_traffic(dom, n), "kernel": dom,
                 "avg_launch_ms": round(ms / cnt, 5),
                 "algorithmic_bytes_per_launch": kernel_bytes(dom, n, s_z=s_z)}
-    # the reverse colour-pair GS launch (VALU-bound): its must-read bytes against the counter traffic
+    # the reverse colour-pair GS launch (texture addresser and VALU): its must-read bytes against the counter traffic
     gs_c, gs_t = prof["fine_gs"]
     gs_pair = None
-    if gs_c and gs_colours_per_launch(n) == 2:
+    if gs_c:
         gb = gs_pair_must_read(n, s_z=s_z)
         gs_ms = gs_t / gs_c
         gtr = measured_traffic("fine_gs", n)
