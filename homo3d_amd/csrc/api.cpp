@@ -1546,8 +1546,16 @@ int homo3d_oc_filter(homo3d_handle* h, float* sens, const float* rho, int pitch,
         HIPCHK(h, hipMemcpyAsync(h->d_ftmp, wk.data(), sizeof(float) * wk.size(), hipMemcpyHostToDevice, h->stream));
         launch_oc_filter(h->stream, n, pitch, hw, periodic, h->d_ftmp, ds, dr, dout);
     }
-    rc = stage_out(h, sens, dout, pitch, on_device);
-    if (rc) return rc;
+    if (here) {
+        rc = stage_out(h, sens, dout, pitch, on_device);
+        if (rc) return rc;
+    } else {
+        // back through the staged copy of sens, padding and all: a copy of the live columns alone moves each
+        // row to the host by itself (109 ms at 128^3 with rows of 160, 1.7 this way)
+        launch_copy_pitched(h->stream, n, pitch, pitch, dout, h->d_stage);
+        HIPCHK(h, hipMemcpyAsync(sens, h->d_stage, sizeof(float) * elems,
+                                 on_device ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost, h->stream));
+    }
     HIPCHK(h, hipStreamSynchronize(h->stream));
     return HOMO3D_OK;
 }
