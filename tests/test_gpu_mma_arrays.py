@@ -13,8 +13,6 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("n,m", [(1000, 1), (70001, 2)])
 def test_host_and_device_arrays(n, m):
-    import torch
-
     print("mma arrays: n=%d m=%d" % (n, m), flush=True)
     rng = np.random.default_rng(n)
     x = rng.uniform(0.2, 0.8, n).astype(np.float32)
@@ -22,21 +20,19 @@ def test_host_and_device_arrays(n, m):
     host, dev = (homo3d_amd.MMAOptimizer(m, n, 1.0, 0.0, 1000.0, 1.0) for _ in range(2))
     host.setBound(0.001, 1.0)
     dev.setBound(0.001, 1.0)
-    xd = torch.from_numpy(x.copy()).cuda()
+    xd = homo3d_amd.DeviceBuffer.from_array(x)
     for it in range(1, 6):
         df = (-(1.0 + np.sin(3 * x.astype(np.float64)))).astype(np.float32)
         g = np.array([(w[i] * x).sum() / n - 0.4 - 0.1 * i for i in range(m)], dtype=np.float32)
         dg = (w / n).astype(np.float32)
-        dfd, dgd = torch.from_numpy(df).cuda(), torch.from_numpy(dg).cuda()
-        torch.cuda.synchronize()
-        ptrs = (ctypes.c_void_p * m)(*[dgd[i].data_ptr() for i in range(m)])
-        rc = homo3d_amd.lib().homo3d_mma_update(dev._h, it, ctypes.c_void_p(xd.data_ptr()),
-                                                ctypes.c_void_p(dfd.data_ptr()),
-                                                g.ctypes.data_as(ctypes.c_void_p), ptrs, 1)
+        dfd = homo3d_amd.DeviceBuffer.from_array(df)
+        dgd = [homo3d_amd.DeviceBuffer.from_array(v) for v in dg]
+        ptrs = (ctypes.c_void_p * m)(*[v.value for v in dgd])
+        rc = homo3d_amd.lib().homo3d_mma_update(dev._h, it, xd.ptr, dfd.ptr, g.ctypes.data_as(ctypes.c_void_p), ptrs, 1)
         assert rc == homo3d_amd.HOMO3D_OK
         xin = x.copy()
         x = host.update(it, xin, df, g, list(dg))
-        assert np.array_equal(xd.cpu().numpy(), x), it
+        assert np.array_equal(xd.download(), x), it
         sh, sd = host.state(), dev.state()
         for a, b in zip(sh[:3], sd[:3]):
             assert np.array_equal(a, b), it
