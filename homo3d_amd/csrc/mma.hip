@@ -36,6 +36,7 @@ constexpr int kMmaThreads = 256;
 constexpr int kMmaCand = 8;        // line-search steps tried per pass: steg, steg / 2, ..., steg / 128
 constexpr int kMmaCtlThreads = 1024;
 constexpr int kMmaSums = kMmaCand * (2 + kMmaMaxM);  // most quantities a pass reduces
+constexpr int kMmaNewton = 200;    // most Newton steps of one epsi
 
 enum { kPhaseNewton = 0, kPhaseSearch = 1, kPhaseResid = 2, kPhaseDone = 3 };
 
@@ -393,7 +394,7 @@ __device__ __forceinline__ void small_residual(const MmaState* __restrict__ st, 
 // After a residual that ends a Newton step or opens an epsi: what comes next.
 __device__ __forceinline__ void next_phase(MmaState* st, double residumax) {
     const double epsi = st->epsi;
-    if (residumax > 0.9 * epsi && st->ittt < 200) {
+    if (residumax > 0.9 * epsi && st->ittt < kMmaNewton) {
         st->phase = kPhaseNewton;
         return;
     }
@@ -512,7 +513,7 @@ __global__ __launch_bounds__(kMmaCtlThreads) void k_mma_solve(MmaState* st, cons
     *st = t;
 }
 
-// The step length and the start of the line search.
+// The step length and the start of the line search (subsolv_g's resinew = 2 residunorm).
 template <int M>
 __global__ __launch_bounds__(kMmaCtlThreads) void k_mma_steplen(MmaState* st, const double* __restrict__ part, int nb) {
     if (st->phase != kPhaseNewton) return;
@@ -533,6 +534,15 @@ __global__ __launch_bounds__(kMmaCtlThreads) void k_mma_steplen(MmaState* st, co
     }
     up(-1.01 * t.dz / t.z);
     up(-1.01 * t.dzet / t.zet);
+    // The line search goes on while the residual is not below the one before, starting from twice that: it is
+    // not entered from a residual that is not a number (a variable with equal bounds, an infinite gradient).
+    // The point stays, and with it all that the further steps of this epsi would compute.
+    if (!(2 * t.residunorm > t.residunorm)) {
+        t.itera += kMmaNewton - t.ittt;
+        t.ittt = kMmaNewton;
+        next_phase(st, 0.0);
+        return;
+    }
     t.steg = 1.0 / stm;
     t.itto = 0;
     t.phase = kPhaseSearch;
@@ -702,9 +712,9 @@ int mma_step(homo3d_mma* h, int itn, float* out) {
                        h->upp, h->part);
     hipLaunchKernelGGL(k_mma_begin<M>, dim3(1), dim3(kMmaCtlThreads), 0, h->stream, h->st, h->part, h->nb);
     // The state is read back behind every kRounds rounds while the next ones are already queued (they
-    // return at once when the method has ended).  8 values of epsi, at most 200 Newton steps each and 50
-    // trials a step bound the rounds.
-    const int most = 8 * (200 * (1 + 50 / kMmaCand + 1) + 1) / kRounds + 2;
+    // return at once when the method has ended).  8 values of epsi, at most kMmaNewton Newton steps each and
+    // 50 trials a step bound the rounds.
+    const int most = 8 * (kMmaNewton * (1 + 50 / kMmaCand + 1) + 1) / kRounds + 2;
     bool done = false;
     for (int k = 0; k < most && !done; k++) {
         for (int r = 0; r < kRounds; r++) launch_round<M>(h, v);
