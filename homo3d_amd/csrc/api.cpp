@@ -61,6 +61,10 @@ constexpr int kSmallLevelN = 32;
 constexpr int kSmallLevelMinN = 16;
 constexpr int kPrecondSmallSweeps = 2;
 
+// floats of a handle's small scratch (d_ftmp)
+constexpr int kTmpFloats = 4096;
+static_assert(kBoxTable * sizeof(double) <= kTmpFloats * sizeof(float), "a box filter's weight sums");
+
 }  // namespace
 
 struct homo3d_handle {
@@ -110,7 +114,7 @@ struct homo3d_handle {
     double* d_partial = nullptr;
     double* d_sc = nullptr;
     double* d_tmp = nullptr;
-    float* d_ftmp = nullptr;
+    float* d_ftmp = nullptr;    // kTmpFloats: filter weights or weight sums, block maxima
     double ke[576];
     bool density_set = false;
     std::string err;
@@ -727,7 +731,7 @@ int homo3d_create(const homo3d_config* cfg, homo3d_handle** out) {
         h->lv[0].N = (size_t)n * n * n;
         h->partial_elems = 21 * kDotBlocks;
         if (hipMalloc(&h->d_partial, sizeof(double) * h->partial_elems) || hipMalloc(&h->d_tmp, sizeof(double) * 64) ||
-            hipMalloc(&h->d_ftmp, sizeof(float) * 4096))
+            hipMalloc(&h->d_ftmp, sizeof(float) * kTmpFloats))
             return fail(HOMO3D_HIP_ERROR);
         *out = h;
         return HOMO3D_OK;
@@ -757,7 +761,7 @@ int homo3d_create(const homo3d_config* cfg, homo3d_handle** out) {
     if (hipMalloc(&h->U64, sizeof(double) * 3 * kRhs * N0) || hipMemset(h->U64, 0, sizeof(double) * 3 * kRhs * N0))
         return fail(HOMO3D_HIP_ERROR);
     if (hipMalloc(&h->d_partial, sizeof(double) * h->partial_elems) || hipMalloc(&h->d_sc, sizeof(double) * 64) ||
-        hipMalloc(&h->d_tmp, sizeof(double) * 64) || hipMalloc(&h->d_ftmp, sizeof(float) * 4096))
+        hipMalloc(&h->d_tmp, sizeof(double) * 64) || hipMalloc(&h->d_ftmp, sizeof(float) * kTmpFloats))
         return fail(HOMO3D_HIP_ERROR);
     // element matrix, macro loads and the level-1 Galerkin table
     element_matrix(cfg->youngs_modulus, cfg->poisson_ratio, h->ke);
@@ -1514,7 +1518,7 @@ int homo3d_oc_filter(homo3d_handle* h, float* sens, const float* rho, int pitch,
     if (pitch < n) return set_err(h, HOMO3D_BAD_ARG, "pitch %d < n %d", pitch, n);
     const int hw = (int)(radius + 0.5);
     const int side = 2 * hw + 1;
-    if (side * side * side > 4096) return set_err(h, HOMO3D_NO_SUPPORT, "filter radius too large");
+    if (side * side * side > kTmpFloats) return set_err(h, HOMO3D_NO_SUPPORT, "filter radius too large");
     std::vector<float> wk(side * side * side);
     double W = 0;
     std::vector<double> wd(wk.size());
@@ -1679,7 +1683,7 @@ int homo3d_density_filter(homo3d_handle* h, const float* in, float* out, int pit
     if (pitch < n) return set_err(h, HOMO3D_BAD_ARG, "pitch %d < n %d", pitch, n);
     const int hw = (int)(radius + 0.5);
     const int side = 2 * hw + 1;
-    if (side * side * side > 4096) return set_err(h, HOMO3D_NO_SUPPORT, "filter radius too large");
+    if (side * side * side > kTmpFloats) return set_err(h, HOMO3D_NO_SUPPORT, "filter radius too large");
     if (2 * hw + 1 > n && periodic) return set_err(h, HOMO3D_NO_SUPPORT, "periodic filter wider than the grid");
     std::vector<double> wd(side * side * side);
     double W = 0;

@@ -499,7 +499,7 @@ __global__ __launch_bounds__(kChains) void k_chan_mean(const float* __restrict__
     sh[1][threadIdx.x] = chains[((long)b * kMeanRow + kOut) * kChains + threadIdx.x];
     __syncthreads();
     for (int k = kChains / 2; k > 0; k >>= 1) {
-        if (threadIdx.x < k) {
+        if ((int)threadIdx.x < k) {
             sh[0][threadIdx.x] += sh[0][threadIdx.x + k];
             sh[1][threadIdx.x] += sh[1][threadIdx.x + k];
         }
@@ -550,7 +550,7 @@ __global__ __launch_bounds__(256) void k_head_loss(const float* __restrict__ P, 
     sh[threadIdx.x] = s;
     __syncthreads();
     for (int k = 128; k > 0; k >>= 1) {
-        if (threadIdx.x < k) sh[threadIdx.x] += sh[threadIdx.x + k];
+        if ((int)threadIdx.x < k) sh[threadIdx.x] += sh[threadIdx.x + k];
         __syncthreads();
     }
     if (threadIdx.x == 0) partial[blockIdx.y * gridDim.x + blockIdx.x] = sh[0];
